@@ -24,7 +24,7 @@ void flyg_ctx_s::release() {
   (void)hipSetDevice(device);
   (void)hipStreamSynchronize(stream);
   if (hflags) (void)hipHostFree(hflags);
-  if (hscal) (void)hipHostFree(hscal);
+  if (hpart) (void)hipHostFree(hpart);
   (void)hipStreamDestroy(stream);
   delete this;   // device buffers are freed by their destructors
 }
@@ -33,6 +33,7 @@ unsigned flyg_ctx_s::take_flags() {
   HIPCHK(hipMemcpyAsync(hflags, dflags.get(), sizeof(unsigned), hipMemcpyDeviceToHost, stream));
   HIPCHK(hipStreamSynchronize(stream));
   unsigned f = hflags[0];
+  hflags[1] = 0;
   if (f) HIPCHK(hipMemsetAsync(dflags.get(), 0, sizeof(unsigned), stream));
   return f;
 }
@@ -95,9 +96,8 @@ int flyg_ctx_create(int device, flyg_ctx* out) {
     noalloc_scratch_init(device);   // the allocation-free gradient's scratch address on this device
     c->dflags.reserve(16);
     HIPCHK(hipMemset(c->dflags.get(), 0, 16 * sizeof(unsigned)));
-    c->dscal.reserve(64);
     HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&c->hflags), 16 * sizeof(unsigned), hipHostMallocDefault));
-    HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&c->hscal), 64 * sizeof(double), hipHostMallocDefault));
+    HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&c->hpart), (VPART + 16) * sizeof(double), hipHostMallocDefault));
     *out = c.release();
   });
 }

@@ -22,7 +22,7 @@
 #include <map>
 #include <mutex>
 
-#include "eam_host.hpp"
+#include "vecops.hpp"
 
 namespace flyg {
 
@@ -573,12 +573,14 @@ namespace flyg {
     E.eatom.reserve(nl.n);
     launch_density<LANES>(E, shifts_of(nl.box), pair_args(E, nl, types, frozen), true, FLYG_FP64, E.posf.get());
     HIPCHK(hipGetLastError());
-    dev_sum(*E.ctx, E.eatom.get(), nl.n, E.ctx->dscal.get());
-    HIPCHK(hipMemcpyAsync(E.ctx->hscal, E.ctx->dscal.get(), sizeof(double), hipMemcpyDeviceToHost, E.ctx->stream));
-    unsigned fl = E.ctx->take_flags();
-    if (fl & ERR_SPLINE_OOB) throw Error(FLYG_SPLINE_OOB, "x is outside tabulated region of a spline");
-    if (fl & ERR_TYPE) throw Error(FLYG_INVALID_ARG, "TypeID out of range");
-    return E.ctx->hscal[0];
+    dev_sum(*E.ctx, E.eatom.get(), nl.n, E.ctx->hpart, E.ctx->hflags + 1);
+    HIPCHK(hipStreamSynchronize(E.ctx->stream));
+    if (E.ctx->hflags[1]) {
+      unsigned fl = E.ctx->take_flags();
+      if (fl & ERR_SPLINE_OOB) throw Error(FLYG_SPLINE_OOB, "x is outside tabulated region of a spline");
+      if (fl & ERR_TYPE) throw Error(FLYG_INVALID_ARG, "TypeID out of range");
+    }
+    return host_sum(E.ctx->hpart, 0, nl.n);
   }
 
   namespace {

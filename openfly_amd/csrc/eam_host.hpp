@@ -36,10 +36,8 @@ struct flyg_ctx_s {
   std::string err;
   int cus = 0;
   flyg::DBuf<unsigned> dflags;   // [0] error bits, [1..] scratch counters
-  flyg::DBuf<double> dscal;      // scalar scratch for reductions
-  flyg::DBuf<double> dpart;      // block partial sums
-  unsigned* hflags = nullptr;    // pinned mirror of small results
-  double* hscal = nullptr;
+  unsigned* hflags = nullptr;    // pinned: [0] error bits read by take_flags, [1] those a kernel left
+  double* hpart = nullptr;       // pinned: block partial sums that kernels write for the host, then scalars
 
   int refs = 1;                  // the context lives until its creator and every handle released it
 
@@ -177,6 +175,6 @@ namespace flyg {
   // Copy device per-atom inputs into the handle's staged buffers.
   void stage_atoms_device(flyg_eam_s& e, uint32_t const* types, uint8_t const* frozen, long n);
 
-  // Deterministic device reductions (vecops.hip).
-  void dev_sum(flyg_ctx_s& ctx, double const* x, long n, double* d_out);
+  // Block partial sums of x and the error flags, for the host (vecops.hip).
+  void dev_sum(flyg_ctx_s& ctx, double const* x, long n, double* part, unsigned* hflag);
 }  // namespace flyg

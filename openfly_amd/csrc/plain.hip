@@ -10,14 +10,6 @@
 
 namespace flyg {
 
-  double read_scalar(flyg_ctx_s& ctx, double const* d, int count, double* out) {
-    HIPCHK(hipMemcpyAsync(ctx.hscal, d, count * sizeof(double), hipMemcpyDeviceToHost, ctx.stream));
-    HIPCHK(hipStreamSynchronize(ctx.stream));
-    if (out)
-      for (int k = 0; k < count; ++k) out[k] = ctx.hscal[k];
-    return ctx.hscal[0];
-  }
-
   namespace {
     void copy(flyg_ctx_s& ctx, double* dst, double const* src, long n) {
       HIPCHK(hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyDeviceToDevice, ctx.stream));
@@ -36,43 +28,6 @@ namespace flyg {
                                       " (returned " + std::to_string(rc) + ")");
       }
     }
-
-    VecArgs lin(long n, double* out, double const* a, Coef ca, double const* b = nullptr, Coef cb = {},
-                double const* c = nullptr, Coef cc = {}) {
-      VecArgs v;
-      v.n = n;
-      v.out = out;
-      v.v[0] = a;
-      v.c[0] = ca;
-      v.v[1] = b;
-      v.c[1] = cb;
-      v.v[2] = c;
-      v.c[2] = cc;
-      return v;
-    }
-
-    VecArgs dots(long n, double* slots, std::initializer_list<std::pair<double const*, double const*>> xy) {
-      VecArgs v;
-      v.n = n;
-      v.slots = slots;
-      for (auto const& p : xy) {
-        v.X[v.ndot] = p.first;
-        v.Y[v.ndot] = p.second;
-        ++v.ndot;
-      }
-      return v;
-    }
-
-    // Adds dot products (null = the output vector) to a lincomb.
-    VecArgs with_dots(VecArgs v, double* slots, std::initializer_list<std::pair<double const*, double const*>> xy) {
-      v.slots = slots;
-      for (auto const& p : xy) {
-        v.X[v.ndot] = p.first;
-        v.Y[v.ndot] = p.second;
-        ++v.ndot;
-      }
-      return v;
-    }
   }  // namespace
 
   // ================================================================================================
@@ -83,10 +38,10 @@ namespace flyg {
   DevLBFGS::DevLBFGS(flyg_ctx_s* ctx, int m) : m_ctx(ctx), m_m(m), m_s(static_cast<std::size_t>(m)), m_y(static_cast<std::size_t>(m)) {
     require(m > 0 && m <= 32, "L-BFGS history length must be in [1, 32]");
     m_sc.reserve(1);
-    m_slots.reserve(8);
+    m_part.reserve(2 * VPART);
   }
 
-  double* DevLBFGS::newton_step(double const* x, double const* g, long N) {
+  double* DevLBFGS::newton_step(double const* x, double const* g, long N, double const* w, double const** sums) {
     flyg_ctx_s& ctx = *m_ctx;
     if (m_k > 0) require(N == m_N, "Call to newton_step() with a different number of atoms than the history");
     if (N != m_N) {
@@ -98,64 +53,39 @@ namespace flyg {
       m_r.p(N);
       m_N = N;
     }
-    LBScalars* sc = m_sc.get();
-    double* slots = m_slots.get();
-    int prev = m_k > 0 ? (m_k - 1) % m_m : 0;
-    if (m_k > 0) {
-      vec(ctx, lin(N, m_s[prev].get(), x, cst(1), m_px.get(), cst(-1)));
-      VecArgs a = with_dots(lin(N, m_y[prev].get(), g, cst(1), m_pg.get(), cst(-1)), slots,
-                            {{m_s[prev].get(), nullptr}, {nullptr, nullptr}});
-      a.post = POST_HIST;
-      a.pj = prev;
-      a.lb = sc;
-      vec(ctx, a);
-    }
-    copy(ctx, m_px.get(), x, N);
-    copy(ctx, m_pg.get(), g, N);
-    copy(ctx, m_q.get(), g, N);
-    int incur = m_k <= m_m ? 0 : m_k - m_m;
-    int bound = m_k <= m_m ? m_k : m_m;
+    LBScalars* lb = m_sc.get();
+    double* in = m_part.get();          // partial sums of the stage before
+    double* out = in + VPART;           // ... and of this one
     double* q = m_q.get();
     double* r = m_r.get();
-    int jprev = -1;
-    for (int i = bound - 1; i >= 0; --i) {   // loop 1: newest -> oldest
-      int j = (i + incur) % m_m;
-      VecArgs a;
-      if (jprev < 0) {
-        a = dots(N, slots, {{m_s[j].get(), q}});
-      } else {
-        a = with_dots(lin(N, q, q, cst(1), m_y[jprev].get(), dev(&sc->alpha[jprev], -1.0)), slots, {{m_s[j].get(), nullptr}});
-      }
-      a.post = POST_ALPHA;
-      a.pj = j;
-      a.lb = sc;
-      vec(ctx, a);
-      jprev = j;
+    if (m_k == 0) {
+      lb_first(ctx, N, x, g, m_px.get(), m_pg.get(), r, w, out);
+      ++m_k;
+      if (sums) *sums = out;
+      return r;
     }
-    if (bound == 0) {
-      copy(ctx, r, q, N);
-    } else {
-      vec(ctx, lin(N, q, q, cst(1), m_y[jprev].get(), dev(&sc->alpha[jprev], -1.0)));
-      int j0 = incur % m_m;
-      VecArgs a = with_dots(lin(N, r, q, dev(&sc->h0)), slots, {{m_y[j0].get(), nullptr}});
-      a.post = POST_BETA;
-      a.pj = j0;
-      a.lb = sc;
-      vec(ctx, a);
-      for (int i = 0; i < bound; ++i) {   // loop 2: oldest -> newest
-        int j = (i + incur) % m_m;
-        VecArgs b = lin(N, r, r, cst(1), m_s[j].get(), dev(&sc->coef[j]));
-        if (i + 1 < bound) {
-          int jn = (i + 1 + incur) % m_m;
-          b = with_dots(b, slots, {{m_y[jn].get(), nullptr}});
-          b.post = POST_BETA;
-          b.pj = jn;
-          b.lb = sc;
-        }
-        vec(ctx, b);
-      }
+    int const bound = m_k <= m_m ? m_k : m_m;
+    int const oldest = m_k <= m_m ? 0 : m_k - m_m;
+    auto pair = [&](int i) { return (i + oldest) % m_m; };   // i = 0 oldest .. bound - 1 newest
+    int const newest = pair(bound - 1);
+    lb_hist(ctx, N, x, g, m_px.get(), m_pg.get(), m_s[newest].get(), m_y[newest].get(), out);
+    std::swap(in, out);
+    double const* from = m_pg.get();    // q before loop 1: the gradient lb_hist kept
+    for (int i = bound - 1; i > 0; --i) {
+      int const j = pair(i);
+      lb_loop1(ctx, N, j == newest, j, lb, in, from, m_y[j].get(), m_s[pair(i - 1)].get(), q, out);
+      std::swap(in, out);
+      from = q;
+    }
+    lb_turn(ctx, N, bound == 1, pair(0), lb, in, from, m_y[pair(0)].get(), r, out);
+    std::swap(in, out);
+    for (int i = 0; i < bound; ++i) {
+      int const j = pair(i);
+      lb_loop2(ctx, N, j, lb, in, r, m_s[j].get(), i + 1 < bound ? m_y[pair(i + 1)].get() : w, out);
+      std::swap(in, out);
     }
     ++m_k;
+    if (sums) *sums = in;
     return r;
   }
 
@@ -169,10 +99,19 @@ namespace flyg {
   }
 
   namespace {
-    void check_flags(flyg_ctx_s& ctx) {
-      unsigned fl = ctx.take_flags();
+    void throw_flags(unsigned fl) {
       if (fl & ERR_SPLINE_OOB) throw Error(FLYG_SPLINE_OOB, "x is outside tabulated region of a spline");
       if (fl & ERR_TYPE) throw Error(FLYG_INVALID_ARG, "TypeID out of range");
+    }
+
+    void check_flags(flyg_ctx_s& ctx) { throw_flags(ctx.take_flags()); }
+
+    void sync(flyg_ctx_s& ctx) { HIPCHK(hipStreamSynchronize(ctx.stream)); }
+
+    // After a kernel that wrote its sums and the error flags to pinned memory.
+    void sync_checked(flyg_ctx_s& ctx) {
+      sync(ctx);
+      if (ctx.hflags[1]) check_flags(ctx);
     }
   }  // namespace
 
@@ -190,41 +129,48 @@ namespace flyg {
     if (!m.nl || m.nl->rc != rc) m.nl = make_list(&ctx, m.basis, m.periodic, rc);
     if (!m.core) m.core = std::make_unique<DevLBFGS>(&ctx, o.n);
     m.core->clear();
-    m.slots.reserve(8);
     double* x = d_pos;
     double* g = d_grad;
-    double* sl = m.slots.get();
+    double* hp = ctx.hpart;
+    double& hstep = hp[VPART];   // |q|^2 of the step under way
+    unsigned* hfl = ctx.hflags + 1;
 
     list_rebuild(*m.nl, x, n);
     eam_gradient(e, *m.nl, d_types, d_frozen, g, FLYG_FP64);
-    vec(ctx, dots(N, sl, {{g, g}}));
-    double mag_g = read_scalar(ctx, sl);
-    check_flags(ctx);
+    vec_dots(ctx, N, g, g, nullptr, nullptr, hp, hfl);
+    sync_checked(ctx);
+    double mag_g = host_sum(hp, 0, N);
     double trust = o.min_trust, acc = 0;
     for (int i = 0; i < o.iter_max; ++i) {
       if (iterations) *iterations = i;
       observe(ctx, m.obs, m.obs_user, i, x, n, m.obs_host);
       if (mag_g < o.f2norm * o.f2norm) return false;
-      double* q = m.core->newton_step(x, g, N);
-      vec(ctx, dots(N, sl, {{q, q}}));
-      double nrm = std::sqrt(read_scalar(ctx, sl));
-      double scale = std::fmin(1.0, trust / nrm);
-      vec(ctx, lin(N, q, q, cst(scale)));
-      acc += nrm * scale;
-      vec(ctx, lin(N, x, x, cst(1), q, cst(-1)));
-      if (acc > 0.5 * skin) {
-        list_rebuild(*m.nl, x, n);
-        acc = 0;
-      } else {
-        list_update(*m.nl, q, n);
+      double const* qq;
+      double* q = m.core->newton_step(x, g, N, nullptr, &qq);
+      vec_step(ctx, N, trust, qq, q, x, list_move(*m.nl), &hstep);
+      // The step is at most the trust radius long: while that cannot use up the skin, its length is read
+      // with the next sums instead of on its own.
+      bool known = false;
+      auto add_step = [&] {
+        double const nrm = std::sqrt(hstep);
+        double const scale = std::fmin(1.0, trust / nrm);
+        acc += nrm * scale;
+        known = true;
+      };
+      if (!(acc + 1.001 * trust < 0.5 * skin)) {
+        sync(ctx);
+        add_step();
+        if (acc > 0.5 * skin) {
+          list_rebuild(*m.nl, x, n);
+          acc = 0;
+        }
       }
       eam_gradient(e, *m.nl, d_types, d_frozen, g, FLYG_FP64);
-      vec(ctx, dots(N, sl, {{g, q}, {g, g}}));
-      double two[2];
-      read_scalar(ctx, sl, 2, two);
-      check_flags(ctx);
-      double proj = two[0];
-      mag_g = two[1];
+      vec_dots(ctx, N, g, q, g, g, hp, hfl);
+      sync_checked(ctx);
+      if (!known) add_step();
+      double proj = host_sum(hp, 0, N);
+      mag_g = host_sum(hp, 1, N);
       if (proj < -o.proj_tol) {
         trust = std::fmax(o.min_trust, o.shrink_trust * trust);
       } else if (proj > o.proj_tol) {
@@ -249,14 +195,18 @@ namespace flyg {
   }  // namespace
 
   // Rotor::eff_gradient on the list nl (ready at the positions; moved by +-delta_r and back, never rebuilt).
-  // Axis in/out in d.ax, effective gradient to d.eff.  Returns the curvature; leaves |g_eff|^2 in d.slots[0].
+  // Axis in/out in d.ax, effective gradient to d.eff.  Returns the curvature; |g_eff|^2 and g_eff.step (step
+  // null: only the first) are left in ctx.hpart with the error flags, for the caller to read after a sync.
   double eff_gradient(flyg_dimer_s& d, flyg_list_s& nl, flyg_eam_s& e, uint32_t const* t, uint8_t const* f, long n,
-                      int count_frozen) {
+                      int count_frozen, double const* step) {
       flyg_ctx_s& ctx = *d.ctx;
       flyg_rotor_options const& o = d.ropt;
       long N = 3 * n;
       double const dr = o.delta_r;
-      double* sl = d.slots.get();
+      d.part.reserve(2 * VPART);
+      double* in = d.part.get();
+      double* out = in + VPART;
+      double* hp = ctx.hpart;
       double* ax = d.ax.get();
       double* g0 = d.g0.get();
       double* g1 = d.g1.get();
@@ -265,96 +215,63 @@ namespace flyg {
       double* dgp = d.delta_g.get();
       double* axp = d.axisp.get();
       double* dprev = d.delta_prev.get();
-      double* u = d.u.get();
-      double const inv_n = 1.0 / static_cast<double>(n);
+      ListMove const lm = list_move(nl);
+      bool const none_frozen = count_frozen == 0;
+      double const mean_k = -(1.0 / static_cast<double>(n));
 
       d.rcore->clear();
       gradient_at(d, nl, e, t, f, g0);
-      vec(ctx, lin(N, dprev, ax, cst(-dr)));
-      list_update(nl, dprev, n);
+      rot_offset(ctx, N, dr, ax, dprev, lm);
       gradient_at(d, nl, e, t, f, g1);
+      rot_diff(ctx, N, g1, g0, ax, dg, out);
 
       double curv = 0;
       for (int i = 0;; ++i) {
-        // Torque: delta_g = (g1 - g0) - ((g1 - g0).n) n, minus its mean when nothing is frozen.
-        vec(ctx, with_dots(lin(N, dg, g1, cst(1), g0, cst(-1)), sl + 0, {{nullptr, ax}}));
-        VecArgs a = lin(N, dgp, dg, cst(1), ax, dev(sl + 0, -1.0));
-        if (count_frozen == 0) {
-          a.comp_sums = 1;
-          a.slots = sl + 4;
-        }
-        vec(ctx, a);
-        if (count_frozen == 0) {
-          VecArgs b = lin(N, dgp, nullptr, cst(0));
-          b.mean3 = sl + 4;
-          b.mean_k = -inv_n;
-          vec(ctx, b);
-        }
-        double* theta = d.rcore->newton_step(ax, dgp, N);
-        vec(ctx, dots(N, sl + 0, {{theta, ax}}));
-        vec(ctx, with_dots(lin(N, theta, theta, cst(1), ax, dev(sl + 0, -1.0)), sl + 1, {{nullptr, nullptr}}));
-        vec(ctx, with_dots(lin(N, theta, theta, dev_rsqrt(sl + 1)), sl + 2, {{dg, nullptr}, {dg, ax}}));
-        double bc[2];
-        read_scalar(ctx, sl + 2, 2, bc);
-        double b_1 = bc[0] / dr;
-        double c_x0 = bc[1] / dr;
+        // Torque: delta_g = (g1 - g0) - ((g1 - g0).n) n, minus its mean when nothing is frozen; `out` holds
+        // the sum (g1 - g0).n.
+        std::swap(in, out);
+        rot_torque(ctx, N, none_frozen, in, dg, ax, dgp, out);
+        if (none_frozen) vec_demean(ctx, N, mean_k, out, dgp, nullptr, nullptr, nullptr);
+        double const* thax;
+        double* theta = d.rcore->newton_step(ax, dgp, N, ax, &thax);
+        rot_orth(ctx, N, thax, ax, theta, out);
+        rot_unit(ctx, N, out, theta, dg, ax, hp);
+        sync(ctx);
+        double b_1 = host_sum(hp, 0, N) / dr;
+        double c_x0 = host_sum(hp, 1, N) / dr;
         double theta_1 = -0.5 * std::atan(b_1 / std::abs(c_x0));
         if (std::abs(theta_1) < o.theta_tol || (i >= o.iter_max_rot && c_x0 < 0) || i > 10 * o.iter_max_rot) {
           curv = c_x0;
           break;
         }
         // Trial rotation; the list moves from the previous end to the trial end.
-        vec(ctx, lin(N, axp, ax, cst(std::cos(theta_1)), theta, cst(std::sin(theta_1))));
-        vec(ctx, lin(N, u, axp, cst(-dr), dprev, cst(-1)));
-        vec(ctx, lin(N, dprev, axp, cst(-dr)));
-        list_update(nl, u, n);
+        rot_trial(ctx, N, std::cos(theta_1), std::sin(theta_1), dr, ax, theta, axp, dprev, lm);
         gradient_at(d, nl, e, t, f, g1p);
-        vec(ctx, with_dots(lin(N, u, g1p, cst(1), g0, cst(-1)), sl + 0, {{nullptr, axp}}));
-        double c_x1 = read_scalar(ctx, sl + 0) / dr;
+        rot_curv(ctx, N, g1p, g0, axp, hp);
+        sync(ctx);
+        double c_x1 = host_sum(hp, 0, N) / dr;
         double a_1 = (c_x0 - c_x1 + b_1 * std::sin(2 * theta_1)) / (1 - std::cos(2 * theta_1));
         double theta_min = 0.5 * std::atan(b_1 / a_1);
         if (a_1 * std::cos(2 * theta_min) - a_1 + b_1 * std::sin(2 * theta_min) > 0) theta_min += M_PI / 2;
-        vec(ctx, lin(N, ax, ax, cst(std::cos(theta_min)), theta, cst(std::sin(theta_min))));
         double w1 = std::sin(theta_1 - theta_min) / std::sin(theta_1);
         double w2 = std::sin(theta_min) / std::sin(theta_1);
         double w3 = 1 - std::cos(theta_min) - std::sin(theta_min) * std::tan(0.5 * theta_1);
-        vec(ctx, lin(N, g1, g1, cst(w1), g1p, cst(w2), g0, cst(w3)));
-        if (std::abs(theta_min) < o.theta_tol) {
-          vec(ctx, with_dots(lin(N, dg, g1, cst(1), g0, cst(-1)), sl + 0, {{nullptr, ax}}));
-          curv = read_scalar(ctx, sl + 0) / dr;
+        bool const last = std::abs(theta_min) < o.theta_tol;
+        rot_accept(ctx, N, std::cos(theta_min), std::sin(theta_min), w1, w2, w3, ax, theta, g1, g1p, g0, dg,
+                   last ? hp : out);
+        if (last) {
+          sync(ctx);
+          curv = host_sum(hp, 0, N) / dr;
           break;
         }
       }
       // Move the list back to the centre.
-      vec(ctx, lin(N, u, dprev, cst(-1)));
-      list_update(nl, u, n);
-
-      vec(ctx, dots(N, sl + 0, {{g0, ax}}));
-      double k = (!o.relax_in_convex && curv > 0) ? -1.0 : -2.0;
-      double* eff = d.eff.get();
-      if (!o.relax_in_convex && curv > 0) {
-        VecArgs a = lin(N, eff, ax, dev(sl + 0, k));
-        if (count_frozen == 0) {
-          a.comp_sums = 1;
-          a.slots = sl + 4;
-        }
-        vec(ctx, a);
-      } else {
-        VecArgs a = lin(N, eff, g0, cst(1), ax, dev(sl + 0, k));
-        if (count_frozen == 0) {
-          a.comp_sums = 1;
-          a.slots = sl + 4;
-        }
-        vec(ctx, a);
-      }
-      if (count_frozen == 0) {
-        VecArgs b = lin(N, eff, nullptr, cst(0));
-        b.mean3 = sl + 4;
-        b.mean_k = -inv_n;
-        vec(ctx, with_dots(b, sl + 0, {{nullptr, nullptr}}));
-      } else {
-        vec(ctx, dots(N, sl + 0, {{eff, eff}}));
-      }
+      rot_back(ctx, N, dprev, g0, ax, lm, in);
+      bool const flat = !o.relax_in_convex && curv > 0;
+      unsigned* hfl = ctx.hflags + 1;
+      rot_eff(ctx, N, none_frozen, !flat, flat ? -1.0 : -2.0, in, g0, ax, d.eff.get(), step, none_frozen ? out : hp,
+              none_frozen ? nullptr : hfl);
+      if (none_frozen) vec_demean(ctx, N, mean_k, out, d.eff.get(), step, hp, hfl);
       return curv;
     }
 
@@ -366,10 +283,9 @@ namespace flyg {
     require(nl.rc >= e.tab.rc + 2 * d.ropt.delta_r, "the list's cut-off is below the rotor's r_cut()");
     long N = 3 * n;
     if (!d.rcore) d.rcore = std::make_unique<DevLBFGS>(&ctx, d.ropt.n);
-    d.slots.reserve(16);
-    for (DVec* v : {&d.ax, &d.eff, &d.g0, &d.g1, &d.g1p, &d.dg, &d.delta_g, &d.axisp, &d.delta_prev, &d.u}) v->p(N);
+    for (DVec* v : {&d.ax, &d.eff, &d.g0, &d.g1, &d.g1p, &d.dg, &d.delta_g, &d.axisp, &d.delta_prev}) v->p(N);
     copy(ctx, d.ax.get(), d_axis, N);
-    double curv = eff_gradient(d, nl, e, t, f, n, count_frozen);
+    double curv = eff_gradient(d, nl, e, t, f, n, count_frozen, nullptr);
     copy(ctx, d_axis, d.ax.get(), N);
     copy(ctx, d_eff, d.eff.get(), N);
     check_flags(ctx);
@@ -389,10 +305,10 @@ namespace flyg {
     if (!d.core) d.core = std::make_unique<DevLBFGS>(&ctx, o.n);
     if (!d.rcore) d.rcore = std::make_unique<DevLBFGS>(&ctx, d.ropt.n);
     d.core->clear();
-    d.slots.reserve(16);
-    for (DVec* v : {&d.x, &d.ax, &d.eff, &d.g0, &d.g1, &d.g1p, &d.dg, &d.delta_g, &d.axisp, &d.delta_prev, &d.u, &d.tmp})
+    for (DVec* v : {&d.x, &d.ax, &d.eff, &d.g0, &d.g1, &d.g1p, &d.dg, &d.delta_g, &d.axisp, &d.delta_prev, &d.tmp})
       v->p(N);
-    double* sl = d.slots.get();
+    double* hp = ctx.hpart;
+    double& hstep = hp[VPART];   // |q|^2 of the step under way
     double* x = d.x.get();
     copy(ctx, x, d_pos, N);
     copy(ctx, d.ax.get(), d_axis, N);
@@ -403,16 +319,17 @@ namespace flyg {
     if (o.use_history && n_hist > 0) {
       if (static_cast<int>(d.hist_d.size()) < n_hist) d.hist_d.resize(static_cast<std::size_t>(n_hist));
       for (int k = 0; k < n_hist; ++k) {
-        vec(ctx, with_dots(lin(N, d.hist_d[k].p(N), d_hist + N * k, cst(1), d_in_min, cst(-1)), sl, {{nullptr, nullptr}}));
-        sn[k] = std::sqrt(read_scalar(ctx, sl));
+        vec_diff(ctx, N, d_hist + N * k, d_in_min, d.hist_d[k].p(N), hp);
+        sync(ctx);
+        sn[k] = std::sqrt(host_sum(hp, 0, N));
       }
     }
 
     int rebuilds = 0;
     list_rebuild(*d.nl, x, n);
-    double curv = eff_gradient(d, *d.nl, e, t, f, n, count_frozen);
-    double mag_g = read_scalar(ctx, sl);
-    check_flags(ctx);
+    double curv = eff_gradient(d, *d.nl, e, t, f, n, count_frozen, nullptr);
+    sync_checked(ctx);
+    double mag_g = host_sum(hp, 0, N);
     double trust = o.min_trust, acc = 0, convex_count = 0;
     int ret = FLYG_EXIT_ITER_MAX, steps = o.max_steps;
     for (int i = 0; i < o.max_steps; ++i) {
@@ -428,13 +345,15 @@ namespace flyg {
       }
       if (o.use_history && n_hist > 0 && i % o.hist_check_freq == 0) {
         double* dx = d.tmp.get();
-        vec(ctx, with_dots(lin(N, dx, x, cst(1), d_in_min, cst(-1)), sl, {{nullptr, nullptr}}));
-        double on = std::sqrt(read_scalar(ctx, sl));
+        vec_diff(ctx, N, x, d_in_min, dx, hp);
+        sync(ctx);
+        double on = std::sqrt(host_sum(hp, 0, N));
         double ctheta = -1;
         bool hit = false;
         for (int k = 0; k < n_hist && !hit; ++k) {
-          vec(ctx, dots(N, sl, {{dx, d.hist_d[k].get()}}));
-          double dt = read_scalar(ctx, sl);
+          vec_dots(ctx, N, dx, d.hist_d[k].get(), nullptr, nullptr, hp, nullptr);
+          sync(ctx);
+          double dt = host_sum(hp, 0, N);
           ctheta = std::fmax(ctheta, dt / (sn[k] * on));
           if (ctheta > std::cos(theta_tol)) hit = true;
         }
@@ -444,28 +363,32 @@ namespace flyg {
           break;
         }
       }
-      double* q = d.core->newton_step(x, d.eff.get(), N);
-      vec(ctx, dots(N, sl, {{q, q}}));
-      double nrm = std::sqrt(read_scalar(ctx, sl));
-      double scale = std::fmin(1.0, trust / nrm);
-      vec(ctx, lin(N, q, q, cst(scale)));
-      acc += nrm * scale;
-      vec(ctx, lin(N, x, x, cst(1), q, cst(-1)));
-      if (acc > 0.5 * skin) {
-        list_rebuild(*d.nl, x, n);
-        acc = 0;
-        ++rebuilds;
-      } else {
-        list_update(*d.nl, q, n);
+      double const* qq;
+      double* q = d.core->newton_step(x, d.eff.get(), N, nullptr, &qq);
+      vec_step(ctx, N, trust, qq, q, x, list_move(*d.nl), &hstep);
+      // As in the minimiser: the step's length is read on its own only when it could use up the skin.
+      bool known = false;
+      auto add_step = [&] {
+        double const nrm = std::sqrt(hstep);
+        double const scale = std::fmin(1.0, trust / nrm);
+        acc += nrm * scale;
+        known = true;
+      };
+      if (!(acc + 1.001 * trust < 0.5 * skin)) {
+        sync(ctx);
+        add_step();
+        if (acc > 0.5 * skin) {
+          list_rebuild(*d.nl, x, n);
+          acc = 0;
+          ++rebuilds;
+        }
       }
-      curv = eff_gradient(d, *d.nl, e, t, f, n, count_frozen);
+      curv = eff_gradient(d, *d.nl, e, t, f, n, count_frozen, q);
       convex_count = curv > 0 ? convex_count + 1 : 0;
-      vec(ctx, dots(N, sl + 8, {{d.eff.get(), q}}));
-      double two[2];
-      read_scalar(ctx, sl, 1, two);
-      mag_g = two[0];
-      double proj = read_scalar(ctx, sl + 8);
-      check_flags(ctx);
+      sync_checked(ctx);
+      if (!known) add_step();
+      mag_g = host_sum(hp, 0, N);
+      double proj = host_sum(hp, 1, N);
       if (proj < -o.proj_tol) {
         trust = std::fmax(o.min_trust, o.shrink_trust * trust);
       } else if (proj > o.proj_tol) {

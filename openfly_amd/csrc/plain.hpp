@@ -1,5 +1,5 @@
 // Plain form of the minimiser and dimer: the reference's control flow on the host, every 3N vector
-// resident on the device, vector algebra in fused kernels with device-side scalars (vecops.hpp).
+// resident on the device, vector algebra in fused kernels (vecops.hpp).
 #pragma once
 
 #include <memory>
@@ -22,8 +22,10 @@ namespace flyg {
   public:
     DevLBFGS(flyg_ctx_s* ctx, int m);
     void clear() { m_k = 0; }
-    // Returns q ~ H^-1 g (device, length N); x and g are device vectors of length N.
-    double* newton_step(double const* x, double const* g, long N);
+    // Returns r ~ H^-1 g (device, length N); x and g are device vectors of length N.  `sums` (if given):
+    // device partial sums of r.w (w null: r.r), valid until the next call.
+    double* newton_step(double const* x, double const* g, long N, double const* w = nullptr,
+                        double const** sums = nullptr);
 
   private:
     flyg_ctx_s* m_ctx;
@@ -33,11 +35,8 @@ namespace flyg {
     std::vector<DVec> m_s, m_y;
     DVec m_px, m_pg, m_q, m_r;
     DBuf<LBScalars> m_sc;
-    DBuf<double> m_slots;
+    DBuf<double> m_part;   // two sets of partial sums, used in turn
   };
-
-  // Host-side copy of a small scalar result (synchronises the stream).
-  double read_scalar(flyg_ctx_s& ctx, double const* d, int count = 1, double* out = nullptr);
 
 }  // namespace flyg
 
@@ -55,8 +54,7 @@ struct flyg_lbfgs_s {
   int periodic[3];
   std::unique_ptr<flyg_list_s> nl;
   std::unique_ptr<flyg::DevLBFGS> core;
-  flyg::DVec x, g, tmp;
-  flyg::DBuf<double> slots;
+  flyg::DVec x, g;
   flyg_step_observer obs = nullptr;   // per-iteration positions to the caller (Options::fout)
   void* obs_user = nullptr;
   std::vector<double> obs_host;
@@ -71,9 +69,9 @@ struct flyg_dimer_s {
   std::unique_ptr<flyg_list_s> nl;
   std::unique_ptr<flyg::DevLBFGS> core;    // translation, m = opt.n
   std::unique_ptr<flyg::DevLBFGS> rcore;   // rotation, m = ropt.n
-  flyg::DVec x, ax, eff, g0, g1, g1p, dg, delta_g, axisp, delta_prev, u, tmp, inmin;
+  flyg::DVec x, ax, eff, g0, g1, g1p, dg, delta_g, axisp, delta_prev, tmp;
   std::vector<flyg::DVec> hist_d;   // sp_k - in_min
-  flyg::DBuf<double> slots;
+  flyg::DBuf<double> part;   // two sets of partial sums, used in turn
   long grads = 0;
   flyg_step_observer obs = nullptr;
   void* obs_user = nullptr;

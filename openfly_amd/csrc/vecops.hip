@@ -1,4 +1,4 @@
-// Fused vector kernel and deterministic reductions (see vecops.hpp).
+// Vector kernels of the plain form and deterministic reductions (see vecops.hpp).
 #include <cmath>
 
 #include "vecops.hpp"
@@ -7,122 +7,573 @@ namespace flyg {
 
   namespace {
 
-    constexpr int VT = 256;        // threads per block
-    constexpr int VMAXB = 240;     // blocks (fixed per length -> reproducible sums)
+    constexpr int VT = 256;   // threads per block
 
-    __device__ inline double coef_val(Coef const& c) {
-      if (!c.s) return c.k;
-      double s = *c.s;
-      return c.k * (c.inv_sqrt ? 1.0 / sqrt(s) : s);
+    // Sum k of the partial sums the kernel before left, in block order, by every thread for itself.
+    // `sh` holds K * VMAXB doubles; starts and ends with no barrier owed to the caller.
+    template <int K>
+    __device__ inline void collect(double const* __restrict__ part, double* sh, double (&tot)[K]) {
+      int const nb = static_cast<int>(gridDim.x);
+      for (int q = threadIdx.x; q < nb; q += VT)
+#pragma unroll
+        for (int k = 0; k < K; ++k) sh[k * VMAXB + q] = part[k * VMAXB + q];
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < K; ++k) tot[k] = 0.0;
+#pragma unroll 8
+      for (int b = 0; b < nb; ++b)
+#pragma unroll
+        for (int k = 0; k < K; ++k) tot[k] += sh[k * VMAXB + b];
     }
 
-    // Partials live in part[block * 4 + k]; `counter` elects the finalising block.
-    __global__ __launch_bounds__(VT) void k_vec(VecArgs a, double* __restrict__ part, unsigned* __restrict__ counter) {
-      __shared__ double sh[VT / 64];
-      __shared__ bool last;
-      double c0 = a.v[0] ? coef_val(a.c[0]) : 0.0;
-      double c1 = a.v[1] ? coef_val(a.c[1]) : 0.0;
-      double c2 = a.v[2] ? coef_val(a.c[2]) : 0.0;
-      double m3[3] = {0, 0, 0};
-      if (a.mean3)
-        for (int k = 0; k < 3; ++k) m3[k] = a.mean_k * a.mean3[k];
-      bool write = a.out && (a.v[0] || a.mean3);
-      double acc[4] = {0, 0, 0, 0};
-      long stride = static_cast<long>(gridDim.x) * VT;
-      for (long i = blockIdx.x * static_cast<long>(VT) + threadIdx.x; i < a.n; i += stride) {
-        double o = 0;
-        if (write) {
-          o = 0;
-          if (a.v[0]) o = c0 * a.v[0][i];
-          if (a.v[1]) o += c1 * a.v[1][i];
-          if (a.v[2]) o += c2 * a.v[2][i];
-          if (!a.v[0]) o = a.out[i];
-          if (a.mean3) o += m3[i % 3];
-          a.out[i] = o;
-        } else if (a.out) {
-          o = a.out[i];
-        }
-        if (a.comp_sums) {
-          acc[i % 3] += o;
-        } else {
-          for (int k = 0; k < a.ndot; ++k) {
-            double x = a.X[k] ? a.X[k][i] : o;
-            double y = a.Y[k] ? a.Y[k][i] : o;
-            acc[k] += x * y;
-          }
-        }
-      }
-      int nacc = a.comp_sums ? 3 : a.ndot;
-      if (nacc == 0) return;
-      for (int k = 0; k < nacc; ++k) {
-        double s = block_sum<VT>(acc[k], sh);
-        if (threadIdx.x == 0) __hip_atomic_store(&part[blockIdx.x * 4 + k], s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-      __threadfence();
-      if (threadIdx.x == 0) {
-        unsigned t = atomicAdd(counter, 1u);
-        last = (t == gridDim.x - 1);
+    // Block sums of acc[0..K) to part[k * VMAXB + block]: the wavefronts' xor trees, then the wavefronts in
+    // order.
+    template <int K>
+    __device__ inline void leave(double const (&acc)[K], double* __restrict__ part) {
+      __shared__ double sw[K][VT / 64];
+      int const w = threadIdx.x >> 6;
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        double const v = group_sum<64>(acc[k]);
+        if ((threadIdx.x & 63) == 0) sw[k][w] = v;
       }
       __syncthreads();
-      if (!last || threadIdx.x != 0) return;
-      __threadfence();
-      double tot[4] = {0, 0, 0, 0};
-      for (unsigned b = 0; b < gridDim.x; ++b)
-        for (int k = 0; k < nacc; ++k) tot[k] += __hip_atomic_load(&part[b * 4 + k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      *counter = 0u;
-      for (int k = 0; k < nacc; ++k) a.slots[k] = tot[k];
-      if (a.post == POST_HIST) {
-        a.lb->rho[a.pj] = 1.0 / fabs(tot[0]);
-        a.lb->h0 = (1.0 / a.lb->rho[a.pj]) / tot[1];
-      } else if (a.post == POST_ALPHA) {
-        a.lb->alpha[a.pj] = a.lb->rho[a.pj] * tot[0];
-      } else if (a.post == POST_BETA) {
-        a.lb->coef[a.pj] = a.lb->alpha[a.pj] - a.lb->rho[a.pj] * tot[0];
+      if (threadIdx.x < K) {
+        double s = 0;
+        for (int q = 0; q < VT / 64; ++q) s += sw[threadIdx.x][q];
+        part[threadIdx.x * VMAXB + blockIdx.x] = s;
       }
     }
 
-    __global__ __launch_bounds__(VT) void k_sum(double const* __restrict__ x, long n, double* __restrict__ part,
-                                               unsigned* __restrict__ counter, double* __restrict__ out) {
-      __shared__ double sh[VT / 64];
-      __shared__ bool last;
-      double acc = 0;
-      long stride = static_cast<long>(gridDim.x) * VT;
-      for (long i = blockIdx.x * static_cast<long>(VT) + threadIdx.x; i < n; i += stride) acc += x[i];
-      double s = block_sum<VT>(acc, sh);
-      if (threadIdx.x == 0) __hip_atomic_store(&part[blockIdx.x * 4], s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __threadfence();
-      if (threadIdx.x == 0) {
-        unsigned t = atomicAdd(counter, 1u);
-        last = (t == gridDim.x - 1);
+    // Element i of thread t of block b: i = b VT + t, then every gridDim VT further, in increasing order;
+    // the loads of four elements are issued before the first of them is worked on (one after the other
+    // they cost a memory round trip each).
+    template <typename Load, typename Body>
+    __device__ inline void vec_loop(long n, Load&& load, Body&& body) {
+      long const step = static_cast<long>(gridDim.x) * VT;
+      for (long i = blockIdx.x * static_cast<long>(VT) + threadIdx.x; i < n; i += 4 * step) {
+        decltype(load(i)) v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (i + u * step < n) v[u] = load(i + u * step);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (i + u * step < n) body(i + u * step, v[u]);
       }
-      __syncthreads();
-      if (!last || threadIdx.x != 0) return;
-      __threadfence();
-      double tot = 0;
-      for (unsigned b = 0; b < gridDim.x; ++b) tot += __hip_atomic_load(&part[b * 4], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      *counter = 0u;
-      *out = tot;
     }
 
-    unsigned blocks_for(long n) {
-      long b = (n + VT * 4 - 1) / (VT * 4);
-      if (b < 1) b = 1;
-      if (b > VMAXB) b = VMAXB;
-      return static_cast<unsigned>(b);
+    struct V1 { double a; };
+    struct V2 { double a, b; };
+    struct V3 { double a, b, c; };
+    struct V4 { double a, b, c, d; };
+    struct V5 { double a, b, c, d, e; };
+
+    // List::update's p -= u for one component: where it lies, and what is there.
+    struct Moved {
+      double p;
+      long at, gat;
+    };
+    __device__ inline Moved to_move(ListMove const& lm, long i) {
+      unsigned const a = static_cast<unsigned>(i) / 3u, c = static_cast<unsigned>(i) - 3u * a;
+      Moved m;
+      m.at = 4l * a + c;
+      m.gat = 4l * lm.rank[a] + c;
+      m.p = lm.pos[m.at];
+      return m;
+    }
+    __device__ inline void move_one(ListMove const& lm, Moved const& m, double u) {
+      double const p = m.p - u;
+      lm.pos[m.at] = p;
+      lm.gpos[m.gat] = p;
+    }
+    struct M1 { double a; Moved m; };
+    struct M2 { double a, b; Moved m; };
+    struct M3 { double a, b, c; Moved m; };
+
+    // acc[i mod 3] += v without indexing registers.
+    __device__ inline void add_comp(double (&acc)[3], long i, double v) {
+      unsigned const c = static_cast<unsigned>(i) % 3u;
+#pragma unroll
+      for (unsigned k = 0; k < 3; ++k)
+        if (k == c) acc[k] += v;
+    }
+
+    __global__ __launch_bounds__(VT) void k_lb_first(long n, double const* __restrict__ x, double const* __restrict__ g,
+                                                     double* __restrict__ px, double* __restrict__ pg,
+                                                     double* __restrict__ r, double const* __restrict__ w,
+                                                     double* __restrict__ out) {
+      double acc[1] = {0};
+      vec_loop(
+          n, [&](long i) { return V3{x[i], g[i], w ? w[i] : g[i]}; },
+          [&](long i, V3 const& v) {
+            px[i] = v.a;
+            pg[i] = v.b;
+            r[i] = v.b;
+            acc[0] += v.b * v.c;
+          });
+      leave(acc, out);
+    }
+
+    __global__ __launch_bounds__(VT) void k_lb_hist(long n, double const* __restrict__ x, double const* __restrict__ g,
+                                                    double* __restrict__ px, double* __restrict__ pg,
+                                                    double* __restrict__ s, double* __restrict__ y,
+                                                    double* __restrict__ out) {
+      double acc[3] = {0, 0, 0};
+      vec_loop(
+          n, [&](long i) { return V4{x[i], g[i], px[i], pg[i]}; },
+          [&](long i, V4 const& v) {
+            double const si = v.a - v.c, yi = v.b - v.d;
+            s[i] = si;
+            y[i] = yi;
+            px[i] = v.a;
+            pg[i] = v.b;
+            acc[0] += si * yi;
+            acc[1] += yi * yi;
+            acc[2] += si * v.b;
+          });
+      leave(acc, out);
+    }
+
+    // alpha_j of loop 1 from the stage before; the newest pair's rho and h0 come from lb_hist's sums.
+    template <bool NEWEST>
+    __device__ inline double alpha_of(double const* __restrict__ in, double* sh, LBScalars* __restrict__ lb, int j,
+                                      double& h0) {
+      double alpha;
+      if constexpr (NEWEST) {
+        double t[3];
+        collect(in, sh, t);
+        double const rho = 1.0 / fabs(t[0]);
+        h0 = (1.0 / rho) / t[1];
+        alpha = rho * t[2];
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+          lb->rho[j] = rho;
+          lb->h0 = h0;
+        }
+      } else {
+        double t[1];
+        collect(in, sh, t);
+        alpha = lb->rho[j] * t[0];
+        h0 = lb->h0;
+      }
+      if (blockIdx.x == 0 && threadIdx.x == 0) lb->alpha[j] = alpha;
+      return alpha;
+    }
+
+    template <bool NEWEST>
+    __global__ __launch_bounds__(VT) void k_lb_loop1(long n, int j, LBScalars* __restrict__ lb, double const* __restrict__ in,
+                                                     double const* q, double const* __restrict__ y,
+                                                     double const* __restrict__ s_next, double* qout,
+                                                     double* __restrict__ out) {
+      __shared__ double sh[3 * VMAXB];
+      double h0;
+      double const c = -1.0 * alpha_of<NEWEST>(in, sh, lb, j, h0);
+      double acc[1] = {0};
+      vec_loop(
+          n, [&](long i) { return V3{q[i], y[i], s_next[i]}; },
+          [&](long i, V3 const& v) {
+            double o = v.a;
+            o += c * v.b;
+            qout[i] = o;
+            acc[0] += v.c * o;
+          });
+      leave(acc, out);
+    }
+
+    template <bool NEWEST>
+    __global__ __launch_bounds__(VT) void k_lb_turn(long n, int j, LBScalars* __restrict__ lb, double const* __restrict__ in,
+                                                    double const* __restrict__ q, double const* __restrict__ y,
+                                                    double* __restrict__ r, double* __restrict__ out) {
+      __shared__ double sh[3 * VMAXB];
+      double h0;
+      double const c = -1.0 * alpha_of<NEWEST>(in, sh, lb, j, h0);
+      double acc[1] = {0};
+      vec_loop(
+          n, [&](long i) { return V2{q[i], y[i]}; },
+          [&](long i, V2 const& v) {
+            double o = v.a;
+            o += c * v.b;
+            double const ri = h0 * o;
+            r[i] = ri;
+            acc[0] += v.b * ri;
+          });
+      leave(acc, out);
+    }
+
+    __global__ __launch_bounds__(VT) void k_lb_loop2(long n, int j, LBScalars const* __restrict__ lb,
+                                                     double const* __restrict__ in, double* __restrict__ r,
+                                                     double const* __restrict__ s, double const* __restrict__ w,
+                                                     double* __restrict__ out) {
+      __shared__ double sh[VMAXB];
+      double t[1];
+      collect(in, sh, t);
+      double const c = lb->alpha[j] - lb->rho[j] * t[0];
+      double acc[1] = {0};
+      vec_loop(
+          n, [&](long i) { return V3{r[i], s[i], w ? w[i] : 0.0}; },
+          [&](long i, V3 const& v) {
+            double o = v.a;
+            o += c * v.b;
+            r[i] = o;
+            acc[0] += o * (w ? v.c : o);
+          });
+      leave(acc, out);
+    }
+
+    __global__ __launch_bounds__(VT) void k_step(long n, double trust, double const* __restrict__ in, double* __restrict__ q,
+                                                 double* __restrict__ x, ListMove lm, double* __restrict__ hsum) {
+      __shared__ double sh[VMAXB];
+      double t[1];
+      collect(in, sh, t);
+      if (blockIdx.x == 0 && threadIdx.x == 0) *hsum = t[0];
+      double const c = fmin(1.0, trust / sqrt(t[0]));
+      vec_loop(
+          n, [&](long i) { return M2{q[i], x[i], to_move(lm, i)}; },
+          [&](long i, M2 const& v) {
+            double const o = c * v.a;
+            q[i] = o;
+            x[i] = v.b - o;
+            move_one(lm, v.m, o);
+          });
+    }
+
+    __global__ __launch_bounds__(VT) void k_dots(long n, double const* __restrict__ a, double const* __restrict__ b,
+                                                 double const* __restrict__ c, double const* __restrict__ d,
+                                                 double* __restrict__ out, unsigned const* __restrict__ flags,
+                                                 unsigned* __restrict__ hflag) {
+      double acc[2] = {0, 0};
+      vec_loop(
+          n, [&](long i) { return V4{a[i], b[i], c ? c[i] : 0.0, c ? d[i] : 0.0}; },
+          [&](long, V4 const& v) {
+            acc[0] += v.a * v.b;
+            acc[1] += v.c * v.d;
+          });
+      leave(acc, out);
+      if (hflag && blockIdx.x == 0 && threadIdx.x == 0) *hflag = *flags;
+    }
+
+    __global__ __launch_bounds__(VT) void k_diff(long n, double const* __restrict__ a, double const* __restrict__ b,
+                                                 double* __restrict__ o, double* __restrict__ out) {
+      double acc[1] = {0};
+      vec_loop(
+          n, [&](long i) { return V2{a[i], b[i]}; },
+          [&](long i, V2 const& w) {
+            double const v = w.a - w.b;
+            o[i] = v;
+            acc[0] += v * v;
+          });
+      leave(acc, out);
+    }
+
+    __global__ __launch_bounds__(VT) void k_rot_offset(long n, double dr, double const* __restrict__ ax,
+                                                       double* __restrict__ delta, ListMove lm) {
+      vec_loop(
+          n, [&](long i) { return M1{ax[i], to_move(lm, i)}; },
+          [&](long i, M1 const& v) {
+            double const o = -dr * v.a;
+            delta[i] = o;
+            move_one(lm, v.m, o);
+          });
+    }
+
+    __global__ __launch_bounds__(VT) void k_rot_diff(long n, double const* __restrict__ g1, double const* __restrict__ g0,
+                                                     double const* __restrict__ ax, double* __restrict__ dg,
+                                                     double* __restrict__ out) {
+      double acc[1] = {0};
+      vec_loop(
+          n, [&](long i) { return V3{g1[i], g0[i], ax[i]}; },
+          [&](long i, V3 const& v) {
+            double const o = v.a - v.b;
+            dg[i] = o;
+            acc[0] += o * v.c;
+          });
+      leave(acc, out);
+    }
+
+    template <bool SUMS>
+    __global__ __launch_bounds__(VT) void k_rot_torque(long n, double const* __restrict__ in, double const* __restrict__ dg,
+                                                       double const* __restrict__ ax, double* __restrict__ o,
+                                                       double* __restrict__ out) {
+      __shared__ double sh[VMAXB];
+      double t[1];
+      collect(in, sh, t);
+      double const c = -1.0 * t[0];
+      double acc[3] = {0, 0, 0};
+      vec_loop(
+          n, [&](long i) { return V2{dg[i], ax[i]}; },
+          [&](long i, V2 const& w) {
+            double v = w.a;
+            v += c * w.b;
+            o[i] = v;
+            if (SUMS) add_comp(acc, i, v);
+          });
+      if (SUMS) leave(acc, out);
+    }
+
+    __global__ __launch_bounds__(VT) void k_demean(long n, double mean_k, double const* __restrict__ in,
+                                                   double* __restrict__ o, double const* __restrict__ w,
+                                                   double* __restrict__ out, unsigned const* __restrict__ flags,
+                                                   unsigned* __restrict__ hflag) {
+      __shared__ double sh[3 * VMAXB];
+      double t[3];
+      collect(in, sh, t);
+      double const m0 = mean_k * t[0], m1 = mean_k * t[1], m2 = mean_k * t[2];
+      double acc[2] = {0, 0};
+      vec_loop(
+          n, [&](long i) { return V2{o[i], w ? w[i] : 0.0}; },
+          [&](long i, V2 const& e) {
+            unsigned const c = static_cast<unsigned>(i) % 3u;
+            double const v = e.a + (c == 0 ? m0 : (c == 1 ? m1 : m2));
+            o[i] = v;
+            acc[0] += v * v;
+            acc[1] += v * e.b;
+          });
+      if (out) leave(acc, out);
+      if (hflag && blockIdx.x == 0 && threadIdx.x == 0) *hflag = *flags;
+    }
+
+    __global__ __launch_bounds__(VT) void k_rot_orth(long n, double const* __restrict__ in, double const* __restrict__ ax,
+                                                     double* __restrict__ theta, double* __restrict__ out) {
+      __shared__ double sh[VMAXB];
+      double t[1];
+      collect(in, sh, t);
+      double const c = -1.0 * t[0];
+      double acc[1] = {0};
+      vec_loop(
+          n, [&](long i) { return V2{theta[i], ax[i]}; },
+          [&](long i, V2 const& v) {
+            double o = v.a;
+            o += c * v.b;
+            theta[i] = o;
+            acc[0] += o * o;
+          });
+      leave(acc, out);
+    }
+
+    __global__ __launch_bounds__(VT) void k_rot_unit(long n, double const* __restrict__ in, double* __restrict__ theta,
+                                                     double const* __restrict__ dg, double const* __restrict__ ax,
+                                                     double* __restrict__ out) {
+      __shared__ double sh[VMAXB];
+      double t[1];
+      collect(in, sh, t);
+      double const c = 1.0 / sqrt(t[0]);
+      double acc[2] = {0, 0};
+      vec_loop(
+          n, [&](long i) { return V3{theta[i], dg[i], ax[i]}; },
+          [&](long i, V3 const& v) {
+            double const o = c * v.a;
+            theta[i] = o;
+            acc[0] += v.b * o;
+            acc[1] += v.b * v.c;
+          });
+      leave(acc, out);
+    }
+
+    __global__ __launch_bounds__(VT) void k_rot_trial(long n, double c, double s, double dr, double const* __restrict__ ax,
+                                                      double const* __restrict__ theta, double* __restrict__ axp,
+                                                      double* __restrict__ delta, ListMove lm) {
+      vec_loop(
+          n, [&](long i) { return M3{ax[i], theta[i], delta[i], to_move(lm, i)}; },
+          [&](long i, M3 const& v) {
+            double o = c * v.a;
+            o += s * v.b;
+            axp[i] = o;
+            double const e = -dr * o;
+            delta[i] = e;
+            move_one(lm, v.m, e - v.c);
+          });
+    }
+
+    __global__ __launch_bounds__(VT) void k_rot_curv(long n, double const* __restrict__ g1p, double const* __restrict__ g0,
+                                                     double const* __restrict__ axp, double* __restrict__ out) {
+      double acc[1] = {0};
+      vec_loop(
+          n, [&](long i) { return V3{g1p[i], g0[i], axp[i]}; },
+          [&](long, V3 const& v) {
+            double const o = v.a - v.b;
+            acc[0] += o * v.c;
+          });
+      leave(acc, out);
+    }
+
+    __global__ __launch_bounds__(VT) void k_rot_accept(long n, double c, double s, double w1, double w2, double w3,
+                                                       double* __restrict__ ax, double const* __restrict__ theta,
+                                                       double* __restrict__ g1, double const* __restrict__ g1p,
+                                                       double const* __restrict__ g0, double* __restrict__ dg,
+                                                       double* __restrict__ out) {
+      double acc[1] = {0};
+      vec_loop(
+          n, [&](long i) { return V5{ax[i], theta[i], g1[i], g1p[i], g0[i]}; },
+          [&](long i, V5 const& v) {
+            double a = c * v.a;
+            a += s * v.b;
+            ax[i] = a;
+            double o = w1 * v.c;
+            o += w2 * v.d;
+            o += w3 * v.e;
+            g1[i] = o;
+            double const d = o - v.e;
+            dg[i] = d;
+            acc[0] += d * a;
+          });
+      leave(acc, out);
+    }
+
+    __global__ __launch_bounds__(VT) void k_rot_back(long n, double const* __restrict__ delta, double const* __restrict__ g0,
+                                                     double const* __restrict__ ax, ListMove lm, double* __restrict__ out) {
+      double acc[1] = {0};
+      vec_loop(
+          n, [&](long i) { return M3{delta[i], g0[i], ax[i], to_move(lm, i)}; },
+          [&](long, M3 const& v) {
+            move_one(lm, v.m, -v.a);
+            acc[0] += v.b * v.c;
+          });
+      leave(acc, out);
+    }
+
+    template <bool SUMS, bool G0>
+    __global__ __launch_bounds__(VT) void k_rot_eff(long n, double k, double const* __restrict__ in,
+                                                    double const* __restrict__ g0, double const* __restrict__ ax,
+                                                    double* __restrict__ eff, double const* __restrict__ w,
+                                                    double* __restrict__ out, unsigned const* __restrict__ flags,
+                                                    unsigned* __restrict__ hflag) {
+      __shared__ double sh[VMAXB];
+      double t[1];
+      collect(in, sh, t);
+      double const c = k * t[0];
+      double acc[3] = {0, 0, 0};
+      vec_loop(
+          n, [&](long i) { return V3{G0 ? g0[i] : 0.0, ax[i], w ? w[i] : 0.0}; },
+          [&](long i, V3 const& v) {
+            double o;
+            if (G0) {
+              o = v.a;
+              o += c * v.b;
+            } else {
+              o = c * v.b;
+            }
+            eff[i] = o;
+            if (SUMS) {
+              add_comp(acc, i, o);
+            } else {
+              acc[0] += o * o;
+              acc[1] += o * v.c;
+            }
+          });
+      leave(acc, out);
+      if (hflag && blockIdx.x == 0 && threadIdx.x == 0) *hflag = *flags;
+    }
+
+    __global__ __launch_bounds__(VT) void k_sum(double const* __restrict__ x, long n, double* __restrict__ out,
+                                                unsigned const* __restrict__ flags, unsigned* __restrict__ hflag) {
+      double acc[1] = {0};
+      vec_loop(
+          n, [&](long i) { return V1{x[i]}; }, [&](long, V1 const& v) { acc[0] += v.a; });
+      leave(acc, out);
+      if (hflag && blockIdx.x == 0 && threadIdx.x == 0) *hflag = *flags;
     }
 
   }  // namespace
 
-  void vec(flyg_ctx_s& ctx, VecArgs const& a) {
-    if (a.n <= 0) return;
-    ctx.dpart.reserve(VMAXB * 4);
-    k_vec<<<blocks_for(a.n), VT, 0, ctx.stream>>>(a, ctx.dpart.get(), ctx.dflags.get() + 3);
-    HIPCHK(hipGetLastError());
+#define FLYG_VEC_LAUNCH(kernel, ...) \
+  kernel<<<vec_blocks(n), VT, 0, ctx.stream>>>(n, __VA_ARGS__); \
+  HIPCHK(hipGetLastError())
+
+  ListMove list_move(flyg_list_s& nl) {
+    return ListMove{reinterpret_cast<double*>(nl.pos.get()), reinterpret_cast<double*>(nl.gpos.get()), nl.rank.get()};
   }
 
-  void dev_sum(flyg_ctx_s& ctx, double const* x, long n, double* d_out) {
-    ctx.dpart.reserve(VMAXB * 4);
-    k_sum<<<blocks_for(n), VT, 0, ctx.stream>>>(x, n, ctx.dpart.get(), ctx.dflags.get() + 3, d_out);
+  void lb_first(flyg_ctx_s& ctx, long n, double const* x, double const* g, double* px, double* pg, double* r,
+                double const* w, double* out) {
+    FLYG_VEC_LAUNCH(k_lb_first, x, g, px, pg, r, w, out);
+  }
+  void lb_hist(flyg_ctx_s& ctx, long n, double const* x, double const* g, double* px, double* pg, double* s, double* y,
+               double* out) {
+    FLYG_VEC_LAUNCH(k_lb_hist, x, g, px, pg, s, y, out);
+  }
+  void lb_loop1(flyg_ctx_s& ctx, long n, bool newest, int j, LBScalars* lb, double const* in, double const* q,
+                double const* y, double const* s_next, double* qout, double* out) {
+    if (newest) {
+      FLYG_VEC_LAUNCH(k_lb_loop1<true>, j, lb, in, q, y, s_next, qout, out);
+    } else {
+      FLYG_VEC_LAUNCH(k_lb_loop1<false>, j, lb, in, q, y, s_next, qout, out);
+    }
+  }
+  void lb_turn(flyg_ctx_s& ctx, long n, bool newest, int j, LBScalars* lb, double const* in, double const* q,
+               double const* y, double* r, double* out) {
+    if (newest) {
+      FLYG_VEC_LAUNCH(k_lb_turn<true>, j, lb, in, q, y, r, out);
+    } else {
+      FLYG_VEC_LAUNCH(k_lb_turn<false>, j, lb, in, q, y, r, out);
+    }
+  }
+  void lb_loop2(flyg_ctx_s& ctx, long n, int j, LBScalars* lb, double const* in, double* r, double const* s,
+                double const* w, double* out) {
+    FLYG_VEC_LAUNCH(k_lb_loop2, j, lb, in, r, s, w, out);
+  }
+  void vec_step(flyg_ctx_s& ctx, long n, double trust, double const* in, double* q, double* x, ListMove lm, double* hsum) {
+    FLYG_VEC_LAUNCH(k_step, trust, in, q, x, lm, hsum);
+  }
+  void vec_dots(flyg_ctx_s& ctx, long n, double const* a, double const* b, double const* c, double const* d, double* out,
+                unsigned* hflag) {
+    FLYG_VEC_LAUNCH(k_dots, a, b, c, d, out, ctx.dflags.get(), hflag);
+  }
+  void vec_diff(flyg_ctx_s& ctx, long n, double const* a, double const* b, double* o, double* out) {
+    FLYG_VEC_LAUNCH(k_diff, a, b, o, out);
+  }
+  void rot_offset(flyg_ctx_s& ctx, long n, double dr, double const* ax, double* delta, ListMove lm) {
+    FLYG_VEC_LAUNCH(k_rot_offset, dr, ax, delta, lm);
+  }
+  void rot_diff(flyg_ctx_s& ctx, long n, double const* g1, double const* g0, double const* ax, double* dg, double* out) {
+    FLYG_VEC_LAUNCH(k_rot_diff, g1, g0, ax, dg, out);
+  }
+  void rot_torque(flyg_ctx_s& ctx, long n, bool sums, double const* in, double const* dg, double const* ax, double* o,
+                  double* out) {
+    if (sums) {
+      FLYG_VEC_LAUNCH(k_rot_torque<true>, in, dg, ax, o, out);
+    } else {
+      FLYG_VEC_LAUNCH(k_rot_torque<false>, in, dg, ax, o, out);
+    }
+  }
+  void vec_demean(flyg_ctx_s& ctx, long n, double mean_k, double const* in, double* o, double const* w, double* out,
+                  unsigned* hflag) {
+    FLYG_VEC_LAUNCH(k_demean, mean_k, in, o, w, out, ctx.dflags.get(), hflag);
+  }
+  void rot_orth(flyg_ctx_s& ctx, long n, double const* in, double const* ax, double* theta, double* out) {
+    FLYG_VEC_LAUNCH(k_rot_orth, in, ax, theta, out);
+  }
+  void rot_unit(flyg_ctx_s& ctx, long n, double const* in, double* theta, double const* dg, double const* ax, double* out) {
+    FLYG_VEC_LAUNCH(k_rot_unit, in, theta, dg, ax, out);
+  }
+  void rot_trial(flyg_ctx_s& ctx, long n, double c, double s, double dr, double const* ax, double const* theta, double* axp,
+                 double* delta, ListMove lm) {
+    FLYG_VEC_LAUNCH(k_rot_trial, c, s, dr, ax, theta, axp, delta, lm);
+  }
+  void rot_curv(flyg_ctx_s& ctx, long n, double const* g1p, double const* g0, double const* axp, double* out) {
+    FLYG_VEC_LAUNCH(k_rot_curv, g1p, g0, axp, out);
+  }
+  void rot_accept(flyg_ctx_s& ctx, long n, double c, double s, double w1, double w2, double w3, double* ax,
+                  double const* theta, double* g1, double const* g1p, double const* g0, double* dg, double* out) {
+    FLYG_VEC_LAUNCH(k_rot_accept, c, s, w1, w2, w3, ax, theta, g1, g1p, g0, dg, out);
+  }
+  void rot_back(flyg_ctx_s& ctx, long n, double const* delta, double const* g0, double const* ax, ListMove lm, double* out) {
+    FLYG_VEC_LAUNCH(k_rot_back, delta, g0, ax, lm, out);
+  }
+  void rot_eff(flyg_ctx_s& ctx, long n, bool sums, bool with_g0, double k, double const* in, double const* g0,
+               double const* ax, double* eff, double const* w, double* out, unsigned* hflag) {
+    unsigned const* fl = ctx.dflags.get();
+    if (sums && with_g0) {
+      FLYG_VEC_LAUNCH((k_rot_eff<true, true>), k, in, g0, ax, eff, w, out, fl, hflag);
+    } else if (sums) {
+      FLYG_VEC_LAUNCH((k_rot_eff<true, false>), k, in, g0, ax, eff, w, out, fl, hflag);
+    } else if (with_g0) {
+      FLYG_VEC_LAUNCH((k_rot_eff<false, true>), k, in, g0, ax, eff, w, out, fl, hflag);
+    } else {
+      FLYG_VEC_LAUNCH((k_rot_eff<false, false>), k, in, g0, ax, eff, w, out, fl, hflag);
+    }
+  }
+
+  void dev_sum(flyg_ctx_s& ctx, double const* x, long n, double* part, unsigned* hflag) {
+    k_sum<<<vec_blocks(n), VT, 0, ctx.stream>>>(x, n, part, ctx.dflags.get(), hflag);
     HIPCHK(hipGetLastError());
   }
 

@@ -1,60 +1,104 @@
-// Device vector engine for the plain-form minimiser and dimer: one fused kernel computes
-//   out = c0 v0 + c1 v1 + c2 v2 (+ per-component mean correction)
-// and up to four dot products (or the three component sums of `out`), reduced deterministically
-// (fixed grid, per-block trees, the last block sums the block partials in order) into device scalar
-// slots, followed by an optional scalar post-op (the L-BFGS two-loop coefficients), so whole chains
-// of vector algebra run without host synchronisation.
+// Device vector algebra of the plain-form minimiser, rotor and dimer: each kernel fuses the element-wise
+// updates of one stage with the dot products of the next, so a chain of L-BFGS or rotor stages is one
+// launch per dependent reduction.
+//
+// Reductions are deterministic: the grid depends on the vector length only (vec_blocks), each block
+// leaves its partial sums in part[k * VMAXB + block], and whoever needs the value adds the partials in
+// block order: the next kernel of the chain (every block for itself, from LDS), or the host, from a buffer
+// in pinned memory that the kernel writes directly.  No block waits for another one.
+//
+// What bounds them: at 16k atoms (48k elements) latency, not bytes.  A launch whose last block collected
+// the partials with device-scope loads in sequence took 14-16 us there, most of it that loop and its two
+// device-scope fences; with the partials left to the consumer a launch takes 3 us.
 #pragma once
 
 #include "eam_host.hpp"
 
 namespace flyg {
 
-  // Coefficient value = k * f(*s) with f = identity, or 1/sqrt when inv_sqrt (s == nullptr: value = k).
-  struct Coef {
-    double k = 0;
-    double const* s = nullptr;
-    int inv_sqrt = 0;
-  };
+  constexpr int VMAXB = 240;               // most blocks of a vector kernel
+  constexpr int VPART = 4 * VMAXB;         // doubles of one set of partial sums
 
-  inline Coef cst(double k) { return Coef{k, nullptr, 0}; }
-  inline Coef dev(double const* s, double k = 1.0) { return Coef{k, s, 0}; }
-  inline Coef dev_rsqrt(double const* s, double k = 1.0) { return Coef{k, s, 1}; }
-
-  // Post-ops applied by the finalising block (acc = the reduced sums):
-  enum PostOp : int {
-    POST_NONE = 0,
-    POST_HIST = 1,    // lb.rho[j] = 1/|acc0|; lb.h0 = (1/rho[j]) / acc1
-    POST_ALPHA = 2,   // lb.alpha[j] = lb.rho[j] * acc0
-    POST_BETA = 3,    // lb.coef[j] = lb.alpha[j] - lb.rho[j] * acc0
-  };
+  inline unsigned vec_blocks(long n) {     // 256 threads a block, at least 4 elements a thread
+    long b = (n + 1023) / 1024;
+    return static_cast<unsigned>(b < 1 ? 1 : (b > VMAXB ? VMAXB : b));
+  }
 
   // Scalars of one device L-BFGS core.
   struct LBScalars {
     double rho[32];
     double alpha[32];
-    double coef[32];
     double h0;
   };
 
-  struct VecArgs {
-    long n = 0;
-    double* out = nullptr;
-    double const* v[3] = {nullptr, nullptr, nullptr};
-    Coef c[3];
-    double const* mean3 = nullptr;   // out[i] += mean_k * mean3[i % 3]
-    double mean_k = 0;
-    // dots: acc_k = sum X_k[i] Y_k[i]; a null X_k/Y_k means `out`.  ndot = number of dots.
-    int ndot = 0;
-    double const* X[4] = {nullptr, nullptr, nullptr, nullptr};
-    double const* Y[4] = {nullptr, nullptr, nullptr, nullptr};
-    int comp_sums = 0;   // acc_{0,1,2} = component sums of out (instead of dots)
-    double* slots = nullptr;   // receives the reduced sums (4 doubles)
-    int post = POST_NONE;
-    int pj = 0;
-    LBScalars* lb = nullptr;
+  // The live positions of a neighbour list, moved by -u beside the kernel's own work (List::update).
+  struct ListMove {
+    double* pos = nullptr;    // by atom, 4 doubles each
+    double* gpos = nullptr;   // by slot
+    int const* rank = nullptr;
   };
+  ListMove list_move(flyg_list_s& nl);
 
-  void vec(flyg_ctx_s& ctx, VecArgs const& a);
+  // L-BFGS two-loop stages (lbfgs_core.cpp:29-87).  `in`: the partial sums of the stage before; `out` must
+  // be another buffer.
+  // First call: px = x, pg = r = g; out: r.w (w = null: r.r).
+  void lb_first(flyg_ctx_s& ctx, long n, double const* x, double const* g, double* px, double* pg, double* r,
+                double const* w, double* out);
+  // s = x - px, y = g - pg, px = x, pg = g; out: s.y, y.y, s.g.
+  void lb_hist(flyg_ctx_s& ctx, long n, double const* x, double const* g, double* px, double* pg, double* s, double* y,
+               double* out);
+  // alpha_j from `in` (newest: rho_j and h0 too), qout = q - alpha_j y; out: s_next.qout.
+  void lb_loop1(flyg_ctx_s& ctx, long n, bool newest, int j, LBScalars* lb, double const* in, double const* q,
+                double const* y, double const* s_next, double* qout, double* out);
+  // The same for the oldest pair, then r = h0 (q - alpha_j y); out: y.r.
+  void lb_turn(flyg_ctx_s& ctx, long n, bool newest, int j, LBScalars* lb, double const* in, double const* q,
+               double const* y, double* r, double* out);
+  // r += (alpha_j - rho_j in) s; out: r.w (w = null: r.r).
+  void lb_loop2(flyg_ctx_s& ctx, long n, int j, LBScalars* lb, double const* in, double* r, double const* s,
+                double const* w, double* out);
+
+  // Trust-region step: q *= min(1, trust / sqrt(in)), x -= q, the list follows; the sum itself goes to *hsum.
+  void vec_step(flyg_ctx_s& ctx, long n, double trust, double const* in, double* q, double* x, ListMove lm, double* hsum);
+  // out: a.b and c.d (c null: one sum); the device error flags go to *hflag (null: not copied).
+  void vec_dots(flyg_ctx_s& ctx, long n, double const* a, double const* b, double const* c, double const* d, double* out,
+                unsigned* hflag);
+  // o = a - b; out: o.o.
+  void vec_diff(flyg_ctx_s& ctx, long n, double const* a, double const* b, double* o, double* out);
+
+  // Rotor stages (rotor.cpp:49-164).
+  // delta = -dr ax, the list follows.
+  void rot_offset(flyg_ctx_s& ctx, long n, double dr, double const* ax, double* delta, ListMove lm);
+  // dg = g1 - g0; out: dg.ax.
+  void rot_diff(flyg_ctx_s& ctx, long n, double const* g1, double const* g0, double const* ax, double* dg, double* out);
+  // o = dg - in ax; out: the component sums of o when `sums`.
+  void rot_torque(flyg_ctx_s& ctx, long n, bool sums, double const* in, double const* dg, double const* ax, double* o,
+                  double* out);
+  // o += mean_k (component sums `in`); out: o.o and o.w (w null: o.o alone; out null: neither).
+  void vec_demean(flyg_ctx_s& ctx, long n, double mean_k, double const* in, double* o, double const* w, double* out,
+                  unsigned* hflag);
+  // theta -= in ax; out: theta.theta.
+  void rot_orth(flyg_ctx_s& ctx, long n, double const* in, double const* ax, double* theta, double* out);
+  // theta /= sqrt(in); out: dg.theta, dg.ax.
+  void rot_unit(flyg_ctx_s& ctx, long n, double const* in, double* theta, double const* dg, double const* ax, double* out);
+  // axp = c ax + s theta; the list moves by -dr axp - delta, delta = -dr axp.
+  void rot_trial(flyg_ctx_s& ctx, long n, double c, double s, double dr, double const* ax, double const* theta, double* axp,
+                 double* delta, ListMove lm);
+  // out: (g1p - g0).axp.
+  void rot_curv(flyg_ctx_s& ctx, long n, double const* g1p, double const* g0, double const* axp, double* out);
+  // ax = c ax + s theta, g1 = w1 g1 + w2 g1p + w3 g0, dg = g1 - g0; out: dg.ax.
+  void rot_accept(flyg_ctx_s& ctx, long n, double c, double s, double w1, double w2, double w3, double* ax,
+                  double const* theta, double* g1, double const* g1p, double const* g0, double* dg, double* out);
+  // The list moves back by delta; out: g0.ax.
+  void rot_back(flyg_ctx_s& ctx, long n, double const* delta, double const* g0, double const* ax, ListMove lm, double* out);
+  // eff = (g0 +) k in ax; out: the component sums of eff when `sums`, else eff.eff and eff.w (w null: none).
+  void rot_eff(flyg_ctx_s& ctx, long n, bool sums, bool with_g0, double k, double const* in, double const* g0,
+               double const* ax, double* eff, double const* w, double* out, unsigned* hflag);
+
+  // Value k of a set of partial sums, added on the host (the kernel wrote them to pinned memory).
+  inline double host_sum(double const* part, int k, long n) {
+    double t = 0;
+    for (unsigned b = 0; b < vec_blocks(n); ++b) t += part[k * VMAXB + b];
+    return t;
+  }
 
 }  // namespace flyg
