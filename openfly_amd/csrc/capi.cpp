@@ -375,7 +375,7 @@ int flyg_eam_hessian_eigenvalues(flyg_eam eam, flyg_list nl, const uint32_t* typ
     uint32_t const* t;
     uint8_t const* f;
     stage_atoms(*eam, types, frozen, n, where, &t, &f);
-    std::vector<double> w = hessian_eigenvalues(*eam, *nl, t, f, hf, ht, nullptr);
+    std::vector<double> w = hessian_eigenvalues(*eam, *nl, t, f, hf, ht);
     std::copy(w.begin(), w.end(), eigenvalues);
     *n_dof = static_cast<int64_t>(w.size());
   });

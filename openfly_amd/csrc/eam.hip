@@ -26,24 +26,16 @@
 
 namespace flyg {
 
+  // t0 >= 0 selects the single-species kernels (constant table indices): always with one species
+  // tabulated, and with several when the staged host types hold one species only.
+  PairArgs pair_args(flyg_eam_s const& E, flyg_list_s& nl, uint32_t const* types, uint8_t const* frozen) {
+    int t0 = E.tab.ntypes == 1 ? 0 : (types == E.types.get() ? E.staged_single : -1);
+    return PairArgs{nl.pos.get(), nl.nbr.get(), nl.ncnt.get(), nl.K, nl.n, types, frozen, t0};
+  }
+
   namespace {
 
     constexpr int NT = 256;
-
-    // Image shift of a packed entry: sum_a s_a * basis column a, s_a in {-1, 0, 1}.  Exact for
-    // orthorhombic boxes (each component is 0 or +-L), computed in registers (no table lookup).
-    struct Shifts {
-      double b[3][3];   // b[row][col]
-      __device__ double3 of(unsigned code) const {
-        int s0 = static_cast<int>(code % 3u) - 1;
-        int s1 = static_cast<int>((code / 3u) % 3u) - 1;
-        int s2 = static_cast<int>(code / 9u) - 1;
-        return make_double3(s0 * b[0][0] + s1 * b[0][1] + s2 * b[0][2], s0 * b[1][0] + s1 * b[1][1] + s2 * b[1][2],
-                            s0 * b[2][0] + s1 * b[2][1] + s2 * b[2][2]);
-      }
-    };
-
-    __device__ inline int vidx(EAMTables const& T, int a, int b) { return a > b ? a + T.ntypes * b : b + T.ntypes * a; }
 
     // Mixed-form pass-1 output: the force pass uses F' only in FP32, so the w slot of (x, y, z, w) carries
     // F' as a float in its low 32 bits and the species in its high 32 bits, and a neighbour's species
@@ -407,20 +399,6 @@ namespace flyg {
       double v = deriv == 0 ? spl64<0>(T, s, x[i], e) : deriv == 1 ? spl64<1>(T, s, x[i], e) : spl64<2>(T, s, x[i], e);
       out[i] = v;
       if (e) atomicOr(err, e);
-    }
-
-    Shifts shifts_of(BoxDesc const& b) {
-      Shifts s;
-      for (int r = 0; r < 3; ++r)
-        for (int c = 0; c < 3; ++c) s.b[r][c] = b.B[r][c];
-      return s;
-    }
-
-    // t0 >= 0 selects the single-species kernels (constant table indices): always with one species
-    // tabulated, and with several when the staged host types hold one species only.
-    PairArgs pair_args(flyg_eam_s const& E, flyg_list_s& nl, uint32_t const* types, uint8_t const* frozen) {
-      int t0 = E.tab.ntypes == 1 ? 0 : (types == E.types.get() ? E.staged_single : -1);
-      return PairArgs{nl.pos.get(), nl.nbr.get(), nl.ncnt.get(), nl.K, nl.n, types, frozen, t0};
     }
 
     __global__ void k_types_by_slot(uint32_t const* __restrict__ types, int const* __restrict__ order, long n,

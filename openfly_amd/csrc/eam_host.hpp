@@ -64,6 +64,8 @@ struct flyg_eam_s {
   long gtype_build = -1, gtype_stamp = -1;   // gtype holds the staged types in the layout of this build
   flyg::DBuf<uint8_t> frozen;
   flyg::DBuf<double> vec_in, vec_out;
+  flyg::DBuf<double> hess;      // workspace of hessian_eigenvalues, kept between calls while it is small
+  flyg::DBuf<int> hess_ids;     // its atom indices
   std::vector<uint32_t> last_types;
   std::vector<uint8_t> last_frozen;
   int lanes = 0;                                   // lanes per atom row, 0 = timed choice
@@ -150,6 +152,27 @@ namespace flyg {
     // its position; set for the slot layout with several species.
     bool type_in_w = false;
   };
+  // Image shift of a packed entry: sum_a s_a * basis column a, s_a in {-1, 0, 1}.  Exact for
+  // orthorhombic boxes (each component is 0 or +-L), computed in registers (no table lookup).
+  struct Shifts {
+    double b[3][3];   // b[row][col]
+    __device__ double3 of(unsigned code) const {
+      int s0 = static_cast<int>(code % 3u) - 1;
+      int s1 = static_cast<int>((code / 3u) % 3u) - 1;
+      int s2 = static_cast<int>(code / 9u) - 1;
+      return make_double3(s0 * b[0][0] + s1 * b[0][1] + s2 * b[0][2], s0 * b[1][0] + s1 * b[1][1] + s2 * b[1][2],
+                          s0 * b[2][0] + s1 * b[2][1] + s2 * b[2][2]);
+    }
+  };
+  inline Shifts shifts_of(BoxDesc const& b) {
+    Shifts s;
+    for (int r = 0; r < 3; ++r)
+      for (int c = 0; c < 3; ++c) s.b[r][c] = b.B[r][c];
+    return s;
+  }
+  __device__ inline int vidx(EAMTables const& T, int a, int b) { return a > b ? a + T.ntypes * b : b + T.ntypes * a; }
+  PairArgs pair_args(flyg_eam_s const& E, flyg_list_s& nl, uint32_t const* types, uint8_t const* frozen);
+
   void eam_setup_tables(flyg_eam_s& e);
   double eam_energy(flyg_eam_s& e, flyg_list_s& nl, uint32_t const* d_types, uint8_t const* d_frozen);
   void eam_gradient(flyg_eam_s& e, flyg_list_s& nl, uint32_t const* d_types, uint8_t const* d_frozen, double* d_grad,
@@ -163,7 +186,7 @@ namespace flyg {
   // Sorted eigenvalues of the mass-weighted Hessian block of the non-frozen atoms (hessian.hip).
   std::vector<double> hessian_eigenvalues(flyg_eam_s& e, flyg_list_s& nl, uint32_t const* d_types,
                                           uint8_t const* d_frozen, std::vector<uint8_t> const& h_frozen,
-                                          std::vector<uint32_t> const& h_types, int* sweeps);
+                                          std::vector<uint32_t> const& h_types);
   void eam_hvp(flyg_eam_s& e, flyg_list_s& nl, uint32_t const* d_types, uint8_t const* d_frozen, double const* d_v,
                double* d_hv);
   void eam_table_eval(flyg_eam_s& e, int kind, int a, int b, double const* x, long m, int deriv, double* out);

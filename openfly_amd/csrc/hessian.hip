@@ -3,37 +3,223 @@
 // (hessian.hpp:86-93; the reference calls Eigen's SelfAdjointEigenSolver), as used by Master for
 // Mechanism::kinetic_pre (find.cpp:838-871) and the minimum's log-product (find.cpp:1094-1144).
 //
-// Assembly: column c of the 3M x 3M block (M = non-frozen atoms) is H e_c from the matrix-free
-// Hessian-vector product kernels, gathered over the non-frozen rows and divided by sqrt(m_i m_j); the
-// lower triangle is kept (the part the reference's solver reads) and mirrored.
-// Diagonalisation: cyclic Jacobi rotations (Golub & Van Loan, Matrix Computations, Alg. 8.4.3) in the
-// parallel round-robin ordering: each of the m - 1 rounds of a sweep rotates m / 2 disjoint index pairs
-// at once (one workgroup per pair updates the pair's two rows, then every row's two columns), so a sweep
-// touches every off-diagonal element once; sweeps repeat until the off-diagonal Frobenius norm is below
-// 1e-14 of the matrix's.  The eigenvalues (the diagonal) come back sorted.
+// Assembly: the analytic block, row by row.  With u = (r_a - r_g) / r along a listed pair,
+//   H = sum over pairs of K (+K on the diagonal blocks, -K between the two atoms),
+//       K = k'' u u^T + (m / r) (I - u u^T),  m = V' + F'_g phi'_{a->g} + F'_a phi'_{g->a}, k'' the same of second derivatives,
+//     + sum over atoms b, frozen ones included, of F''_b (grad rho_b)(grad rho_b)^T.
+// D holds dF'_b by moved coordinate for every atom b next to a mobile one; a row of H is then the pair
+// blocks plus a short sum of rows of D (one per neighbour), so both kernels stream whole rows.  Assembly from
+// the columns' Hessian-vector products took five launches and two passes over the whole system for
+// each of the 3M coordinates: 11 ms at 120 mobile atoms in a 2000-atom cell, now 60 us.
+//
+// Eigenvalues: Householder reduction to tridiagonal form (Golub & Van Loan, Matrix Computations, Alg. 8.3.1),
+// one launch a column that applies the previous reflection and multiplies by the next one in the same
+// pass over the block; then each eigenvalue by multisection on Sturm counts (Givens; Barth, Martin & Wilkinson,
+// Numer. Math. 9 (1967) 386), a wavefront per eigenvalue testing 64 points of its interval at once.  Both are
+// backward stable: errors of a few units of 1e-16 of the largest eigenvalue.  Bound by one launch per column
+// up to some 1000 coordinates, then by the memory traffic of the shrinking block.  Cyclic Jacobi rotations
+// needed ten sweeps of 3M rounds of two launches: 36 ms at 360 coordinates.
 #include <algorithm>
 #include <cmath>
 #include <vector>
 
-#include "eam_host.hpp"
+#include "vecops.hpp"
 
 namespace flyg {
-
-  void eam_hvp(flyg_eam_s& E, flyg_list_s& nl, uint32_t const* types, uint8_t const* frozen, double const* d_v,
-               double* d_hv);
 
   namespace {
 
     constexpr int NTB = 256;
+    constexpr std::size_t HESS_KEEP = 64u << 20;   // largest workspace kept in the potential handle between calls
 
-    __global__ void k_set(double* v, long i, double x) { v[i] = x; }
+    constexpr int EC = 256;   // neighbour entries staged at a time
 
-    // H[r][c] = hv[dof[r]] / sqrt(m_r m_c) for the non-frozen degrees of freedom r (column c).
-    __global__ void k_gather_column(double const* __restrict__ hv, long const* __restrict__ dof,
-                                    double const* __restrict__ rmass, long n3m, long c, double* __restrict__ H) {
-      long r = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
-      if (r >= n3m) return;
-      H[r * n3m + c] = hv[dof[r]] * (rmass[r] * rmass[c]);
+    // F' and F'' of every atom.
+    template <int L>
+    __global__ __launch_bounds__(NTB) void k_embed(EAMTables T, Shifts S, PairArgs A, double2* __restrict__ ff,
+                                                   unsigned* __restrict__ err) {
+      long const gid = blockIdx.x * static_cast<long>(NTB) + threadIdx.x;
+      long const i = gid / L;
+      int const lane = static_cast<int>(gid % L);
+      bool const act = i < A.n;
+      unsigned e = 0;
+      double rho = 0;
+      int ti = 0;
+      if (act) {
+        double4 const pi = A.pos[i];
+        ti = A.t0 < 0 ? checked_type(A.types[i], T.ntypes, e) : A.t0;
+        int const c = min(A.cnt[i], A.K);
+        for (int k = lane; k < c; k += L) {
+          unsigned const en = A.nbr[i * static_cast<long>(A.K) + k];
+          unsigned const j = en & NB_IDX_MASK;
+          double3 const sh = S.of(en >> NB_SHIFT_BITS);
+          double4 const pj = A.pos[j];
+          double const dx = (pj.x + sh.x) - pi.x, dy = (pj.y + sh.y) - pi.y, dz = (pj.z + sh.z) - pi.z;
+          double const r2 = dx * dx + dy * dy + dz * dz;
+          if (r2 < T.rc2) {
+            int const tj = A.t0 < 0 ? checked_type(A.types[j], T.ntypes, e) : A.t0;
+            rho += spl64<0>(T, T.phi[tj + T.ntypes * ti], sqrt(r2), e);
+          }
+        }
+      }
+      rho = group_sum<L>(rho);
+      if (act && lane == 0) ff[i] = make_double2(spl64<1>(T, T.F[ti], rho, e), spl64<2>(T, T.F[ti], rho, e));
+      if (e) atomicOr(err, e);
+    }
+
+    // Marks the mobile atoms and their neighbours (one wavefront per mobile atom).
+    __global__ void k_mark(PairArgs A, int const* __restrict__ atoms, long nm, int* __restrict__ mark) {
+      long const w = (blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x) / 64;
+      int const lane = threadIdx.x & 63;
+      if (w >= nm) return;
+      long const i = atoms[w];
+      if (lane == 0) mark[i] = 1;
+      int const c = min(A.cnt[i], A.K);
+      for (int k = lane; k < c; k += 64) mark[A.nbr[i * static_cast<long>(A.K) + k] & NB_IDX_MASK] = 1;
+    }
+
+    // loc = exclusive scan of the marks: the atom of each row of D.
+    __global__ void k_region(int const* __restrict__ loc, long n, int* __restrict__ region) {
+      long const i = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
+      if (i < n && loc[i + 1] > loc[i]) region[loc[i]] = static_cast<int>(i);
+    }
+
+    struct Pair {
+      double ux, uy, uz, r;
+      int j, ti, tj;
+      bool in;
+    };
+
+    __device__ inline Pair pair_at(EAMTables const& T, Shifts const& S, PairArgs const& A, long i, double4 const& pi, int ti,
+                                   int k, unsigned& e) {
+      Pair p;
+      unsigned const en = A.nbr[i * static_cast<long>(A.K) + k];
+      p.j = static_cast<int>(en & NB_IDX_MASK);
+      double3 const sh = S.of(en >> NB_SHIFT_BITS);
+      double4 const pj = A.pos[p.j];
+      double const dx = (pj.x + sh.x) - pi.x, dy = (pj.y + sh.y) - pi.y, dz = (pj.z + sh.z) - pi.z;
+      double const r2 = dx * dx + dy * dy + dz * dz;
+      p.in = r2 < T.rc2;
+      p.r = p.in ? sqrt(r2) : 1.0;
+      p.ux = dx / p.r;
+      p.uy = dy / p.r;
+      p.uz = dz / p.r;
+      p.ti = ti;
+      p.tj = A.t0 < 0 ? checked_type(A.types[p.j], T.ntypes, e) : A.t0;
+      return p;
+    }
+
+    // Row b of D: F''_b d rho_b / d (coordinate) for the 3 nm mobile coordinates.  One workgroup per region atom:
+    // its entries are staged in LDS, then every thread sums those that touch its columns, in row order.
+    __global__ __launch_bounds__(NTB) void k_drow(EAMTables T, Shifts S, PairArgs A, double2 const* __restrict__ ff,
+                                                  int const* __restrict__ region, int const* __restrict__ mob, long n3m,
+                                                  double* __restrict__ D, unsigned* __restrict__ err) {
+      __shared__ double s_g[3][EC];
+      __shared__ int s_m[EC];
+      long const b = region[blockIdx.x];
+      unsigned e = 0;
+      double4 const pb = A.pos[b];
+      int const tb = A.t0 < 0 ? checked_type(A.types[b], T.ntypes, e) : A.t0;
+      int const mb = mob[b];
+      double const fpp = ff[b].y;
+      int const c = min(A.cnt[b], A.K);
+      double* row = D + blockIdx.x * n3m;
+      for (int k0 = 0; k0 == 0 || k0 < c; k0 += EC) {
+        int const nk = min(EC, c - k0);
+        __syncthreads();
+        for (int k = threadIdx.x; k < nk; k += NTB) {
+          Pair const p = pair_at(T, S, A, b, pb, tb, k0 + k, e);
+          double const f = p.in ? fpp * spl64<1>(T, T.phi[p.tj + T.ntypes * tb], p.r, e) : 0.0;
+          s_g[0][k] = f * p.ux;
+          s_g[1][k] = f * p.uy;
+          s_g[2][k] = f * p.uz;
+          s_m[k] = p.in ? mob[p.j] : -2;
+        }
+        __syncthreads();
+        for (long col = threadIdx.x; col < n3m; col += NTB) {
+          int const m = static_cast<int>(col / 3), d = static_cast<int>(col % 3);
+          double v = k0 ? row[col] : 0.0;
+          if (m == mb) {
+            for (int k = 0; k < nk; ++k) v += (s_m[k] == m ? s_g[d][k] : 0.0) - s_g[d][k];
+          } else {
+            for (int k = 0; k < nk; ++k)
+              if (s_m[k] == m) v += s_g[d][k];
+          }
+          row[col] = v;
+        }
+      }
+      if (e) atomicOr(err, e);
+    }
+
+    // Rows 3g .. 3g + 2 of the mass-weighted block.  One workgroup per mobile atom g.
+    __global__ __launch_bounds__(NTB) void k_hrow(EAMTables T, Shifts S, PairArgs A, double2 const* __restrict__ ff,
+                                                  int const* __restrict__ atoms, int const* __restrict__ mob,
+                                                  int const* __restrict__ loc, double const* __restrict__ rmass, long n3m,
+                                                  double const* __restrict__ D, double* __restrict__ H,
+                                                  unsigned* __restrict__ err) {
+      __shared__ double s_u[3][EC], s_g[EC], s_a[EC], s_k[EC], s_t[EC];   // u, phi'_{a->g}, phi'_{g->a}, k'' - m / r, m / r
+      __shared__ int s_m[EC], s_l[EC];
+      int const mg = static_cast<int>(blockIdx.x);
+      long const g = atoms[mg];
+      unsigned e = 0;
+      double4 const pg = A.pos[g];
+      int const tg = A.t0 < 0 ? checked_type(A.types[g], T.ntypes, e) : A.t0;
+      double const fg = ff[g].x;
+      int const c = min(A.cnt[g], A.K);
+      double const* Dg = D + static_cast<long>(loc[g]) * n3m;
+      double* h0 = H + 3l * mg * n3m;
+      for (int k0 = 0; k0 == 0 || k0 < c; k0 += EC) {
+        int const nk = min(EC, c - k0);
+        __syncthreads();
+        for (int k = threadIdx.x; k < nk; k += NTB) {
+          Pair const p = pair_at(T, S, A, g, pg, tg, k0 + k, e);
+          double ga = 0, gb = 0, kk = 0, tt = 0;
+          if (p.in) {
+            SplineDesc const& sv = T.V[vidx(T, tg, p.tj)];
+            SplineDesc const& sa = T.phi[p.tj + T.ntypes * tg];
+            SplineDesc const& sb = T.phi[tg + T.ntypes * p.tj];
+            double const fa = ff[p.j].x;
+            ga = spl64<1>(T, sa, p.r, e);
+            gb = spl64<1>(T, sb, p.r, e);
+            double const m = spl64<1>(T, sv, p.r, e) + fg * ga + fa * gb;
+            tt = m / p.r;
+            kk = spl64<2>(T, sv, p.r, e) + fg * spl64<2>(T, sa, p.r, e) + fa * spl64<2>(T, sb, p.r, e) - tt;
+          }
+          s_u[0][k] = p.ux;
+          s_u[1][k] = p.uy;
+          s_u[2][k] = p.uz;
+          s_g[k] = ga;
+          s_a[k] = gb;
+          s_k[k] = kk;
+          s_t[k] = tt;
+          s_m[k] = p.in ? mob[p.j] : -2;
+          s_l[k] = p.in ? loc[p.j] : loc[g];
+        }
+        __syncthreads();
+        for (long col = threadIdx.x; col < n3m; col += NTB) {
+          int const m = static_cast<int>(col / 3), d = static_cast<int>(col % 3);
+          double const dg = Dg[col], rc = rmass[col];
+          double h[3] = {0, 0, 0};
+#pragma unroll 4
+          for (int k = 0; k < nk; ++k) {
+            double const q = s_g[k] * dg + s_a[k] * D[s_l[k] * n3m + col];
+#pragma unroll
+            for (int r = 0; r < 3; ++r) h[r] -= s_u[r][k] * q;
+            double const w = (m == mg ? 1.0 : 0.0) - (m == s_m[k] ? 1.0 : 0.0);
+            if (w != 0.0) {
+              double const ud = s_u[d][k] * s_k[k];
+#pragma unroll
+              for (int r = 0; r < 3; ++r) h[r] += w * (s_u[r][k] * ud + (r == d ? s_t[k] : 0.0));
+            }
+          }
+#pragma unroll
+          for (int r = 0; r < 3; ++r) {
+            double const v = h[r] * (rmass[3 * mg + r] * rc);
+            h0[r * n3m + col] = k0 ? h0[r * n3m + col] + v : v;
+          }
+        }
+      }
+      if (e) atomicOr(err, e);
     }
 
     // Keep the lower triangle: H[c][r] = H[r][c] for r > c.
@@ -44,99 +230,183 @@ namespace flyg {
       if (r > c) H[c * n + r] = H[r * n + c];
     }
 
-    // Pair k of round `round` in the round-robin ordering of m (even) indices: (round, m - 1) for k = 0,
-    // ((round + k) mod (m - 1), (round - k) mod (m - 1)) otherwise; returned as p < q.
-    __device__ inline void pair_of(int round, int k, int m, int& p, int& q) {
-      int a, b;
-      if (k == 0) {
-        a = round;
-        b = m - 1;
-      } else {
-        a = (round + k) % (m - 1);
-        b = (round - k + (m - 1)) % (m - 1);
-      }
-      p = min(a, b);
-      q = max(a, b);
-    }
-
-    // Symmetric Schur decomposition of the 2x2 block (Golub & Van Loan Alg. 8.4.1): c, s with
-    // [c s; -s c]^T [app apq; apq aqq] [c s; -s c] diagonal.
-    __device__ inline void schur2(double app, double aqq, double apq, double& c, double& s) {
-      if (apq == 0.0) {
-        c = 1.0;
-        s = 0.0;
-        return;
-      }
-      double tau = (aqq - app) / (2.0 * apq);
-      double t = fabs(tau) > 1e150 ? 0.5 / tau : (tau >= 0 ? 1.0 : -1.0) / (fabs(tau) + sqrt(1.0 + tau * tau));
-      c = 1.0 / sqrt(1.0 + t * t);
-      s = t * c;
-    }
-
-    // One workgroup per pair: rotation from the current block, then the pair's two rows.
-    __global__ void k_jacobi_rows(double* __restrict__ A, int n, int m, int round, double2* __restrict__ cs) {
-      int p, q;
-      pair_of(round, blockIdx.x, m, p, q);
-      bool const live = q < n;   // an index >= n pads an odd n
-      double c = 1.0, s = 0.0;
-      if (live) schur2(A[static_cast<long>(p) * n + p], A[static_cast<long>(q) * n + q], A[static_cast<long>(p) * n + q], c, s);
-      __syncthreads();   // every thread has read the 2x2 block before the rows change
-      if (threadIdx.x == 0) cs[blockIdx.x] = make_double2(c, s);
-      if (!live) return;
-      double* rp = A + static_cast<long>(p) * n;
-      double* rq = A + static_cast<long>(q) * n;
-      for (int j = threadIdx.x; j < n; j += blockDim.x) {
-        double a = rp[j], b = rq[j];
-        rp[j] = c * a - s * b;
-        rq[j] = s * a + c * b;
-      }
-    }
-
-    // Every row's two columns of every pair of the round.
-    __global__ void k_jacobi_cols(double* __restrict__ A, int n, int m, int round, double2 const* __restrict__ cs) {
-      long idx = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
-      long const npairs = m / 2;
-      if (idx >= npairs * n) return;
-      int k = static_cast<int>(idx / n);
-      long i = idx % n;
-      int p, q;
-      pair_of(round, k, m, p, q);
-      if (q >= n) return;
-      double2 r = cs[k];
-      double* row = A + i * n;
-      double a = row[p], b = row[q];
-      row[p] = r.x * a - r.y * b;
-      row[q] = r.y * a + r.x * b;
-    }
-
-    // Off-diagonal and total squared Frobenius norms, one block, fixed order.
-    __global__ void k_norms(double const* __restrict__ A, long n, double* __restrict__ out) {
-      __shared__ double so[NTB], st[NTB];
-      double o = 0, t = 0;
-      for (long idx = threadIdx.x; idx < n * n; idx += NTB) {
-        double v = A[idx];
-        t += v * v;
-        if (idx / n != idx % n) o += v * v;
-      }
-      so[threadIdx.x] = o;
-      st[threadIdx.x] = t;
+    // Block sums of two values, to every thread.
+    __device__ inline void sum2(double& x, double& y, double (*sh)[NTB / 64]) {
+      x = group_sum<64>(x);
+      y = group_sum<64>(y);
       __syncthreads();
-      for (int w = NTB / 2; w > 0; w >>= 1) {
-        if (threadIdx.x < w) {
-          so[threadIdx.x] += so[threadIdx.x + w];
-          st[threadIdx.x] += st[threadIdx.x + w];
-        }
-        __syncthreads();
+      if ((threadIdx.x & 63) == 0) {
+        sh[0][threadIdx.x >> 6] = x;
+        sh[1][threadIdx.x >> 6] = y;
       }
-      if (threadIdx.x == 0) {
-        out[0] = so[0];
-        out[1] = st[0];
+      __syncthreads();
+      x = y = 0;
+#pragma unroll
+      for (int w = 0; w < NTB / 64; ++w) {
+        x += sh[0][w];
+        y += sh[1][w];
       }
     }
 
-    __global__ void k_diag(double const* __restrict__ A, long n, double* __restrict__ d) {
-      long i = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
-      if (i < n) d[i] = A[i * n + i];
+    // Step k of the reduction.  A holds the block before reflection k - 1 is applied (its vector v, scale b and
+    // product p = A v are in vp, bt and pp); rows above k are done.  Every workgroup for itself: w = b p - (b^2 (p.v) / 2) v,
+    // row k of the updated block, its diagonal and the next reflection; then, a wavefront per row,
+    // A_ij -= v_i w_j + w_i v_j and the row's part of A v_new.  Row k itself is only read.
+    __global__ __launch_bounds__(NTB) void k_tridiag(double* __restrict__ A, long n, long k, double const* __restrict__ vp,
+                                                     double const* __restrict__ pp, double const* __restrict__ bt,
+                                                     double* __restrict__ vn, double* __restrict__ pn,
+                                                     double* __restrict__ bn, double* __restrict__ diag,
+                                                     double* __restrict__ off) {
+      __shared__ double sh[2][NTB / 64];
+      double const* Ak = A + k * n;
+      bool const first = k == 0;
+      double const b = first ? 0.0 : *bt;
+      double pv = 0, dummy = 0;
+      if (!first)
+        for (long j = k + threadIdx.x; j < n; j += NTB) pv += pp[j] * vp[j];
+      sum2(pv, dummy, sh);
+      double const kk = 0.5 * b * b * pv;
+      // v_j and w_j of the reflection before (zero at the first step).
+      auto vw = [&](long j, double& v, double& w) {
+        v = first ? 0.0 : vp[j];
+        w = first ? 0.0 : b * pp[j] - kk * v;
+      };
+      double vk, wk;
+      vw(k, vk, wk);
+      auto rowk = [&](long j, double& v, double& w) {
+        vw(j, v, w);
+        return Ak[j] - (vk * w + wk * v);
+      };
+      double ss = 0;
+      for (long j = k + 2 + threadIdx.x; j < n; j += NTB) {
+        double v, w;
+        double const x = rowk(j, v, w);
+        ss += x * x;
+      }
+      double zero = 0;
+      sum2(ss, zero, sh);
+      double v1, w1;
+      double const x1 = rowk(k + 1, v1, w1);
+      double alpha = x1, top = 0, beta = 0;
+      if (ss != 0.0) {
+        alpha = -copysign(sqrt(ss + x1 * x1), x1);
+        top = x1 - alpha;
+        beta = 2.0 / (ss + top * top);
+      }
+      auto next = [&](long j, double& v, double& w) {   // new reflection's vector (zero where there is none)
+        double const x = rowk(j, v, w);
+        return j == k + 1 ? top : (beta != 0.0 ? x : 0.0);
+      };
+      if (blockIdx.x == 0) {
+        if (threadIdx.x == 0) {
+          double v, w;
+          diag[k] = rowk(k, v, w);
+          off[k] = alpha;
+          *bn = beta;
+        }
+        for (long j = k + 1 + threadIdx.x; j < n; j += NTB) {
+          double v, w;
+          vn[j] = next(j, v, w);
+        }
+      }
+      int const lane = threadIdx.x & 63;
+      long const waves = static_cast<long>(gridDim.x) * (NTB / 64);
+      for (long i = k + 1 + blockIdx.x * (NTB / 64) + (threadIdx.x >> 6); i < n; i += waves) {
+        double vi, wi;
+        vw(i, vi, wi);
+        double* Ai = A + i * n;
+        double p = 0;
+        for (long j = k + 1 + lane; j < n; j += 64) {
+          double v, w;
+          double const x = next(j, v, w);
+          double const a = Ai[j] - (vi * w + wi * v);
+          Ai[j] = a;
+          p += a * x;
+        }
+        p = group_sum<64>(p);
+        if (lane == 0) pn[i] = p;
+      }
+    }
+
+    // The last 2 x 2 (or 1 x 1) block once no reflection is left.
+    __global__ void k_tridiag_end(double const* __restrict__ A, long n, double const* __restrict__ vp,
+                                  double const* __restrict__ pp, double const* __restrict__ bt, double* __restrict__ diag,
+                                  double* __restrict__ off) {
+      if (threadIdx.x) return;
+      long const k = n >= 2 ? n - 2 : 0;
+      bool const none = n < 3;
+      double const b = none ? 0.0 : *bt;
+      double pv = 0;
+      if (!none)
+        for (long j = k; j < n; ++j) pv += pp[j] * vp[j];
+      double const kk = 0.5 * b * b * pv;
+      for (long i = k; i < n; ++i) {
+        double const vi = none ? 0.0 : vp[i], wi = none ? 0.0 : b * pp[i] - kk * vi;
+        diag[i] = A[i * n + i] - 2.0 * (vi * wi);
+        if (i > k) {
+          double const v = none ? 0.0 : vp[k], w = none ? 0.0 : b * pp[k] - kk * v;
+          off[k] = A[k * n + i] - (vi * w + wi * v);
+        }
+      }
+    }
+
+    // Squares of the off-diagonal and Gershgorin bounds (one workgroup): lim = (low, high, least pivot).
+    __global__ __launch_bounds__(NTB) void k_bounds(double const* __restrict__ d, double const* __restrict__ off, long n,
+                                                    double* __restrict__ e2, double* __restrict__ lim) {
+      __shared__ double s0[NTB], s1[NTB], s2[NTB];
+      double lo = INFINITY, hi = -INFINITY, em = 0;
+      bool bad = false;
+      for (long i = threadIdx.x; i < n; i += NTB) {
+        double const l = i > 0 ? fabs(off[i - 1]) : 0.0, r = i + 1 < n ? fabs(off[i]) : 0.0;
+        double const a = d[i] - (l + r), z = d[i] + (l + r);
+        bad = bad || !isfinite(a) || !isfinite(z);
+        lo = fmin(lo, a);
+        hi = fmax(hi, z);
+        e2[i] = l * l;   // couples i - 1 and i
+        em = fmax(em, l * l);
+      }
+      s0[threadIdx.x] = bad ? NAN : lo;
+      s1[threadIdx.x] = hi;
+      s2[threadIdx.x] = em;
+      __syncthreads();
+      if (threadIdx.x) return;
+      for (int q = 1; q < NTB; ++q) {
+        s0[0] = isnan(s0[0]) || isnan(s0[q]) ? NAN : fmin(s0[0], s0[q]);
+        s1[0] = fmax(s1[0], s1[q]);
+        s2[0] = fmax(s2[0], s2[q]);
+      }
+      double const pad = 1e-15 * fmax(fabs(s0[0]), fabs(s1[0])) + 1e-300;
+      lim[0] = s0[0] - pad;
+      lim[1] = s1[0] + pad;
+      lim[2] = 2.3e-308 * fmax(1.0, s2[0]);
+    }
+
+    // Eigenvalue m of the tridiagonal matrix: one wavefront narrows its interval 65-fold per pass.  The number of
+    // negative terms of q_i = (d_i - x) - e_i^2 / q_{i-1} is the number of eigenvalues below x.
+    constexpr int STURM_PASSES = 9;   // 65^9 = 2^54: down to the rounding of the interval's own width
+
+    __global__ __launch_bounds__(NTB) void k_sturm(double const* __restrict__ d, double const* __restrict__ e2, long n,
+                                                   double const* __restrict__ lim, double* __restrict__ out) {
+      long const m = blockIdx.x * static_cast<long>(NTB / 64) + (threadIdx.x >> 6);
+      int const lane = threadIdx.x & 63;
+      if (m >= n) return;
+      double lo = lim[0], hi = lim[1];
+      double const piv = lim[2];
+      for (int pass = 0; pass < STURM_PASSES; ++pass) {
+        double const x = lo + (hi - lo) * (static_cast<double>(lane + 1) / 65.0);
+        double q = 1.0;
+        long below = 0;
+        for (long i = 0; i < n; ++i) {
+          q = (d[i] - x) - e2[i] / q;
+          if (fabs(q) <= piv) q = -piv;
+          below += q < 0 ? 1 : 0;
+        }
+        int const t = __popcll(__ballot(below <= m));   // points that eigenvalue m is not below
+        double const nlo = __shfl(x, t > 0 ? t - 1 : 0, 64), nhi = __shfl(x, t < 64 ? t : 63, 64);
+        if (t > 0) lo = nlo;
+        if (t < 64) hi = nhi;
+      }
+      if (lane == 0) out[m] = 0.5 * (lo + hi);
     }
 
     unsigned blocks(long n, int t) { return static_cast<unsigned>((n + t - 1) / t); }
@@ -146,7 +416,7 @@ namespace flyg {
   // Returns the sorted eigenvalues of the mass-weighted Hessian block of the non-frozen atoms.
   std::vector<double> hessian_eigenvalues(flyg_eam_s& E, flyg_list_s& nl, uint32_t const* d_types,
                                           uint8_t const* d_frozen, std::vector<uint8_t> const& h_frozen,
-                                          std::vector<uint32_t> const& h_types, int* sweeps_out) {
+                                          std::vector<uint32_t> const& h_types) {
     flyg_ctx_s& ctx = *E.ctx;
     hipStream_t st = ctx.stream;
     long const n = nl.n;
@@ -166,53 +436,73 @@ namespace flyg {
     long const n3m = static_cast<long>(dof.size());
     if (n3m == 0) return {};
     require(n3m <= 16384, "the Hessian block is limited to 16384 degrees of freedom");
-    DBuf<double> v, hv, H, rm, nrm, diag;
-    DBuf<long> ddof;
-    DBuf<double2> cs;
-    v.reserve(3 * n);
-    hv.reserve(3 * n);
-    H.reserve(n3m * n3m);
-    rm.reserve(n3m);
-    ddof.reserve(n3m);
-    nrm.reserve(2);
-    diag.reserve(n3m);
-    long const m = n3m + (n3m % 2);
-    cs.reserve(m / 2);
-    HIPCHK(hipMemsetAsync(v.get(), 0, 3 * n * sizeof(double), st));
-    HIPCHK(hipMemcpyAsync(ddof.get(), dof.data(), n3m * sizeof(long), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(rm.get(), rmass.data(), n3m * sizeof(double), hipMemcpyHostToDevice, st));
-    for (long c = 0; c < n3m; ++c) {
-      k_set<<<1, 1, 0, st>>>(v.get(), dof[c], 1.0);
-      eam_hvp(E, nl, d_types, d_frozen, v.get(), hv.get());
-      k_set<<<1, 1, 0, st>>>(v.get(), dof[c], 0.0);
-      k_gather_column<<<blocks(n3m, NTB), NTB, 0, st>>>(hv.get(), ddof.get(), rm.get(), n3m, c, H.get());
+    require(nl.built, "List used before rebuild");
+    require(E.tab.rc <= nl.rc, "r_cut is bigger than the internal r_cut of the list");
+    long const nm = n3m / 3;
+    PairArgs const A = pair_args(E, nl, d_types, d_frozen);
+    Shifts const S = shifts_of(nl.box);
+    unsigned* err = ctx.dflags.get();
+
+    // Mobile atoms, their neighbours (the rows of D) and F', F''.
+    std::vector<int> host(static_cast<std::size_t>(n + nm), -1);   // mobile index by atom, then the mobile atoms
+    for (long q = 0; q < nm; ++q) {
+      long const a = dof[3 * q] / 3;
+      host[a] = static_cast<int>(q);
+      host[n + q] = static_cast<int>(a);
     }
-    k_mirror_lower<<<blocks(n3m * n3m, NTB), NTB, 0, st>>>(H.get(), n3m);
+    E.hess_ids.reserve(3 * n + 1 + nm);
+    int* mob = E.hess_ids.get();
+    int* atoms = mob + n;
+    int* loc = atoms + nm;          // n + 1: marks, then their exclusive scan
+    int* region = loc + n + 1;      // up to n
+    HIPCHK(hipMemcpyAsync(mob, host.data(), host.size() * sizeof(int), hipMemcpyHostToDevice, st));
+    HIPCHK(hipMemsetAsync(loc, 0, (n + 1) * sizeof(int), st));
+    k_mark<<<blocks(nm * 64, NTB), NTB, 0, st>>>(A, atoms, nm, loc);
+    exclusive_scan(ctx, loc, static_cast<int>(n + 1), nl.scan_tmp);
+    k_region<<<blocks(n, NTB), NTB, 0, st>>>(loc, n, region);
+    HIPCHK(hipMemcpyAsync(ctx.hflags + 2, loc + n, sizeof(int), hipMemcpyDeviceToHost, st));
+    HIPCHK(hipStreamSynchronize(st));
+    long const nreg = static_cast<long>(ctx.hflags[2]);
+
+    // One workspace: H, D, (F', F'') by atom, 1 / sqrt(m), and eight vectors of the reduction.
+    std::size_t const need = static_cast<std::size_t>(n3m) * (n3m + nreg + 9) + 2 * n + 16;
+    DBuf<double> own;
+    bool const keep = need * sizeof(double) <= HESS_KEEP;
+    DBuf<double>& work = keep ? E.hess : own;
+    work.reserve(need);
+    double2* ff = reinterpret_cast<double2*>(work.get());
+    double* H = work.get() + 2 * n;
+    double* D = H + n3m * n3m;
+    double* rm = D + nreg * n3m;
+    double* v[2] = {rm + n3m, rm + 2 * n3m};
+    double* p[2] = {rm + 3 * n3m, rm + 4 * n3m};
+    double* diag = rm + 5 * n3m;
+    double* off = rm + 6 * n3m;
+    double* e2 = rm + 7 * n3m;
+    double* lam = rm + 8 * n3m;
+    double* bt[2] = {rm + 9 * n3m, rm + 9 * n3m + 1};
+    double* lim = rm + 9 * n3m + 2;
+    HIPCHK(hipMemcpyAsync(rm, rmass.data(), n3m * sizeof(double), hipMemcpyHostToDevice, st));
+    k_embed<8><<<blocks(n * 8, NTB), NTB, 0, st>>>(E.tab, S, A, ff, err);
+    k_drow<<<static_cast<unsigned>(nreg), NTB, 0, st>>>(E.tab, S, A, ff, region, mob, n3m, D, err);
+    k_hrow<<<static_cast<unsigned>(nm), NTB, 0, st>>>(E.tab, S, A, ff, atoms, mob, loc, rm, n3m, D, H, err);
+    k_mirror_lower<<<blocks(n3m * n3m, NTB), NTB, 0, st>>>(H, n3m);
+    for (long k = 0; k + 2 < n3m; ++k) {
+      long const rows = n3m - k - 1;
+      unsigned const g = static_cast<unsigned>(std::min<long>((rows + NTB / 64 - 1) / (NTB / 64), 512));
+      k_tridiag<<<g, NTB, 0, st>>>(H, n3m, k, v[k & 1], p[k & 1], bt[k & 1], v[(k + 1) & 1], p[(k + 1) & 1], bt[(k + 1) & 1],
+                                   diag, off);
+    }
+    k_tridiag_end<<<1, 64, 0, st>>>(H, n3m, v[n3m & 1], p[n3m & 1], bt[n3m & 1], diag, off);
+    k_bounds<<<1, NTB, 0, st>>>(diag, off, n3m, e2, lim);
+    k_sturm<<<blocks(n3m, NTB / 64), NTB, 0, st>>>(diag, e2, n3m, lim, lam);
     HIPCHK(hipGetLastError());
-    int sweeps = 0;
-    double hn[2];
-    for (; sweeps < 60; ++sweeps) {
-      k_norms<<<1, NTB, 0, st>>>(H.get(), n3m, nrm.get());
-      HIPCHK(hipMemcpyAsync(hn, nrm.get(), sizeof(hn), hipMemcpyDeviceToHost, st));
-      HIPCHK(hipStreamSynchronize(st));
-      if (!(hn[0] > 1e-28 * hn[1])) break;   // off-diagonal norm below 1e-14 of the matrix's
-      for (int r = 0; r < m - 1; ++r) {
-        k_jacobi_rows<<<static_cast<unsigned>(m / 2), NTB, 0, st>>>(H.get(), static_cast<int>(n3m), static_cast<int>(m), r,
-                                                                    cs.get());
-        k_jacobi_cols<<<blocks((m / 2) * n3m, NTB), NTB, 0, st>>>(H.get(), static_cast<int>(n3m), static_cast<int>(m), r,
-                                                                  cs.get());
-      }
-      HIPCHK(hipGetLastError());
-    }
-    require(sweeps < 60, "Jacobi sweeps did not converge");
     std::vector<double> w(n3m);
-    k_diag<<<blocks(n3m, NTB), NTB, 0, st>>>(H.get(), n3m, diag.get());
-    HIPCHK(hipMemcpyAsync(w.data(), diag.get(), n3m * sizeof(double), hipMemcpyDeviceToHost, st));
+    HIPCHK(hipMemcpyAsync(w.data(), lam, n3m * sizeof(double), hipMemcpyDeviceToHost, st));
     unsigned fl = ctx.take_flags();   // synchronises
     if (fl & ERR_SPLINE_OOB) throw Error(FLYG_SPLINE_OOB, "x is outside tabulated region of a spline");
     if (fl & ERR_TYPE) throw Error(FLYG_INVALID_ARG, "TypeID out of range");
     std::sort(w.begin(), w.end());
-    if (sweeps_out) *sweeps_out = sweeps;
     return w;
   }
 

@@ -64,6 +64,33 @@ def test_hessian_spectrum_vs_oracle(ctx, wen, frozen_radius):
         assert np.sum(np.abs(w) < 1e-6) == 3
 
 
+@pytest.mark.parametrize("species,mobile", [("wen", 1), ("wen", 2), ("wen", 22), ("Fe X", 1), ("Fe X", 43)])
+def test_spectrum_of_few_atoms(ctx, wen, species, mobile):
+    # Blocks of 3 (no reflection), 6, 66 and 129 coordinates (more than one wavefront, odd), one and two species.
+    # Bound: the reduction and the Sturm counts are backward stable, n x 1e-16 of the largest eigenvalue each.
+    if species == "wen":
+        pot, data = wen
+        pos, basis = vacancy_cell(6)
+        t = np.zeros(len(pos), np.uint32)
+    else:
+        path = systems.potential_path(("Fe", "X"))
+        pot, data = fa.EAM(ctx, path), po.DataEAM(path)
+        s = systems.fe_x_alloy(3, cells=6)
+        pos, basis, t = s.pos, s.basis, s.types
+    rng = np.random.default_rng(mobile)
+    pos = pos + rng.normal(0, 0.05, pos.shape)
+    f = np.ones(len(pos), np.uint8)
+    d = pos - pos[-1]
+    d -= np.diag(basis) * np.round(d / np.diag(basis))
+    f[np.argsort(np.einsum("ij,ij->i", d, d))[:mobile]] = 0
+    nl = fa.List(ctx, fa.Box(basis), pot.r_cut() + 0.3)
+    nl.rebuild(pos)
+    w = pot.hessian_eigenvalues(t, f, nl)
+    wo = oracle_block(data, basis, pos, t, f)
+    assert len(w) == 3 * mobile and np.all(np.diff(w) >= 0)
+    assert np.max(np.abs(w - wo)) <= 1e-12 * np.abs(wo).max()
+
+
 def test_saddle_spectrum_and_prefactor(ctx, wen):
     # The vacancy hop's saddle (found by the oracle's dimer from a nudge towards the vacancy) and the relaxed
     # minimum: one negative mode at the saddle, none at the minimum, three zero modes each; the prefactor
