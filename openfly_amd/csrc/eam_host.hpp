@@ -98,7 +98,8 @@ struct flyg_list_s {
   flyg::DBuf<double4> ent;       // reals + ghost images at build time (chained positions)
   flyg::DBuf<unsigned> eid;      // packed (shift, real) of ent
   flyg::DBuf<int> ecell;         // cell of ent
-  flyg::DBuf<int> ccount, cstart, ccursor;
+  flyg::DBuf<int> earr;          // its place in the cell in arrival order
+  flyg::DBuf<int> ccount, cstart;
   flyg::DBuf<double4> spos;      // ent sorted by cell (packed-id order inside a cell)
   flyg::DBuf<unsigned> usid;     // packed ids scattered by cell, unordered inside a cell
   flyg::DBuf<int> rslot;         // sorted slot of each real atom
@@ -118,7 +119,9 @@ struct flyg_list_s {
   flyg::DBuf<int> gcnt;
   flyg::DBuf<int> scan_tmp;
   flyg::DBuf<double> stage;      // host staging of xyz vectors
-  flyg::DBuf<unsigned> lstate;   // device build counters
+  flyg::DBuf<unsigned> lstate;   // device build counters: two sets, used in turn
+  int parity = 0;                // the set of the next build
+  bool counters_clear = false;   // ccount and that set are zero
   unsigned* hstate = nullptr;    // pinned mirror
   long gcap = 0;                 // ghost slots
   ~flyg_list_s() {
@@ -133,7 +136,10 @@ namespace flyg {
   // neigh.hip
   void list_rebuild(flyg_list_s& nl, double const* d_xyz, long n);
   void list_update(flyg_list_s& nl, double const* d_delta, long n);
-  void exclusive_scan(flyg_ctx_s& ctx, int* data, int n, flyg::DBuf<int>& tmp);
+  // Exclusive scan of src into dst (they may be the same; both hold scan_room(n) values, whatever lies past the
+  // n-th); clear_state: src and the four words there are zeroed.
+  constexpr long scan_room(long n) { return (n + 3) & ~3l; }
+  void exclusive_scan(flyg_ctx_s& ctx, int* src, int* dst, int n, flyg::DBuf<int>& tmp, unsigned* clear_state = nullptr);
 
   // eam.hip
   struct PairArgs {

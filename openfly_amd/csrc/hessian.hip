@@ -450,15 +450,16 @@ namespace flyg {
       host[a] = static_cast<int>(q);
       host[n + q] = static_cast<int>(a);
     }
-    E.hess_ids.reserve(3 * n + 1 + nm);
-    int* mob = E.hess_ids.get();
+    long const nloc = scan_room(n + 1);
+    E.hess_ids.reserve(2 * n + nloc + nm);
+    int* loc = E.hess_ids.get();    // n + 1: marks, then their exclusive scan
+    int* region = loc + nloc;       // up to n
+    int* mob = region + n;
     int* atoms = mob + n;
-    int* loc = atoms + nm;          // n + 1: marks, then their exclusive scan
-    int* region = loc + n + 1;      // up to n
     HIPCHK(hipMemcpyAsync(mob, host.data(), host.size() * sizeof(int), hipMemcpyHostToDevice, st));
     HIPCHK(hipMemsetAsync(loc, 0, (n + 1) * sizeof(int), st));
     k_mark<<<blocks(nm * 64, NTB), NTB, 0, st>>>(A, atoms, nm, loc);
-    exclusive_scan(ctx, loc, static_cast<int>(n + 1), nl.scan_tmp);
+    exclusive_scan(ctx, loc, loc, static_cast<int>(n + 1), nl.scan_tmp);
     k_region<<<blocks(n, NTB), NTB, 0, st>>>(loc, n, region);
     HIPCHK(hipMemcpyAsync(ctx.hflags + 2, loc + n, sizeof(int), hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));

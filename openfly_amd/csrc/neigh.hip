@@ -1,12 +1,16 @@
 // Neighbour-list build and update on gfx950 (replaces neigh::List, list.cpp:37-165).
 //
 // Rebuild pipeline (all on the device, one HIP stream):
-//   1. canonicalise real positions                       (List::rebuild copy-in, list.cpp:68-72)
-//   2. ghost images, axis by axis, chained               (List::make_ghosts, list.cpp:100-132)
-//   3. counting-sort binning of reals + ghosts into the HyperGrid cells (atomic histogram, exclusive
-//      scan, scatter, then each cell sorted by packed id so the result does not depend on atomics)
-//   4. one thread per real atom scans its 27 cells and appends every (real, image) with d^2 < r_cut^2
-//      (strict, list.cpp:146,159) to its row of an ELL table: n rows x K packed 32-bit entries.
+//   1. k_entries: canonical real positions (List::rebuild copy-in, list.cpp:68-72) and their ghost images
+//      (List::make_ghosts, list.cpp:100-132)
+//   2. k_cell_count: the HyperGrid cell of each, counted with atomics whose return value is the entry's
+//      place in arrival order
+//   3. exclusive scan of the cell counts (which clears them for the next build)
+//   4. scatter of the packed ids by cell, then each cell sorted by packed id, so the result does not
+//      depend on the atomics
+//   5. k_build_rows: every (real, image) of an atom's 27 cells with d^2 < r_cut^2 (strict,
+//      list.cpp:146,159) goes to its row of an ELL table: n rows x K packed 32-bit entries.
+// Six launches and one synchronisation; the state the host needs is written to pinned memory.
 // The distance tests, canonical images and ghost chains round exactly like the reference's FP64
 // expressions (no FMA contraction), so the pair sets equal the reference's at rebuild time.
 // Ghosts are not kept after the build: an entry stores (shift code, real index) and the pair kernels
@@ -164,52 +168,45 @@ namespace flyg {
     // lstate[0] ghosts generated, [1] longest row, [3] overflow bits.
     enum : unsigned { OV_GHOST = 1u };
 
-    // Canonical images of the reals; the same launch clears the build's counters (cell counts za[0..na),
-    // cell cursors zb[0..nb), the four state words), which only later kernels of the build use.
-    __global__ void k_canon_reals(BoxDesc b, double const* __restrict__ xyz, long n, double4* __restrict__ pos,
-                                  double4* __restrict__ ent, unsigned* __restrict__ eid, int* __restrict__ za, long na,
-                                  int* __restrict__ zb, long nb, unsigned* __restrict__ st) {
-      long i = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
-      if (i < na) za[i] = 0;
-      if (i < nb) zb[i] = 0;
-      if (i < 4) st[i] = 0u;
-      if (i >= n) return;
-      double x[3] = {xyz[3 * i], xyz[3 * i + 1], xyz[3 * i + 2]};
-      canon_image(b, x);
-      double4 p = make_double4(x[0], x[1], x[2], 0.0);
-      pos[i] = p;
-      ent[i] = p;
-      eid[i] = (13u << NB_SHIFT_BITS) | static_cast<unsigned>(i);
-    }
+    // Slots for g images per thread, one atomic per workgroup of ETPB threads (prefix sums of the lanes' counts and
+    // of the wavefronts' totals): the counter is one address, and an atomic per wavefront on it took 100 us
+    // at a million atoms.  Slot order is free: the rank placement sorts every cell by packed id
+    // afterwards.  Every thread of the workgroup must call it.
+    constexpr int ETPB = 1024;
 
-    // Slots for g images per lane, one atomic per wavefront (a prefix sum of the lanes' counts): one per
-    // atom on the single counter serialises the kernel.  Slot order is free: the rank placement sorts
-    // every cell by packed id afterwards.  Every lane of the wavefront must call it.
     __device__ inline unsigned ghost_slots(unsigned g, unsigned* st) {
-      int const wl = static_cast<int>(threadIdx.x & 63);
+      __shared__ unsigned wsum[ETPB / 64];
+      __shared__ unsigned wbase;
+      int const wl = static_cast<int>(threadIdx.x & 63), w = static_cast<int>(threadIdx.x >> 6);
       unsigned incl = g;
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) {
         unsigned t = __shfl_up(incl, o, 64);
         if (wl >= o) incl += t;
       }
-      unsigned const total = __shfl(incl, 63, 64);
-      unsigned wbase = 0;
-      if (wl == 63 && total > 0) wbase = atomicAdd(&st[0], total);
-      wbase = __shfl(wbase, 63, 64);
-      return wbase + (incl - g);
+      if (wl == 63) wsum[w] = incl;
+      __syncthreads();
+      if (threadIdx.x == 0) {
+        unsigned total = 0;
+        for (int q = 0; q < ETPB / 64; ++q) total += wsum[q];
+        wbase = total > 0 ? atomicAdd(&st[0], total) : 0u;
+      }
+      __syncthreads();
+      unsigned before = wbase;
+      for (int q = 0; q < w; ++q) before += wsum[q];
+      return before + (incl - g);
     }
 
     // The reference's chain of gen_image calls (any box): images of images, axis by axis.
-    __device__ inline void ghosts_chain(BoxDesc const& b, double rc, double4 const& p, bool inr, long i, long n,
+    __device__ inline void ghosts_chain(BoxDesc const& b, GridDesc const& g, double const* x, bool inr, long i, long n,
                                         double4* __restrict__ ent, unsigned* __restrict__ eid, unsigned* __restrict__ st,
                                         long gcap) {
       double cx[27][3];
       int cs[27];
       int m = 1;
-      cx[0][0] = p.x;
-      cx[0][1] = p.y;
-      cx[0][2] = p.z;
+      cx[0][0] = x[0];
+      cx[0][1] = x[1];
+      cx[0][2] = x[2];
       cs[0] = 13;
       int const pow3[3] = {1, 3, 9};
       for (int ax = 0; ax < 3 && inr; ++ax) {
@@ -218,7 +215,7 @@ namespace flyg {
         for (int sgn = 1; sgn >= -1; sgn -= 2) {
           for (int c = 0; c < end; ++c) {
             double im[3] = {cx[c][0], cx[c][1], cx[c][2]};
-            if (gen_image(b, rc, sgn, im, ax)) {
+            if (gen_image(b, g.rc, sgn, im, ax)) {
               cx[m][0] = im[0];
               cx[m][1] = im[1];
               cx[m][2] = im[2];
@@ -228,11 +225,10 @@ namespace flyg {
           }
         }
       }
-      unsigned const g = static_cast<unsigned>(m - 1);
-      unsigned const base = ghost_slots(g, st);
-      if (g == 0) return;
+      unsigned const ng = static_cast<unsigned>(m - 1);
+      unsigned const base = ghost_slots(ng, st);
       for (int k = 1; k < m; ++k) {
-        long slot = static_cast<long>(base) + (k - 1);
+        long const slot = static_cast<long>(base) + (k - 1);
         if (slot >= gcap) {
           atomicOr(&st[3], static_cast<unsigned>(OV_GHOST));
           return;
@@ -242,63 +238,67 @@ namespace flyg {
       }
     }
 
-    // make_ghosts with a fixed capacity; the counter keeps counting past it so the host can resize.
-    // Launched with whole wavefronts.  Orthorhombic boxes: whether an axis contributes a +1 / -1 image
-    // depends only on the atom's own coordinate on that axis, so the images are the product of the
+    // Reals and ghosts (capacity gcap; the counter keeps counting past it so the host can resize).  Launched with whole wavefronts.  Orthorhombic boxes: whether an axis contributes a
+    // +1 / -1 image depends only on the atom's own coordinate on that axis, so the images are the product of the
     // per-axis choices (the same set, and the same coordinates, as the reference's chain) and live in
     // registers; other boxes follow the chain of gen_image calls.  One instantiation per box kind: the
     // chain's per-lane arrays live in scratch memory, which the orthorhombic form does not need.
     template <bool ORTHO>
-    __global__ void k_ghosts_cap(BoxDesc b, double rc, double4 const* __restrict__ pos, long n, double4* __restrict__ ent,
-                                 unsigned* __restrict__ eid, unsigned* __restrict__ st, long gcap) {
-      long i = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
+    __global__ __launch_bounds__(ETPB) void k_entries(BoxDesc b, GridDesc g, double const* __restrict__ xyz, long n, double4* __restrict__ pos,
+                              double4* __restrict__ ent, unsigned* __restrict__ eid, unsigned* __restrict__ st,
+                              long gcap) {
+      long const i = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
       bool const inr = i < n;
-      double4 p = inr ? pos[i] : make_double4(0.0, 0.0, 0.0, 0.0);
+      double x[3] = {0, 0, 0};
+      if (inr) {
+        x[0] = xyz[3 * i];
+        x[1] = xyz[3 * i + 1];
+        x[2] = xyz[3 * i + 2];
+        canon_image(b, x);
+        double4 const p = make_double4(x[0], x[1], x[2], 0.0);
+        pos[i] = p;
+        ent[i] = p;
+        eid[i] = (13u << NB_SHIFT_BITS) | static_cast<unsigned>(i);
+      }
       if constexpr (ORTHO) {
-        double const x[3] = {p.x, p.y, p.z};
         bool up[3], dn[3];
-        unsigned g = 1;
+        unsigned ng = inr ? 1 : 0;
 #pragma unroll
         for (int ax = 0; ax < 3; ++ax) {
-          up[ax] = inr && b.per[ax] && x[ax] < rc;
-          dn[ax] = inr && b.per[ax] && x[ax] > b.ext[ax] - rc;
-          g *= 1u + (up[ax] ? 1u : 0u) + (dn[ax] ? 1u : 0u);
+          up[ax] = inr && b.per[ax] && x[ax] < g.rc;
+          dn[ax] = inr && b.per[ax] && x[ax] > b.ext[ax] - g.rc;
+          ng *= 1u + (up[ax] ? 1u : 0u) + (dn[ax] ? 1u : 0u);
         }
-        g -= 1u;
-        unsigned const base = ghost_slots(g, st);
-        if (g == 0) return;
+        ng = inr ? ng - 1u : 0u;
+        unsigned const base = ghost_slots(ng, st);
+        if (ng == 0) return;
         unsigned k = 0;
-#pragma unroll
-        for (int s2 = -1; s2 <= 1; ++s2)
-#pragma unroll
-          for (int s1 = -1; s1 <= 1; ++s1)
-#pragma unroll
-            for (int s0 = -1; s0 <= 1; ++s0) {
-              if (s0 == 0 && s1 == 0 && s2 == 0) continue;
-              bool const use = (s0 == 0 || (s0 > 0 ? up[0] : dn[0])) && (s1 == 0 || (s1 > 0 ? up[1] : dn[1])) &&
-                               (s2 == 0 || (s2 > 0 ? up[2] : dn[2]));
-              if (!use) continue;
-              long const slot = static_cast<long>(base) + k;
-              ++k;
-              if (slot >= gcap) {
-                atomicOr(&st[3], static_cast<unsigned>(OV_GHOST));
-                return;
-              }
-              double im[3] = {x[0], x[1], x[2]};
-              {
+        for (int code = 0; code < 27; ++code) {
+          int const s0 = code % 3 - 1, s1 = code / 3 % 3 - 1, s2 = code / 9 - 1;
+          bool const use = (s0 == 0 || (s0 > 0 ? up[0] : dn[0])) && (s1 == 0 || (s1 > 0 ? up[1] : dn[1])) &&
+                           (s2 == 0 || (s2 > 0 ? up[2] : dn[2]));
+          if (code == 13 || !use) continue;
+          long const slot = static_cast<long>(base) + k;
+          ++k;
+          if (slot >= gcap) {
+            atomicOr(&st[3], static_cast<unsigned>(OV_GHOST));
+            return;
+          }
+          double im[3] = {x[0], x[1], x[2]};
+          {
 #pragma clang fp contract(off)
-                if (s0 > 0) im[0] += b.ext[0];
-                if (s0 < 0) im[0] -= b.ext[0];
-                if (s1 > 0) im[1] += b.ext[1];
-                if (s1 < 0) im[1] -= b.ext[1];
-                if (s2 > 0) im[2] += b.ext[2];
-                if (s2 < 0) im[2] -= b.ext[2];
-              }
-              ent[n + slot] = make_double4(im[0], im[1], im[2], 0.0);
-              eid[n + slot] = (static_cast<unsigned>(shift_code(s0, s1, s2)) << NB_SHIFT_BITS) | static_cast<unsigned>(i);
-            }
+            if (s0 > 0) im[0] += b.ext[0];
+            if (s0 < 0) im[0] -= b.ext[0];
+            if (s1 > 0) im[1] += b.ext[1];
+            if (s1 < 0) im[1] -= b.ext[1];
+            if (s2 > 0) im[2] += b.ext[2];
+            if (s2 < 0) im[2] -= b.ext[2];
+          }
+          ent[n + slot] = make_double4(im[0], im[1], im[2], 0.0);
+          eid[n + slot] = (static_cast<unsigned>(code) << NB_SHIFT_BITS) | static_cast<unsigned>(i);
+        }
       } else {
-        ghosts_chain(b, rc, p, inr, i, n, ent, eid, st, gcap);
+        ghosts_chain(b, g, x, inr, i, n, ent, eid, st, gcap);
       }
     }
 
@@ -307,11 +307,13 @@ namespace flyg {
       return n + (g < gcap ? g : gcap);
     }
 
-    // Entries per cell in cnt[0 .. nc1), real atoms per cell in cnt[nc1 .. 2 nc1) (one scan of both gives
-    // the cell starts and, less the first half's total, the first slot of each cell's reals).
-    __global__ void k_cell_count_cap(GridDesc g, double4 const* __restrict__ ent, long n, long gcap,
-                                     unsigned const* __restrict__ st, int* __restrict__ ecell, int* __restrict__ cnt,
-                                     long nc1) {
+    // Cell of every entry and its place in the cell in arrival order.  Counts: cnt[c] entries of cell c,
+    // cnt[nc1 + c] real ones (one scan of both gives the cell starts and, less the first half's total, the
+    // first slot of each cell's reals).  A launch of its own: inside k_entries a corner atom's 26 ghosts would wait
+    // for one atomic's return after the other (28 us instead of 6 + 7 at 54.5k atoms).
+    __global__ void k_cell_count(GridDesc g, double4 const* __restrict__ ent, long n, long gcap,
+                                 unsigned const* __restrict__ st, int* __restrict__ ecell, int* __restrict__ earr,
+                                 int* __restrict__ cnt, long nc1) {
       long e = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
       if (e >= live_entries(st, n, gcap)) return;
       double4 p = ent[e];
@@ -319,18 +321,17 @@ namespace flyg {
       int c3[3];
       int c = cell_idx(g, x, c3);
       ecell[e] = c;
-      atomicAdd(&cnt[c], 1);
       if (e < n) atomicAdd(&cnt[nc1 + c], 1);
+      earr[e] = atomicAdd(&cnt[c], 1);
     }
 
     // Counting-sort scatter of the packed ids only (order inside a cell follows the atomics).
-    __global__ void k_scatter_ids(unsigned const* __restrict__ eid, int const* __restrict__ ecell, long n, long gcap,
-                                  unsigned const* __restrict__ st, int const* __restrict__ cstart, int* __restrict__ cursor,
-                                  unsigned* __restrict__ usid) {
+    __global__ void k_scatter_ids(unsigned const* __restrict__ eid, int const* __restrict__ ecell,
+                                  int const* __restrict__ earr, long n, long gcap, unsigned const* __restrict__ st,
+                                  int const* __restrict__ cstart, unsigned* __restrict__ usid) {
       long e = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
       if (e >= live_entries(st, n, gcap)) return;
-      int c = ecell[e];
-      usid[cstart[c] + atomicAdd(&cursor[c], 1)] = eid[e];
+      usid[cstart[ecell[e]] + earr[e]] = eid[e];
     }
 
     // Places every entry at cell start + its rank among the cell's packed ids: cells come out sorted by
@@ -365,92 +366,180 @@ namespace flyg {
       }
     }
 
-    // List::build_neigh_list (list.cpp:134-165): BL lanes per real atom walk the 3x3x3 block of cells
-    // around it (z outermost, x innermost; each cell in packed-id order) with the strict r < r_c test
-    // of the reference; the lanes split each cell and write their hits in candidate order (ballot +
-    // prefix count), so a row is the same sequence a single thread would produce.
-    constexpr int BL = 8;
-    constexpr int BU = 4;   // candidate chunks loaded per step of the row build
+    // List::build_neigh_list (list.cpp:134-165): a wavefront walks the 3x3x3 block of cells around A
+    // consecutive slots (atoms in cell order) with the strict r < r_c test of the reference, z outermost, x
+    // innermost, each cell in packed-id order.  The up-to-three x-neighbouring cells of a (y, z) line are
+    // consecutive cells (x fastest), so their sorted atoms are one contiguous range: 9 ranges, whose ends the
+    // first nine lanes fetch at once.  A range holds 36 to 60 candidates in a metal at these cut-offs, one
+    // coalesced chunk of 64; the chunks of three ranges are loaded before the first is tested, and hits are
+    // taken in candidate order (ballot + prefix count), so a row is the sequence a single thread would produce.
+    // A chunk yields about eight hits: they wait in a ring in LDS until 64 of them leave as one coalesced store.
+    // Slots of one cell share the candidates' loads; a wavefront whose slots straddle cells walks each
+    // cell's block in turn.
+    // Small systems are bound by the chain of loads (A = 1: every atom a wavefront), large ones by the
+    // candidates' L1 lookups (A = 4 loads them a quarter as often); BUILD_WIDE is where the two cross.
+    //
+    // Each row is written twice: by atom with atom indices (nbr) and by slot with slot indices (grow, the
+    // gradient layout).  hst (pinned): [0] ghosts, [1] set when a row overflowed, [3] overflow bits.
+    constexpr long BUILD_WIDE = 24000;
 
-    // Atoms are taken in slot (cell) order, so a workgroup's candidates overlap; each row is written
-    // twice: by atom with atom indices (nbr) and by slot with slot indices (grow, the gradient layout).
-    __global__ void k_build_rows(GridDesc g, double4 const* __restrict__ spos, unsigned const* __restrict__ sid,
-                                 int const* __restrict__ cstart, int const* __restrict__ rslot, long n,
-                                 unsigned* __restrict__ nbr, int* __restrict__ ncnt, int K, unsigned* __restrict__ st,
-                                 int const* __restrict__ order, int const* __restrict__ rank_of,
-                                 unsigned* __restrict__ grow, int* __restrict__ gcnt) {
-      long gid = xcd_block(blockIdx.x, gridDim.x) * static_cast<long>(blockDim.x) + threadIdx.x;
-      long const slot = gid / BL;
-      int const lane = static_cast<int>(gid % BL);
-      if (slot >= n) return;   // whole groups leave together (blockDim is a multiple of BL)
-      long const i = order[slot];
-      int const gbase = static_cast<int>(threadIdx.x & 63) - lane;
-      int const self = rslot[i];
-      double4 p = spos[self];
-      double xi[3] = {p.x, p.y, p.z};
-      int c3[3];
-      cell_idx(g, xi, c3);
+    template <int A>
+    __global__ __launch_bounds__(TPB) void k_build_rows(GridDesc g, double4 const* __restrict__ spos,
+                                                        unsigned const* __restrict__ sid, int const* __restrict__ cstart,
+                                                        int const* __restrict__ rslot, long n, unsigned* __restrict__ nbr,
+                                                        int* __restrict__ ncnt, int K, unsigned* __restrict__ st,
+                                                        int const* __restrict__ order, int const* __restrict__ rank_of,
+                                                        unsigned* __restrict__ grow, int* __restrict__ gcnt,
+                                                        unsigned* __restrict__ hst) {
+      if (blockIdx.x == 0 && threadIdx.x == 0) {
+        hst[0] = st[0];
+        hst[3] = st[3];
+      }
+      int const lane = static_cast<int>(threadIdx.x & 63);
+      int const wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+      long const slot0 = (xcd_block(blockIdx.x, gridDim.x) * static_cast<long>(TPB / 64) + wave) * A;
+      if (slot0 >= n) return;   // whole wavefronts leave together
+      int const na = static_cast<int>(min(static_cast<long>(A), n - slot0));
+      __shared__ unsigned ring[TPB / 64][A][128];
       double const rc2 = g.rc * g.rc;
-      int cnt = 0;
-      unsigned* row = nbr + i * static_cast<long>(K);
-      unsigned* srow = grow + slot * static_cast<long>(K);
-      // The up-to-three x-neighbouring cells of a (y, z) line are consecutive cells (x fastest), so their
-      // sorted atoms form one contiguous range: 9 ranges instead of 27 cells, in the same order.  Each
-      // step loads BU chunks of BL candidates (positions and packed ids) before testing them, then the
-      // slots of all its hits, then writes the hits in order (more loads in flight, the same rows).
-      int const x0 = max(c3[0] - 1, 0), x1 = min(c3[0] + 2, g.shape[0]);
-      for (int z = max(c3[2] - 1, 0); z < min(c3[2] + 2, g.shape[2]); ++z)
-        for (int y = max(c3[1] - 1, 0); y < min(c3[1] + 2, g.shape[1]); ++y) {
-          int const line = y * g.prod[1] + z * g.prod[2];
-          int const b = cstart[x0 * g.prod[0] + line], end = cstart[(x1 - 1) * g.prod[0] + line + 1];
-          for (int s0 = b; s0 < end; s0 += BU * BL) {
-            bool hit[BU];
-            unsigned en[BU];
+      int atom[A], self[A], cell[A], cx[A], cy[A], cz[A], cnt[A];
+      double xi[A][3];
 #pragma unroll
-            for (int u = 0; u < BU; ++u) {
-              int const s = s0 + u * BL + lane;
-              hit[u] = false;
-              en[u] = 0;
-              if (s < end && s != self) {
-                double4 q = spos[s];
-                en[u] = sid[s];
-                double xn[3] = {q.x, q.y, q.z};
-                hit[u] = dist2(xi, xn) < rc2;
-              }
+      for (int a = 0; a < A; ++a) {
+        atom[a] = order[slot0 + min(a, na - 1)];
+        self[a] = rslot[atom[a]];
+      }
+#pragma unroll
+      for (int a = 0; a < A; ++a) {
+        double4 const p = spos[self[a]];
+        xi[a][0] = p.x;
+        xi[a][1] = p.y;
+        xi[a][2] = p.z;
+        int c3[3];
+        cell[a] = cell_idx(g, xi[a], c3);
+        cx[a] = c3[0];
+        cy[a] = c3[1];
+        cz[a] = c3[2];
+        cnt[a] = 0;
+      }
+      // Entries [k0, k0 + 64) of slot a's row, those below `c` (a wavefront runs in lockstep: its LDS accesses
+      // need no barrier, only their program order).
+      auto flush = [&](int a, int k0, int c) {
+        int const k = k0 + lane;
+        __builtin_amdgcn_wave_barrier();
+        if (k < c && k < K) {
+          unsigned const en = ring[wave][a][k & 127];
+          nbr[atom[a] * static_cast<long>(K) + k] = en;
+          grow[(slot0 + a) * K + k] = (en & ~NB_IDX_MASK) | static_cast<unsigned>(rank_of[en & NB_IDX_MASK]);
+        }
+        __builtin_amdgcn_wave_barrier();
+      };
+      int done = 0;   // slots whose rows are written
+      while (done < na) {
+        int c0 = cell[0], x = cx[0], y0 = cy[0], z0 = cz[0];
+#pragma unroll
+        for (int a = 1; a < A; ++a)
+          if (a == done) {
+            c0 = cell[a];
+            x = cx[a];
+            y0 = cy[a];
+            z0 = cz[a];
+          }
+        int rb = 0, re = 0;   // lane l < 9: range l
+        if (lane < 9) {
+          int const y = y0 - 1 + lane % 3, z = z0 - 1 + lane / 3;
+          if (y >= 0 && y < g.shape[1] && z >= 0 && z < g.shape[2]) {
+            int const line = y * g.prod[1] + z * g.prod[2];
+            rb = cstart[max(x - 1, 0) * g.prod[0] + line];
+            re = cstart[min(x + 1, g.shape[0] - 1) * g.prod[0] + line + 1];
+          }
+        }
+        auto test = [&](double4 const& q, unsigned en, int s) {
+          double const xn[3] = {q.x, q.y, q.z};   // far away on lanes without a candidate
+#pragma unroll
+          for (int a = 0; a < A; ++a) {
+            if (a >= na || cell[a] != c0) continue;
+            bool const hit = s != self[a] && dist2(xi[a], xn) < rc2;
+            unsigned long long const m = __ballot(hit);
+            int const before = __builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(m >> 32),
+                                                         __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(m), 0u));
+            if (hit) ring[wave][a][(cnt[a] + before) & 127] = en;
+            int const c = cnt[a] + __popcll(m);
+            if ((c ^ cnt[a]) & ~63) flush(a, cnt[a] & ~63, c & ~63);   // a block of 64 is full
+            cnt[a] = c;
+          }
+        };
+        for (int z = 0; z < 3; ++z) {
+          int b[3], e[3];
+          double4 q[3];
+          unsigned en[3];
+#pragma unroll
+          for (int u = 0; u < 3; ++u) {
+            b[u] = __builtin_amdgcn_readlane(rb, 3 * z + u);
+            e[u] = __builtin_amdgcn_readlane(re, 3 * z + u);
+            int const s = b[u] + lane;
+            en[u] = 0;
+            q[u] = make_double4(1e200, 0.0, 0.0, 0.0);
+            if (s < e[u]) {
+              q[u] = spos[s];
+              en[u] = sid[s];
             }
-            int rk[BU];
+          }
 #pragma unroll
-            for (int u = 0; u < BU; ++u) rk[u] = hit[u] ? rank_of[en[u] & NB_IDX_MASK] : 0;
-#pragma unroll
-            for (int u = 0; u < BU; ++u) {
-              unsigned long long m = __ballot(hit[u]);
-              unsigned gm = static_cast<unsigned>((m >> gbase) & ((1ull << BL) - 1ull));
-              if (hit[u]) {
-                int k = cnt + __popc(gm & ((1u << lane) - 1u));
-                if (k < K) {
-                  row[k] = en[u];
-                  srow[k] = (en[u] & ~NB_IDX_MASK) | static_cast<unsigned>(rk[u]);
-                }
+          for (int u = 0; u < 3; ++u) {
+            test(q[u], en[u], b[u] + lane);
+            for (int s0 = b[u] + 64; s0 < e[u]; s0 += 64) {   // the rest of a long range
+              int const s = s0 + lane;
+              double4 c = make_double4(1e200, 0.0, 0.0, 0.0);
+              unsigned id = 0;
+              if (s < e[u]) {
+                c = spos[s];
+                id = sid[s];
               }
-              cnt += __popc(gm);
+              test(c, id, s);
             }
           }
         }
-      if (lane == 0) {
-        ncnt[i] = cnt;
-        gcnt[slot] = cnt;
+        int next = na;   // the first later slot of another cell (slots are in cell order)
+#pragma unroll
+        for (int a = A - 1; a > 0; --a)
+          if (a > done && a < na && cell[a] != c0) next = a;
+        done = next;
+      }
+#pragma unroll
+      for (int a = 0; a < A; ++a)
+        if (a < na) flush(a, cnt[a] & ~63, cnt[a]);
+      if (lane < A && lane < na) {
+        int c = cnt[0], i = atom[0];
+#pragma unroll
+        for (int a = 1; a < A; ++a)
+          if (a == lane) {
+            c = cnt[a];
+            i = atom[a];
+          }
+        ncnt[i] = c;
+        gcnt[slot0 + lane] = c;
         // Only overflowing rows report their length (the host widens the rows to the longest one): an
         // atomic per atom on the one counter serialised the kernel (half of its time).
-        if (cnt > K) atomicMax(&st[1], static_cast<unsigned>(cnt));
+        if (c > K) {
+          atomicMax(&st[1], static_cast<unsigned>(c));
+          hst[1] = 1u;
+        }
       }
     }
 
     constexpr int SCAN_B = 1024;
 
-    __global__ void k_scan_block(int* __restrict__ data, int n, int* __restrict__ sums) {
+    // First level of an exclusive scan of src into dst (which may be src); clear: src is zeroed, and so are
+    // the four words at cst.
+    __global__ void k_scan_block(int* src, int* dst, int n, int* __restrict__ sums, bool clear, unsigned* cst) {
       __shared__ int wsum[SCAN_B / 64];
       int gi = blockIdx.x * SCAN_B + threadIdx.x;
-      int v = gi < n ? data[gi] : 0;
+      int v = gi < n ? src[gi] : 0;
+      if (clear) {
+        if (gi < n) src[gi] = 0;
+        if (gi < 4) cst[gi] = 0u;
+      }
       int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
       int inc = v;
 #pragma unroll
@@ -471,21 +560,37 @@ namespace flyg {
       }
       __syncthreads();
       int before = (w > 0 ? wsum[w - 1] : 0) + inc - v;
-      if (gi < n) data[gi] = before;
+      if (gi < n) dst[gi] = before;
       if (threadIdx.x == SCAN_B - 1) sums[blockIdx.x] = wsum[SCAN_B / 64 - 1];
     }
 
-    // Exclusive scan of up to SCAN_B * SCAN_RUN values in one workgroup: thread t owns a run of
-    // consecutive values, the runs' totals are scanned across the block, then each run is written out.
+    // Exclusive scan of up to SCAN_B * SCAN_RUN values in one workgroup: thread t owns a run of `per`
+    // consecutive values (a multiple of four, kept in registers), the runs' totals are scanned across the block.
+    // Both arrays hold scan_room(n) values and are 16-byte aligned: a run is read and written four values at a time.
     constexpr int SCAN_RUN = 16;
 
-    __global__ void k_scan_one(int* __restrict__ data, int n) {
+    __global__ __launch_bounds__(SCAN_B) void k_scan_one(int* src, int* dst, int n, bool clear, unsigned* cst) {
       __shared__ int wsum[SCAN_B / 64];
-      int const per = (n + SCAN_B - 1) / SCAN_B;
+      int const per = ((n + SCAN_B - 1) / SCAN_B + 3) & ~3;
       int const b = static_cast<int>(threadIdx.x) * per;
-      int const e = min(n, b + per);
+      int val[SCAN_RUN];
       int v = 0;
-      for (int q = b; q < e; ++q) v += data[q];
+#pragma unroll
+      for (int q = 0; q < SCAN_RUN; q += 4) {
+        int4 t = make_int4(0, 0, 0, 0);
+        if (q < per && b + q < n) t = *reinterpret_cast<int4 const*>(src + b + q);
+        val[q] = t.x;
+        val[q + 1] = b + q + 1 < n ? t.y : 0;
+        val[q + 2] = b + q + 2 < n ? t.z : 0;
+        val[q + 3] = b + q + 3 < n ? t.w : 0;
+        v += val[q] + val[q + 1] + val[q + 2] + val[q + 3];
+      }
+      if (clear) {
+#pragma unroll
+        for (int q = 0; q < SCAN_RUN; q += 4)
+          if (q < per && b + q < n) *reinterpret_cast<int4*>(src + b + q) = make_int4(0, 0, 0, 0);
+        if (threadIdx.x < 4) cst[threadIdx.x] = 0u;
+      }
       int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
       int inc = v;
 #pragma unroll
@@ -506,10 +611,15 @@ namespace flyg {
       }
       __syncthreads();
       int run = (w > 0 ? wsum[w - 1] : 0) + inc - v;
-      for (int q = b; q < e; ++q) {
-        int const x = data[q];
-        data[q] = run;
-        run += x;
+#pragma unroll
+      for (int q = 0; q < SCAN_RUN; q += 4) {
+        int4 t;
+        t.x = run;
+        t.y = t.x + val[q];
+        t.z = t.y + val[q + 1];
+        t.w = t.z + val[q + 2];
+        run = t.w + val[q + 3];
+        if (q < per && b + q < n) *reinterpret_cast<int4*>(dst + b + q) = t;
       }
     }
 
@@ -522,10 +632,11 @@ namespace flyg {
 
   }  // namespace
 
-  void exclusive_scan(flyg_ctx_s& ctx, int* data, int n, DBuf<int>& tmp) {
+  void exclusive_scan(flyg_ctx_s& ctx, int* src, int* dst, int n, DBuf<int>& tmp, unsigned* clear_state) {
     if (n <= 0) return;
+    bool const clear = clear_state != nullptr;
     if (n <= SCAN_B * SCAN_RUN) {   // one launch: each launch in a stream costs several microseconds
-      k_scan_one<<<1, SCAN_B, 0, ctx.stream>>>(data, n);
+      k_scan_one<<<1, SCAN_B, 0, ctx.stream>>>(src, dst, n, clear, clear_state);
       HIPCHK(hipGetLastError());
       return;
     }
@@ -543,11 +654,12 @@ namespace flyg {
     }
     tmp.reserve(static_cast<std::size_t>(total) + 1);
     // Down-sweep of block sums.
-    int* level_data = data;
+    int* level_data = dst;
     int level_n = n;
     for (std::size_t l = 0; l < offs.size(); ++l) {
       int blocks = (level_n + SCAN_B - 1) / SCAN_B;
-      k_scan_block<<<blocks, SCAN_B, 0, ctx.stream>>>(level_data, level_n, tmp.get() + offs[l]);
+      k_scan_block<<<blocks, SCAN_B, 0, ctx.stream>>>(l == 0 ? src : level_data, level_data, level_n, tmp.get() + offs[l],
+                                                     clear && l == 0, clear_state);
       if (blocks == 1) break;
       level_data = tmp.get() + offs[l];
       level_n = blocks;
@@ -555,7 +667,7 @@ namespace flyg {
     // Up-sweep: add scanned block sums back, deepest level first.
     for (std::size_t l = offs.size(); l-- > 0;) {
       int ln = l == 0 ? n : sizes[l - 1];
-      int* ld = l == 0 ? data : tmp.get() + offs[l - 1];
+      int* ld = l == 0 ? dst : tmp.get() + offs[l - 1];
       int blocks = (ln + SCAN_B - 1) / SCAN_B;
       if (blocks == 1) continue;
       k_scan_add<<<blocks, SCAN_B, 0, ctx.stream>>>(ld, ln, tmp.get() + offs[l]);
@@ -581,7 +693,6 @@ namespace flyg {
     flyg_ctx_s& ctx = *nl.ctx;
     hipStream_t st = ctx.stream;
     if (!nl.hstate) HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&nl.hstate), 4 * sizeof(unsigned), hipHostMallocDefault));
-    nl.lstate.reserve(4);
     nl.built = false;
     if (n != nl.n) {
       nl.gcap = 0;
@@ -591,64 +702,81 @@ namespace flyg {
     if (nl.gcap == 0) nl.gcap = std::max(4096l, n);
     if (nl.K == 0) nl.K = 64;
     int const nc = nl.grid.ncells;
+    long const nc1 = nc + 1;
+    nl.lstate.reserve(8);
+    nl.ccount.reserve(scan_room(2 * nc1));
+    nl.cstart.reserve(scan_room(2 * nc1));   // cell starts, then the first real slot of each cell (offset)
     nl.pos.reserve(n);
-    nl.cstart.reserve(2 * (nc + 1));   // cell starts, then the first real slot of each cell (offset)
-    nl.ccursor.reserve(nc);
     nl.ncnt.reserve(n);
     nl.rslot.reserve(n);
     nl.order.reserve(n);
     nl.rank.reserve(n);
     nl.gpos.reserve(n);
     nl.gcnt.reserve(n);
-    unsigned* dst = nl.lstate.get();
+    if (!nl.counters_clear) {   // a first build, or one that ended in an error half way
+      HIPCHK(hipMemsetAsync(nl.ccount.get(), 0, scan_room(2 * nc1) * sizeof(int), st));
+      HIPCHK(hipMemsetAsync(nl.lstate.get(), 0, 8 * sizeof(unsigned), st));
+    }
+    nl.counters_clear = false;
 
     for (int attempt = 0; attempt < 3; ++attempt) {
+      // Two sets of state words in turn: the scan clears the other build's.
+      unsigned* dst = nl.lstate.get() + 4 * nl.parity;
+      unsigned* other = nl.lstate.get() + 4 * (1 - nl.parity);
+      nl.parity = 1 - nl.parity;
       long const cap = n + nl.gcap;
       nl.ent.reserve(cap);
       nl.eid.reserve(cap);
       nl.ecell.reserve(cap);
+      nl.earr.reserve(cap);
       nl.spos.reserve(cap);
       nl.sid.reserve(cap);
       nl.usid.reserve(cap);
       nl.nbr.reserve(static_cast<std::size_t>(n) * nl.K);
       nl.grow.reserve(static_cast<std::size_t>(n) * nl.K);
-      long const nc1 = nc + 1;
-      long const nz = std::max<long>(std::max<long>(n, 2 * nc1), 4);
-      k_canon_reals<<<nblk(nz, TPB), TPB, 0, st>>>(nl.box, d_xyz, n, nl.pos.get(), nl.ent.get(), nl.eid.get(),
-                                                   nl.cstart.get(), 2 * nc1, nl.ccursor.get(), nc, dst);
+      nl.hstate[1] = 0;
       if (nl.box.ortho) {
-        k_ghosts_cap<true><<<nblk(n, TPB), TPB, 0, st>>>(nl.box, nl.rc, nl.pos.get(), n, nl.ent.get(), nl.eid.get(), dst,
-                                                         nl.gcap);
+        k_entries<true><<<nblk(n, ETPB), ETPB, 0, st>>>(nl.box, nl.grid, d_xyz, n, nl.pos.get(), nl.ent.get(),
+                                                        nl.eid.get(), dst, nl.gcap);
       } else {
-        k_ghosts_cap<false><<<nblk(n, TPB), TPB, 0, st>>>(nl.box, nl.rc, nl.pos.get(), n, nl.ent.get(), nl.eid.get(), dst,
-                                                          nl.gcap);
+        k_entries<false><<<nblk(n, ETPB), ETPB, 0, st>>>(nl.box, nl.grid, d_xyz, n, nl.pos.get(), nl.ent.get(),
+                                                        nl.eid.get(), dst, nl.gcap);
       }
-      k_cell_count_cap<<<nblk(cap, TPB), TPB, 0, st>>>(nl.grid, nl.ent.get(), n, nl.gcap, dst, nl.ecell.get(),
-                                                       nl.cstart.get(), nc1);
-      exclusive_scan(ctx, nl.cstart.get(), static_cast<int>(2 * nc1), nl.scan_tmp);
-      k_scatter_ids<<<nblk(cap, TPB), TPB, 0, st>>>(nl.eid.get(), nl.ecell.get(), n, nl.gcap, dst, nl.cstart.get(),
-                                                    nl.ccursor.get(), nl.usid.get());
+      k_cell_count<<<nblk(cap, TPB), TPB, 0, st>>>(nl.grid, nl.ent.get(), n, nl.gcap, dst, nl.ecell.get(), nl.earr.get(),
+                                                   nl.ccount.get(), nc1);
+      exclusive_scan(ctx, nl.ccount.get(), nl.cstart.get(), static_cast<int>(2 * nc1), nl.scan_tmp, other);
+      k_scatter_ids<<<nblk(cap, TPB), TPB, 0, st>>>(nl.eid.get(), nl.ecell.get(), nl.earr.get(), n, nl.gcap, dst,
+                                                    nl.cstart.get(), nl.usid.get());
       k_rank_place<<<nblk(cap, TPB), TPB, 0, st>>>(nl.ent.get(), nl.eid.get(), nl.ecell.get(), n, nl.gcap, dst,
                                                    nl.cstart.get(), nc1, nl.usid.get(), nl.spos.get(), nl.sid.get(),
                                                    nl.rslot.get(), nl.order.get(), nl.rank.get(), nl.gpos.get());
-      k_build_rows<<<nblk(n * BL, TPB), TPB, 0, st>>>(nl.grid, nl.spos.get(), nl.sid.get(), nl.cstart.get(), nl.rslot.get(),
-                                                 n, nl.nbr.get(), nl.ncnt.get(), nl.K, dst, nl.order.get(),
-                                                 nl.rank.get(), nl.grow.get(), nl.gcnt.get());
+      auto rows = [&](auto k, int A) {
+        k<<<nblk(n, A * (TPB / 64)), TPB, 0, st>>>(nl.grid, nl.spos.get(), nl.sid.get(), nl.cstart.get(), nl.rslot.get(), n,
+                                                   nl.nbr.get(), nl.ncnt.get(), nl.K, dst, nl.order.get(), nl.rank.get(),
+                                                   nl.grow.get(), nl.gcnt.get(), nl.hstate);
+      };
+      if (n < BUILD_WIDE) {
+        rows(k_build_rows<1>, 1);
+      } else {
+        rows(k_build_rows<4>, 4);
+      }
       HIPCHK(hipGetLastError());
-      HIPCHK(hipMemcpyAsync(nl.hstate, dst, 4 * sizeof(unsigned), hipMemcpyDeviceToHost, st));
       HIPCHK(hipStreamSynchronize(st));
-      unsigned const G = nl.hstate[0], maxrow = nl.hstate[1], flags = nl.hstate[3];
+      unsigned const G = nl.hstate[0], flags = nl.hstate[3];
       if (flags & OV_GHOST) {   // more ghost images than slots: grow and start again
         nl.gcap = static_cast<long>(G) + static_cast<long>(G) / 4 + 4096;
         continue;
       }
       nl.nghost = G;
-      if (static_cast<int>(maxrow) > nl.K) {   // a row overflowed: widen the rows and build again
-        nl.K = (static_cast<int>(maxrow) + 15) / 16 * 16 + 16;
+      if (nl.hstate[1]) {   // a row overflowed: widen the rows and build again
+        HIPCHK(hipMemcpyAsync(nl.hstate, dst, 4 * sizeof(unsigned), hipMemcpyDeviceToHost, st));
+        HIPCHK(hipStreamSynchronize(st));
+        nl.K = (static_cast<int>(nl.hstate[1]) + 15) / 16 * 16 + 16;
         continue;
       }
       static std::atomic<long> builds{0};
       nl.build_id = ++builds;
+      nl.counters_clear = true;
       nl.built = true;
       return;
     }

@@ -66,6 +66,25 @@ def test_small_box_multiple_images(ctx):
     assert np.array_equal(H.pair_set(go, gj, gs), H.pair_set(oo, oj, os_))
 
 
+@pytest.mark.parametrize("n,rc,tilt", [(23999, 3.1, 0.0), (24001, 3.1, 0.0), (25003, 4.4, 3.0), (30002, 1.2, 0.0)])
+def test_large_lists_equal_pair_sets(ctx, n, rc, tilt):
+    # Both forms of the row build (one or four atoms a wavefront), with 3 to 100 candidates per range of cells:
+    # partly filled, full and repeated chunks of 64, rows longer than 64 and than the first row table, and
+    # wavefronts whose atoms straddle cells.  A list is built twice: the second build reuses the counters.
+    rng = np.random.default_rng(n)
+    basis = np.diag([41.0, 38.0, 44.0])
+    basis[0, 1] = tilt
+    periodic = np.array([1, 0, 1], np.int32)
+    pos = rng.random((n, 3)) @ basis.T
+    nl = fa.List(ctx, fa.Box(basis, periodic), rc)
+    nl.rebuild(pos[::-1].copy())
+    nl.rebuild(pos)
+    _, (oo, oj, os_, _) = oracle_pairs(basis, periodic, pos, rc)
+    go, gj, gs, _ = nl.pairs()
+    assert np.array_equal(go, oo)
+    assert np.array_equal(H.pair_set(go, gj, gs), H.pair_set(oo, oj, os_))
+
+
 def test_update_matches_brute_force(ctx):
     rng = np.random.default_rng(77)
     for _ in range(4):
