@@ -93,8 +93,9 @@ int flyg_eam_destroy(flyg_eam eam);
 int flyg_eam_info(flyg_eam eam, int* ntypes, double* r_cut, double* masses, char* names);
 /* FLYG_FP64 (default) or FLYG_MIXED for gradient / HVP pair arithmetic.  Energies are always FP64. */
 int flyg_eam_set_precision(flyg_eam eam, int precision);
-/* Lanes of a wavefront that share one atom's neighbour row in the gradient kernels: 4, 8 or 16, or 0
- * (default) to time the three once per system size.  Results are bitwise identical for every choice. */
+/* Lanes of a wavefront that share one atom's neighbour row: 4, 8 or 16, which also selects the row-by-row
+ * gradient and energy kernels, or 0 (default) for the library's choice of kernel by size.  Results are bitwise
+ * identical for every choice. */
 int flyg_eam_set_lanes(flyg_eam eam, int lanes);
 /* Kernel timing of gradient calls (no reference counterpart; for benchmarks): while on, each gradient
  * call records a HIP event pair on the context's stream around its density + force kernels.
@@ -152,8 +153,7 @@ int flyg_eam_gradient(flyg_eam eam, flyg_list nl, const uint32_t* types, const u
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).  Same kernels and results as
  * flyg_eam_gradient with FLYG_DEVICE pointers (types, frozen, grad on the context's device), but the
  * density pass's output goes to a library-held device array of at most 131072 atoms (32 B per atom, one
- * copy per GPU, held until the process ends) instead of a per-handle buffer, and the lanes per atom are
- * not tuned (set_lanes, an earlier tuning for this size, else 8).  Larger systems are refused
+ * copy per GPU, held until the process ends) instead of a per-handle buffer.  Larger systems are refused
  * (FLYG_INVALID_ARG).  Calls that overlap on one GPU share that array and race.  Asynchronous on the
  * context's stream; spline and type errors surface at the next synchronising call. */
 int flyg_eam_gradient_noalloc(flyg_eam eam, flyg_list nl, const uint32_t* types, const uint8_t* frozen, int64_t n,

@@ -295,6 +295,37 @@ namespace flyg {
   }
 
   // ----------------------------------------------------------------------------------------------
+  // Tiles of cells.  Tile t of an axis owns d cells of the grid's interior; the first and last tile
+  // also own the ghost layer beside them (an atom on the box face can be binned there).  Its halo is one
+  // more cell on every side.  With d <= 2 a halo has at most four lines of cells in y and in z.
+  // ----------------------------------------------------------------------------------------------
+  struct TileGrid {
+    int d[3], nt[3], shape[3], prod[3];
+    int ntiles;
+    long nc1;   // cells + 1: the offset of the real slots' part in the cell starts
+
+    __host__ __device__ int of(int ax, int c) const {
+      int const t = (c - 1) / d[ax];
+      return t < 0 ? 0 : (t > nt[ax] - 1 ? nt[ax] - 1 : t);
+    }
+    __host__ __device__ int lo(int ax, int t) const { return t == 0 ? 0 : 1 + t * d[ax]; }
+    __host__ __device__ int hi(int ax, int t) const { return t == nt[ax] - 1 ? shape[ax] : 1 + (t + 1) * d[ax]; }
+    __host__ __device__ int halo_lo(int ax, int t) const { return lo(ax, t) > 0 ? lo(ax, t) - 1 : 0; }
+    __host__ __device__ int halo_hi(int ax, int t) const { return hi(ax, t) < shape[ax] ? hi(ax, t) + 1 : shape[ax]; }
+    // Cell range [b, e) of line q = y + 4 z (counted from the halo's or the tile's first) of tile (tx, ty, tz);
+    // empty where there is no such line.
+    __host__ __device__ void line(bool halo, int tx, int ty, int tz, int q, int& b, int& e) const {
+      int const y = (halo ? halo_lo(1, ty) : lo(1, ty)) + (q & 3), z = (halo ? halo_lo(2, tz) : lo(2, tz)) + (q >> 2);
+      b = e = 0;
+      if (y >= (halo ? halo_hi(1, ty) : hi(1, ty)) || z >= (halo ? halo_hi(2, tz) : hi(2, tz))) return;
+      int const l = y * prod[1] + z * prod[2];
+      b = (halo ? halo_lo(0, tx) : lo(0, tx)) * prod[0] + l;
+      e = (halo ? halo_hi(0, tx) : hi(0, tx)) * prod[0] + l;
+    }
+  };
+  constexpr int TILE_MOST = 1900;   // entries a tile may stage: with species and tables below 64 KB
+
+  // ----------------------------------------------------------------------------------------------
   // Wavefront helpers (64 lanes on CDNA).
   // ----------------------------------------------------------------------------------------------
 
@@ -349,6 +380,19 @@ namespace flyg {
       return v[0];
     }
   };
+
+  // Acc16<16>'s tree (8, 4, 2, 1) within each row of 16 lanes, by DPP instead of LDS shuffles.  Once lanes 8 apart
+  // hold the same sum a rotation by 4 reads the lane the xor by 4 would.
+  template <int CTRL>
+  __device__ inline double dpp_add(double v) {
+    return __dadd_rn(v, __builtin_amdgcn_update_dpp(0.0, v, CTRL, 0xF, 0xF, false));
+  }
+  __device__ inline double total16(double v) {
+    v = dpp_add<0x128>(v);   // row_ror:8
+    v = dpp_add<0x124>(v);   // row_ror:4
+    v = dpp_add<0x4E>(v);    // quad_perm [2,3,0,1]
+    return dpp_add<0xB1>(v); // quad_perm [1,0,3,2]
+  }
 
   // Deterministic block reduction of one double (fixed tree order); result valid in thread 0.
   template <int NT>

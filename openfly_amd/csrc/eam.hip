@@ -19,7 +19,6 @@
 //      which is H v for the analytic Hessian of eam.cpp:122-233 (pinned against it in the tests).
 #include <atomic>
 #include <cstring>
-#include <map>
 #include <mutex>
 
 #include "vecops.hpp"
@@ -137,7 +136,7 @@ namespace flyg {
         unsigned const* row = A.nbr + i * static_cast<long>(A.K);
         walk_row<L>(row, c, lane, S, A.pos, pi, [&](int q, PairGeo const& p) {
           if (p.r2 < T.rc2) {
-            int tj = MULTI ? checked_type(A.type_in_w ? static_cast<uint32_t>(p.w) : A.types[p.j], T.ntypes, e) : A.t0;
+            int tj = MULTI ? checked_type(A.types[p.j], T.ntypes, e) : A.t0;
             if (MIX && !ENERGY) {
               float r2f = static_cast<float>(p.r2);
               float rf = r2f * __frsqrt_rn(r2f);
@@ -189,12 +188,10 @@ namespace flyg {
         }
       };
       long gid = xcd_block(blockIdx.x, gridDim.x) * static_cast<long>(NT) + threadIdx.x;
-      long i = gid / L;   // row: the atom, or its slot when A.order is set
+      long i = gid / L;
       int lane = static_cast<int>(gid % L);
       bool inr = i < A.n;
-      long const ia = inr && A.order ? A.order[i] : i;   // the atom, for its frozen flag and gradient
       unsigned e = 0;
-      // The row's own data is loaded beside the frozen flag (not after it): the flag waits on `order`.
       double4 pi = make_double4(0.0, 0.0, 0.0, 0.0);
       int ti = MULTI ? 0 : A.t0;
       int c = 0;
@@ -204,7 +201,7 @@ namespace flyg {
         // Mixed form: the species the density pass packed beside F' (checked there).
         if (MULTI) ti = MIX ? packed_type(pi.w) : checked_type(A.types[i], T.ntypes, e);
       }
-      bool act = inr && !A.frozen[ia];
+      bool act = inr && !A.frozen[i];
       Acc16<L> gx, gy, gz;
       if (act) {
         unsigned const* row = A.nbr + i * static_cast<long>(A.K);
@@ -238,12 +235,358 @@ namespace flyg {
       double tx = gx.total(), ty = gy.total(), tz = gz.total();
       if (L >= 3 && inr && lane < 3) {
         double v = lane == 0 ? tx : (lane == 1 ? ty : tz);
-        grad[3 * ia + lane] = act ? v : 0.0;
+        grad[3 * i + lane] = act ? v : 0.0;
       }
       if (L < 3 && inr && lane == 0) {
-        grad[3 * ia] = act ? tx : 0.0;
-        grad[3 * ia + 1] = act ? ty : 0.0;
-        grad[3 * ia + 2] = act ? tz : 0.0;
+        grad[3 * i] = act ? tx : 0.0;
+        grad[3 * i + 1] = act ? ty : 0.0;
+        grad[3 * i + 2] = act ? tz : 0.0;
+      }
+      if (e) atomicOr(err, e);
+    }
+
+    // ---- Tiled passes -------------------------------------------------------------------------------
+    // One workgroup per tile of cells (TileGrid).  It stages the entries of the tile's halo in LDS, image
+    // shifts applied, and walks the rows of the tile's atoms 16 lanes a row through 16-bit indices into the stage.
+    //
+    // Why: the row-gather kernels above are bound by L1 lookups, one cache line a clock and CU.  64 pairs need 128 of
+    // them for the neighbours' positions, 64 per spline segment read and 8 for the row; at 54.5k atoms the
+    // density pass counts 8.8M lookups, 14 us of its 18.  From LDS a position costs no lookup, and a 2x2x2
+    // tile stages eight entries per atom, read in order, where it gathered 65.  A stage of one cell (27 entries per
+    // atom, little work between barriers) was slower than the gathers.
+    // Entries, their order and every expression are those of the row-gather kernels: the same bits.
+
+    constexpr int TT = 512;   // threads: 32 rows at a time
+
+    struct TileArgs {
+      TileGrid G;
+      int const* cstart;       // entries by cell, then (from nc1) real slots by cell
+      unsigned const* sslot;
+      unsigned const* rows;
+      int rowW;                // words a row
+      int K;
+      int const* cnt;          // by slot
+      int const* order;
+      double4 const* pos;      // by slot; w: species (several species, density pass) or F'
+      uint32_t const* types;   // by slot (several species)
+      uint8_t const* frozen;   // by atom
+      int t0;
+      int cap;                 // entries of room in the stage
+    };
+
+    struct TileLds {
+      int ls[16], off[17];     // halo lines: first sorted entry, place in the stage
+      int os[16], oo[17];      // own lines: first slot, rows before it
+    };
+
+    // The last of 16 lines that starts at or before x.
+    __device__ inline int line_of(int const* off, int x) {
+      int q = 0;
+#pragma unroll
+      for (int b = 8; b > 0; b >>= 1)
+        if (off[q + b] <= x) q += b;
+      return q;
+    }
+
+    // Fills the line tables and the stage (xy, zw; types where `st` is given).  Ends with a barrier.
+    template <typename F>
+    __device__ inline void stage_tile(TileArgs const& A, Shifts const& S, TileLds& L, double2* xy, double2* zw, F&& extra) {
+      int const t = static_cast<int>(xcd_block(blockIdx.x, gridDim.x));
+      if (threadIdx.x < 64) {   // lanes 0..15 the halo's lines, 16..31 the tile's own
+        int const q = threadIdx.x & 15;
+        bool const own = threadIdx.x >= 16;
+        int cb, ce;
+        A.G.line(!own, t % A.G.nt[0], t / A.G.nt[0] % A.G.nt[1], t / (A.G.nt[0] * A.G.nt[1]), q, cb, ce);
+        int const* c = A.cstart + (own ? A.G.nc1 : 0);
+        int const b = c[cb], len = c[ce] - b;
+        int incl = len;
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) {
+          int const v = __shfl_up(incl, o, 16);
+          if (q >= o) incl += v;
+        }
+        if (threadIdx.x < 16) {
+          L.ls[q] = b;
+          L.off[q] = incl - len;
+          if (q == 15) L.off[16] = incl;
+        } else if (threadIdx.x < 32) {
+          L.os[q] = b - A.cstart[A.G.nc1];
+          L.oo[q] = incl - len;
+          if (q == 15) L.oo[16] = incl;
+        }
+      }
+      __syncthreads();
+      int const total = min(L.off[16], A.cap);
+      for (int e0 = threadIdx.x; e0 < total; e0 += 4 * TT) {
+        unsigned en[4];
+        double4 p[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          int const e = e0 + u * TT;
+          if (e < total) {
+            int const q = line_of(L.off, e);
+            en[u] = A.sslot[L.ls[q] + (e - L.off[q])];
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (e0 + u * TT < total) p[u] = A.pos[en[u] & NB_IDX_MASK];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          int const e = e0 + u * TT;
+          if (e < total) {
+            unsigned const code = en[u] >> NB_SHIFT_BITS;
+            if (code != 13u) {
+              double3 const sh = S.of(code);
+              p[u].x += sh.x;
+              p[u].y += sh.y;
+              p[u].z += sh.z;
+            }
+            xy[e] = make_double2(p[u].x, p[u].y);
+            zw[e] = make_double2(p[u].z, p[u].w);
+            extra(e, en[u] & NB_IDX_MASK);
+          }
+        }
+      }
+      __syncthreads();
+    }
+
+    // NB entries of a lane's row: geometry, and whether each is a pair within the cut-off.
+    template <int NB>
+    struct Pairs {
+      PairGeo p[NB];
+      bool in[NB];
+    };
+
+    // Lane l of 16 walks entries l, l + 16, ... of a row.  Entries go to one() four at a time so that their table
+    // loads are in flight together (entry by entry a row is a chain of five L2 round trips); those past the row's end
+    // or the cut-off are marked, not branched around.  The number of steps is that of the wavefront's
+    // longest row, so no control flow diverges.  Every lane of the wavefront must call it (lanes without a row with
+    // c = 0).  The next group's words are loaded ahead.
+    template <typename F>
+    __device__ inline void walk_tile_grouped(unsigned const* __restrict__ row, int c, int l, double4 const& pi, double rc2,
+                                             double2 const* xy, double2 const* zw, F&& one) {
+      int const c0 = __builtin_amdgcn_readlane(c, 0), c1 = __builtin_amdgcn_readlane(c, 16);
+      int const c2 = __builtin_amdgcn_readlane(c, 32), c3 = __builtin_amdgcn_readlane(c, 48);
+      int const steps = (max(max(c0, c1), max(c2, c3)) + 15) / 16;
+      unsigned w0 = 0, w1 = 0;
+      if (c > 0) w0 = row[l];
+      if (c > 32) w1 = row[16 + l];
+      auto group = [&](auto nb, unsigned a, unsigned b, int k) {
+        constexpr int NB = decltype(nb)::value;
+        Pairs<NB> G;
+#pragma unroll
+        for (int n = 0; n < NB; ++n) {
+          unsigned const word = n < 2 ? a : b;
+          bool const valid = k + 16 * n < c;
+          unsigned const j = valid ? ((n & 1) ? word >> 16 : word & 0xffffu) : 0u;
+          PairGeo& p = G.p[n];
+          double2 const u = xy[j], v = zw[j];
+          p.dx = u.x - pi.x;
+          p.dy = u.y - pi.y;
+          p.dz = v.x - pi.z;
+          p.w = v.y;
+          p.j = j;
+          p.r2 = p.dx * p.dx + p.dy * p.dy + p.dz * p.dz;
+          G.in[n] = valid && p.r2 < rc2;
+        }
+        one(G);
+      };
+      for (int s = 0; s < steps; s += 4) {
+        int const k = 16 * s + l, left = steps - s;
+        unsigned n0 = 0, n1 = 0;
+        if (16 * (s + 4) < c) n0 = row[8 * (s + 4) + l];
+        if (16 * (s + 6) < c) n1 = row[8 * (s + 6) + l];
+        if (left >= 4) {
+          group(std::integral_constant<int, 4>{}, w0, w1, k);
+        } else if (left == 1) {
+          group(std::integral_constant<int, 1>{}, w0, 0u, k);
+        } else {
+          group(std::integral_constant<int, 2>{}, w0, 0u, k);
+          if (left == 3) group(std::integral_constant<int, 1>{}, w1, 0u, k + 32);
+        }
+        w0 = n0;
+        w1 = n1;
+      }
+    }
+
+    // The same, entry by entry, pairs outside the cut-off branched around: for the forms whose table loads and
+    // arithmetic of several entries would not fit in the registers that leave three workgroups a CU.
+    template <typename F>
+    __device__ inline void walk_tile(unsigned const* __restrict__ row, int c, int l, double4 const& pi, double rc2,
+                                     double2 const* xy, double2 const* zw, F&& one) {
+      unsigned w[4];   // the first 128 entries: a row's words are in flight together
+#pragma unroll
+      for (int u = 0; u < 4; ++u) w[u] = 32 * u < c ? row[16 * u + l] : 0u;
+      auto pair = [&](unsigned word, int k) {
+        unsigned const j[2] = {word & 0xffffu, word >> 16};
+        PairGeo p[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          if (k + 16 * h < c) {
+            double2 const a = xy[j[h]], b = zw[j[h]];
+            p[h].dx = a.x - pi.x;
+            p[h].dy = a.y - pi.y;
+            p[h].dz = b.x - pi.z;
+            p[h].w = b.y;
+            p[h].j = j[h];
+          }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          if (k + 16 * h < c) {
+            p[h].r2 = p[h].dx * p[h].dx + p[h].dy * p[h].dy + p[h].dz * p[h].dz;
+            if (p[h].r2 < rc2) one(p[h]);
+          }
+      };
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (32 * u < c) pair(w[u], 32 * u + l);
+      for (int k = 128; k < c; k += 32) pair(row[k / 2 + l], k + l);
+    }
+
+    // Density pass: posf by slot; ENERGY: eatom by atom (FP64 densities and pair energies).
+    template <bool MULTI, bool ENERGY, bool MIX>
+    __global__ __launch_bounds__(TT) void k_tile_density(EAMTables T, Shifts S, TileArgs A, double4* __restrict__ posf,
+                                                         double* __restrict__ eatom, unsigned* __restrict__ err) {
+      extern __shared__ double2 s_stage[];
+      double2* const xy = s_stage;
+      double2* const zw = s_stage + A.cap;
+      __shared__ TileLds L;
+      __shared__ SplineDesc s_phi[MULTI ? MAX_TYPES * MAX_TYPES : 1], s_V[MULTI && ENERGY ? MAX_TYPES * MAX_TYPES : 1];
+      if (MULTI && threadIdx.x < T.ntypes * T.ntypes) {
+        s_phi[threadIdx.x] = T.phi[threadIdx.x];
+        if (ENERGY) s_V[threadIdx.x] = T.V[threadIdx.x];
+      }
+      unsigned e = 0;
+      stage_tile(A, S, L, xy, zw, [](int, unsigned) {});
+      int const rows = L.oo[16];
+      int const l = threadIdx.x & 15;
+      // Four rows a wavefront; its lanes stay together (walk_tile_grouped reads across them): lanes without a
+      // row get the last one with no entries.
+      for (int r0 = (threadIdx.x >> 6) * 4; r0 < rows; r0 += TT / 16) {
+        int const r = r0 + static_cast<int>((threadIdx.x & 63) >> 4);
+        int const rr = min(r, rows - 1);
+        int const q = line_of(L.oo, rr);
+        long const i = L.os[q] + (rr - L.oo[q]);
+        double4 const pi = A.pos[i];
+        int const ti = MULTI ? checked_type(static_cast<uint32_t>(pi.w), T.ntypes, e) : A.t0;
+        int const c = r < rows ? min(A.cnt[i], A.K) : 0;
+        double rho = 0.0, vs = 0.0;
+        auto phi_of = [&](double w) -> SplineDesc const& {
+          int const tj = MULTI ? checked_type(static_cast<uint32_t>(w), T.ntypes, e) : A.t0;
+          return MULTI ? s_phi[tj + T.ntypes * ti] : T.phi[tj + T.ntypes * ti];
+        };
+        if constexpr (MIX && !ENERGY) {
+          walk_tile_grouped(A.rows + i * A.rowW, c, l, pi, T.rc2, xy, zw, [&](auto const& G) {
+            constexpr int NB = sizeof(G.in) / sizeof(bool);
+            Seg<true> g[NB];
+            float4 co[NB];
+#pragma unroll
+            for (int n = 0; n < NB; ++n) {
+              SplineDesc const& sp = phi_of(G.p[n].w);
+              float const r2f = G.in[n] ? static_cast<float>(G.p[n].r2) : 1.0f;
+              g[n] = seg_of<true>(sp, r2f * __frsqrt_rn(r2f), G.in[n], e);
+              co[n] = coef_of<true>(T, sp, g[n]);
+            }
+#pragma unroll
+            for (int n = 0; n < NB; ++n) {
+              double const f = static_cast<double>(poly0(co[n], g[n].t));
+              rho = g[n].use ? __dadd_rn(rho, f) : rho;
+            }
+          });
+        } else {
+          walk_tile(A.rows + i * A.rowW, c, l, pi, T.rc2, xy, zw, [&](PairGeo const& p) {
+            double const d = sqrt(p.r2);
+            rho = __dadd_rn(rho, spl64<0>(T, phi_of(p.w), d, e));
+            if (ENERGY) {
+              int const tj = MULTI ? checked_type(static_cast<uint32_t>(p.w), T.ntypes, e) : A.t0;
+              vs = __dadd_rn(vs, spl64<0>(T, MULTI ? s_V[vidx(T, ti, tj)] : T.V[vidx(T, ti, tj)], d, e));
+            }
+          });
+        }
+        rho = total16(rho);
+        if (ENERGY) vs = total16(vs);
+        if (l == 0 && r < rows) {
+          posf[i] = make_double4(pi.x, pi.y, pi.z, rho);
+          if (ENERGY) eatom[A.order[i]] = vs;
+        }
+      }
+      // The embedding spline once per row and thread, instead of by one lane in 16 beside the walks.
+      __syncthreads();
+      for (int r = threadIdx.x; r < rows; r += TT) {
+        int const q = line_of(L.oo, r);
+        long const i = L.os[q] + (r - L.oo[q]);
+        int const ti = MULTI ? checked_type(A.types[i], T.ntypes, e) : A.t0;
+        double f, fp;
+        spl64_ffp(T, T.F[ti], posf[i].w, f, fp, e);
+        posf[i].w = MIX && !ENERGY ? pack_fp_type(static_cast<float>(fp), ti) : fp;
+        if (ENERGY) {
+          int const a = A.order[i];
+          eatom[a] = 0.5 * eatom[a] + f;
+        }
+      }
+      if (e) atomicOr(err, e);
+    }
+
+    template <bool MULTI, bool MIX>
+    __global__ __launch_bounds__(TT) void k_tile_force(EAMTables T, Shifts S, TileArgs A, double* __restrict__ grad,
+                                                       unsigned* __restrict__ err) {
+      extern __shared__ double2 s_stage[];
+      double2* const xy = s_stage;
+      double2* const zw = s_stage + A.cap;
+      uint8_t* const typ = reinterpret_cast<uint8_t*>(zw + A.cap);   // FP64 with several species
+      __shared__ TileLds L;
+      __shared__ SplineDesc s_phi[MULTI ? MAX_TYPES * MAX_TYPES : 1], s_V[MULTI ? MAX_TYPES * MAX_TYPES : 1];
+      if (MULTI && threadIdx.x < T.ntypes * T.ntypes) {
+        s_phi[threadIdx.x] = T.phi[threadIdx.x];
+        s_V[threadIdx.x] = T.V[threadIdx.x];
+      }
+      unsigned e = 0;
+      stage_tile(A, S, L, xy, zw, [&](int k, unsigned slot) {
+        if (MULTI && !MIX) typ[k] = static_cast<uint8_t>(checked_type(A.types[slot], T.ntypes, e));
+      });
+      int const rows = L.oo[16];
+      int const l = threadIdx.x & 15;
+      for (int r = threadIdx.x >> 4; r < rows; r += TT / 16) {
+        int const q = line_of(L.oo, r);
+        long const i = L.os[q] + (r - L.oo[q]);
+        int const ia = A.order[i];
+        double4 const pi = A.pos[i];
+        int const c = min(A.cnt[i], A.K);
+        // Mixed form: the species the density pass packed beside F' (checked there).
+        int const ti = MULTI ? (MIX ? packed_type(pi.w) : checked_type(A.types[i], T.ntypes, e)) : A.t0;
+        bool const act = !A.frozen[ia];
+        double gx = 0.0, gy = 0.0, gz = 0.0;
+        walk_tile(A.rows + i * A.rowW, act ? c : 0, l, pi, T.rc2, xy, zw, [&](PairGeo const& p) {
+          int const tj = MULTI ? (MIX ? packed_type(p.w) : typ[p.j]) : A.t0;
+          SplineDesc const& sv = MULTI ? s_V[vidx(T, ti, tj)] : T.V[vidx(T, ti, tj)];
+          SplineDesc const& sa = MULTI ? s_phi[tj + T.ntypes * ti] : T.phi[tj + T.ntypes * ti];
+          double cf;
+          if (MIX) {
+            float r2f = static_cast<float>(p.r2);
+            float rinv = __frsqrt_rn(r2f);
+            float rf = r2f * rinv;
+            float vp = spl32f<1>(T, sv, rf, e);
+            float pa = spl32f<1>(T, sa, rf, e);
+            // phi_{g->a} is phi_{a->g} for a same-species pair: no second table load.
+            float pb = MULTI && ti != tj ? spl32f<1>(T, s_phi[MULTI ? ti + T.ntypes * tj : 0], rf, e) : pa;
+            float mag = vp + packed_fp(pi.w) * pa + packed_fp(p.w) * pb;
+            cf = static_cast<double>(mag * rinv);
+          } else {
+            double d = sqrt(p.r2);
+            double vp = spl64<1>(T, sv, d, e);
+            double pa = spl64<1>(T, sa, d, e);
+            double pb = MULTI && ti != tj ? spl64<1>(T, s_phi[MULTI ? ti + T.ntypes * tj : 0], d, e) : pa;
+            cf = (vp + pi.w * pa + p.w * pb) / d;
+          }
+          gx = __dadd_rn(gx, -cf * p.dx);
+          gy = __dadd_rn(gy, -cf * p.dy);
+          gz = __dadd_rn(gz, -cf * p.dz);
+        });
+        gx = total16(gx);
+        gy = total16(gy);
+        gz = total16(gz);
+        if (l < 3) grad[3l * ia + l] = act ? (l == 0 ? gx : (l == 1 ? gy : gz)) : 0.0;
       }
       if (e) atomicOr(err, e);
     }
@@ -411,20 +754,17 @@ namespace flyg {
       }
     }
 
-    // The gradient passes run in the list's cell-order layout: a workgroup's atoms are neighbours in
-    // space and so are the rows they gather, which raises the L1/L2 hit rate of the gathers.  Rows hold
-    // the same entries in the same order, so the sums (and the bits) are those of the atom layout.  With
-    // several species the types are gathered into slot order, and into the w slot of the slot-ordered
+    // The tiled passes run in the list's slot (cell) order: a workgroup's atoms are neighbours in space.
+    // With several species the types are gathered into slot order, and into the w slot of the slot-ordered
     // positions (the density pass reads a neighbour's species from there): once per list build for staged
     // host types (the library sees every change of them), on every call for device types.  Type stamps
     // are unique across handles, so a list shared by several potentials or type arrays is re-gathered
     // whenever another one wrote its w slots last.
-    PairArgs slot_args(flyg_eam_s& E, flyg_list_s& nl, uint32_t const* types, uint8_t const* frozen) {
-      PairArgs A = pair_args(E, nl, types, frozen);
-      A.pos = nl.gpos.get();
-      A.nbr = nl.grow.get();
-      A.cnt = nl.gcnt.get();
-      A.order = nl.order.get();
+    TileArgs tile_args(flyg_eam_s& E, flyg_list_s& nl, uint32_t const* types, uint8_t const* frozen) {
+      PairArgs const P = pair_args(E, nl, types, frozen);
+      TileArgs A{nl.tile,        nl.cstart.get(), nl.sslot.get(), nl.rows.get(), nl.rowK / 2, nl.K, nl.gcnt.get(),
+                 nl.order.get(), nl.gpos.get(),   nullptr,        frozen,        P.t0,        0};
+      A.cap = (nl.tile_most + 15) & ~15;
       if (A.t0 < 0) {
         bool const staged = types == E.types.get();
         bool const cached = staged && E.gtype_build == nl.build_id && E.gtype_stamp == E.types_stamp &&
@@ -444,13 +784,11 @@ namespace flyg {
           }
         }
         A.types = E.gtype.get();
-        A.type_in_w = true;
       }
       return A;
     }
 
-    // Lanes per atom for the full-system kernels (a row of ~60 entries split 8 ways keeps ~8 pairs
-    // in flight per lane and the grid at >= 8 wavefronts per SIMD for >= 30k atoms).
+    // Lanes per atom for the energy, HVP and density kernels.
     constexpr int LANES = 8;
 
     unsigned grid_for(long n, int L) { return static_cast<unsigned>((n * L + NT - 1) / NT); }
@@ -544,12 +882,46 @@ namespace flyg {
     }
   }  // namespace
 
+  namespace {
+    void tile_density(flyg_eam_s& E, Shifts const& S, TileArgs const& A, bool energy, int precision, double4* pf) {
+      unsigned const g = static_cast<unsigned>(A.G.ntiles);
+      std::size_t const lds = static_cast<std::size_t>(A.cap) * sizeof(double4);
+      unsigned* err = E.ctx->dflags.get();
+      auto run = [&](auto k) { k<<<g, TT, lds, E.ctx->stream>>>(E.tab, S, A, pf, E.eatom.get(), err); };
+      bool const mix = precision == FLYG_MIXED;
+      if (A.t0 < 0) {
+        energy ? run(k_tile_density<true, true, false>)
+               : (mix ? run(k_tile_density<true, false, true>) : run(k_tile_density<true, false, false>));
+      } else {
+        energy ? run(k_tile_density<false, true, false>)
+               : (mix ? run(k_tile_density<false, false, true>) : run(k_tile_density<false, false, false>));
+      }
+    }
+
+    void tile_force(flyg_eam_s& E, Shifts const& S, TileArgs const& A, double* grad, int precision) {
+      unsigned const g = static_cast<unsigned>(A.G.ntiles);
+      bool const mix = precision == FLYG_MIXED;
+      std::size_t const lds = static_cast<std::size_t>(A.cap) * (sizeof(double4) + (A.t0 < 0 && !mix ? 1 : 0));
+      auto run = [&](auto k) { k<<<g, TT, lds, E.ctx->stream>>>(E.tab, S, A, grad, E.ctx->dflags.get()); };
+      if (A.t0 < 0) {
+        mix ? run(k_tile_force<true, true>) : run(k_tile_force<true, false>);
+      } else {
+        mix ? run(k_tile_force<false, true>) : run(k_tile_force<false, false>);
+      }
+    }
+  }  // namespace
+
   double eam_energy(flyg_eam_s& E, flyg_list_s& nl, uint32_t const* types, uint8_t const* frozen) {
     require(nl.built, "List used before rebuild");
     require(E.tab.rc <= nl.rc, "r_cut is bigger than the internal r_cut of the list");
     E.posf.reserve(nl.n);
     E.eatom.reserve(nl.n);
-    launch_density<LANES>(E, shifts_of(nl.box), pair_args(E, nl, types, frozen), true, FLYG_FP64, E.posf.get());
+    Shifts const S = shifts_of(nl.box);
+    if (nl.tiled && E.lanes <= 0) {
+      tile_density(E, S, tile_args(E, nl, types, frozen), true, FLYG_FP64, E.posf.get());
+    } else {
+      launch_density<LANES>(E, S, pair_args(E, nl, types, frozen), true, FLYG_FP64, E.posf.get());
+    }
     HIPCHK(hipGetLastError());
     dev_sum(*E.ctx, E.eatom.get(), nl.n, E.ctx->hpart, E.ctx->hflags + 1);
     HIPCHK(hipStreamSynchronize(E.ctx->stream));
@@ -563,10 +935,6 @@ namespace flyg {
 
   namespace {
     // Density then force pass; pf holds the pass-1 output (positions + F') of every atom.
-    // Lanes per atom row of the two passes, packed as density | force << 8 (either count gives the same
-    // sums, Acc16, so each pass takes its own).
-    constexpr int pack_lanes(int ld, int lf) { return ld | (lf << 8); }
-
     void density_with(flyg_eam_s& E, Shifts const& S, PairArgs const& A, int precision, int L, double4* pf) {
       switch (L) {
         case 4:
@@ -594,49 +962,15 @@ namespace flyg {
       }
     }
 
-    void gradient_with(flyg_eam_s& E, Shifts const& S, PairArgs const& A, double* d_grad, int precision, int lanes,
-                       double4* pf) {
-      density_with(E, S, A, precision, lanes & 0xff, pf);
-      force_with(E, S, A, d_grad, precision, lanes >> 8, pf);
-    }
-
-    // Lanes per atom row of each pass: the row sums do not depend on it (Acc16), so each pass's count is
-    // picked by timing that pass alone (the force pass reads the density pass's output of the last run).
-    int tuned_lanes(flyg_eam_s& E, Shifts const& S, PairArgs const& A, double* d_grad, int precision) {
-      if (E.lanes > 0) return pack_lanes(E.lanes, E.lanes);
-      auto key = std::make_pair(A.n, precision);
-      auto it = E.tuned.find(key);
-      if (it != E.tuned.end()) return it->second;
-      hipStream_t st = E.ctx->stream;
-      hipEvent_t a, b;
-      HIPCHK(hipEventCreate(&a));
-      HIPCHK(hipEventCreate(&b));
-      auto best_of = [&](auto&& run) {
-        int best = 8;
-        float best_ms = 1e30f;
-        for (int L : {4, 8, 16}) {
-          run(L);   // warm
-          HIPCHK(hipEventRecord(a, st));
-          for (int r = 0; r < 3; ++r) run(L);
-          HIPCHK(hipEventRecord(b, st));
-          HIPCHK(hipEventSynchronize(b));
-          float ms = 0;
-          HIPCHK(hipEventElapsedTime(&ms, a, b));
-          if (ms < best_ms) {
-            best_ms = ms;
-            best = L;
-          }
-        }
-        return best;
-      };
-      int const ld = best_of([&](int L) { density_with(E, S, A, precision, L, E.posf.get()); });
-      density_with(E, S, A, precision, ld, E.posf.get());
-      int const lf = best_of([&](int L) { force_with(E, S, A, d_grad, precision, L, E.posf.get()); });
-      (void)hipEventDestroy(a);
-      (void)hipEventDestroy(b);
-      int const lanes = pack_lanes(ld, lf);
-      E.tuned[key] = lanes;
-      return lanes;
+    // Lanes per atom row of the plain-row passes.  The row sums do not depend on them (Acc16).  16 unless the handle
+    // names a count: more lanes shorten each row's chain of dependent gathers, which is what bounds the sizes left to
+    // these passes.  Density / force, us, FP64 at 16, 8 and 4 lanes: 8.2k atoms 6.6/8.1, 9.6/11.5, 13.4/17.8; 16k
+    // 9.4/10.2, 8.5/13.4, 11.3/14.8.  Timing the three counts on a potential's first call cost 24 launches and
+    // could keep a slower one.
+    void gradient_with(flyg_eam_s& E, Shifts const& S, PairArgs const& A, double* d_grad, int precision, double4* pf) {
+      int const L = E.lanes > 0 ? E.lanes : 16;
+      density_with(E, S, A, precision, L, pf);
+      force_with(E, S, A, d_grad, precision, L, pf);
     }
   }  // namespace
 
@@ -646,7 +980,7 @@ namespace flyg {
     require(E.tab.rc <= nl.rc, "r_cut is bigger than the internal r_cut of the list");
     E.posf.reserve(nl.n);
     Shifts S = shifts_of(nl.box);
-    if (E.timing) {   // the pair covers the species gather too (and, on a first call, the lane tuning)
+    if (E.timing) {   // the pair covers the species gather too
       if (E.events_used == E.events.size()) {
         hipEvent_t a, b;
         HIPCHK(hipEventCreate(&a));
@@ -655,9 +989,14 @@ namespace flyg {
       }
       HIPCHK(hipEventRecord(E.events[E.events_used].first, E.ctx->stream));
     }
-    PairArgs A = slot_args(E, nl, types, frozen);
-    int const lanes = tuned_lanes(E, S, A, d_grad, precision);
-    gradient_with(E, S, A, d_grad, precision, lanes, E.posf.get());
+    if (nl.tiled && E.lanes <= 0) {
+      TileArgs A = tile_args(E, nl, types, frozen);
+      tile_density(E, S, A, false, precision, E.posf.get());
+      A.pos = E.posf.get();
+      tile_force(E, S, A, d_grad, precision);
+    } else {
+      gradient_with(E, S, pair_args(E, nl, types, frozen), d_grad, precision, E.posf.get());
+    }
     if (E.timing) HIPCHK(hipEventRecord(E.events[E.events_used++].second, E.ctx->stream));
     HIPCHK(hipGetLastError());
   }
@@ -702,11 +1041,7 @@ namespace flyg {
     require(pf != nullptr, "no scratch address for this device (its context was not created)");
     Shifts S = shifts_of(nl.box);
     PairArgs A = pair_args(E, nl, d_types, d_frozen);
-    // The lanes per atom row change no result bit: a fixed choice, or an earlier tuning, without timing.
-    int lanes = E.lanes > 0 ? pack_lanes(E.lanes, E.lanes) : pack_lanes(8, 8);
-    auto it = E.tuned.find(std::make_pair(A.n, precision));
-    if (E.lanes <= 0 && it != E.tuned.end()) lanes = it->second;
-    gradient_with(E, S, A, d_grad, precision, lanes, pf);
+    gradient_with(E, S, A, d_grad, precision, pf);
     HIPCHK(hipGetLastError());
   }
 

@@ -2,7 +2,6 @@
 #pragma once
 
 #include <istream>
-#include <map>
 #include <memory>
 #include <string>
 #include <vector>
@@ -68,10 +67,9 @@ struct flyg_eam_s {
   flyg::DBuf<int> hess_ids;     // its atom indices
   std::vector<uint32_t> last_types;
   std::vector<uint8_t> last_frozen;
-  int lanes = 0;                                   // lanes per atom row, 0 = timed choice
-  int staged_single = -1;                          // one species in the staged host types, else -1
-  long staged_n = -1;                              // atoms in the staged copy (types/frozen), -1 = none
-  std::map<std::pair<long, int>, int> tuned;       // (atoms, precision) -> lanes: density | force << 8
+  int lanes = 0;                // lanes per atom row, 0 = the library's choice
+  int staged_single = -1;       // one species in the staged host types, else -1
+  long staged_n = -1;           // atoms in the staged copy (types/frozen), -1 = none
   // Optional kernel timing of gradient calls: one event pair around each call's kernels.
   bool timing = false;
   std::vector<std::pair<hipEvent_t, hipEvent_t>> events;
@@ -107,16 +105,25 @@ struct flyg_list_s {
   flyg::DBuf<unsigned> nbr;      // n x K packed entries
   flyg::DBuf<int> ncnt;          // entries per atom
   // The gradient passes' layout, made at each rebuild: the real atoms in cell order (slot k holds atom
-  // order[k], rank[i] is atom i's slot), their positions by slot (kept current by update), and the rows
-  // by slot with neighbour indices given as slots (the same entries in the same order as nbr).
+  // order[k], rank[i] is atom i's slot) and their positions by slot (kept current by update).
   flyg::DBuf<int> order, rank;
   // gpos's w slot holds the species of each slot for a multi-species gradient (written with the slot-order
   // types; update keeps it): those of the staged host types with stamp wtype_stamp, if wtype_build is the
   // current build_id, else of the last gradient call's types.
   flyg::DBuf<double4> gpos;
   long wtype_stamp = -1, wtype_build = -1;
-  flyg::DBuf<unsigned> grow;
-  flyg::DBuf<int> gcnt;
+  // Tiles (boxes of cells): a pair kernel's workgroup stages the positions of a tile's cells and of the cells
+  // around it in LDS and walks its atoms' rows through 16-bit indices into that stage.  sslot: the
+  // sorted entries (reals and images, cell by cell) as (shift, slot); rows: by slot, rowK entries of
+  // room, in blocks of 32 whose entry k lies at 2 (k mod 16) + (k / 16 mod 2), so a lane of 16 loads two at a time.
+  flyg::TileGrid tile{};
+  bool tiled = false;            // rows and sslot belong to this build
+  int tile_level = 0;            // tile shapes found too full for LDS with this atom count are skipped
+  int tile_most = 0;             // entries staged by the fullest tile
+  int rowK = 0;
+  flyg::DBuf<unsigned> sslot;
+  flyg::DBuf<unsigned> rows;     // two entries a word
+  flyg::DBuf<int> gcnt;          // entries per slot
   flyg::DBuf<int> scan_tmp;
   flyg::DBuf<double> stage;      // host staging of xyz vectors
   flyg::DBuf<unsigned> lstate;   // device build counters: two sets, used in turn
@@ -151,12 +158,6 @@ namespace flyg {
     uint32_t const* types;
     uint8_t const* frozen;
     int t0;   // the one species present (-1: several or unknown); read by the single-species kernels
-    // Null: rows, positions and types are by atom.  Otherwise they are by slot of the list's cell-order
-    // layout (types gathered into slot order) and order[slot] is the atom, for frozen flags and gradients.
-    int const* order = nullptr;
-    // The w slot of pos holds each atom's species (as a double), so a neighbour's species arrives with
-    // its position; set for the slot layout with several species.
-    bool type_in_w = false;
   };
   // Image shift of a packed entry: sum_a s_a * basis column a, s_a in {-1, 0, 1}.  Exact for
   // orthorhombic boxes (each component is 0 or +-L), computed in registers (no table lookup).

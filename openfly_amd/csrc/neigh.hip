@@ -9,7 +9,8 @@
 //   4. scatter of the packed ids by cell, then each cell sorted by packed id, so the result does not
 //      depend on the atomics
 //   5. k_build_rows: every (real, image) of an atom's 27 cells with d^2 < r_cut^2 (strict,
-//      list.cpp:146,159) goes to its row of an ELL table: n rows x K packed 32-bit entries.
+//      list.cpp:146,159) goes to its row of an ELL table: n rows x K packed 32-bit entries, and, when the list
+//      is tiled, to its row of 16-bit indices into the tile's staged entries.
 // Six launches and one synchronisation; the state the host needs is written to pinned memory.
 // The distance tests, canonical images and ghost chains round exactly like the reference's FP64
 // expressions (no FMA contraction), so the pair sets equal the reference's at rebuild time.
@@ -342,8 +343,19 @@ namespace flyg {
                                  int const* __restrict__ ecell, long n, long gcap, unsigned const* __restrict__ st,
                                  int const* __restrict__ cstart, long nc1, unsigned const* __restrict__ usid,
                                  double4* __restrict__ spos, unsigned* __restrict__ sid, int* __restrict__ rslot,
-                                 int* __restrict__ order, int* __restrict__ rank_of, double4* __restrict__ gpos) {
+                                 int* __restrict__ order, int* __restrict__ rank_of, double4* __restrict__ gpos,
+                                 TileGrid tg, unsigned* __restrict__ most) {
       long e = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
+      if (e < tg.ntiles) {   // entries that tile e stages
+        int const t = static_cast<int>(e);
+        int sum = 0;
+        for (int q = 0; q < 16; ++q) {
+          int cb, ce;
+          tg.line(true, t % tg.nt[0], t / tg.nt[0] % tg.nt[1], t / (tg.nt[0] * tg.nt[1]), q, cb, ce);
+          sum += cstart[ce] - cstart[cb];
+        }
+        atomicMax(most, static_cast<unsigned>(sum));
+      }
       if (e >= live_entries(st, n, gcap)) return;
       int c = ecell[e];
       unsigned id = eid[e];
@@ -379,21 +391,31 @@ namespace flyg {
     // Small systems are bound by the chain of loads (A = 1: every atom a wavefront), large ones by the
     // candidates' L1 lookups (A = 4 loads them a quarter as often); BUILD_WIDE is where the two cross.
     //
-    // Each row is written twice: by atom with atom indices (nbr) and by slot with slot indices (grow, the
-    // gradient layout).  hst (pinned): [0] ghosts, [1] set when a row overflowed, [3] overflow bits.
+    // A tiled list gets each row twice: by atom with atom indices (nbr), and by slot with indices into the tile's stage
+    // (the candidate's place in the tile's halo: the lines' entries one after the other).  hst (pinned): [0] ghosts,
+    // [1] set when a row overflowed, [2] entries of the fullest tile, [3] overflow bits.
     constexpr long BUILD_WIDE = 24000;
 
-    template <int A>
+    template <int A, bool TILED>
     __global__ __launch_bounds__(TPB) void k_build_rows(GridDesc g, double4 const* __restrict__ spos,
                                                         unsigned const* __restrict__ sid, int const* __restrict__ cstart,
                                                         int const* __restrict__ rslot, long n, unsigned* __restrict__ nbr,
                                                         int* __restrict__ ncnt, int K, unsigned* __restrict__ st,
                                                         int const* __restrict__ order, int const* __restrict__ rank_of,
-                                                        unsigned* __restrict__ grow, int* __restrict__ gcnt,
+                                                        TileGrid tg, unsigned* __restrict__ sslot, long live_cap,
+                                                        unsigned* __restrict__ rows, int rowK, int* __restrict__ gcnt,
                                                         unsigned* __restrict__ hst) {
       if (blockIdx.x == 0 && threadIdx.x == 0) {
         hst[0] = st[0];
+        hst[2] = st[2];
         hst[3] = st[3];
+      }
+      if constexpr (TILED) {
+        long const live = live_entries(st, n, live_cap);
+        for (long s = blockIdx.x * static_cast<long>(TPB) + threadIdx.x; s < live; s += static_cast<long>(gridDim.x) * TPB) {
+          unsigned const en = sid[s];
+          sslot[s] = (en & ~NB_IDX_MASK) | static_cast<unsigned>(rank_of[en & NB_IDX_MASK]);
+        }
       }
       int const lane = static_cast<int>(threadIdx.x & 63);
       int const wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
@@ -401,6 +423,7 @@ namespace flyg {
       if (slot0 >= n) return;   // whole wavefronts leave together
       int const na = static_cast<int>(min(static_cast<long>(A), n - slot0));
       __shared__ unsigned ring[TPB / 64][A][128];
+      __shared__ unsigned short ring16[TILED ? TPB / 64 : 1][A][128];
       double const rc2 = g.rc * g.rc;
       int atom[A], self[A], cell[A], cx[A], cy[A], cz[A], cnt[A];
       double xi[A][3];
@@ -430,7 +453,13 @@ namespace flyg {
         if (k < c && k < K) {
           unsigned const en = ring[wave][a][k & 127];
           nbr[atom[a] * static_cast<long>(K) + k] = en;
-          grow[(slot0 + a) * K + k] = (en & ~NB_IDX_MASK) | static_cast<unsigned>(rank_of[en & NB_IDX_MASK]);
+        }
+        if constexpr (TILED) {   // two blocks of 32 entries, two entries a lane
+          int const k2 = k0 + (lane >> 4) * 32 + (lane & 15);
+          if (lane < 32 && k2 < c && k2 < K) {
+            unsigned const w = ring16[wave][a][k2 & 127] | (static_cast<unsigned>(ring16[wave][a][(k2 + 16) & 127]) << 16);
+            rows[((slot0 + a) * rowK + k0) / 2 + lane] = w;
+          }
         }
         __builtin_amdgcn_wave_barrier();
       };
@@ -446,6 +475,23 @@ namespace flyg {
             z0 = cz[a];
           }
         int rb = 0, re = 0;   // lane l < 9: range l
+        int loc = 0;          // ... and what turns a place in the sorted entries into one in the tile's stage
+        if constexpr (TILED) {
+          int const tx = tg.of(0, x), ty = tg.of(1, y0), tz = tg.of(2, z0);
+          int const q = lane & 15;
+          int cb, ce;
+          tg.line(true, tx, ty, tz, q, cb, ce);
+          int const lb = cstart[cb], len = cstart[ce] - lb;
+          int incl = len;
+#pragma unroll
+          for (int o = 1; o < 16; o <<= 1) {
+            int const t = __shfl_up(incl, o, 16);
+            if (q >= o) incl += t;
+          }
+          int const shift = (incl - len) - lb;   // by line of the tile
+          int const ly = y0 - 1 + lane % 3 - tg.halo_lo(1, ty), lz = z0 - 1 + lane / 3 - tg.halo_lo(2, tz);
+          loc = __shfl(shift, (ly + 4 * lz) & 15, 64);   // of a line outside the grid: not used
+        }
         if (lane < 9) {
           int const y = y0 - 1 + lane % 3, z = z0 - 1 + lane / 3;
           if (y >= 0 && y < g.shape[1] && z >= 0 && z < g.shape[2]) {
@@ -454,7 +500,7 @@ namespace flyg {
             re = cstart[min(x + 1, g.shape[0] - 1) * g.prod[0] + line + 1];
           }
         }
-        auto test = [&](double4 const& q, unsigned en, int s) {
+        auto test = [&](double4 const& q, unsigned en, int s, int shift) {
           double const xn[3] = {q.x, q.y, q.z};   // far away on lanes without a candidate
 #pragma unroll
           for (int a = 0; a < A; ++a) {
@@ -463,20 +509,24 @@ namespace flyg {
             unsigned long long const m = __ballot(hit);
             int const before = __builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(m >> 32),
                                                          __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(m), 0u));
-            if (hit) ring[wave][a][(cnt[a] + before) & 127] = en;
+            if (hit) {
+              ring[wave][a][(cnt[a] + before) & 127] = en;
+              if constexpr (TILED) ring16[wave][a][(cnt[a] + before) & 127] = static_cast<unsigned short>(s + shift);
+            }
             int const c = cnt[a] + __popcll(m);
             if ((c ^ cnt[a]) & ~63) flush(a, cnt[a] & ~63, c & ~63);   // a block of 64 is full
             cnt[a] = c;
           }
         };
         for (int z = 0; z < 3; ++z) {
-          int b[3], e[3];
+          int b[3], e[3], sh[3];
           double4 q[3];
           unsigned en[3];
 #pragma unroll
           for (int u = 0; u < 3; ++u) {
             b[u] = __builtin_amdgcn_readlane(rb, 3 * z + u);
             e[u] = __builtin_amdgcn_readlane(re, 3 * z + u);
+            sh[u] = TILED ? __builtin_amdgcn_readlane(loc, 3 * z + u) : 0;
             int const s = b[u] + lane;
             en[u] = 0;
             q[u] = make_double4(1e200, 0.0, 0.0, 0.0);
@@ -487,7 +537,7 @@ namespace flyg {
           }
 #pragma unroll
           for (int u = 0; u < 3; ++u) {
-            test(q[u], en[u], b[u] + lane);
+            test(q[u], en[u], b[u] + lane, sh[u]);
             for (int s0 = b[u] + 64; s0 < e[u]; s0 += 64) {   // the rest of a long range
               int const s = s0 + lane;
               double4 c = make_double4(1e200, 0.0, 0.0, 0.0);
@@ -496,7 +546,7 @@ namespace flyg {
                 c = spos[s];
                 id = sid[s];
               }
-              test(c, id, s);
+              test(c, id, s, sh[u]);
             }
           }
         }
@@ -685,6 +735,47 @@ namespace flyg {
     }
   }
 
+  namespace {
+    // Tile shapes (cells), largest first.  A larger tile stages fewer entries per atom (8, 12, 18 of them) but
+    // there are fewer workgroups, each walking more rows: the largest shape that leaves TILE_LEAST tiles, a little
+    // over two for each of the 256 CUs, is taken.  Update + gradient, us, mixed form, one species, 2x2x2 / 1x2x2 / 1x1x2 /
+    // plain rows: 27.6k atoms (216 / 396 / 726 tiles) 86 / 67 / 53 / 53, 44k (343 / 637 / 1183) 96 / 75 / 78 / 81,
+    // 93k (729 / 1377 / 2601) 122 / 134 / 134 / 153, 1.03M 500 / 550 / 640 / 750; below, the plain rows are faster
+    // (16k: 40 us against 47).
+    constexpr int TILE_SHAPES[][3] = {{2, 2, 2}, {1, 2, 2}, {1, 1, 2}};
+    constexpr int TILE_KINDS = 3;
+    constexpr int TILE_LEAST = 600;
+
+    TileGrid tile_grid(GridDesc const& g, int level) {
+      TileGrid t{};
+      t.ntiles = 1;
+      for (int k = 0; k < 3; ++k) {
+        t.d[k] = TILE_SHAPES[level][k];
+        t.shape[k] = g.shape[k];
+        t.prod[k] = g.prod[k];
+        t.nt[k] = std::max(1, (g.shape[k] - 2 + t.d[k] - 1) / t.d[k]);
+        t.ntiles *= t.nt[k];
+      }
+      t.nc1 = g.ncells + 1l;
+      return t;
+    }
+
+    bool choose_tiles(flyg_list_s& nl, long n) {
+      GridDesc const& g = nl.grid;
+      double const inner = static_cast<double>(g.shape[0] - 2) * (g.shape[1] - 2) * (g.shape[2] - 2);
+      for (int level = nl.tile_level; level < TILE_KINDS; ++level) {
+        TileGrid const t = tile_grid(g, level);
+        double const staged = n / inner * (t.d[0] + 2) * (t.d[1] + 2) * (t.d[2] + 2);
+        if (staged > 0.9 * TILE_MOST || t.ntiles < TILE_LEAST) continue;
+        if (n < 16l * t.ntiles) return false;   // a gas: tiles of a few atoms
+        nl.tile = t;
+        nl.tile_level = level;
+        return true;
+      }
+      return false;
+    }
+  }  // namespace
+
   // One rebuild costs one host synchronisation: capacities (ghost slots, row length) come from the
   // previous build; the device records what it needed and the build is redone only on overflow.
   void list_rebuild(flyg_list_s& nl, double const* d_xyz, long n) {
@@ -697,6 +788,7 @@ namespace flyg {
     if (n != nl.n) {
       nl.gcap = 0;
       nl.K = 0;
+      nl.tile_level = 0;
     }
     nl.n = n;
     if (nl.gcap == 0) nl.gcap = std::max(4096l, n);
@@ -719,7 +811,7 @@ namespace flyg {
     }
     nl.counters_clear = false;
 
-    for (int attempt = 0; attempt < 3; ++attempt) {
+    for (int attempt = 0; attempt < 3 + TILE_KINDS; ++attempt) {
       // Two sets of state words in turn: the scan clears the other build's.
       unsigned* dst = nl.lstate.get() + 4 * nl.parity;
       unsigned* other = nl.lstate.get() + 4 * (1 - nl.parity);
@@ -733,7 +825,13 @@ namespace flyg {
       nl.sid.reserve(cap);
       nl.usid.reserve(cap);
       nl.nbr.reserve(static_cast<std::size_t>(n) * nl.K);
-      nl.grow.reserve(static_cast<std::size_t>(n) * nl.K);
+      nl.tiled = choose_tiles(nl, n);
+      TileGrid const tg = nl.tiled ? nl.tile : TileGrid{};
+      nl.rowK = (nl.K + 31) / 32 * 32;
+      if (nl.tiled) {
+        nl.sslot.reserve(cap);
+        nl.rows.reserve(static_cast<std::size_t>(n) * nl.rowK / 2);
+      }
       nl.hstate[1] = 0;
       if (nl.box.ortho) {
         k_entries<true><<<nblk(n, ETPB), ETPB, 0, st>>>(nl.box, nl.grid, d_xyz, n, nl.pos.get(), nl.ent.get(),
@@ -747,18 +845,19 @@ namespace flyg {
       exclusive_scan(ctx, nl.ccount.get(), nl.cstart.get(), static_cast<int>(2 * nc1), nl.scan_tmp, other);
       k_scatter_ids<<<nblk(cap, TPB), TPB, 0, st>>>(nl.eid.get(), nl.ecell.get(), nl.earr.get(), n, nl.gcap, dst,
                                                     nl.cstart.get(), nl.usid.get());
-      k_rank_place<<<nblk(cap, TPB), TPB, 0, st>>>(nl.ent.get(), nl.eid.get(), nl.ecell.get(), n, nl.gcap, dst,
+      k_rank_place<<<nblk(std::max<long>(cap, tg.ntiles), TPB), TPB, 0, st>>>(nl.ent.get(), nl.eid.get(), nl.ecell.get(), n, nl.gcap, dst,
                                                    nl.cstart.get(), nc1, nl.usid.get(), nl.spos.get(), nl.sid.get(),
-                                                   nl.rslot.get(), nl.order.get(), nl.rank.get(), nl.gpos.get());
+                                                   nl.rslot.get(), nl.order.get(), nl.rank.get(), nl.gpos.get(), tg, dst + 2);
       auto rows = [&](auto k, int A) {
         k<<<nblk(n, A * (TPB / 64)), TPB, 0, st>>>(nl.grid, nl.spos.get(), nl.sid.get(), nl.cstart.get(), nl.rslot.get(), n,
                                                    nl.nbr.get(), nl.ncnt.get(), nl.K, dst, nl.order.get(), nl.rank.get(),
-                                                   nl.grow.get(), nl.gcnt.get(), nl.hstate);
+                                                   tg, nl.sslot.get(), nl.gcap, nl.rows.get(), nl.rowK, nl.gcnt.get(),
+                                                   nl.hstate);
       };
       if (n < BUILD_WIDE) {
-        rows(k_build_rows<1>, 1);
+        nl.tiled ? rows(k_build_rows<1, true>, 1) : rows(k_build_rows<1, false>, 1);
       } else {
-        rows(k_build_rows<4>, 4);
+        nl.tiled ? rows(k_build_rows<4, true>, 4) : rows(k_build_rows<4, false>, 4);
       }
       HIPCHK(hipGetLastError());
       HIPCHK(hipStreamSynchronize(st));
@@ -772,6 +871,11 @@ namespace flyg {
         HIPCHK(hipMemcpyAsync(nl.hstate, dst, 4 * sizeof(unsigned), hipMemcpyDeviceToHost, st));
         HIPCHK(hipStreamSynchronize(st));
         nl.K = (static_cast<int>(nl.hstate[1]) + 15) / 16 * 16 + 16;
+        continue;
+      }
+      nl.tile_most = static_cast<int>(nl.hstate[2]);
+      if (nl.tiled && nl.tile_most > TILE_MOST) {   // a tile too full for its stage: smaller tiles, or none
+        ++nl.tile_level;
         continue;
       }
       static std::atomic<long> builds{0};

@@ -435,3 +435,58 @@ def test_staged_atoms_follow_stage_calls_and_rebuilds(ctx, wen_orc):
     pot.stage(t1[:-1], f[:-1])
     with pytest.raises(fa.FlyError, match="staged"):
         pot.gradient(None, None, nl)
+
+
+TILED = {   # cells: the tile shape a list with 0.6 A of skin takes
+    24: "1x1x2", 30: "1x2x2", 36: "2x2x2"}
+
+
+@pytest.mark.parametrize("cells,tilt,slab,single", [(24, 0.0, False, False), (24, 0.1, True, True), (30, 0.07, False, False),
+                                                    (30, 0.0, True, True), (36, 0.0, False, False)])
+def test_tiled_passes_equal_plain_rows(ctx, cells, tilt, slab, single):
+    # Lists of these sizes evaluate tile by tile; a handle with a fixed lane count walks the plain rows.  The
+    # same entries in the same order: gradients and energies are equal bit for bit, in periodic, sheared and slab boxes
+    # (edge tiles, image shifts), with frozen atoms, after moves, and with atoms on the box faces.
+    print(f"case tiles {TILED[cells]} tilt={tilt} slab={slab} single={single}", flush=True)
+    s = systems.fe_x_alloy(cells, cells=cells)
+    basis = s.basis.copy()
+    pos = s.pos.copy()
+    pos = np.where(np.abs(pos) < 0.1, 0.0, pos)   # a layer of atoms exactly on the box faces
+    shear = np.eye(3)
+    shear[0, 1] = tilt
+    basis, pos = shear @ basis, pos @ shear.T
+    if slab:
+        basis[2, 2] += 9.0
+    types = np.zeros_like(s.types) if single else s.types
+    rng = np.random.default_rng(cells)
+    frozen = (rng.random(s.n) < 0.2).astype(np.uint8)
+    nl = fa.List(ctx, fa.Box(basis, (1, 1, 0 if slab else 1)), 5.9)
+    nl.rebuild(pos)
+    nl.update(rng.uniform(-0.05, 0.05, pos.shape))
+    pot = fa.EAM(ctx, systems.potential_path(("Fe", "X")))
+    for precision in (fa.FP64, fa.MIXED):
+        pot.set_precision(precision)
+        got = {}
+        for lanes in (0, 8):
+            pot.set_lanes(lanes)
+            got[lanes] = pot.energy(types, frozen, nl), pot.gradient(types, frozen, nl).copy()
+        assert got[0][0] == got[8][0]
+        assert np.array_equal(got[0][1], got[8][1])
+
+
+def test_crowded_cell_falls_back(ctx):
+    # 1300 more atoms around one cell of a 28k-atom system: no tile there fits the stage, the plain rows are used.
+    s = systems.fe_x_alloy(5, cells=24)
+    g = np.stack(np.meshgrid(np.arange(10), np.arange(10), np.arange(13), indexing="ij"), axis=-1).reshape(-1, 3)
+    pos = np.concatenate([s.pos, 10.0 + 1.85 * g])
+    types = np.concatenate([s.types, np.ones(len(g), np.uint32)])
+    frozen = np.zeros(len(pos), np.uint8)
+    pot = fa.EAM(ctx, systems.potential_path(("Fe", "X")))
+    nl = fa.List(ctx, fa.Box(s.basis), 5.9)
+    for p, t in ((s.pos, s.types), (pos, types), (s.pos, s.types)):   # tiles, too full for them, tiles again
+        nl.rebuild(p)
+        f = frozen[:len(p)]
+        pot.set_lanes(0)
+        a = pot.gradient(t, f, nl).copy()
+        pot.set_lanes(8)
+        assert np.array_equal(a, pot.gradient(t, f, nl))
