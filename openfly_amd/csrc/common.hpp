@@ -225,6 +225,20 @@ namespace flyg {
     fp = c.y + t * (2.0 * c.z + t * 3.0 * c.w);
   }
 
+  // f' and f'' from one segment fetch.
+  __device__ inline void spl64_12(EAMTables const& T, SplineDesc const& s, double x, double& fp, double& fpp, unsigned& err) {
+    int i;
+    double t;
+    if (!seg64(s, x, i, t)) {
+      err |= ERR_SPLINE_OOB;
+      fp = fpp = 0.0;
+      return;
+    }
+    double4 c = T.c64[s.off + i];
+    fp = c.y + t * (2.0 * c.z + t * 3.0 * c.w);
+    fpp = 2.0 * c.z + 6.0 * t * c.w;
+  }
+
   // FP32 pair arithmetic on FP32 coefficients (mixed-precision form).
   template <int D>
   __device__ inline float spl32f(EAMTables const& T, SplineDesc const& s, float x, unsigned& err) {

@@ -591,6 +591,45 @@ namespace flyg {
       if (e) atomicOr(err, e);
     }
 
+    // ---- Hessian-vector product ---------------------------------------------------------------------
+    // One reciprocal and one segment fetch per table and pair; rows from the plain list (L lanes an atom, small
+    // systems) or tile by tile with positions, the masked direction v and (F', dF') staged in LDS, where
+    // a pair takes no gather but its table segments (row gathers: 51 + 122 us at 54.5k atoms).
+
+    struct HvpSum {
+      double x = 0, y = 0, z = 0;
+    };
+
+    __device__ inline void hvp_density_pair(EAMTables const& T, SplineDesc const& sa, double dx, double dy, double dz, double r2,
+                                            double vx, double vy, double vz, double& rho, double& drho, unsigned& e) {
+      double const r = sqrt(r2);
+      double f, fp;
+      spl64_ffp(T, sa, r, f, fp, e);
+      rho += f;
+      drho += fp * ((dx * vx + dy * vy + dz * vz) / r);
+    }
+
+    // dv = v_a - v_g, (F', dF') of the row's atom (di) and of the neighbour (dj).
+    template <bool MULTI>
+    __device__ inline void hvp_force_pair(EAMTables const& T, SplineDesc const& sv, SplineDesc const& sa, SplineDesc const& sb,
+                                          bool same, double dx, double dy, double dz, double r2, double vx, double vy,
+                                          double vz, double2 di, double2 dj, HvpSum& h, unsigned& e) {
+      double const r = sqrt(r2), inv = 1.0 / r;
+      double const ux = dx * inv, uy = dy * inv, uz = dz * inv;
+      double const s = ux * vx + uy * vy + uz * vz;
+      double vp, vpp, pa, paa;
+      spl64_12(T, sv, r, vp, vpp, e);
+      spl64_12(T, sa, r, pa, paa, e);   // phi_{a->g}
+      double pb = pa, pbb = paa;        // phi_{g->a}
+      if (MULTI && !same) spl64_12(T, sb, r, pb, pbb, e);
+      double const m = vp + di.x * pa + dj.x * pb;
+      double const dm = (vpp + di.x * paa + dj.x * pbb) * s + di.y * pa + dj.y * pb;
+      double const q = m * inv;
+      h.x -= dm * ux + q * (vx - ux * s);
+      h.y -= dm * uy + q * (vy - uy * s);
+      h.z -= dm * uz + q * (vz - uz * s);
+    }
+
     template <int L, bool MULTI>
     __global__ __launch_bounds__(NT) void k_hvp_density(EAMTables T, Shifts S, PairArgs A, double const* __restrict__ v,
                                                         double2* __restrict__ dfp, unsigned* __restrict__ err) {
@@ -609,30 +648,20 @@ namespace flyg {
         int const c = min(A.cnt[i], A.K);
         unsigned const* row = A.nbr + i * static_cast<long>(A.K);
         for (int k = lane; k < c; k += L) {
-          unsigned en = row[k];
-          unsigned j = en & NB_IDX_MASK;
-          double3 sh = S.of(en >> NB_SHIFT_BITS);
-          double4 pj = A.pos[j];
-          double dx = (pj.x + sh.x) - pi.x, dy = (pj.y + sh.y) - pi.y, dz = (pj.z + sh.z) - pi.z;
-          double r2 = dx * dx + dy * dy + dz * dz;
-          if (r2 < T.rc2) {
-            double r = sqrt(r2);
-            int tj = MULTI ? checked_type(A.types[j], T.ntypes, e) : A.t0;
-            double f, fp;
-            spl64_ffp(T, T.phi[tj + T.ntypes * ti], r, f, fp, e);
-            rho += f;
-            bool fj = A.frozen[j];
-            double vjx = fj ? 0 : v[3 * j], vjy = fj ? 0 : v[3 * j + 1], vjz = fj ? 0 : v[3 * j + 2];
-            double s = (dx * (vjx - vix) + dy * (vjy - viy) + dz * (vjz - viz)) / r;
-            drho += fp * s;
-          }
+          PairGeo const p = geo(S, A.pos, row[k], pi);
+          long const j = p.j;
+          bool const fj = A.frozen[j];
+          double vjx = fj ? 0 : v[3 * j], vjy = fj ? 0 : v[3 * j + 1], vjz = fj ? 0 : v[3 * j + 2];
+          int tj = MULTI ? checked_type(A.types[j], T.ntypes, e) : A.t0;
+          if (p.r2 < T.rc2)
+            hvp_density_pair(T, T.phi[tj + T.ntypes * ti], p.dx, p.dy, p.dz, p.r2, vjx - vix, vjy - viy, vjz - viz, rho, drho, e);
         }
       }
       rho = group_sum<L>(rho);
       drho = group_sum<L>(drho);
       if (act && lane == 0) {
-        double fp = spl64<1>(T, T.F[ti], rho, e);
-        double fpp = spl64<2>(T, T.F[ti], rho, e);
+        double fp, fpp;
+        spl64_12(T, T.F[ti], rho, fp, fpp, e);
         dfp[i] = make_double2(fp, fpp * drho);
       }
       if (e) atomicOr(err, e);
@@ -647,7 +676,7 @@ namespace flyg {
       int lane = static_cast<int>(gid % L);
       bool inr = i < A.n;
       bool act = inr && !A.frozen[i];
-      double hx = 0, hy = 0, hz = 0;
+      HvpSum h;
       unsigned e = 0;
       if (act) {
         double4 pi = A.pos[i];
@@ -657,46 +686,97 @@ namespace flyg {
         int const c = min(A.cnt[i], A.K);
         unsigned const* row = A.nbr + i * static_cast<long>(A.K);
         for (int k = lane; k < c; k += L) {
-          unsigned en = row[k];
-          unsigned j = en & NB_IDX_MASK;
-          double3 sh = S.of(en >> NB_SHIFT_BITS);
-          double4 pj = A.pos[j];
-          double dx = (pj.x + sh.x) - pi.x, dy = (pj.y + sh.y) - pi.y, dz = (pj.z + sh.z) - pi.z;
-          double r2 = dx * dx + dy * dy + dz * dz;
-          if (r2 < T.rc2) {
-            double r = sqrt(r2);
-            int tj = MULTI ? checked_type(A.types[j], T.ntypes, e) : A.t0;
-            double2 dj = dfp[j];
-            bool fj = A.frozen[j];
-            double vjx = fj ? 0 : v[3 * j], vjy = fj ? 0 : v[3 * j + 1], vjz = fj ? 0 : v[3 * j + 2];
-            double ux = dx / r, uy = dy / r, uz = dz / r;
-            double dvx = vjx - vix, dvy = vjy - viy, dvz = vjz - viz;
-            double s = ux * dvx + uy * dvy + uz * dvz;
-            double vp = spl64<1>(T, T.V[vidx(T, ti, tj)], r, e);
-            double vpp = spl64<2>(T, T.V[vidx(T, ti, tj)], r, e);
-            double pa = spl64<1>(T, T.phi[tj + T.ntypes * ti], r, e);   // phi'_{a->g}
-            double paa = spl64<2>(T, T.phi[tj + T.ntypes * ti], r, e);
-            double pb = pa, pbb = paa;
-            if (MULTI) {
-              pb = spl64<1>(T, T.phi[ti + T.ntypes * tj], r, e);          // phi'_{g->a}
-              pbb = spl64<2>(T, T.phi[ti + T.ntypes * tj], r, e);
-            }
-            double m = vp + di.x * pa + dj.x * pb;
-            double dm = (vpp + di.x * paa + dj.x * pbb) * s + di.y * pa + dj.y * pb;
-            double q = m / r;
-            hx -= dm * ux + q * (dvx - ux * s);
-            hy -= dm * uy + q * (dvy - uy * s);
-            hz -= dm * uz + q * (dvz - uz * s);
-          }
+          PairGeo const p = geo(S, A.pos, row[k], pi);
+          long const j = p.j;
+          bool const fj = A.frozen[j];
+          double vjx = fj ? 0 : v[3 * j], vjy = fj ? 0 : v[3 * j + 1], vjz = fj ? 0 : v[3 * j + 2];
+          double2 const dj = dfp[j];
+          int tj = MULTI ? checked_type(A.types[j], T.ntypes, e) : A.t0;
+          if (p.r2 < T.rc2)
+            hvp_force_pair<MULTI>(T, T.V[vidx(T, ti, tj)], T.phi[tj + T.ntypes * ti], T.phi[ti + T.ntypes * tj], ti == tj, p.dx,
+                                  p.dy, p.dz, p.r2, vjx - vix, vjy - viy, vjz - viz, di, dj, h, e);
         }
       }
-      hx = group_sum<L>(hx);
-      hy = group_sum<L>(hy);
-      hz = group_sum<L>(hz);
-      if (inr && lane == 0) {
-        hv[3 * i] = act ? hx : 0.0;
-        hv[3 * i + 1] = act ? hy : 0.0;
-        hv[3 * i + 2] = act ? hz : 0.0;
+      h.x = group_sum<L>(h.x);
+      h.y = group_sum<L>(h.y);
+      h.z = group_sum<L>(h.z);
+      if (inr && lane < 3) hv[3 * i + lane] = act ? (lane == 0 ? h.x : (lane == 1 ? h.y : h.z)) : 0.0;
+      if (e) atomicOr(err, e);
+    }
+
+    // Tiled passes: the stage holds (x, y), (z, vz), (vx, vy) and, in the force pass, (F', dF') of every entry, and its
+    // species with several.  dfp by slot.
+    template <bool MULTI, bool FORCE>
+    __global__ __launch_bounds__(TT) void k_tile_hvp(EAMTables T, Shifts S, TileArgs A, double const* __restrict__ v,
+                                                     double2* __restrict__ dfp, double* __restrict__ hv,
+                                                     unsigned* __restrict__ err) {
+      extern __shared__ double2 s_stage[];
+      double2* const xy = s_stage;
+      double2* const zv = xy + A.cap;
+      double2* const vv = zv + A.cap;
+      double2* const df = vv + A.cap;
+      uint8_t* const typ = reinterpret_cast<uint8_t*>(df + (FORCE ? A.cap : 0));
+      __shared__ TileLds L;
+      __shared__ SplineDesc s_phi[MULTI ? MAX_TYPES * MAX_TYPES : 1], s_V[MULTI && FORCE ? MAX_TYPES * MAX_TYPES : 1];
+      if (MULTI && threadIdx.x < T.ntypes * T.ntypes) {
+        s_phi[threadIdx.x] = T.phi[threadIdx.x];
+        if (FORCE) s_V[threadIdx.x] = T.V[threadIdx.x];
+      }
+      unsigned e = 0;
+      stage_tile(A, S, L, xy, zv, [&](int k, unsigned slot) {
+        long const a = A.order[slot];
+        bool const f = A.frozen[a];
+        vv[k] = make_double2(f ? 0 : v[3 * a], f ? 0 : v[3 * a + 1]);
+        zv[k].y = f ? 0 : v[3 * a + 2];
+        if (FORCE) df[k] = dfp[slot];
+        if (MULTI) typ[k] = static_cast<uint8_t>(checked_type(A.types[slot], T.ntypes, e));
+      });
+      int const rows = L.oo[16];
+      int const l = threadIdx.x & 15;
+      for (int r = threadIdx.x >> 4; r < rows; r += TT / 16) {
+        int const q = line_of(L.oo, r);
+        long const i = L.os[q] + (r - L.oo[q]);
+        long const ia = A.order[i];
+        double4 const pi = A.pos[i];
+        int const c = min(A.cnt[i], A.K);
+        int const ti = MULTI ? checked_type(A.types[i], T.ntypes, e) : A.t0;
+        bool const fi = A.frozen[ia];
+        double const vix = fi ? 0 : v[3 * ia], viy = fi ? 0 : v[3 * ia + 1], viz = fi ? 0 : v[3 * ia + 2];
+        double2 const di = FORCE ? dfp[i] : make_double2(0, 0);
+        double rho = 0, drho = 0;
+        HvpSum h;
+        walk_tile(A.rows + i * A.rowW, FORCE && fi ? 0 : c, l, pi, T.rc2, xy, zv, [&](PairGeo const& p) {
+          double2 const w = vv[p.j];
+          int const tj = MULTI ? typ[p.j] : A.t0;
+          SplineDesc const& sa = MULTI ? s_phi[tj + T.ntypes * ti] : T.phi[tj + T.ntypes * ti];
+          if constexpr (FORCE) {
+            SplineDesc const& sv = MULTI ? s_V[vidx(T, ti, tj)] : T.V[vidx(T, ti, tj)];
+            hvp_force_pair<MULTI>(T, sv, sa, s_phi[MULTI ? ti + T.ntypes * tj : 0], ti == tj, p.dx, p.dy, p.dz, p.r2, w.x - vix,
+                                  w.y - viy, p.w - viz, di, df[p.j], h, e);
+          } else {
+            hvp_density_pair(T, sa, p.dx, p.dy, p.dz, p.r2, w.x - vix, w.y - viy, p.w - viz, rho, drho, e);
+          }
+        });
+        if constexpr (FORCE) {
+          double const hx = total16(h.x), hy = total16(h.y), hz = total16(h.z);
+          if (l < 3) hv[3 * ia + l] = fi ? 0.0 : (l == 0 ? hx : (l == 1 ? hy : hz));
+        } else {
+          rho = total16(rho);
+          drho = total16(drho);
+          if (l == 0) dfp[i] = make_double2(rho, drho);
+        }
+      }
+      if constexpr (!FORCE) {   // the embedding spline, a row a thread
+        __syncthreads();
+        for (int r = threadIdx.x; r < rows; r += TT) {
+          int const q = line_of(L.oo, r);
+          long const i = L.os[q] + (r - L.oo[q]);
+          int const ti = MULTI ? checked_type(A.types[i], T.ntypes, e) : A.t0;
+          double2 const d = dfp[i];
+          double fp, fpp;
+          spl64_12(T, T.F[ti], d.x, fp, fpp, e);
+          dfp[i] = make_double2(fp, fpp * d.y);
+        }
       }
       if (e) atomicOr(err, e);
     }
@@ -1051,16 +1131,32 @@ namespace flyg {
     require(E.tab.rc <= nl.rc, "r_cut is bigger than the internal r_cut of the list");
     E.dfp.reserve(nl.n);
     Shifts S = shifts_of(nl.box);
-    PairArgs A = pair_args(E, nl, types, frozen);
     hipStream_t st = E.ctx->stream;
     unsigned* err = E.ctx->dflags.get();
-    unsigned g = grid_for(nl.n, LANES);
+    if (nl.tiled && E.lanes <= 0) {
+      TileArgs const A = tile_args(E, nl, types, frozen);
+      unsigned const g = static_cast<unsigned>(A.G.ntiles);
+      std::size_t const t = A.t0 < 0 ? 1 : 0;
+      std::size_t const ld = static_cast<std::size_t>(A.cap) * (48 + t), lf = static_cast<std::size_t>(A.cap) * (64 + t);
+      if (A.t0 < 0) {
+        k_tile_hvp<true, false><<<g, TT, ld, st>>>(E.tab, S, A, d_v, E.dfp.get(), d_hv, err);
+        k_tile_hvp<true, true><<<g, TT, lf, st>>>(E.tab, S, A, d_v, E.dfp.get(), d_hv, err);
+      } else {
+        k_tile_hvp<false, false><<<g, TT, ld, st>>>(E.tab, S, A, d_v, E.dfp.get(), d_hv, err);
+        k_tile_hvp<false, true><<<g, TT, lf, st>>>(E.tab, S, A, d_v, E.dfp.get(), d_hv, err);
+      }
+      HIPCHK(hipGetLastError());
+      return;
+    }
+    PairArgs A = pair_args(E, nl, types, frozen);
+    constexpr int L = 16;
+    unsigned g = grid_for(nl.n, L);
     if (A.t0 < 0) {
-      k_hvp_density<LANES, true><<<g, NT, 0, st>>>(E.tab, S, A, d_v, E.dfp.get(), err);
-      k_hvp_force<LANES, true><<<g, NT, 0, st>>>(E.tab, S, A, d_v, E.dfp.get(), d_hv, err);
+      k_hvp_density<L, true><<<g, NT, 0, st>>>(E.tab, S, A, d_v, E.dfp.get(), err);
+      k_hvp_force<L, true><<<g, NT, 0, st>>>(E.tab, S, A, d_v, E.dfp.get(), d_hv, err);
     } else {
-      k_hvp_density<LANES, false><<<g, NT, 0, st>>>(E.tab, S, A, d_v, E.dfp.get(), err);
-      k_hvp_force<LANES, false><<<g, NT, 0, st>>>(E.tab, S, A, d_v, E.dfp.get(), d_hv, err);
+      k_hvp_density<L, false><<<g, NT, 0, st>>>(E.tab, S, A, d_v, E.dfp.get(), err);
+      k_hvp_force<L, false><<<g, NT, 0, st>>>(E.tab, S, A, d_v, E.dfp.get(), d_hv, err);
     }
     HIPCHK(hipGetLastError());
   }

@@ -18,6 +18,7 @@
 // add the shift vector to the live real position, so update() touches only the N real atoms.
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <numeric>
 
 #include "eam_host.hpp"
@@ -792,7 +793,14 @@ namespace flyg {
     }
     nl.n = n;
     if (nl.gcap == 0) nl.gcap = std::max(4096l, n);
-    if (nl.K == 0) nl.K = 64;
+    if (nl.K == 0) {
+      // Room for the rows of a uniform system and a fifth more: a first guess of 64 built most lists twice.
+      double const vol = std::fabs(nl.box.B[0][0] * (nl.box.B[1][1] * nl.box.B[2][2] - nl.box.B[1][2] * nl.box.B[2][1]) -
+                                   nl.box.B[0][1] * (nl.box.B[1][0] * nl.box.B[2][2] - nl.box.B[1][2] * nl.box.B[2][0]) +
+                                   nl.box.B[0][2] * (nl.box.B[1][0] * nl.box.B[2][1] - nl.box.B[1][1] * nl.box.B[2][0]));
+      double const mean = static_cast<double>(n) / vol * 4.18879 * nl.rc * nl.rc * nl.rc;
+      nl.K = std::max(64, (static_cast<int>(std::min(1.2 * mean, 512.0)) + 15) / 16 * 16);
+    }
     int const nc = nl.grid.ncells;
     long const nc1 = nc + 1;
     nl.lstate.reserve(8);

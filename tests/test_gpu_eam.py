@@ -472,6 +472,13 @@ def test_tiled_passes_equal_plain_rows(ctx, cells, tilt, slab, single):
             got[lanes] = pot.energy(types, frozen, nl), pot.gradient(types, frozen, nl).copy()
         assert got[0][0] == got[8][0]
         assert np.array_equal(got[0][1], got[8][1])
+    # Hessian-vector product, whose row sums are 60 terms in FP64: 60 roundings of 1e-16 of the largest term
+    v = rng.normal(size=pos.shape)
+    hv = {}
+    for lanes in (0, 8):
+        pot.set_lanes(lanes)
+        hv[lanes] = pot.hvp(types, frozen, nl, v).copy()
+    assert np.max(np.abs(hv[0] - hv[8])) <= 1e-13 * np.max(np.abs(hv[8]))
 
 
 def test_crowded_cell_falls_back(ctx):
