@@ -136,7 +136,7 @@ namespace flyg {
         unsigned const* row = A.nbr + i * static_cast<long>(A.K);
         walk_row<L>(row, c, lane, S, A.pos, pi, [&](int q, PairGeo const& p) {
           if (p.r2 < T.rc2) {
-            int tj = MULTI ? checked_type(A.types[p.j], T.ntypes, e) : A.t0;
+            int tj = MULTI ? checked_type(A.type_in_w ? static_cast<uint32_t>(p.w) : A.types[p.j], T.ntypes, e) : A.t0;
             if (MIX && !ENERGY) {
               float r2f = static_cast<float>(p.r2);
               float rf = r2f * __frsqrt_rn(r2f);
@@ -156,7 +156,7 @@ namespace flyg {
         spl64_ffp(T, T.F[ti], rt, f, fp, e);
         double const w = MIX && !ENERGY ? pack_fp_type(static_cast<float>(fp), ti) : fp;
         posf[i] = make_double4(pi.x, pi.y, pi.z, w);
-        if (ENERGY) eatom[i] = 0.5 * vt + f;
+        if (ENERGY) eatom[A.order ? A.order[i] : i] = 0.5 * vt + f;
       }
       if (e) atomicOr(err, e);
     }
@@ -188,10 +188,12 @@ namespace flyg {
         }
       };
       long gid = xcd_block(blockIdx.x, gridDim.x) * static_cast<long>(NT) + threadIdx.x;
-      long i = gid / L;
+      long i = gid / L;   // row: the atom, or its slot when A.order is set
       int lane = static_cast<int>(gid % L);
       bool inr = i < A.n;
+      long const ia = inr && A.order ? A.order[i] : i;   // the atom, for its frozen flag and gradient
       unsigned e = 0;
+      // The row's own data is loaded beside the frozen flag (not after it): the flag waits on `order`.
       double4 pi = make_double4(0.0, 0.0, 0.0, 0.0);
       int ti = MULTI ? 0 : A.t0;
       int c = 0;
@@ -201,7 +203,7 @@ namespace flyg {
         // Mixed form: the species the density pass packed beside F' (checked there).
         if (MULTI) ti = MIX ? packed_type(pi.w) : checked_type(A.types[i], T.ntypes, e);
       }
-      bool act = inr && !A.frozen[i];
+      bool act = inr && !A.frozen[ia];
       Acc16<L> gx, gy, gz;
       if (act) {
         unsigned const* row = A.nbr + i * static_cast<long>(A.K);
@@ -235,12 +237,12 @@ namespace flyg {
       double tx = gx.total(), ty = gy.total(), tz = gz.total();
       if (L >= 3 && inr && lane < 3) {
         double v = lane == 0 ? tx : (lane == 1 ? ty : tz);
-        grad[3 * i + lane] = act ? v : 0.0;
+        grad[3 * ia + lane] = act ? v : 0.0;
       }
       if (L < 3 && inr && lane == 0) {
-        grad[3 * i] = act ? tx : 0.0;
-        grad[3 * i + 1] = act ? ty : 0.0;
-        grad[3 * i + 2] = act ? tz : 0.0;
+        grad[3 * ia] = act ? tx : 0.0;
+        grad[3 * ia + 1] = act ? ty : 0.0;
+        grad[3 * ia + 2] = act ? tz : 0.0;
       }
       if (e) atomicOr(err, e);
     }
@@ -834,41 +836,58 @@ namespace flyg {
       }
     }
 
-    // The tiled passes run in the list's slot (cell) order: a workgroup's atoms are neighbours in space.
-    // With several species the types are gathered into slot order, and into the w slot of the slot-ordered
-    // positions (the density pass reads a neighbour's species from there): once per list build for staged
-    // host types (the library sees every change of them), on every call for device types.  Type stamps
-    // are unique across handles, so a list shared by several potentials or type arrays is re-gathered
+    // The gradient and energy passes run in the list's slot (cell) order: a workgroup's atoms are neighbours in
+    // space and so are the rows they read.  With several species the types are gathered into slot order, and into the
+    // w slot of the slot-ordered positions (the density pass reads a neighbour's species from there): once per list
+    // build for staged host types (the library sees every change of them), on every call for device types.  Type
+    // stamps are unique across handles, so a list shared by several potentials or type arrays is re-gathered
     // whenever another one wrote its w slots last.
+    uint32_t const* types_by_slot(flyg_eam_s& E, flyg_list_s& nl, uint32_t const* types) {
+      bool const staged = types == E.types.get();
+      bool const cached = staged && E.gtype_build == nl.build_id && E.gtype_stamp == E.types_stamp &&
+                          nl.wtype_build == nl.build_id && nl.wtype_stamp == E.types_stamp;
+      if (!cached) {
+        E.gtype_build = -1;   // the buffer may be reallocated: its contents are no longer known
+        nl.wtype_build = -1;
+        E.gtype.reserve(nl.n);
+        k_types_by_slot<<<static_cast<unsigned>((nl.n + 255) / 256), 256, 0, E.ctx->stream>>>(
+            types, nl.order.get(), nl.n, E.gtype.get(), nl.gpos.get());
+        HIPCHK(hipGetLastError());
+        if (staged) {
+          E.gtype_build = nl.build_id;
+          E.gtype_stamp = E.types_stamp;
+          nl.wtype_build = nl.build_id;
+          nl.wtype_stamp = E.types_stamp;
+        }
+      }
+      return E.gtype.get();
+    }
+
+    // Plain rows in slot order (a tiled list keeps them by atom only).
+    PairArgs slot_args(flyg_eam_s& E, flyg_list_s& nl, uint32_t const* types, uint8_t const* frozen) {
+      PairArgs A = pair_args(E, nl, types, frozen);
+      if (nl.tiled) return A;
+      A.pos = nl.gpos.get();
+      A.nbr = nl.rows.get();
+      A.cnt = nl.gcnt.get();
+      A.order = nl.order.get();
+      if (A.t0 < 0) {
+        A.types = types_by_slot(E, nl, types);
+        A.type_in_w = true;
+      }
+      return A;
+    }
+
     TileArgs tile_args(flyg_eam_s& E, flyg_list_s& nl, uint32_t const* types, uint8_t const* frozen) {
       PairArgs const P = pair_args(E, nl, types, frozen);
       TileArgs A{nl.tile,        nl.cstart.get(), nl.sslot.get(), nl.rows.get(), nl.rowK / 2, nl.K, nl.gcnt.get(),
                  nl.order.get(), nl.gpos.get(),   nullptr,        frozen,        P.t0,        0};
       A.cap = (nl.tile_most + 15) & ~15;
-      if (A.t0 < 0) {
-        bool const staged = types == E.types.get();
-        bool const cached = staged && E.gtype_build == nl.build_id && E.gtype_stamp == E.types_stamp &&
-                            nl.wtype_build == nl.build_id && nl.wtype_stamp == E.types_stamp;
-        if (!cached) {
-          E.gtype_build = -1;   // the buffer may be reallocated: its contents are no longer known
-          nl.wtype_build = -1;
-          E.gtype.reserve(nl.n);
-          k_types_by_slot<<<static_cast<unsigned>((nl.n + 255) / 256), 256, 0, E.ctx->stream>>>(
-              types, nl.order.get(), nl.n, E.gtype.get(), nl.gpos.get());
-          HIPCHK(hipGetLastError());
-          if (staged) {
-            E.gtype_build = nl.build_id;
-            E.gtype_stamp = E.types_stamp;
-            nl.wtype_build = nl.build_id;
-            nl.wtype_stamp = E.types_stamp;
-          }
-        }
-        A.types = E.gtype.get();
-      }
+      if (A.t0 < 0) A.types = types_by_slot(E, nl, types);
       return A;
     }
 
-    // Lanes per atom for the energy, HVP and density kernels.
+    // Lanes per atom for the base densities of batched searches.
     constexpr int LANES = 8;
 
     unsigned grid_for(long n, int L) { return static_cast<unsigned>((n * L + NT - 1) / NT); }
@@ -1000,7 +1019,7 @@ namespace flyg {
     if (nl.tiled && E.lanes <= 0) {
       tile_density(E, S, tile_args(E, nl, types, frozen), true, FLYG_FP64, E.posf.get());
     } else {
-      launch_density<LANES>(E, S, pair_args(E, nl, types, frozen), true, FLYG_FP64, E.posf.get());
+      launch_density<16>(E, S, slot_args(E, nl, types, frozen), true, FLYG_FP64, E.posf.get());
     }
     HIPCHK(hipGetLastError());
     dev_sum(*E.ctx, E.eatom.get(), nl.n, E.ctx->hpart, E.ctx->hflags + 1);
@@ -1075,7 +1094,7 @@ namespace flyg {
       A.pos = E.posf.get();
       tile_force(E, S, A, d_grad, precision);
     } else {
-      gradient_with(E, S, pair_args(E, nl, types, frozen), d_grad, precision, E.posf.get());
+      gradient_with(E, S, slot_args(E, nl, types, frozen), d_grad, precision, E.posf.get());
     }
     if (E.timing) HIPCHK(hipEventRecord(E.events[E.events_used++].second, E.ctx->stream));
     HIPCHK(hipGetLastError());

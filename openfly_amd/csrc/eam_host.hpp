@@ -116,13 +116,14 @@ struct flyg_list_s {
   // around it in LDS and walks its atoms' rows through 16-bit indices into that stage.  sslot: the
   // sorted entries (reals and images, cell by cell) as (shift, slot); rows: by slot, rowK entries of
   // room, in blocks of 32 whose entry k lies at 2 (k mod 16) + (k / 16 mod 2), so a lane of 16 loads two at a time.
+  // Lists that are not tiled keep packed (shift, slot) entries there instead, nbr's in the slot order.
   flyg::TileGrid tile{};
   bool tiled = false;            // rows and sslot belong to this build
   int tile_level = 0;            // tile shapes found too full for LDS with this atom count are skipped
   int tile_most = 0;             // entries staged by the fullest tile
   int rowK = 0;
   flyg::DBuf<unsigned> sslot;
-  flyg::DBuf<unsigned> rows;     // two entries a word
+  flyg::DBuf<unsigned> rows;
   flyg::DBuf<int> gcnt;          // entries per slot
   flyg::DBuf<int> scan_tmp;
   flyg::DBuf<double> stage;      // host staging of xyz vectors
@@ -158,6 +159,12 @@ namespace flyg {
     uint32_t const* types;
     uint8_t const* frozen;
     int t0;   // the one species present (-1: several or unknown); read by the single-species kernels
+    // Null: rows, positions and types are by atom.  Otherwise they are by slot of the list's cell-order
+    // layout (types gathered into slot order) and order[slot] is the atom, for frozen flags and gradients.
+    int const* order = nullptr;
+    // The w slot of pos holds each atom's species (as a double), so a neighbour's species arrives with
+    // its position; set for the slot layout with several species.
+    bool type_in_w = false;
   };
   // Image shift of a packed entry: sum_a s_a * basis column a, s_a in {-1, 0, 1}.  Exact for
   // orthorhombic boxes (each component is 0 or +-L), computed in registers (no table lookup).

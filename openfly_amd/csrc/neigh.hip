@@ -9,8 +9,9 @@
 //   4. scatter of the packed ids by cell, then each cell sorted by packed id, so the result does not
 //      depend on the atomics
 //   5. k_build_rows: every (real, image) of an atom's 27 cells with d^2 < r_cut^2 (strict,
-//      list.cpp:146,159) goes to its row of an ELL table: n rows x K packed 32-bit entries, and, when the list
-//      is tiled, to its row of 16-bit indices into the tile's staged entries.
+//      list.cpp:146,159) goes to its row of an ELL table: n rows x K packed 32-bit entries, and to a second table
+//      by slot (cell order): 16-bit indices into the tile's staged entries when the list is tiled, else packed entries
+//      that name slots.
 // Six launches and one synchronisation; the state the host needs is written to pinned memory.
 // The distance tests, canonical images and ghost chains round exactly like the reference's FP64
 // expressions (no FMA contraction), so the pair sets equal the reference's at rebuild time.
@@ -392,8 +393,9 @@ namespace flyg {
     // Small systems are bound by the chain of loads (A = 1: every atom a wavefront), large ones by the
     // candidates' L1 lookups (A = 4 loads them a quarter as often); BUILD_WIDE is where the two cross.
     //
-    // A tiled list gets each row twice: by atom with atom indices (nbr), and by slot with indices into the tile's stage
-    // (the candidate's place in the tile's halo: the lines' entries one after the other).  hst (pinned): [0] ghosts,
+    // Each row is written twice: by atom with atom indices (nbr), and by slot, in a tiled list with indices into the
+    // tile's stage (the candidate's place in the tile's halo: the lines' entries one after the other), otherwise with
+    // slots.  hst (pinned): [0] ghosts,
     // [1] set when a row overflowed, [2] entries of the fullest tile, [3] overflow bits.
     constexpr long BUILD_WIDE = 24000;
 
@@ -454,6 +456,8 @@ namespace flyg {
         if (k < c && k < K) {
           unsigned const en = ring[wave][a][k & 127];
           nbr[atom[a] * static_cast<long>(K) + k] = en;
+          if constexpr (!TILED)
+            rows[(slot0 + a) * rowK + k] = (en & ~NB_IDX_MASK) | static_cast<unsigned>(rank_of[en & NB_IDX_MASK]);
         }
         if constexpr (TILED) {   // two blocks of 32 entries, two entries a lane
           int const k2 = k0 + (lane >> 4) * 32 + (lane & 15);
@@ -835,11 +839,9 @@ namespace flyg {
       nl.nbr.reserve(static_cast<std::size_t>(n) * nl.K);
       nl.tiled = choose_tiles(nl, n);
       TileGrid const tg = nl.tiled ? nl.tile : TileGrid{};
-      nl.rowK = (nl.K + 31) / 32 * 32;
-      if (nl.tiled) {
-        nl.sslot.reserve(cap);
-        nl.rows.reserve(static_cast<std::size_t>(n) * nl.rowK / 2);
-      }
+      nl.rowK = nl.tiled ? (nl.K + 31) / 32 * 32 : nl.K;
+      if (nl.tiled) nl.sslot.reserve(cap);
+      nl.rows.reserve(static_cast<std::size_t>(n) * nl.rowK / (nl.tiled ? 2 : 1));
       nl.hstate[1] = 0;
       if (nl.box.ortho) {
         k_entries<true><<<nblk(n, ETPB), ETPB, 0, st>>>(nl.box, nl.grid, d_xyz, n, nl.pos.get(), nl.ent.get(),
