@@ -129,7 +129,9 @@ struct flyg_list_s {
   flyg::DBuf<double> stage;      // host staging of xyz vectors
   flyg::DBuf<unsigned> lstate;   // device build counters: two sets, used in turn
   int parity = 0;                // the set of the next build
-  bool counters_clear = false;   // ccount and that set are zero
+  // ccount and that set are zero for a grid of so many cells + 1 (the search server gives one list object
+  // system after system, each with its own box and grid).
+  long clear_cells = -1;
   unsigned* hstate = nullptr;    // pinned mirror
   long gcap = 0;                 // ghost slots
   ~flyg_list_s() {

@@ -793,8 +793,8 @@ namespace flyg {
     if (n != nl.n) {
       nl.gcap = 0;
       nl.K = 0;
-      nl.tile_level = 0;
     }
+    if (n != nl.n || nl.clear_cells != nl.grid.ncells + 1) nl.tile_level = 0;
     nl.n = n;
     if (nl.gcap == 0) nl.gcap = std::max(4096l, n);
     if (nl.K == 0) {
@@ -817,11 +817,11 @@ namespace flyg {
     nl.rank.reserve(n);
     nl.gpos.reserve(n);
     nl.gcnt.reserve(n);
-    if (!nl.counters_clear) {   // a first build, or one that ended in an error half way
+    if (nl.clear_cells != nc1) {   // a first build, another grid, or a build that ended in an error half way
       HIPCHK(hipMemsetAsync(nl.ccount.get(), 0, scan_room(2 * nc1) * sizeof(int), st));
       HIPCHK(hipMemsetAsync(nl.lstate.get(), 0, 8 * sizeof(unsigned), st));
     }
-    nl.counters_clear = false;
+    nl.clear_cells = -1;
 
     for (int attempt = 0; attempt < 3 + TILE_KINDS; ++attempt) {
       // Two sets of state words in turn: the scan clears the other build's.
@@ -890,7 +890,7 @@ namespace flyg {
       }
       static std::atomic<long> builds{0};
       nl.build_id = ++builds;
-      nl.counters_clear = true;
+      nl.clear_cells = nc1;
       nl.built = true;
       return;
     }

@@ -184,3 +184,26 @@ def test_serve_loop_small(ctx, wen):
     assert out["systems_admitted"] <= 3
     assert all(r.done >= r.t for r in reqs)
     assert srv.status()["systems"] == 0
+
+
+def test_admission_scratch_over_changing_grids(ctx, wen):
+    # One server admits systems of growing and shrinking boxes: the list object that gives their base densities is
+    # reused with another cell grid each time.  Every system's searches equal a batch's on that system alone.
+    pot = wen["pot"]
+    server = fa.Server(ctx, pot, dimer=dict(f2norm=1e-3, max_steps=12), precision=fa.FP64, **SHAPE)
+    for q, cells in enumerate((7, 11, 8, 12, 7)):
+        pos, basis = vacancy_system(cells, drop=q)
+        rng = np.random.default_rng(cells + q)
+        pos = np.mod(pos + rng.normal(0, 0.03, pos.shape), np.diag(basis))
+        t = np.zeros(len(pos), np.uint32)
+        print(f"case admit {cells}^3 cells", flush=True)
+        sid = server.add_system(fa.Box(basis), pos, t)
+        centres, radii = rng.integers(0, len(pos), 2), np.array([4.0, 6.0])
+        states = rng.integers(1, 2 ** 63, size=(2, 4), dtype=np.uint64)
+        served = drain(server, server.submit_perturbed(sid, centres, radii, states.copy()))
+        b = fa.Batch(ctx, pot, fa.Box(basis), pos, t, dimer=dict(f2norm=1e-3, max_steps=12), precision=fa.FP64, **SHAPE)
+        ids = b.submit_perturbed(centres, radii, states.copy())
+        b.run()
+        for s, i in zip(served, ids):
+            r = b.result(i)
+            assert (s["exit"], s["steps"], s["grads"], s["barrier"]) == (r["exit"], r["steps"], r["grads"], r["barrier"])
