@@ -14,8 +14,8 @@
 //
 // Eigenvalues: Householder reduction to tridiagonal form (Golub & Van Loan, Matrix Computations, Alg. 8.3.1),
 // one launch a column that applies the previous reflection and multiplies by the next one in the same
-// pass over the block; then each eigenvalue by multisection on Sturm counts (Givens; Barth, Martin & Wilkinson,
-// Numer. Math. 9 (1967) 386), a wavefront per eigenvalue testing 64 points of its interval at once.  Both are
+// pass over the block; then each eigenvalue by multisection on Sturm counts (Givens' bisection), a
+// wavefront per eigenvalue testing 64 points of its interval at once.  Both are
 // backward stable: errors of a few units of 1e-16 of the largest eigenvalue.  Bound by one launch per column
 // up to some 1000 coordinates, then by the memory traffic of the shrinking block.  Cyclic Jacobi rotations
 // needed ten sweeps of 3M rounds of two launches: 36 ms at 360 coordinates.
@@ -252,76 +252,153 @@ namespace flyg {
     // product p = A v are in vp, bt and pp); rows above k are done.  Every workgroup for itself: w = b p - (b^2 (p.v) / 2) v,
     // row k of the updated block, its diagonal and the next reflection; then, a wavefront per row,
     // A_ij -= v_i w_j + w_i v_j and the row's part of A v_new.  Row k itself is only read.
+    //
+    // A step is a launch and a chain of loads, two block sums and a row sum: what it costs at 360
+    // coordinates is latency.  NC > 0 (blocks of up to 64 NC coordinates): vectors and rows are loaded at once
+    // before the first sum, v, w and the new vector wait in LDS (6.4 -> 4.6 us a step).  NC = 0: any size,
+    // everything read again from the caches where it is used.
+    template <int NC>
     __global__ __launch_bounds__(NTB) void k_tridiag(double* __restrict__ A, long n, long k, double const* __restrict__ vp,
                                                      double const* __restrict__ pp, double const* __restrict__ bt,
                                                      double* __restrict__ vn, double* __restrict__ pn,
                                                      double* __restrict__ bn, double* __restrict__ diag,
                                                      double* __restrict__ off) {
-      __shared__ double sh[2][NTB / 64];
+      constexpr int NV = NC > 0 ? (64 * NC + NTB - 1) / NTB : 1;   // elements of a vector per thread
+      __shared__ double sh[2][2][NTB / 64];
+      __shared__ double sv[NC > 0 ? 64 * NC : 1], sw[NC > 0 ? 64 * NC : 1], sx[NC > 0 ? 64 * NC : 1];
       double const* Ak = A + k * n;
       bool const first = k == 0;
       double const b = first ? 0.0 : *bt;
+      int const lane = threadIdx.x & 63;
+      long const waves = static_cast<long>(gridDim.x) * (NTB / 64);
+      long const i0 = k + 1 + blockIdx.x * (NTB / 64) + (threadIdx.x >> 6);   // this wavefront's first row
+      double ev[NV], ep[NV], ea[NV];   // v, p and row k
+      double row[NC > 0 ? NC : 1];
+      if constexpr (NC > 0) {
+#pragma unroll
+        for (int u = 0; u < NV; ++u) {
+          long const j = k + threadIdx.x + u * NTB;
+          bool const in = j < n;
+          ev[u] = in && !first ? vp[j] : 0.0;
+          ep[u] = in && !first ? pp[j] : 0.0;
+          ea[u] = in ? Ak[j] : 0.0;
+        }
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          long const j = k + 1 + lane + 64 * c;
+          row[c] = i0 < n && j < n ? A[i0 * n + j] : 0.0;
+        }
+      }
       double pv = 0, dummy = 0;
-      if (!first)
-        for (long j = k + threadIdx.x; j < n; j += NTB) pv += pp[j] * vp[j];
-      sum2(pv, dummy, sh);
+      if constexpr (NC > 0) {
+#pragma unroll
+        for (int u = 0; u < NV; ++u) pv += ep[u] * ev[u];
+      } else {
+        if (!first)
+          for (long j = k + threadIdx.x; j < n; j += NTB) pv += pp[j] * vp[j];
+      }
+      sum2(pv, dummy, sh[0]);
       double const kk = 0.5 * b * b * pv;
+      if constexpr (NC > 0) {
+#pragma unroll
+        for (int u = 0; u < NV; ++u) {
+          int const q = threadIdx.x + u * NTB;   // place of element k + q
+          if (q < 64 * NC) {
+            sv[q] = ev[u];
+            sw[q] = b * ep[u] - kk * ev[u];
+          }
+        }
+        __syncthreads();
+      }
       // v_j and w_j of the reflection before (zero at the first step).
       auto vw = [&](long j, double& v, double& w) {
-        v = first ? 0.0 : vp[j];
-        w = first ? 0.0 : b * pp[j] - kk * v;
+        if constexpr (NC > 0) {
+          v = sv[j - k];
+          w = sw[j - k];
+        } else {
+          v = first ? 0.0 : vp[j];
+          w = first ? 0.0 : b * pp[j] - kk * v;
+        }
       };
       double vk, wk;
       vw(k, vk, wk);
+      double ss = 0;
+      if constexpr (NC > 0) {
+#pragma unroll
+        for (int u = 0; u < NV; ++u) {
+          int const q = threadIdx.x + u * NTB;
+          if (q < 64 * NC) {
+            double const x = ea[u] - (vk * sw[q] + wk * sv[q]);   // row k of the updated block
+            sx[q] = x;
+            if (q >= 2) ss += x * x;
+          }
+        }
+      }
       auto rowk = [&](long j, double& v, double& w) {
         vw(j, v, w);
         return Ak[j] - (vk * w + wk * v);
       };
-      double ss = 0;
-      for (long j = k + 2 + threadIdx.x; j < n; j += NTB) {
-        double v, w;
-        double const x = rowk(j, v, w);
-        ss += x * x;
-      }
+      if constexpr (NC == 0)
+        for (long j = k + 2 + threadIdx.x; j < n; j += NTB) {
+          double v, w;
+          double const x = rowk(j, v, w);
+          ss += x * x;
+        }
       double zero = 0;
-      sum2(ss, zero, sh);
-      double v1, w1;
-      double const x1 = rowk(k + 1, v1, w1);
+      sum2(ss, zero, sh[1]);
+      double x0, x1;
+      if constexpr (NC > 0) {
+        x0 = sx[0];
+        x1 = sx[1];
+      } else {
+        double v, w;
+        x0 = rowk(k, v, w);
+        x1 = rowk(k + 1, v, w);
+      }
       double alpha = x1, top = 0, beta = 0;
       if (ss != 0.0) {
         alpha = -copysign(sqrt(ss + x1 * x1), x1);
         top = x1 - alpha;
         beta = 2.0 / (ss + top * top);
       }
-      auto next = [&](long j, double& v, double& w) {   // new reflection's vector (zero where there is none)
-        double const x = rowk(j, v, w);
+      auto next = [&](long j) {   // new reflection's vector (zero where there is none)
+        double x;
+        if constexpr (NC > 0) {
+          x = sx[j - k];
+        } else {
+          double v, w;
+          x = rowk(j, v, w);
+        }
         return j == k + 1 ? top : (beta != 0.0 ? x : 0.0);
       };
       if (blockIdx.x == 0) {
         if (threadIdx.x == 0) {
-          double v, w;
-          diag[k] = rowk(k, v, w);
+          diag[k] = x0;
           off[k] = alpha;
           *bn = beta;
         }
-        for (long j = k + 1 + threadIdx.x; j < n; j += NTB) {
-          double v, w;
-          vn[j] = next(j, v, w);
-        }
+        for (long j = k + 1 + threadIdx.x; j < n; j += NTB) vn[j] = next(j);
       }
-      int const lane = threadIdx.x & 63;
-      long const waves = static_cast<long>(gridDim.x) * (NTB / 64);
-      for (long i = k + 1 + blockIdx.x * (NTB / 64) + (threadIdx.x >> 6); i < n; i += waves) {
+      for (long i = i0; i < n; i += waves) {
         double vi, wi;
         vw(i, vi, wi);
         double* Ai = A + i * n;
         double p = 0;
-        for (long j = k + 1 + lane; j < n; j += 64) {
+        auto one = [&](long j, double a0) {
           double v, w;
-          double const x = next(j, v, w);
-          double const a = Ai[j] - (vi * w + wi * v);
+          vw(j, v, w);
+          double const a = a0 - (vi * w + wi * v);
           Ai[j] = a;
-          p += a * x;
+          p += a * next(j);
+        };
+        if constexpr (NC > 0) {
+#pragma unroll
+          for (int c = 0; c < NC; ++c) {
+            long const j = k + 1 + lane + 64 * c;
+            if (j < n) one(j, i == i0 ? row[c] : Ai[j]);
+          }
+        } else {
+          for (long j = k + 1 + lane; j < n; j += 64) one(j, Ai[j]);
         }
         p = group_sum<64>(p);
         if (lane == 0) pn[i] = p;
@@ -350,63 +427,111 @@ namespace flyg {
       }
     }
 
-    // Squares of the off-diagonal and Gershgorin bounds (one workgroup): lim = (low, high, least pivot).
+    // Gershgorin bounds of the tridiagonal matrix and, for the Sturm counts, the matrix scaled by a power of two to a
+    // norm in [1/2, 1) (exact): ds, and e2 = squares of the off-diagonal (one workgroup).  lim = (low, high,
+    // scale) in scaled units.
     __global__ __launch_bounds__(NTB) void k_bounds(double const* __restrict__ d, double const* __restrict__ off, long n,
-                                                    double* __restrict__ e2, double* __restrict__ lim) {
-      __shared__ double s0[NTB], s1[NTB], s2[NTB];
-      double lo = INFINITY, hi = -INFINITY, em = 0;
-      bool bad = false;
+                                                    double* __restrict__ ds, double* __restrict__ e2,
+                                                    double* __restrict__ lim) {
+      __shared__ double s0[NTB / 64], s1[NTB / 64];
+      __shared__ int s2[NTB / 64];
+      double lo = INFINITY, hi = -INFINITY;
+      int bad = 0;
       for (long i = threadIdx.x; i < n; i += NTB) {
         double const l = i > 0 ? fabs(off[i - 1]) : 0.0, r = i + 1 < n ? fabs(off[i]) : 0.0;
         double const a = d[i] - (l + r), z = d[i] + (l + r);
-        bad = bad || !isfinite(a) || !isfinite(z);
+        bad |= !isfinite(a) || !isfinite(z);
         lo = fmin(lo, a);
         hi = fmax(hi, z);
-        e2[i] = l * l;   // couples i - 1 and i
-        em = fmax(em, l * l);
       }
-      s0[threadIdx.x] = bad ? NAN : lo;
-      s1[threadIdx.x] = hi;
-      s2[threadIdx.x] = em;
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) {
+        lo = fmin(lo, __shfl_xor(lo, o, 64));
+        hi = fmax(hi, __shfl_xor(hi, o, 64));
+        bad |= __shfl_xor(bad, o, 64);
+      }
+      if ((threadIdx.x & 63) == 0) {
+        s0[threadIdx.x >> 6] = lo;
+        s1[threadIdx.x >> 6] = hi;
+        s2[threadIdx.x >> 6] = bad;
+      }
       __syncthreads();
-      if (threadIdx.x) return;
-      for (int q = 1; q < NTB; ++q) {
-        s0[0] = isnan(s0[0]) || isnan(s0[q]) ? NAN : fmin(s0[0], s0[q]);
-        s1[0] = fmax(s1[0], s1[q]);
-        s2[0] = fmax(s2[0], s2[q]);
+      for (int q = 0; q < NTB / 64; ++q) {
+        lo = fmin(lo, s0[q]);
+        hi = fmax(hi, s1[q]);
+        bad |= s2[q];
       }
-      double const pad = 1e-15 * fmax(fabs(s0[0]), fabs(s1[0])) + 1e-300;
-      lim[0] = s0[0] - pad;
-      lim[1] = s1[0] + pad;
-      lim[2] = 2.3e-308 * fmax(1.0, s2[0]);
+      int ex = 0;
+      double const norm = fmax(fabs(lo), fabs(hi));
+      if (norm > 0) (void)frexp(norm, &ex);
+      double const sc = ldexp(1.0, -ex), pad = 1e-15 * norm * sc + 1e-300;
+      for (long i = threadIdx.x; i < n; i += NTB) {
+        double const l = i > 0 ? off[i - 1] * sc : 0.0;
+        ds[i] = d[i] * sc;
+        e2[i] = fmax(l * l, 1e-36);   // couples i - 1 and i; a coupling of 1e-18 of the norm keeps p from sticking at zero
+      }
+      if (threadIdx.x == 0) {
+        lim[0] = bad ? NAN : lo * sc - pad;
+        lim[1] = bad ? NAN : hi * sc + pad;
+        lim[2] = ldexp(1.0, ex);
+      }
     }
 
     // Eigenvalue m of the tridiagonal matrix: one wavefront narrows its interval 65-fold per pass.  The number of
-    // negative terms of q_i = (d_i - x) - e_i^2 / q_{i-1} is the number of eigenvalues below x.
+    // eigenvalues below x is the number of sign changes in p_i = (d_i - x) p_{i-1} - e_i^2 p_{i-2}: a chain of one
+    // FMA a term (with q_i = p_i / p_{i-1} it is a division, 250 cycles).  The pair is rescaled every eight
+    // terms, which cannot leave the range of a double for a matrix of norm 1; the sign of a term that vanishes does
+    // not matter, since its neighbours' differ.  LDS: the matrix waits there (up to STURM_LDS coordinates), the
+    // next eight terms are read while these are worked on.
     constexpr int STURM_PASSES = 9;   // 65^9 = 2^54: down to the rounding of the interval's own width
+    constexpr int STURM_LDS = 3072;
 
+    template <bool LDS>
     __global__ __launch_bounds__(NTB) void k_sturm(double const* __restrict__ d, double const* __restrict__ e2, long n,
                                                    double const* __restrict__ lim, double* __restrict__ out) {
-      long const m = blockIdx.x * static_cast<long>(NTB / 64) + (threadIdx.x >> 6);
+      extern __shared__ double2 s_t[];   // (d, e2), padded by two groups with terms that keep p's sign
+      if constexpr (LDS) {
+        for (long i = threadIdx.x; i < n + 16; i += NTB) s_t[i] = i < n ? make_double2(d[i], e2[i]) : make_double2(2.0, 0.0);
+        __syncthreads();
+      }
+      long const m = blockIdx.x * static_cast<long>(NTB / 64) +
+                     __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
       int const lane = threadIdx.x & 63;
       if (m >= n) return;
+      auto term = [&](long i) {
+        if constexpr (LDS) return s_t[i];
+        return i < n ? make_double2(d[i], e2[i]) : make_double2(2.0, 0.0);
+      };
       double lo = lim[0], hi = lim[1];
-      double const piv = lim[2];
       for (int pass = 0; pass < STURM_PASSES; ++pass) {
         double const x = lo + (hi - lo) * (static_cast<double>(lane + 1) / 65.0);
-        double q = 1.0;
-        long below = 0;
-        for (long i = 0; i < n; ++i) {
-          q = (d[i] - x) - e2[i] / q;
-          if (fabs(q) <= piv) q = -piv;
-          below += q < 0 ? 1 : 0;
+        double p0 = 0.0, p1 = 1.0;   // p_{i-2}, p_{i-1}
+        int below = 0;
+        double2 t8[8], n8[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) t8[u] = term(u);
+        for (long i8 = 0; i8 < n; i8 += 8) {
+#pragma unroll
+          for (int u = 0; u < 8; ++u) n8[u] = term(i8 + 8 + u);
+#pragma unroll
+          for (int u = 0; u < 8; ++u) {
+            double const p = fma(t8[u].x - x, p1, -(t8[u].y * p0));
+            below += static_cast<int>(static_cast<unsigned>(__double2hiint(p) ^ __double2hiint(p1)) >> 31);
+            p0 = p1;
+            p1 = p;
+          }
+          int const ex = max(__builtin_amdgcn_frexp_exp(p0), __builtin_amdgcn_frexp_exp(p1));
+          p0 = ldexp(p0, -ex);
+          p1 = ldexp(p1, -ex);
+#pragma unroll
+          for (int u = 0; u < 8; ++u) t8[u] = n8[u];
         }
         int const t = __popcll(__ballot(below <= m));   // points that eigenvalue m is not below
         double const nlo = __shfl(x, t > 0 ? t - 1 : 0, 64), nhi = __shfl(x, t < 64 ? t : 63, 64);
         if (t > 0) lo = nlo;
         if (t < 64) hi = nhi;
       }
-      if (lane == 0) out[m] = 0.5 * (lo + hi);
+      if (lane == 0) out[m] = 0.5 * (lo + hi) * lim[2];
     }
 
     unsigned blocks(long n, int t) { return static_cast<unsigned>((n + t - 1) / t); }
@@ -491,12 +616,21 @@ namespace flyg {
     for (long k = 0; k + 2 < n3m; ++k) {
       long const rows = n3m - k - 1;
       unsigned const g = static_cast<unsigned>(std::min<long>((rows + NTB / 64 - 1) / (NTB / 64), 512));
-      k_tridiag<<<g, NTB, 0, st>>>(H, n3m, k, v[k & 1], p[k & 1], bt[k & 1], v[(k + 1) & 1], p[(k + 1) & 1], bt[(k + 1) & 1],
-                                   diag, off);
+      auto step = [&](auto f) {
+        f<<<g, NTB, 0, st>>>(H, n3m, k, v[k & 1], p[k & 1], bt[k & 1], v[(k + 1) & 1], p[(k + 1) & 1], bt[(k + 1) & 1], diag,
+                             off);
+      };
+      long const left = n3m - k;   // coordinates of the block, row k among them
+      left <= 128 ? step(k_tridiag<2>) : left <= 256 ? step(k_tridiag<4>) : left <= 512 ? step(k_tridiag<8>)
+                                       : step(k_tridiag<0>);
     }
     k_tridiag_end<<<1, 64, 0, st>>>(H, n3m, v[n3m & 1], p[n3m & 1], bt[n3m & 1], diag, off);
-    k_bounds<<<1, NTB, 0, st>>>(diag, off, n3m, e2, lim);
-    k_sturm<<<blocks(n3m, NTB / 64), NTB, 0, st>>>(diag, e2, n3m, lim, lam);
+    k_bounds<<<1, NTB, 0, st>>>(diag, off, n3m, rm, e2, lim);   // rm: the scaled diagonal (the masses are done with)
+    if (n3m <= STURM_LDS) {
+      k_sturm<true><<<blocks(n3m, NTB / 64), NTB, (n3m + 16) * sizeof(double2), st>>>(rm, e2, n3m, lim, lam);
+    } else {
+      k_sturm<false><<<blocks(n3m, NTB / 64), NTB, 0, st>>>(rm, e2, n3m, lim, lam);
+    }
     HIPCHK(hipGetLastError());
     std::vector<double> w(n3m);
     HIPCHK(hipMemcpyAsync(w.data(), lam, n3m * sizeof(double), hipMemcpyDeviceToHost, st));
