@@ -31,6 +31,9 @@ namespace flyg {
   inline void require(bool ok, std::string const& msg) {
     if (!ok) throw Error(FLYG_INVALID_ARG, msg);
   }
+  inline void require(bool ok, char const* msg) {   // no string is built for a check that passes
+    if (!ok) throw Error(FLYG_INVALID_ARG, msg);
+  }
 
   // Device-side error flags (bit set, read back by the host after a call).
   enum : unsigned { ERR_SPLINE_OOB = 1u, ERR_LIST_OVERFLOW = 2u, ERR_REGION = 4u, ERR_NAN = 8u, ERR_TYPE = 16u };

@@ -96,8 +96,9 @@ namespace flyg {
 
     // Density pass.  MIX (and not ENERGY): r and the density spline in FP32, sums in FP64.
     template <int L, bool MULTI, bool ENERGY, bool MIX>
-    __global__ __launch_bounds__(NT) void k_density(EAMTables T, Shifts S, PairArgs A, double4* __restrict__ posf,
+    __global__ __launch_bounds__(NT) void k_density(EAMTables const* __restrict__ Tp, Shifts S, PairArgs A, double4* __restrict__ posf,
                                                     double* __restrict__ eatom, unsigned* __restrict__ err) {
+      EAMTables const& T = *Tp;
       __shared__ SplineDesc s_phi[MAX_TYPES * MAX_TYPES], s_V[MAX_TYPES * MAX_TYPES];
       if (MULTI) {   // per-lane species pairs: table descriptors from LDS, not from the argument block
         int t = threadIdx.x;
@@ -162,8 +163,9 @@ namespace flyg {
     }
 
     template <int L, bool MULTI, bool MIX>
-    __global__ __launch_bounds__(NT) void k_force(EAMTables T, Shifts S, PairArgs A, double4 const* __restrict__ posf,
+    __global__ __launch_bounds__(NT) void k_force(EAMTables const* __restrict__ Tp, Shifts S, PairArgs A, double4 const* __restrict__ posf,
                                                   double* __restrict__ grad, unsigned* __restrict__ err) {
+      EAMTables const& T = *Tp;
       __shared__ SplineDesc s_phi[MAX_TYPES * MAX_TYPES], s_V[MAX_TYPES * MAX_TYPES];
       if (MULTI) {   // per-lane species pairs: table descriptors from LDS, not from the argument block
         int t = threadIdx.x;
@@ -448,8 +450,9 @@ namespace flyg {
 
     // Density pass: posf by slot; ENERGY: eatom by atom (FP64 densities and pair energies).
     template <bool MULTI, bool ENERGY, bool MIX>
-    __global__ __launch_bounds__(TT) void k_tile_density(EAMTables T, Shifts S, TileArgs A, double4* __restrict__ posf,
+    __global__ __launch_bounds__(TT) void k_tile_density(EAMTables const* __restrict__ Tp, Shifts S, TileArgs A, double4* __restrict__ posf,
                                                          double* __restrict__ eatom, unsigned* __restrict__ err) {
+      EAMTables const& T = *Tp;
       extern __shared__ double2 s_stage[];
       double2* const xy = s_stage;
       double2* const zw = s_stage + A.cap;
@@ -531,8 +534,9 @@ namespace flyg {
     }
 
     template <bool MULTI, bool MIX>
-    __global__ __launch_bounds__(TT) void k_tile_force(EAMTables T, Shifts S, TileArgs A, double* __restrict__ grad,
+    __global__ __launch_bounds__(TT) void k_tile_force(EAMTables const* __restrict__ Tp, Shifts S, TileArgs A, double* __restrict__ grad,
                                                        unsigned* __restrict__ err) {
+      EAMTables const& T = *Tp;
       extern __shared__ double2 s_stage[];
       double2* const xy = s_stage;
       double2* const zw = s_stage + A.cap;
@@ -633,8 +637,9 @@ namespace flyg {
     }
 
     template <int L, bool MULTI>
-    __global__ __launch_bounds__(NT) void k_hvp_density(EAMTables T, Shifts S, PairArgs A, double const* __restrict__ v,
+    __global__ __launch_bounds__(NT) void k_hvp_density(EAMTables const* __restrict__ Tp, Shifts S, PairArgs A, double const* __restrict__ v,
                                                         double2* __restrict__ dfp, unsigned* __restrict__ err) {
+      EAMTables const& T = *Tp;
       long gid = xcd_block(blockIdx.x, gridDim.x) * static_cast<long>(NT) + threadIdx.x;
       long i = gid / L;
       int lane = static_cast<int>(gid % L);
@@ -670,9 +675,10 @@ namespace flyg {
     }
 
     template <int L, bool MULTI>
-    __global__ __launch_bounds__(NT) void k_hvp_force(EAMTables T, Shifts S, PairArgs A, double const* __restrict__ v,
+    __global__ __launch_bounds__(NT) void k_hvp_force(EAMTables const* __restrict__ Tp, Shifts S, PairArgs A, double const* __restrict__ v,
                                                       double2 const* __restrict__ dfp, double* __restrict__ hv,
                                                       unsigned* __restrict__ err) {
+      EAMTables const& T = *Tp;
       long gid = xcd_block(blockIdx.x, gridDim.x) * static_cast<long>(NT) + threadIdx.x;
       long i = gid / L;
       int lane = static_cast<int>(gid % L);
@@ -709,9 +715,10 @@ namespace flyg {
     // Tiled passes: the stage holds (x, y), (z, vz), (vx, vy) and, in the force pass, (F', dF') of every entry, and its
     // species with several.  dfp by slot.
     template <bool MULTI, bool FORCE>
-    __global__ __launch_bounds__(TT) void k_tile_hvp(EAMTables T, Shifts S, TileArgs A, double const* __restrict__ v,
+    __global__ __launch_bounds__(TT) void k_tile_hvp(EAMTables const* __restrict__ Tp, Shifts S, TileArgs A, double const* __restrict__ v,
                                                      double2* __restrict__ dfp, double* __restrict__ hv,
                                                      unsigned* __restrict__ err) {
+      EAMTables const& T = *Tp;
       extern __shared__ double2 s_stage[];
       double2* const xy = s_stage;
       double2* const zv = xy + A.cap;
@@ -785,8 +792,9 @@ namespace flyg {
 
     // FP64 densities only (base state of batched searches).
     template <int L, bool MULTI>
-    __global__ __launch_bounds__(NT) void k_rho(EAMTables T, Shifts S, PairArgs A, double* __restrict__ rho_out,
+    __global__ __launch_bounds__(NT) void k_rho(EAMTables const* __restrict__ Tp, Shifts S, PairArgs A, double* __restrict__ rho_out,
                                                 unsigned* __restrict__ err) {
+      EAMTables const& T = *Tp;
       long gid = xcd_block(blockIdx.x, gridDim.x) * static_cast<long>(NT) + threadIdx.x;
       long i = gid / L;
       int lane = static_cast<int>(gid % L);
@@ -930,6 +938,8 @@ namespace flyg {
     T.c64 = E.c64.get();
     T.c32 = E.c32.get();
     E.tab = T;
+    E.dtab.reserve(1);
+    HIPCHK(hipMemcpy(E.dtab.get(), &E.tab, sizeof(EAMTables), hipMemcpyHostToDevice));
   }
 
   namespace {
@@ -944,18 +954,18 @@ namespace flyg {
       unsigned g = grid_for(A.n, L);
       if (multi) {
         if (energy)
-          k_density<L, true, true, false><<<g, NT, 0, st>>>(E.tab, S, A, pf, E.eatom.get(), err);
+          k_density<L, true, true, false><<<g, NT, 0, st>>>(E.dtab.get(), S, A, pf, E.eatom.get(), err);
         else if (mix)
-          k_density<L, true, false, true><<<g, NT, 0, st>>>(E.tab, S, A, pf, nullptr, err);
+          k_density<L, true, false, true><<<g, NT, 0, st>>>(E.dtab.get(), S, A, pf, nullptr, err);
         else
-          k_density<L, true, false, false><<<g, NT, 0, st>>>(E.tab, S, A, pf, nullptr, err);
+          k_density<L, true, false, false><<<g, NT, 0, st>>>(E.dtab.get(), S, A, pf, nullptr, err);
       } else {
         if (energy)
-          k_density<L, false, true, false><<<g, NT, 0, st>>>(E.tab, S, A, pf, E.eatom.get(), err);
+          k_density<L, false, true, false><<<g, NT, 0, st>>>(E.dtab.get(), S, A, pf, E.eatom.get(), err);
         else if (mix)
-          k_density<L, false, false, true><<<g, NT, 0, st>>>(E.tab, S, A, pf, nullptr, err);
+          k_density<L, false, false, true><<<g, NT, 0, st>>>(E.dtab.get(), S, A, pf, nullptr, err);
         else
-          k_density<L, false, false, false><<<g, NT, 0, st>>>(E.tab, S, A, pf, nullptr, err);
+          k_density<L, false, false, false><<<g, NT, 0, st>>>(E.dtab.get(), S, A, pf, nullptr, err);
       }
     }
 
@@ -969,14 +979,14 @@ namespace flyg {
       unsigned g = grid_for(A.n, L);
       if (multi) {
         if (mix)
-          k_force<L, true, true><<<g, NT, 0, st>>>(E.tab, S, A, pf, grad, err);
+          k_force<L, true, true><<<g, NT, 0, st>>>(E.dtab.get(), S, A, pf, grad, err);
         else
-          k_force<L, true, false><<<g, NT, 0, st>>>(E.tab, S, A, pf, grad, err);
+          k_force<L, true, false><<<g, NT, 0, st>>>(E.dtab.get(), S, A, pf, grad, err);
       } else {
         if (mix)
-          k_force<L, false, true><<<g, NT, 0, st>>>(E.tab, S, A, pf, grad, err);
+          k_force<L, false, true><<<g, NT, 0, st>>>(E.dtab.get(), S, A, pf, grad, err);
         else
-          k_force<L, false, false><<<g, NT, 0, st>>>(E.tab, S, A, pf, grad, err);
+          k_force<L, false, false><<<g, NT, 0, st>>>(E.dtab.get(), S, A, pf, grad, err);
       }
     }
   }  // namespace
@@ -986,7 +996,7 @@ namespace flyg {
       unsigned const g = static_cast<unsigned>(A.G.ntiles);
       std::size_t const lds = static_cast<std::size_t>(A.cap) * sizeof(double4);
       unsigned* err = E.ctx->dflags.get();
-      auto run = [&](auto k) { k<<<g, TT, lds, E.ctx->stream>>>(E.tab, S, A, pf, E.eatom.get(), err); };
+      auto run = [&](auto k) { k<<<g, TT, lds, E.ctx->stream>>>(E.dtab.get(), S, A, pf, E.eatom.get(), err); };
       bool const mix = precision == FLYG_MIXED;
       if (A.t0 < 0) {
         energy ? run(k_tile_density<true, true, false>)
@@ -1001,7 +1011,7 @@ namespace flyg {
       unsigned const g = static_cast<unsigned>(A.G.ntiles);
       bool const mix = precision == FLYG_MIXED;
       std::size_t const lds = static_cast<std::size_t>(A.cap) * (sizeof(double4) + (A.t0 < 0 && !mix ? 1 : 0));
-      auto run = [&](auto k) { k<<<g, TT, lds, E.ctx->stream>>>(E.tab, S, A, grad, E.ctx->dflags.get()); };
+      auto run = [&](auto k) { k<<<g, TT, lds, E.ctx->stream>>>(E.dtab.get(), S, A, grad, E.ctx->dflags.get()); };
       if (A.t0 < 0) {
         mix ? run(k_tile_force<true, true>) : run(k_tile_force<true, false>);
       } else {
@@ -1158,11 +1168,11 @@ namespace flyg {
       std::size_t const t = A.t0 < 0 ? 1 : 0;
       std::size_t const ld = static_cast<std::size_t>(A.cap) * (48 + t), lf = static_cast<std::size_t>(A.cap) * (64 + t);
       if (A.t0 < 0) {
-        k_tile_hvp<true, false><<<g, TT, ld, st>>>(E.tab, S, A, d_v, E.dfp.get(), d_hv, err);
-        k_tile_hvp<true, true><<<g, TT, lf, st>>>(E.tab, S, A, d_v, E.dfp.get(), d_hv, err);
+        k_tile_hvp<true, false><<<g, TT, ld, st>>>(E.dtab.get(), S, A, d_v, E.dfp.get(), d_hv, err);
+        k_tile_hvp<true, true><<<g, TT, lf, st>>>(E.dtab.get(), S, A, d_v, E.dfp.get(), d_hv, err);
       } else {
-        k_tile_hvp<false, false><<<g, TT, ld, st>>>(E.tab, S, A, d_v, E.dfp.get(), d_hv, err);
-        k_tile_hvp<false, true><<<g, TT, lf, st>>>(E.tab, S, A, d_v, E.dfp.get(), d_hv, err);
+        k_tile_hvp<false, false><<<g, TT, ld, st>>>(E.dtab.get(), S, A, d_v, E.dfp.get(), d_hv, err);
+        k_tile_hvp<false, true><<<g, TT, lf, st>>>(E.dtab.get(), S, A, d_v, E.dfp.get(), d_hv, err);
       }
       HIPCHK(hipGetLastError());
       return;
@@ -1171,11 +1181,11 @@ namespace flyg {
     constexpr int L = 16;
     unsigned g = grid_for(nl.n, L);
     if (A.t0 < 0) {
-      k_hvp_density<L, true><<<g, NT, 0, st>>>(E.tab, S, A, d_v, E.dfp.get(), err);
-      k_hvp_force<L, true><<<g, NT, 0, st>>>(E.tab, S, A, d_v, E.dfp.get(), d_hv, err);
+      k_hvp_density<L, true><<<g, NT, 0, st>>>(E.dtab.get(), S, A, d_v, E.dfp.get(), err);
+      k_hvp_force<L, true><<<g, NT, 0, st>>>(E.dtab.get(), S, A, d_v, E.dfp.get(), d_hv, err);
     } else {
-      k_hvp_density<L, false><<<g, NT, 0, st>>>(E.tab, S, A, d_v, E.dfp.get(), err);
-      k_hvp_force<L, false><<<g, NT, 0, st>>>(E.tab, S, A, d_v, E.dfp.get(), d_hv, err);
+      k_hvp_density<L, false><<<g, NT, 0, st>>>(E.dtab.get(), S, A, d_v, E.dfp.get(), err);
+      k_hvp_force<L, false><<<g, NT, 0, st>>>(E.dtab.get(), S, A, d_v, E.dfp.get(), d_hv, err);
     }
     HIPCHK(hipGetLastError());
   }
@@ -1186,9 +1196,9 @@ namespace flyg {
     PairArgs A = pair_args(E, nl, d_types, nullptr);
     unsigned g = grid_for(nl.n, LANES);
     if (A.t0 < 0) {
-      k_rho<LANES, true><<<g, NT, 0, E.ctx->stream>>>(E.tab, S, A, d_rho, E.ctx->dflags.get());
+      k_rho<LANES, true><<<g, NT, 0, E.ctx->stream>>>(E.dtab.get(), S, A, d_rho, E.ctx->dflags.get());
     } else {
-      k_rho<LANES, false><<<g, NT, 0, E.ctx->stream>>>(E.tab, S, A, d_rho, E.ctx->dflags.get());
+      k_rho<LANES, false><<<g, NT, 0, E.ctx->stream>>>(E.dtab.get(), S, A, d_rho, E.ctx->dflags.get());
     }
     HIPCHK(hipGetLastError());
   }
