@@ -68,6 +68,36 @@ namespace flyg {
     int const oldest = m_k <= m_m ? 0 : m_k - m_m;
     auto pair = [&](int i) { return (i + oldest) % m_m; };   // i = 0 oldest .. bound - 1 newest
     int const newest = pair(bound - 1);
+    if (vec_blocks(N) <= NEWTON_BLOCKS) {   // one launch (longer vectors: a launch a stage, bound by their bytes)
+      if (m_slots_n != N) {
+        m_slots.reserve(2 * NEWTON_SLOTS);
+        lb_empty_slots(ctx, m_slots.get(), 2 * NEWTON_SLOTS);
+        m_slots_n = N;
+      }
+      NewtonArgs a{};
+      a.n = N;
+      a.bound = bound;
+      a.x = x;
+      a.g = g;
+      a.px = m_px.get();
+      a.pg = m_pg.get();
+      a.r = r;
+      a.w = w;
+      a.lb = lb;
+      a.slots = m_slots.get() + m_slots_used * NEWTON_SLOTS;
+      m_slots_used = 1 - m_slots_used;
+      a.spare = m_slots.get() + m_slots_used * NEWTON_SLOTS;
+      a.out = out;
+      for (int i = 0; i < bound; ++i) {
+        a.j[i] = pair(i);
+        a.s[i] = m_s[a.j[i]].get();
+        a.y[i] = m_y[a.j[i]].get();
+      }
+      lb_newton(ctx, a);
+      ++m_k;
+      if (sums) *sums = out;
+      return r;
+    }
     lb_hist(ctx, N, x, g, m_px.get(), m_pg.get(), m_s[newest].get(), m_y[newest].get(), out);
     std::swap(in, out);
     double const* from = m_pg.get();    // q before loop 1: the gradient lb_hist kept
@@ -102,6 +132,7 @@ namespace flyg {
     void throw_flags(unsigned fl) {
       if (fl & ERR_SPLINE_OOB) throw Error(FLYG_SPLINE_OOB, "x is outside tabulated region of a spline");
       if (fl & ERR_TYPE) throw Error(FLYG_INVALID_ARG, "TypeID out of range");
+      if (fl & ERR_STALL) throw Error(FLYG_DEVICE_ERROR, "an L-BFGS step waited in vain for the rest of its workgroups");
     }
 
     void check_flags(flyg_ctx_s& ctx) { throw_flags(ctx.take_flags()); }

@@ -36,6 +36,9 @@ namespace flyg {
     DVec m_px, m_pg, m_q, m_r;
     DBuf<LBScalars> m_sc;
     DBuf<double> m_part;   // two sets of partial sums, used in turn
+    DBuf<unsigned long long> m_slots;   // of the one-launch step (lb_newton), two sets
+    long m_slots_n = -1;                // they are in order for vectors of this length
+    int m_slots_used = 0;               // the set of the next call
   };
 
 }  // namespace flyg

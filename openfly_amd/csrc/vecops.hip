@@ -219,6 +219,189 @@ namespace flyg {
       leave(acc, out);
     }
 
+    // ---- The two-loop in one launch ------------------------------------------------------------------
+    // Its 2 m sums are a chain, each needed by every element before the next.  As launches a link costs 4 us at
+    // 48k elements (an empty launch 2.35); here it is a store and a poll through the device's memory, under 2.  A
+    // thread keeps its (at most four) elements of q and r in registers from the first stage to the last, so no
+    // vector data crosses workgroups, only partial sums do: a workgroup writes its sum to a slot of its own, and one
+    // wavefront of every workgroup reads all of them until none is empty.  An empty slot holds a
+    // signalling NaN, which no sum can be.  Sums and expressions are those of the stage kernels: the same bits.
+    // Every workgroup must be resident at once.  At most NEWTON_BLOCKS = 64 of 256 threads are launched, on a chip that
+    // holds 2048, and whatever else runs on it ends by itself; should one still wait for two seconds it
+    // raises ERR_STALL and all of them run to their end.
+    constexpr unsigned long long EMPTY_SLOT = 0x7ff4deadbeef0badull;
+
+    __global__ void k_empty_slots(unsigned long long* slots, long count) {
+      long const i = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
+      if (i < count) slots[i] = EMPTY_SLOT;
+    }
+
+    struct NewtonLds {
+      double sw[3][VT / 64];
+      double sh[3][NEWTON_BLOCKS];
+      double alpha[32], rho[32];
+      int dead;
+    };
+
+    // Totals over the grid of acc[0..K), by sum numbers id .. id + K - 1.
+    template <int K>
+    __device__ inline void grid_sum(NewtonArgs const& A, NewtonLds& L, int id, double const (&acc)[K], double (&tot)[K]) {
+      int const nb = static_cast<int>(gridDim.x), w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        double const v = group_sum<64>(acc[k]);
+        if (lane == 0) L.sw[k][w] = v;
+      }
+      __syncthreads();
+      if (threadIdx.x < K) {
+        double s = 0;
+        for (int q = 0; q < VT / 64; ++q) s += L.sw[threadIdx.x][q];
+        __hip_atomic_store(&A.slots[(id + threadIdx.x) * NEWTON_BLOCKS + blockIdx.x],
+                           static_cast<unsigned long long>(__double_as_longlong(s)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      if (w == 0) {
+        long long const t0 = wall_clock64();
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          unsigned long long const* slot = &A.slots[(id + k) * NEWTON_BLOCKS + (lane < nb ? lane : 0)];
+          unsigned long long v;
+          while (true) {   // ends when every slot is filled, when this workgroup has given up, or after two seconds
+            v = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (__all(v != EMPTY_SLOT) || L.dead) break;
+            if (wall_clock64() - t0 > 200000000ll) {   // 100 MHz
+              L.dead = 1;
+              break;
+            }
+          }
+          L.sh[k][lane] = __longlong_as_double(static_cast<long long>(v));
+        }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < K; ++k) tot[k] = 0.0;
+#pragma unroll 8
+      for (int b = 0; b < nb; ++b)
+#pragma unroll
+        for (int k = 0; k < K; ++k) tot[k] += L.sh[k][b];
+    }
+
+    __global__ __launch_bounds__(VT) void k_lb_newton(NewtonArgs A, unsigned* __restrict__ err) {
+      __shared__ NewtonLds L;
+      long const step = static_cast<long>(gridDim.x) * VT;
+      long const i0 = blockIdx.x * static_cast<long>(VT) + threadIdx.x;
+      int const bound = A.bound;
+      for (int q = threadIdx.x; q < NEWTON_SUMS; q += VT) A.spare[q * NEWTON_BLOCKS + blockIdx.x] = EMPTY_SLOT;
+      if (threadIdx.x == 0) L.dead = 0;
+      if (threadIdx.x < bound - 1) L.rho[threadIdx.x] = A.lb->rho[A.j[threadIdx.x]];
+      auto load = [&](double const* p, double (&v)[4]) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = i0 + u * step < A.n ? p[i0 + u * step] : 0.0;
+      };
+      double q[4], y[4], s[4], yn[4];   // q, later r; the pair's y; s and y of the stage to come
+      double acc[1], tot[1];
+      double h0;
+      {
+        double x[4], px[4], pg[4], acc3[3] = {0, 0, 0}, t[3];
+        load(A.x, x);
+        load(A.g, q);
+        load(A.px, px);
+        load(A.pg, pg);
+        if (bound > 1) {
+          load(A.s[bound - 2], s);
+          load(A.y[bound - 2], yn);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          long const i = i0 + u * step;
+          if (i < A.n) {
+            double const si = x[u] - px[u], yi = q[u] - pg[u];
+            A.s[bound - 1][i] = si;
+            A.y[bound - 1][i] = yi;
+            A.px[i] = x[u];
+            A.pg[i] = q[u];
+            acc3[0] += si * yi;
+            acc3[1] += yi * yi;
+            acc3[2] += si * q[u];
+            y[u] = yi;
+          }
+        }
+        grid_sum<3>(A, L, 0, acc3, t);
+        double const rho = 1.0 / fabs(t[0]);
+        h0 = (1.0 / rho) / t[1];
+        tot[0] = rho * t[2];   // alpha of the newest pair
+        if (threadIdx.x == 0) {
+          L.rho[bound - 1] = rho;
+          if (blockIdx.x == 0) {
+            A.lb->rho[A.j[bound - 1]] = rho;
+            A.lb->h0 = h0;
+          }
+        }
+      }
+      int id = 3;
+      double alpha = tot[0];
+      for (int i = bound - 1; i > 0; --i) {   // loop 1, newest to oldest; s, yn: pair i - 1
+        if (threadIdx.x == 0) L.alpha[i] = alpha;
+        double const c = -1.0 * alpha;
+        acc[0] = 0;
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (i0 + u * step < A.n) {
+            double o = q[u];
+            o += c * y[u];
+            q[u] = o;
+            acc[0] += s[u] * o;
+          }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) y[u] = yn[u];
+        if (i > 1) {
+          load(A.s[i - 2], s);
+          load(A.y[i - 2], yn);
+        }
+        grid_sum<1>(A, L, id++, acc, tot);
+        alpha = L.rho[i - 1] * tot[0];
+      }
+      if (threadIdx.x == 0) L.alpha[0] = alpha;
+      {
+        double const c = -1.0 * alpha;
+        acc[0] = 0;
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (i0 + u * step < A.n) {
+            double o = q[u];
+            o += c * y[u];
+            double const ri = h0 * o;
+            q[u] = ri;
+            acc[0] += y[u] * ri;
+          }
+      }
+      for (int i = 0; i < bound; ++i) {   // loop 2, oldest to newest
+        load(A.s[i], s);
+        bool const last = i + 1 == bound;
+        if (!last) {
+          load(A.y[i + 1], yn);
+        } else if (A.w) {
+          load(A.w, yn);
+        }
+        grid_sum<1>(A, L, id++, acc, tot);
+        double const al = L.alpha[i], rho = L.rho[i];
+        double const c = al - rho * tot[0];
+        acc[0] = 0;
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (i0 + u * step < A.n) {
+            double o = q[u];
+            o += c * s[u];
+            q[u] = o;
+            acc[0] += o * (last && !A.w ? o : yn[u]);
+          }
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (i0 + u * step < A.n) A.r[i0 + u * step] = q[u];
+      leave(acc, A.out);
+      if (threadIdx.x == 0 && L.dead) atomicOr(err, static_cast<unsigned>(ERR_STALL));
+    }
+
     __global__ __launch_bounds__(VT) void k_step(long n, double trust, double const* __restrict__ in, double* __restrict__ q,
                                                  double* __restrict__ x, ListMove lm, double* __restrict__ hsum) {
       __shared__ double sh[VMAXB];
@@ -509,6 +692,14 @@ namespace flyg {
   void lb_loop2(flyg_ctx_s& ctx, long n, int j, LBScalars* lb, double const* in, double* r, double const* s,
                 double const* w, double* out) {
     FLYG_VEC_LAUNCH(k_lb_loop2, j, lb, in, r, s, w, out);
+  }
+  void lb_newton(flyg_ctx_s& ctx, NewtonArgs const& a) {
+    k_lb_newton<<<vec_blocks(a.n), VT, 0, ctx.stream>>>(a, ctx.dflags.get());
+    HIPCHK(hipGetLastError());
+  }
+  void lb_empty_slots(flyg_ctx_s& ctx, unsigned long long* slots, long count) {
+    k_empty_slots<<<static_cast<unsigned>((count + VT - 1) / VT), VT, 0, ctx.stream>>>(slots, count);
+    HIPCHK(hipGetLastError());
   }
   void vec_step(flyg_ctx_s& ctx, long n, double trust, double const* in, double* q, double* x, ListMove lm, double* hsum) {
     FLYG_VEC_LAUNCH(k_step, trust, in, q, x, lm, hsum);

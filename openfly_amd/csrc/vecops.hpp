@@ -57,6 +57,33 @@ namespace flyg {
   void lb_loop2(flyg_ctx_s& ctx, long n, int j, LBScalars* lb, double const* in, double* r, double const* s,
                 double const* w, double* out);
 
+  // The whole two-loop in one launch, for vectors of at most NEWTON_BLOCKS blocks.  Pairs in order, oldest first (the
+  // newest is written); j: their places in lb.  slots: two sets of NEWTON_SLOTS words in turn, those of `slots`
+  // empty, `spare` emptied for the next call.  out: r.w (w = null: r.r).  A workgroup that waits in vain (seconds)
+  // sets ERR_STALL and leaves.
+  constexpr int NEWTON_BLOCKS = 64;
+  constexpr int NEWTON_SUMS = 2 * 32 + 3;
+  constexpr int NEWTON_SLOTS = NEWTON_SUMS * NEWTON_BLOCKS;
+  struct NewtonArgs {
+    long n;
+    int bound;
+    double const* x;
+    double const* g;
+    double* px;
+    double* pg;
+    double* r;
+    double const* w;
+    LBScalars* lb;
+    unsigned long long* slots;
+    unsigned long long* spare;
+    double* out;
+    double* s[32];
+    double* y[32];
+    int j[32];
+  };
+  void lb_newton(flyg_ctx_s& ctx, NewtonArgs const& a);
+  void lb_empty_slots(flyg_ctx_s& ctx, unsigned long long* slots, long count);
+
   // Trust-region step: q *= min(1, trust / sqrt(in)), x -= q, the list follows; the sum itself goes to *hsum.
   void vec_step(flyg_ctx_s& ctx, long n, double trust, double const* in, double* q, double* x, ListMove lm, double* hsum);
   // out: a.b and c.d (c null: one sum); the device error flags go to *hflag (null: not copied).

@@ -52,6 +52,22 @@ def test_steplbfgs_matches_oracle(ctx):
     assert np.array_equal(g_s.newton_step(x, A @ x), A @ x)
 
 
+@pytest.mark.parametrize("N", [1, 1023, 1025, 65536, 65537, 250000])
+def test_steplbfgs_sizes(ctx, N):
+    # One workgroup, a few, the most that take the step in one launch (64), one more than that, and more elements than
+    # the launched threads hold at once; histories shorter than, equal to and longer than m.
+    # Bound: sums of N terms in another order differ by up to N roundings.
+    rng = np.random.default_rng(N)
+    d = rng.uniform(1.0, 3.0, N)
+    g_s, o_s = fa.StepLBFGS(ctx, 3), po.StepLBFGS(3)
+    x = rng.normal(size=N)
+    for it in range(7):
+        g = d * x + 0.1 * np.sin(x)
+        qg, qo = g_s.newton_step(x, g), o_s.newton_step(x, g)
+        assert np.max(np.abs(qg - qo)) <= max(1e-12, N * 2.2e-16) * np.max(np.abs(qo)), it
+        x = x - 0.5 * qo
+
+
 def test_minimise_matches_oracle(ctx, wen):
     pot, data = wen
     pos, basis = small_vacancy_system(a=2.855324)
