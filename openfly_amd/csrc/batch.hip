@@ -845,7 +845,7 @@ namespace flyg {
                   o_hv = in.add<double>(nhv), o_hn = in.add<double>(nhn), o_rs = in.add<double>(nrs);
       Layout sc;
       std::size_t o_cur = sc.add<double4>(nreg), o_base = sc.add<double4>(nreg), o_type = sc.add<uint8_t>(nreg),
-                  o_rhof = sc.add<double>(nreg), o_fp = sc.add<double>(nreg), o_act = sc.add<unsigned>(nent),
+                  o_rhof = sc.add<double>(nreg), o_fp = sc.add<double>(nreg), o_act = sc.add<unsigned>(nent + sk::U),
                   o_alen = sc.add<int>(nreg), o_ws = sc.add<double>(nws),
                   o_q = sc.add<unsigned>(1), o_rsc = sc.add<unsigned>(1);
       std::size_t zero_end = sc.size;

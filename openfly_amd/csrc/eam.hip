@@ -1,12 +1,14 @@
 // EAM / Finnis-Sinclair energy, gradient and Hessian-vector product on gfx950
 // (replaces potential::EAM::energy / gradient / hessian, eam.cpp:33-233).
 //
-// Work mapping: L lanes of a wavefront cooperate on one atom's neighbour row (ELL layout, 32-bit
-// packed entries), each lane striding the row by L; partial sums are combined with cross-lane
-// shuffles in a fixed order, so results are bitwise reproducible run to run.  No atomics touch
-// floating-point data.  Positions are double4 (x, y, z, w): a neighbour gather is one 32-byte load,
-// and pass 1 writes (x, y, z, F'(rho)) so pass 2 gets the neighbour's position and F' in that load (in
-// the mixed form w holds F' as FP32 and the species, see pack_fp_type).
+// Work mapping: systems with enough cells run in tiles (a workgroup stages a box of cells and its halo in LDS
+// and walks 16-bit rows, see TILED PASSES below); smaller ones and calls that ask for it run row by row: L lanes
+// (16 by default) of a wavefront cooperate on one atom's neighbour row (ELL layout, 32-bit packed entries), each
+// lane striding the row by L.  Either way a row's sums go through Acc16's 16 slots, so the two give the same bits
+// and results are reproducible run to run.  No atomics touch floating-point data.  In the rows positions are
+// double4 (x, y, z, w): a neighbour gather is one 32-byte load, and pass 1 writes (x, y, z, F'(rho)) so pass 2 gets
+// the neighbour's position and F' in that load (in the mixed form w holds F' as FP32 and the species, see
+// pack_fp_type).
 //
 //   pass 1 (density):  rho_b = sum_a phi_{t_a->t_b}(r_ab);  F'_b = F_{t_b}'(rho_b)     (eam.cpp:62-86)
 //   pass 2 (force):    dE/dr_g = -sum_a [V'(r) + F'_g phi'_{a->g}(r) + F'_a phi'_{g->a}(r)] (r_a - r_g)/r

@@ -387,15 +387,30 @@ namespace flyg {
       R r[U], rinv[U];
     };
 
-    template <bool MIX>
-    __device__ inline void load_quad(SView const& v, unsigned const* ent, double rc2, double4 const& pi, int k0,
-                                     int stride, int b, int c, Quad<MIX>& Q) {
-      unsigned en[U];
+    // A thread's U entries of one step (k0, k0 + stride, ...) of the row b..c.  Past its end the row's first entry
+    // stands in, in an empty row entry 0.
+    __device__ __forceinline__ void load_step(unsigned const* ent, int k0, int stride, int b, int c, unsigned (&en)[U]) {
 #pragma unroll
       for (int q = 0; q < U; ++q) {
-        int k = k0 + q * stride;
-        en[q] = ent[k < c ? k : b];
+        int const k = k0 + q * stride;
+        unsigned const e = ent[k < c ? k : b];
+        en[q] = c > b ? e : 0u;
       }
+    }
+    // The same for stride 1, as one load: a row may start at any entry (4-byte alignment), and up to U entries
+    // past a row may be read, which the array has room for and no lane uses.
+    struct __attribute__((packed, aligned(4))) Entries {
+      unsigned e[U];
+    };
+    __device__ __forceinline__ void load_step_run(unsigned const* ent, int k0, int b, int c, unsigned (&en)[U]) {
+      Entries const run = *reinterpret_cast<Entries const*>(ent + k0);
+#pragma unroll
+      for (int q = 0; q < U; ++q) en[q] = k0 + q < c ? run.e[q] : (k0 < c ? run.e[0] : 0u);
+    }
+
+    template <bool MIX>
+    __device__ __forceinline__ void load_quad(SView const& v, unsigned const (&en)[U], double rc2, double4 const& pi, int k0,
+                                              int stride, int c, Quad<MIX>& Q) {
       double4 pj[U];
       double3 sh[U];
 #pragma unroll
@@ -441,7 +456,7 @@ namespace flyg {
       double const cf2 = cf * cf, cm2 = cm * cm;
       int const lane = tm.tid % L;
       int const gbase = (tm.tid & 63) - lane;   // first lane of this row group in the wavefront
-      for (int r0 = tm.tid / L; r0 < v.nm; r0 += T / L) {
+      for (int r0 = tm.tid / L; r0 < v.nr; r0 += T / L) {
         double4 pi = v.cur[r0];
         int b = v.rowptr[r0], c = v.rowptr[r0 + 1];
         int cnt = 0;
@@ -456,7 +471,7 @@ namespace flyg {
             double4 pj = v.cur[j];
             double dx = (pj.x + sh.x) - pi.x, dy = (pj.y + sh.y) - pi.y, dz = (pj.z + sh.z) - pi.z;
             double r2 = dx * dx + dy * dy + dz * dz;
-            keep = r2 < (j < v.nm ? cm2 : cf2);
+            keep = r2 < (r0 < v.nm && j < v.nm ? cm2 : cf2);
           }
           unsigned long long m = __ballot(keep);
           unsigned gm = static_cast<unsigned>((m >> gbase) & ((1ull << L) - 1ull));
@@ -464,20 +479,6 @@ namespace flyg {
           cnt += __popc(gm);
         }
         if (lane == 0) v.alen[r0] = cnt;
-      }
-      for (int r0 = v.nm + tm.tid; r0 < v.nr; r0 += T) {
-        double4 pi = v.cur[r0];
-        int b = v.rowptr[r0], c = v.rowptr[r0 + 1];
-        int cnt = 0;
-        for (int k = b; k < c; ++k) {
-          unsigned en = v.ent[k];
-          int j = static_cast<int>(en & NB_IDX_MASK);
-          double3 sh = v.S[en >> NB_SHIFT_BITS];
-          double4 pj = v.cur[j];
-          double dx = (pj.x + sh.x) - pi.x, dy = (pj.y + sh.y) - pi.y, dz = (pj.z + sh.z) - pi.z;
-          if (dx * dx + dy * dy + dz * dz < cf2) v.act[b + cnt++] = en;
-        }
-        v.alen[r0] = cnt;
       }
       __syncthreads();
     }
@@ -520,53 +521,104 @@ namespace flyg {
 #pragma unroll
         for (int q = 0; q < U; ++q) out[q] = sg[q].use ? static_cast<double>(poly0(cf[q], sg[q].t)) : 0.0;
       };
-      // Mobile rows (long: every region neighbour): L lanes per row, 16-slot sums.
-      for (int r0 = tm.tid / L; r0 < v.nm; r0 += T / L) {
-        double4 pi = v.cur[r0];
-        int ti = MULTI ? v.type[r0] : t0;
-        Acc16<L> rho_acc;
-        int b = v.rowptr[r0], c = b + v.alen[r0];
-        for (int k0 = b + lane; k0 < c; k0 += U * L) {
-          Quad<MIX> Q;
-          load_quad<MIX>(v, v.act, Tb.rc2, pi, k0, L, b, c, Q);
-          double d[U];
-          densities(Q, ti, d);
-#pragma unroll
-          for (int q = 0; q < U; ++q)
-            if (Q.in[q]) rho_acc.add_slot(q % NS, d[q]);
+      // A thread's rows, first, first + step, ... (< n), in steps of W entries: row(r0) starts a row, body(en, k0, c,
+      // ahead) does a step and calls ahead() once its positions are loaded, end(r0) ends the row.  ahead() issues the
+      // entry loads of the next step, at a row's last step those of the next row's first, so that no step begins
+      // with a wait for its entries.  All lanes of a row take the same steps.
+      auto walk = [&](int first, int n, int step, int W, auto const& load, auto const& row, auto const& body, auto const& end) {
+        int r0 = first, b = 0, c = 0;
+        unsigned en[U] = {};
+        if (r0 < n) {
+          b = v.rowptr[r0];
+          c = b + v.alen[r0];
+          load(b, b, c, en);
         }
-        double rho = rho_acc.total();
-        if (lane == 0) v.cur[r0].w = spl64<1>(Tb, FF(ti), rho, e);
-      }
+        for (; r0 < n; r0 += step) {
+          int nb = b, nc = c;
+          if (r0 + step < n) {
+            nb = v.rowptr[r0 + step];
+            nc = nb + v.alen[r0 + step];
+          }
+          row(r0);
+          for (int s = b;; s += W) {
+            bool const last = s + W >= c;
+            unsigned nx[U];
+            body(en, s, c, [&]() { load(last ? nb : s + W, last ? nb : b, last ? nc : c, nx); });
+#pragma unroll
+            for (int q = 0; q < U; ++q) en[q] = nx[q];
+            if (last) break;
+          }
+          end(r0);
+          b = nb;
+          c = nc;
+        }
+      };
+      auto const lanes_load = [&](int s, int b, int c, unsigned (&en)[U]) { load_step(v.act, s + lane, L, b, c, en); };
+      auto const run_load = [&](int s, int b, int c, unsigned (&en)[U]) { load_step_run(v.act, s, b, c, en); };
+      // Mobile rows (long: every region neighbour): L lanes per row, 16-slot sums.
+      double4 pi;
+      int ti = t0;
+      Acc16<L> rho_acc;
+      walk(
+          tm.tid / L, v.nm, T / L, U * L, lanes_load,
+          [&](int r0) {
+            pi = v.cur[r0];
+            if (MULTI) ti = v.type[r0];
+            rho_acc = Acc16<L>{};
+          },
+          [&](unsigned const(&en)[U], int s, int c, auto const& ahead) {
+            Quad<MIX> Q;
+            load_quad<MIX>(v, en, Tb.rc2, pi, s + lane, L, c, Q);
+            ahead();
+            double d[U];
+            densities(Q, ti, d);
+#pragma unroll
+            for (int q = 0; q < U; ++q)
+              if (Q.in[q]) rho_acc.add_slot(q % NS, d[q]);
+          },
+          [&](int r0) {
+            double const rho = rho_acc.total();
+            if (lane == 0) v.cur[r0].w = spl64<1>(Tb, FF(ti), rho, e);
+          });
       // Frozen-shell rows (short: mobile neighbours only): one thread per row, entries summed in order,
       // then the frozen part of the density.  Neither order depends on the workgroup shape.
-      for (int r0 = v.nm + tm.tid; r0 < v.nr; r0 += T) {
-        double4 pi = v.cur[r0];
-        int ti = MULTI ? v.type[r0] : t0;
-        int b = v.rowptr[r0], c = b + v.alen[r0];
-        double rho = 0.0;
-        for (int k0 = b; k0 < c; k0 += U) {
-          Quad<MIX> Q;
-          load_quad<MIX>(v, v.act, Tb.rc2, pi, k0, 1, b, c, Q);
-          double d[U];
-          densities(Q, ti, d);
+      double rho = 0.0;
+      walk(
+          v.nm + tm.tid, v.nr, T, U, run_load,
+          [&](int r0) {
+            pi = v.cur[r0];
+            if (MULTI) ti = v.type[r0];
+            rho = 0.0;
+          },
+          [&](unsigned const(&en)[U], int s, int c, auto const& ahead) {
+            Quad<MIX> Q;
+            load_quad<MIX>(v, en, Tb.rc2, pi, s, 1, c, Q);
+            ahead();
+            double d[U];
+            densities(Q, ti, d);
 #pragma unroll
-          for (int q = 0; q < U; ++q)
-            if (Q.in[q]) rho = __dadd_rn(rho, d[q]);
-        }
-        rho = __dadd_rn(rho, v.rhof[r0]);
-        v.cur[r0].w = spl64<1>(Tb, FF(ti), rho, e);
-      }
+            for (int q = 0; q < U; ++q)
+              if (Q.in[q]) rho = __dadd_rn(rho, d[q]);
+          },
+          [&](int r0) {
+            rho = __dadd_rn(rho, v.rhof[r0]);
+            v.cur[r0].w = spl64<1>(Tb, FF(ti), rho, e);
+          });
       __syncthreads();
-      for (int r0 = tm.tid / L; r0 < v.nm; r0 += T / L) {
-        double4 pi = v.cur[r0];
-        double fpi = pi.w;
-        int ti = MULTI ? v.type[r0] : t0;
-        Acc16<L> gx, gy, gz;
-        int b = v.rowptr[r0], c = b + v.alen[r0];
-        for (int k0 = b + lane; k0 < c; k0 += U * L) {
+      double fpi = 0.0;
+      Acc16<L> gx, gy, gz;
+      walk(
+        tm.tid / L, v.nm, T / L, U * L, lanes_load,
+        [&](int r0) {
+          pi = v.cur[r0];
+          fpi = pi.w;
+          if (MULTI) ti = v.type[r0];
+          gx = gy = gz = Acc16<L>{};
+        },
+        [&](unsigned const(&en)[U], int s, int c, auto const& ahead) {
           Quad<MIX> Q;
-          load_quad<MIX>(v, v.act, Tb.rc2, pi, k0, L, b, c, Q);
+          load_quad<MIX>(v, en, Tb.rc2, pi, s + lane, L, c, Q);
+          ahead();
           Seg<MIX> sv[U], sa[U], sb[U];
           decltype(coef_of<MIX>(Tb, phi0, sv[0])) cv[U], ca[U], cb[U];
 #pragma unroll
@@ -602,14 +654,15 @@ namespace flyg {
               gz.add_slot(q % NS, -cf * Q.dz[q]);
             }
           }
-        }
-        double tx = gx.total(), ty = gy.total(), tz = gz.total();
-        if (lane == 0) {
-          g[3 * r0] = tx;
-          g[3 * r0 + 1] = ty;
-          g[3 * r0 + 2] = tz;
-        }
-      }
+        },
+        [&](int r0) {
+          double tx = gx.total(), ty = gy.total(), tz = gz.total();
+          if (lane == 0) {
+            g[3 * r0] = tx;
+            g[3 * r0 + 1] = ty;
+            g[3 * r0 + 2] = tz;
+          }
+        });
       // Spline errors gather in one LDS word (sticky for the search): every thread reads it after the barrier.
       if (e) atomicOr(v.errw, e);
       __syncthreads();
@@ -1001,7 +1054,19 @@ namespace flyg {
       long gticks = 0;
       auto timed_gradient = [&](double* g) -> unsigned {
         long t = static_cast<long>(wall_clock64());
-        unsigned r = region_gradient<T, L, MIX, MULTI>(A, v, tm, g);
+        // Twice the code, by where the positions are: the compiler then addresses them as LDS.  Through a generic
+        // pointer each access is a flat load, which returns later than an LDS read and is waited for together with
+        // every global load before it.  With the walks' early entry loads: 27.9 -> 24.4 us a region gradient (mixed,
+        // 256 searches on 16k atoms, 512 threads), 36.3 -> 31.4 us (FP64, 2k atoms).  The vector algebra gains
+        // nothing from LDS addresses (20.2 us with both), so it stays one copy.
+        unsigned r;
+        if (pos_lds) {
+          SView w = v;
+          w.cur = lds_area;
+          r = region_gradient<T, L, MIX, MULTI>(A, w, tm, g);
+        } else {
+          r = region_gradient<T, L, MIX, MULTI>(A, v, tm, g);
+        }
         gticks += static_cast<long>(wall_clock64()) - t;
         return r;
       };

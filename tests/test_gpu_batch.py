@@ -147,6 +147,43 @@ def test_results_independent_of_kernel_shape(ctx, setup):
             assert np.array_equal(a["pos"], m["pos"])
 
 
+@pytest.mark.parametrize("precision", [fa.FP64, fa.MIXED])
+@pytest.mark.parametrize("radius", [2.0, 9.0])
+def test_small_and_large_regions(ctx, setup, radius, precision):
+    # A single mobile atom (shell rows of one entry, fewer rows than lanes), and more region rows than 256 threads
+    # keep in LDS and 1024 do: the same bits in every shape, FP64 equal to the oracle.
+    # Bound: three steps from a start 0.1 A off; sums in another order differ by 1e-13 of a force of about 1 eV/A,
+    # each step of at most 0.5 A amplifies that by less than 1e2.
+    cells = 11
+    pos = np.delete(systems.bcc_sites(A_WEN, cells), 0, axis=0)
+    basis = np.diag([cells * A_WEN] * 3)
+    t = np.zeros(len(pos), np.uint32)
+    L = np.diag(basis)
+    centre = 700
+    d = pos - pos[centre]
+    d -= L * np.round(d / L)
+    frozen = (np.einsum("ij,ij->i", d, d) > radius * radius).astype(np.uint8)
+    rng = np.random.default_rng(int(radius))
+    x, ax = pos.copy(), np.zeros_like(pos)
+    x[frozen == 0] += rng.normal(0.0, 0.1, (int((frozen == 0).sum()), 3))
+    ax[frozen == 0] = rng.normal(size=(int((frozen == 0).sum()), 3))
+    opt = dict(f2norm=1e-8, max_steps=3)
+    outs = []
+    for T, lanes in ((256, 8), (256, 16), (512, 8), (1024, 16)):
+        b = fa.Batch(ctx, setup["pot"], fa.Box(basis), pos, t, dimer=opt, precision=precision, block_threads=T,
+                     lanes_per_atom=lanes)
+        ids = b.submit([centre], [radius], x[None], ax[None])
+        b.run()
+        outs.append(b.result(ids[0], positions=True))
+    for o in outs[1:]:
+        assert all(o[k] == outs[0][k] for k in ("exit", "steps", "grads", "barrier"))
+        assert np.array_equal(o["pos"], outs[0]["pos"])
+    if precision == fa.FP64:
+        r = po.find_sp(po.Box(basis), setup["data"], x, ax, t, frozen, pos, threads=8, dimer=opt)
+        assert r["exit"] == outs[0]["exit"] and r["steps"] == outs[0]["steps"]
+        assert np.max(np.abs(r["pos"] - outs[0]["pos"].reshape(-1, 3))) < 1e-7
+
+
 def test_tuned_shape_is_reported_and_reusable(ctx, setup):
     # flyg_batch_shape: (0, 0) before the first run, then the autotuned (block threads, lanes per atom);
     # a batch given that shape skips the tuning and reproduces the results bit for bit.
