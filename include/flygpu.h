@@ -73,6 +73,11 @@ int flyg_ctx_create(int device, flyg_ctx* out);
 int flyg_ctx_destroy(flyg_ctx ctx);
 const char* flyg_ctx_last_error(flyg_ctx ctx);
 int flyg_ctx_synchronize(flyg_ctx ctx);
+/* How often a workgroup of the one-launch L-BFGS step (StepLBFGS on host arrays, LBFGS, Dimer, Rotor; vectors of at
+ * most 65536 elements) looks for the other workgroups' sums before it gives up and the step is finished by one
+ * launch per stage: the same result bit for bit, and how a step gets on beside long kernels that fill the chip.
+ * Default 16384 (about 10 ms); 0: every step gives up at once. */
+int flyg_ctx_set_step_polls(flyg_ctx ctx, unsigned polls);
 /* The hipStream_t of the context, for callers that time or order work around it. */
 void* flyg_ctx_stream(flyg_ctx ctx);
 /* Device name and compute-unit count. */

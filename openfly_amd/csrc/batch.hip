@@ -229,9 +229,7 @@ namespace flyg {
         HIPCHK(hipMemcpyAsync(A.types.get(), types, n * sizeof(uint32_t), hipMemcpyHostToDevice, st));
         list_rebuild(*A.nl, A.pos.get(), n);
         eam_density(*eam, *A.nl, A.types.get(), S->d_rho.get());
-        unsigned fl = ctx->take_flags();   // synchronises the stream before the scratch goes away
-        if (fl & ERR_SPLINE_OOB) throw Error(FLYG_SPLINE_OOB, "x is outside tabulated region of a spline");
-        if (fl & ERR_TYPE) throw Error(FLYG_INVALID_ARG, "TypeID out of range");
+        throw_flags(ctx->take_flags());   // synchronises the stream before the scratch goes away
       }
       return S;
     }

@@ -66,12 +66,7 @@ namespace {
     return stage.get();
   }
 
-  void check_errors(flyg_ctx_s& ctx) {
-    unsigned fl = ctx.take_flags();
-    if (fl & ERR_SPLINE_OOB) throw Error(FLYG_SPLINE_OOB, "x is outside tabulated region of a spline");
-    if (fl & ERR_TYPE) throw Error(FLYG_INVALID_ARG, "TypeID out of range");
-    if (fl) throw Error(FLYG_DEVICE_ERROR, "device error flag set");
-  }
+  void check_errors(flyg_ctx_s& ctx) { throw_flags(ctx.take_flags()); }
 }  // namespace
 
 extern "C" {
@@ -97,6 +92,7 @@ int flyg_ctx_create(int device, flyg_ctx* out) {
     c->dflags.reserve(16);
     HIPCHK(hipMemset(c->dflags.get(), 0, 16 * sizeof(unsigned)));
     HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&c->hflags), 16 * sizeof(unsigned), hipHostMallocDefault));
+    std::memset(c->hflags, 0, 16 * sizeof(unsigned));
     HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&c->hpart), (VPART + 16) * sizeof(double), hipHostMallocDefault));
     *out = c.release();
   });
@@ -111,6 +107,10 @@ const char* flyg_ctx_last_error(flyg_ctx ctx) { return ctx ? ctx->err.c_str() : 
 
 int flyg_ctx_synchronize(flyg_ctx ctx) {
   return guard(ctx, [&] { check_errors(*ctx); });
+}
+
+int flyg_ctx_set_step_polls(flyg_ctx ctx, unsigned polls) {
+  return guard(ctx, [&] { ctx->step_polls = polls; });
 }
 
 void* flyg_ctx_stream(flyg_ctx ctx) { return ctx ? static_cast<void*>(ctx->stream) : nullptr; }
@@ -470,10 +470,18 @@ int flyg_steplbfgs_newton_step(flyg_steplbfgs s, const double* x, const double* 
       dx = s->x.get();
       dg = s->g.get();
     }
-    double* r = s->core->newton_step(dx, dg, len);
-    HIPCHK(hipMemcpyAsync(q, r, len * sizeof(double), where == FLYG_HOST ? hipMemcpyDeviceToHost : hipMemcpyDeviceToDevice,
-                          ctx.stream));
-    if (where == FLYG_HOST) HIPCHK(hipStreamSynchronize(ctx.stream));
+    bool const host = where == FLYG_HOST;
+    // A device caller gets no chance to see that a step gave up: its steps do not wait.
+    double* r = s->core->newton_step(dx, dg, len, nullptr, nullptr, host);
+    auto give = [&] {
+      HIPCHK(hipMemcpyAsync(q, r, len * sizeof(double), host ? hipMemcpyDeviceToHost : hipMemcpyDeviceToDevice, ctx.stream));
+      if (host) HIPCHK(hipStreamSynchronize(ctx.stream));
+    };
+    give();
+    if (host && s->core->stalled()) {
+      r = s->core->again(nullptr, nullptr);
+      give();
+    }
   });
 }
 

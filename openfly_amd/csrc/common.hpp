@@ -36,7 +36,7 @@ namespace flyg {
   }
 
   // Device-side error flags (bit set, read back by the host after a call).
-  enum : unsigned { ERR_SPLINE_OOB = 1u, ERR_LIST_OVERFLOW = 2u, ERR_REGION = 4u, ERR_NAN = 8u, ERR_TYPE = 16u, ERR_STALL = 32u };
+  enum : unsigned { ERR_SPLINE_OOB = 1u, ERR_LIST_OVERFLOW = 2u, ERR_REGION = 4u, ERR_NAN = 8u, ERR_TYPE = 16u };
 
   // A device-resident TypeID the host could not check: out of range sets ERR_TYPE (reported as
   // FLYG_INVALID_ARG at the next synchronisation) and species 0 is used so no table index leaves its array.

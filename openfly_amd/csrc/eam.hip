@@ -1036,11 +1036,7 @@ namespace flyg {
     HIPCHK(hipGetLastError());
     dev_sum(*E.ctx, E.eatom.get(), nl.n, E.ctx->hpart, E.ctx->hflags + 1);
     HIPCHK(hipStreamSynchronize(E.ctx->stream));
-    if (E.ctx->hflags[1]) {
-      unsigned fl = E.ctx->take_flags();
-      if (fl & ERR_SPLINE_OOB) throw Error(FLYG_SPLINE_OOB, "x is outside tabulated region of a spline");
-      if (fl & ERR_TYPE) throw Error(FLYG_INVALID_ARG, "TypeID out of range");
-    }
+    if (E.ctx->hflags[1]) throw_flags(E.ctx->take_flags());
     return host_sum(E.ctx->hpart, 0, nl.n);
   }
 
@@ -1218,9 +1214,7 @@ namespace flyg {
     k_table_eval<<<static_cast<unsigned>((m + 255) / 256), 256, 0, st>>>(E.tab, s, dx.get(), m, deriv, dout.get(),
                                                                          E.ctx->dflags.get());
     HIPCHK(hipMemcpyAsync(out, dout.get(), m * sizeof(double), hipMemcpyDeviceToHost, st));
-    unsigned fl = E.ctx->take_flags();
-    if (fl & ERR_SPLINE_OOB) throw Error(FLYG_SPLINE_OOB, "x is outside tabulated region of a spline");
-    if (fl & ERR_TYPE) throw Error(FLYG_INVALID_ARG, "TypeID out of range");
+    throw_flags(E.ctx->take_flags());
   }
 
   namespace {

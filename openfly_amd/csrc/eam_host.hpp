@@ -35,8 +35,12 @@ struct flyg_ctx_s {
   std::string err;
   int cus = 0;
   flyg::DBuf<unsigned> dflags;   // [0] error bits, [1..] scratch counters
-  unsigned* hflags = nullptr;    // pinned: [0] error bits read by take_flags, [1] those a kernel left
+  // Pinned: [0] error bits read by take_flags, [1] those a kernel left, [2] a count, [3] set by an L-BFGS step that
+  // gave up waiting (lb_newton), [4] by one of a rotor, which may be under way beside it.
+  unsigned* hflags = nullptr;
   double* hpart = nullptr;       // pinned: block partial sums that kernels write for the host, then scalars
+
+  unsigned step_polls = 1u << 14;   // polls before a workgroup of lb_newton gives up (about 10 ms)
 
   int refs = 1;                  // the context lives until its creator and every handle released it
 
@@ -145,6 +149,13 @@ struct flyg_list_s {
 namespace flyg {
   // Shift vectors of the 27 image codes (sum of +-basis columns), for pair arithmetic.
   void shift_table(BoxDesc const& b, double3* out27);
+
+  // What take_flags returned, as an error: whoever clears the bits reports every one of them.
+  inline void throw_flags(unsigned fl) {
+    if (fl & ERR_SPLINE_OOB) throw Error(FLYG_SPLINE_OOB, "x is outside tabulated region of a spline");
+    if (fl & ERR_TYPE) throw Error(FLYG_INVALID_ARG, "TypeID out of range");
+    if (fl) throw Error(FLYG_DEVICE_ERROR, "device error flag set");
+  }
 
   // neigh.hip
   void list_rebuild(flyg_list_s& nl, double const* d_xyz, long n);

@@ -634,9 +634,7 @@ namespace flyg {
     HIPCHK(hipGetLastError());
     std::vector<double> w(n3m);
     HIPCHK(hipMemcpyAsync(w.data(), lam, n3m * sizeof(double), hipMemcpyDeviceToHost, st));
-    unsigned fl = ctx.take_flags();   // synchronises
-    if (fl & ERR_SPLINE_OOB) throw Error(FLYG_SPLINE_OOB, "x is outside tabulated region of a spline");
-    if (fl & ERR_TYPE) throw Error(FLYG_INVALID_ARG, "TypeID out of range");
+    throw_flags(ctx.take_flags());   // synchronises
     std::sort(w.begin(), w.end());
     return w;
   }

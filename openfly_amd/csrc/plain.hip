@@ -35,13 +35,15 @@ namespace flyg {
   // newest pair; the first call returns g).
   // ================================================================================================
 
-  DevLBFGS::DevLBFGS(flyg_ctx_s* ctx, int m) : m_ctx(ctx), m_m(m), m_s(static_cast<std::size_t>(m)), m_y(static_cast<std::size_t>(m)) {
+  DevLBFGS::DevLBFGS(flyg_ctx_s* ctx, int m, bool rotor)
+      : m_ctx(ctx), m_hstalled(ctx->hflags + (rotor ? 4 : 3)), m_m(m), m_s(static_cast<std::size_t>(m)), m_y(static_cast<std::size_t>(m)) {
     require(m > 0 && m <= 32, "L-BFGS history length must be in [1, 32]");
     m_sc.reserve(1);
     m_part.reserve(2 * VPART);
   }
 
-  double* DevLBFGS::newton_step(double const* x, double const* g, long N, double const* w, double const** sums) {
+  double* DevLBFGS::newton_step(double const* x, double const* g, long N, double const* w, double const** sums,
+                                bool may_wait) {
     flyg_ctx_s& ctx = *m_ctx;
     if (m_k > 0) require(N == m_N, "Call to newton_step() with a different number of atoms than the history");
     if (N != m_N) {
@@ -54,26 +56,22 @@ namespace flyg {
       m_N = N;
     }
     LBScalars* lb = m_sc.get();
-    double* in = m_part.get();          // partial sums of the stage before
-    double* out = in + VPART;           // ... and of this one
-    double* q = m_q.get();
+    double* out = m_part.get() + VPART;
     double* r = m_r.get();
     if (m_k == 0) {
-      lb_first(ctx, N, x, g, m_px.get(), m_pg.get(), r, w, out);
+      lb_first(ctx, N, lb, x, g, m_px.get(), m_pg.get(), r, w, out);
       ++m_k;
       if (sums) *sums = out;
       return r;
     }
     int const bound = m_k <= m_m ? m_k : m_m;
-    int const oldest = m_k <= m_m ? 0 : m_k - m_m;
-    auto pair = [&](int i) { return (i + oldest) % m_m; };   // i = 0 oldest .. bound - 1 newest
-    int const newest = pair(bound - 1);
-    if (vec_blocks(N) <= NEWTON_BLOCKS) {   // one launch (longer vectors: a launch a stage, bound by their bytes)
+    // One launch, for longer vectors a launch a stage.
+    if (may_wait && vec_blocks(N) <= NEWTON_BLOCKS && m_rest == 0) {
       if (m_slots_n != N) {
         m_slots.reserve(2 * NEWTON_SLOTS);
         lb_empty_slots(ctx, m_slots.get(), 2 * NEWTON_SLOTS);
-        m_slots_n = N;
       }
+      m_slots_n = -1;   // until the launch has succeeded
       NewtonArgs a{};
       a.n = N;
       a.bound = bound;
@@ -87,36 +85,69 @@ namespace flyg {
       a.slots = m_slots.get() + m_slots_used * NEWTON_SLOTS;
       m_slots_used = 1 - m_slots_used;
       a.spare = m_slots.get() + m_slots_used * NEWTON_SLOTS;
+      a.polls = ctx.step_polls;
+      a.hstalled = m_hstalled;
       a.out = out;
       for (int i = 0; i < bound; ++i) {
-        a.j[i] = pair(i);
+        a.j[i] = pair(m_k, i);
         a.s[i] = m_s[a.j[i]].get();
         a.y[i] = m_y[a.j[i]].get();
       }
+      *m_hstalled = 0;
       lb_newton(ctx, a);
+      m_slots_n = N;
       ++m_k;
       if (sums) *sums = out;
       return r;
     }
+    if (m_rest > 0) --m_rest;
+    int const newest = pair(m_k, bound - 1);
     lb_hist(ctx, N, x, g, m_px.get(), m_pg.get(), m_s[newest].get(), m_y[newest].get(), out);
-    std::swap(in, out);
+    ++m_k;
+    return stages(m_k - 1, w, sums);
+  }
+
+  // The step of call k + 1 from the sums that lb_hist left, a launch a stage.
+  double* DevLBFGS::stages(int k, double const* w, double const** sums) {
+    flyg_ctx_s& ctx = *m_ctx;
+    long const N = m_N;
+    LBScalars* lb = m_sc.get();
+    double* out = m_part.get();         // partial sums of this stage
+    double* in = out + VPART;           // ... and of the one before
+    double* q = m_q.get();
+    double* r = m_r.get();
+    int const bound = k <= m_m ? k : m_m;
+    int const newest = pair(k, bound - 1);
     double const* from = m_pg.get();    // q before loop 1: the gradient lb_hist kept
     for (int i = bound - 1; i > 0; --i) {
-      int const j = pair(i);
-      lb_loop1(ctx, N, j == newest, j, lb, in, from, m_y[j].get(), m_s[pair(i - 1)].get(), q, out);
+      int const j = pair(k, i);
+      lb_loop1(ctx, N, j == newest, j, lb, in, from, m_y[j].get(), m_s[pair(k, i - 1)].get(), q, out);
       std::swap(in, out);
       from = q;
     }
-    lb_turn(ctx, N, bound == 1, pair(0), lb, in, from, m_y[pair(0)].get(), r, out);
+    int const oldest = pair(k, 0);
+    lb_turn(ctx, N, bound == 1, oldest, lb, in, from, m_y[oldest].get(), r, out);
     std::swap(in, out);
     for (int i = 0; i < bound; ++i) {
-      int const j = pair(i);
-      lb_loop2(ctx, N, j, lb, in, r, m_s[j].get(), i + 1 < bound ? m_y[pair(i + 1)].get() : w, out);
+      int const j = pair(k, i);
+      lb_loop2(ctx, N, j, lb, in, r, m_s[j].get(), i + 1 < bound ? m_y[pair(k, i + 1)].get() : w, out);
       std::swap(in, out);
     }
-    ++m_k;
     if (sums) *sums = in;
     return r;
+  }
+
+  bool DevLBFGS::stalled() {
+    bool const s = *m_hstalled != 0;
+    *m_hstalled = 0;
+    return s;
+  }
+
+  double* DevLBFGS::again(double const* w, double const** sums) {
+    int const k = m_k - 1, newest = pair(k, (k <= m_m ? k : m_m) - 1);
+    m_rest = m_ctx->step_polls / 64;   // the chip is busy: a wait in vain is spread over so many steps
+    lb_again(*m_ctx, m_N, m_sc.get(), m_s[newest].get(), m_y[newest].get(), m_pg.get(), m_part.get() + VPART);
+    return stages(k, w, sums);
   }
 
   std::unique_ptr<flyg_list_s> make_list(flyg_ctx_s* ctx, double const* basis, int const* periodic, double rc) {
@@ -129,12 +160,6 @@ namespace flyg {
   }
 
   namespace {
-    void throw_flags(unsigned fl) {
-      if (fl & ERR_SPLINE_OOB) throw Error(FLYG_SPLINE_OOB, "x is outside tabulated region of a spline");
-      if (fl & ERR_TYPE) throw Error(FLYG_INVALID_ARG, "TypeID out of range");
-      if (fl & ERR_STALL) throw Error(FLYG_DEVICE_ERROR, "an L-BFGS step waited in vain for the rest of its workgroups");
-    }
-
     void check_flags(flyg_ctx_s& ctx) { throw_flags(ctx.take_flags()); }
 
     void sync(flyg_ctx_s& ctx) { HIPCHK(hipStreamSynchronize(ctx.stream)); }
@@ -177,8 +202,13 @@ namespace flyg {
       observe(ctx, m.obs, m.obs_user, i, x, n, m.obs_host);
       if (mag_g < o.f2norm * o.f2norm) return false;
       double const* qq;
-      double* q = m.core->newton_step(x, g, N, nullptr, &qq);
-      vec_step(ctx, N, trust, qq, q, x, list_move(*m.nl), &hstep);
+      double* q = m.core->newton_step(x, g, N, nullptr, &qq, true);
+      auto step = [&] { vec_step(ctx, N, trust, qq, q, x, list_move(*m.nl), m.core->stalled_word(), &hstep); };
+      step();
+      auto redo = [&] {   // the step gave up: x and the list are where they were
+        q = m.core->again(nullptr, &qq);
+        step();
+      };
       // The step is at most the trust radius long: while that cannot use up the skin, its length is read
       // with the next sums instead of on its own.
       bool known = false;
@@ -190,15 +220,26 @@ namespace flyg {
       };
       if (!(acc + 1.001 * trust < 0.5 * skin)) {
         sync(ctx);
+        if (m.core->stalled()) {
+          redo();
+          sync(ctx);
+        }
         add_step();
         if (acc > 0.5 * skin) {
           list_rebuild(*m.nl, x, n);
           acc = 0;
         }
       }
-      eam_gradient(e, *m.nl, d_types, d_frozen, g, FLYG_FP64);
-      vec_dots(ctx, N, g, q, g, g, hp, hfl);
-      sync_checked(ctx);
+      auto look = [&] {
+        eam_gradient(e, *m.nl, d_types, d_frozen, g, FLYG_FP64);
+        vec_dots(ctx, N, g, q, g, g, hp, hfl);
+        sync_checked(ctx);
+      };
+      look();
+      if (m.core->stalled()) {
+        redo();
+        look();
+      }
       if (!known) add_step();
       double proj = host_sum(hp, 0, N);
       mag_g = host_sum(hp, 1, N);
@@ -228,8 +269,10 @@ namespace flyg {
   // Rotor::eff_gradient on the list nl (ready at the positions; moved by +-delta_r and back, never rebuilt).
   // Axis in/out in d.ax, effective gradient to d.eff.  Returns the curvature; |g_eff|^2 and g_eff.step (step
   // null: only the first) are left in ctx.hpart with the error flags, for the caller to read after a sync.
+  // `by` (if given): the list was just moved by a step of this core; should that step have given up, *lost is set
+  // and neither the list nor the axis has changed.
   double eff_gradient(flyg_dimer_s& d, flyg_list_s& nl, flyg_eam_s& e, uint32_t const* t, uint8_t const* f, long n,
-                      int count_frozen, double const* step) {
+                      int count_frozen, double const* step, DevLBFGS* by = nullptr, bool* lost = nullptr) {
       flyg_ctx_s& ctx = *d.ctx;
       flyg_rotor_options const& o = d.ropt;
       long N = 3 * n;
@@ -250,9 +293,10 @@ namespace flyg {
       bool const none_frozen = count_frozen == 0;
       double const mean_k = -(1.0 / static_cast<double>(n));
 
+      long const grads = d.grads;
       d.rcore->clear();
       gradient_at(d, nl, e, t, f, g0);
-      rot_offset(ctx, N, dr, ax, dprev, lm);
+      rot_offset(ctx, N, dr, ax, dprev, lm, by ? by->stalled_word() : nullptr);
       gradient_at(d, nl, e, t, f, g1);
       rot_diff(ctx, N, g1, g0, ax, dg, out);
 
@@ -264,10 +308,22 @@ namespace flyg {
         rot_torque(ctx, N, none_frozen, in, dg, ax, dgp, out);
         if (none_frozen) vec_demean(ctx, N, mean_k, out, dgp, nullptr, nullptr, nullptr);
         double const* thax;
-        double* theta = d.rcore->newton_step(ax, dgp, N, ax, &thax);
-        rot_orth(ctx, N, thax, ax, theta, out);
-        rot_unit(ctx, N, out, theta, dg, ax, hp);
-        sync(ctx);
+        double* theta = d.rcore->newton_step(ax, dgp, N, ax, &thax, true);
+        auto unit = [&] {
+          rot_orth(ctx, N, thax, ax, theta, out);
+          rot_unit(ctx, N, out, theta, dg, ax, hp);
+          sync(ctx);
+        };
+        unit();
+        if (i == 0 && by && by->stalled()) {
+          d.grads = grads;
+          *lost = true;
+          return 0;
+        }
+        if (d.rcore->stalled()) {
+          theta = d.rcore->again(ax, &thax);
+          unit();
+        }
         double b_1 = host_sum(hp, 0, N) / dr;
         double c_x0 = host_sum(hp, 1, N) / dr;
         double theta_1 = -0.5 * std::atan(b_1 / std::abs(c_x0));
@@ -313,7 +369,7 @@ namespace flyg {
     require(nl.n == n, "rotor size mismatch");
     require(nl.rc >= e.tab.rc + 2 * d.ropt.delta_r, "the list's cut-off is below the rotor's r_cut()");
     long N = 3 * n;
-    if (!d.rcore) d.rcore = std::make_unique<DevLBFGS>(&ctx, d.ropt.n);
+    if (!d.rcore) d.rcore = std::make_unique<DevLBFGS>(&ctx, d.ropt.n, true);
     for (DVec* v : {&d.ax, &d.eff, &d.g0, &d.g1, &d.g1p, &d.dg, &d.delta_g, &d.axisp, &d.delta_prev}) v->p(N);
     copy(ctx, d.ax.get(), d_axis, N);
     double curv = eff_gradient(d, nl, e, t, f, n, count_frozen, nullptr);
@@ -334,7 +390,7 @@ namespace flyg {
     double rc = rot_rc + skin;
     if (!d.nl || d.nl->rc != rc) d.nl = make_list(&ctx, d.basis, d.periodic, rc);
     if (!d.core) d.core = std::make_unique<DevLBFGS>(&ctx, o.n);
-    if (!d.rcore) d.rcore = std::make_unique<DevLBFGS>(&ctx, d.ropt.n);
+    if (!d.rcore) d.rcore = std::make_unique<DevLBFGS>(&ctx, d.ropt.n, true);
     d.core->clear();
     for (DVec* v : {&d.x, &d.ax, &d.eff, &d.g0, &d.g1, &d.g1p, &d.dg, &d.delta_g, &d.axisp, &d.delta_prev, &d.tmp})
       v->p(N);
@@ -395,8 +451,13 @@ namespace flyg {
         }
       }
       double const* qq;
-      double* q = d.core->newton_step(x, d.eff.get(), N, nullptr, &qq);
-      vec_step(ctx, N, trust, qq, q, x, list_move(*d.nl), &hstep);
+      double* q = d.core->newton_step(x, d.eff.get(), N, nullptr, &qq, true);
+      auto step = [&] { vec_step(ctx, N, trust, qq, q, x, list_move(*d.nl), d.core->stalled_word(), &hstep); };
+      step();
+      auto redo = [&] {   // the step gave up: x and the list are where they were
+        q = d.core->again(nullptr, &qq);
+        step();
+      };
       // As in the minimiser: the step's length is read on its own only when it could use up the skin.
       bool known = false;
       auto add_step = [&] {
@@ -407,6 +468,10 @@ namespace flyg {
       };
       if (!(acc + 1.001 * trust < 0.5 * skin)) {
         sync(ctx);
+        if (d.core->stalled()) {
+          redo();
+          sync(ctx);
+        }
         add_step();
         if (acc > 0.5 * skin) {
           list_rebuild(*d.nl, x, n);
@@ -414,7 +479,12 @@ namespace flyg {
           ++rebuilds;
         }
       }
-      curv = eff_gradient(d, *d.nl, e, t, f, n, count_frozen, q);
+      bool lost = false;
+      curv = eff_gradient(d, *d.nl, e, t, f, n, count_frozen, q, d.core.get(), &lost);
+      if (lost) {
+        redo();
+        curv = eff_gradient(d, *d.nl, e, t, f, n, count_frozen, q);
+      }
       convex_count = curv > 0 ? convex_count + 1 : 0;
       sync_checked(ctx);
       if (!known) add_step();

@@ -20,15 +20,29 @@ namespace flyg {
   // StepLBFGS (lbfgs_core.hpp:37-119, lbfgs_core.cpp:29-87) with history on the device.
   class DevLBFGS {
   public:
-    DevLBFGS(flyg_ctx_s* ctx, int m);
-    void clear() { m_k = 0; }
+    DevLBFGS(flyg_ctx_s* ctx, int m, bool rotor = false);
+    void clear() {
+      m_k = 0;
+      *m_hstalled = 0;
+    }
     // Returns r ~ H^-1 g (device, length N); x and g are device vectors of length N.  `sums` (if given):
     // device partial sums of r.w (w null: r.r), valid until the next call.
-    double* newton_step(double const* x, double const* g, long N, double const* w = nullptr,
-                        double const** sums = nullptr);
+    // may_wait: the caller synchronises before it uses r for anything it cannot undo, then asks stalled(); if
+    // so the one-launch step gave up waiting, r and the sums are not valid, and again() makes them.  Kernels
+    // launched in between can look at stalled_word().
+    double* newton_step(double const* x, double const* g, long N, double const* w, double const** sums, bool may_wait);
+    bool stalled();
+    double* again(double const* w, double const** sums);
+    unsigned const* stalled_word() const { return &m_sc.get()->stalled; }
 
   private:
+    int pair(int k, int i) const {   // place of pair i (0 oldest) before call k + 1
+      return (i + (k <= m_m ? 0 : k - m_m)) % m_m;
+    }
+    double* stages(int k, double const* w, double const** sums);
+
     flyg_ctx_s* m_ctx;
+    unsigned* m_hstalled;   // pinned, of the context
     int m_m;
     int m_k = 0;
     long m_N = -1;
@@ -39,6 +53,7 @@ namespace flyg {
     DBuf<unsigned long long> m_slots;   // of the one-launch step (lb_newton), two sets
     long m_slots_n = -1;                // they are in order for vectors of this length
     int m_slots_used = 0;               // the set of the next call
+    unsigned m_rest = 0;                // steps to go by stage kernels after one gave up
   };
 
 }  // namespace flyg

@@ -98,10 +98,11 @@ namespace flyg {
         if (k == c) acc[k] += v;
     }
 
-    __global__ __launch_bounds__(VT) void k_lb_first(long n, double const* __restrict__ x, double const* __restrict__ g,
-                                                     double* __restrict__ px, double* __restrict__ pg,
-                                                     double* __restrict__ r, double const* __restrict__ w,
-                                                     double* __restrict__ out) {
+    __global__ __launch_bounds__(VT) void k_lb_first(long n, LBScalars* __restrict__ lb, double const* __restrict__ x,
+                                                     double const* __restrict__ g, double* __restrict__ px,
+                                                     double* __restrict__ pg, double* __restrict__ r,
+                                                     double const* __restrict__ w, double* __restrict__ out) {
+      if (blockIdx.x == 0 && threadIdx.x == 0) lb->stalled = 0;
       double acc[1] = {0};
       vec_loop(
           n, [&](long i) { return V3{x[i], g[i], w ? w[i] : g[i]}; },
@@ -130,6 +131,21 @@ namespace flyg {
             acc[0] += si * yi;
             acc[1] += yi * yi;
             acc[2] += si * v.b;
+          });
+      leave(acc, out);
+    }
+
+    __global__ __launch_bounds__(VT) void k_lb_again(long n, LBScalars* __restrict__ lb, double const* __restrict__ s,
+                                                     double const* __restrict__ y, double const* __restrict__ pg,
+                                                     double* __restrict__ out) {
+      if (blockIdx.x == 0 && threadIdx.x == 0) lb->stalled = 0;
+      double acc[3] = {0, 0, 0};
+      vec_loop(
+          n, [&](long i) { return V3{s[i], y[i], pg[i]}; },
+          [&](long, V3 const& v) {
+            acc[0] += v.a * v.b;
+            acc[1] += v.b * v.b;
+            acc[2] += v.a * v.c;
           });
       leave(acc, out);
     }
@@ -227,8 +243,11 @@ namespace flyg {
     // wavefront of every workgroup reads all of them until none is empty.  An empty slot holds a
     // signalling NaN, which no sum can be.  Sums and expressions are those of the stage kernels: the same bits.
     // Every workgroup must be resident at once.  At most NEWTON_BLOCKS = 64 of 256 threads are launched, on a chip that
-    // holds 2048, and whatever else runs on it ends by itself; should one still wait for two seconds it
-    // raises ERR_STALL and all of them run to their end.
+    // holds 2048; but long kernels of other streams (the search server's) can leave no room for some of them until
+    // they end.  So the wait is bounded, by polls and not by the clock, which runs on while a queue is switched
+    // out: a workgroup that polls in vain stops waiting, the step is marked as given up, and every workgroup
+    // runs to its end, publishing its sums on the way so that nobody waits for it.  What the step writes besides r
+    // and the sums (px, pg, the newest pair) does not depend on them, so the caller finishes it by stage kernels.
     constexpr unsigned long long EMPTY_SLOT = 0x7ff4deadbeef0badull;
 
     __global__ void k_empty_slots(unsigned long long* slots, long count) {
@@ -260,15 +279,15 @@ namespace flyg {
                            static_cast<unsigned long long>(__double_as_longlong(s)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
       if (w == 0) {
-        long long const t0 = wall_clock64();
+        unsigned polls = 0;
 #pragma unroll
         for (int k = 0; k < K; ++k) {
           unsigned long long const* slot = &A.slots[(id + k) * NEWTON_BLOCKS + (lane < nb ? lane : 0)];
           unsigned long long v;
-          while (true) {   // ends when every slot is filled, when this workgroup has given up, or after two seconds
+          while (true) {   // ends when every slot is filled or after `polls` rounds
             v = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (__all(v != EMPTY_SLOT) || L.dead) break;
-            if (wall_clock64() - t0 > 200000000ll) {   // 100 MHz
+            if (++polls > A.polls) {
               L.dead = 1;
               break;
             }
@@ -285,13 +304,13 @@ namespace flyg {
         for (int k = 0; k < K; ++k) tot[k] += L.sh[k][b];
     }
 
-    __global__ __launch_bounds__(VT) void k_lb_newton(NewtonArgs A, unsigned* __restrict__ err) {
+    __global__ __launch_bounds__(VT) void k_lb_newton(NewtonArgs A) {
       __shared__ NewtonLds L;
       long const step = static_cast<long>(gridDim.x) * VT;
       long const i0 = blockIdx.x * static_cast<long>(VT) + threadIdx.x;
       int const bound = A.bound;
       for (int q = threadIdx.x; q < NEWTON_SUMS; q += VT) A.spare[q * NEWTON_BLOCKS + blockIdx.x] = EMPTY_SLOT;
-      if (threadIdx.x == 0) L.dead = 0;
+      if (threadIdx.x == 0) L.dead = A.polls == 0;   // told not to wait
       if (threadIdx.x < bound - 1) L.rho[threadIdx.x] = A.lb->rho[A.j[threadIdx.x]];
       auto load = [&](double const* p, double (&v)[4]) {
 #pragma unroll
@@ -399,14 +418,20 @@ namespace flyg {
       for (int u = 0; u < 4; ++u)
         if (i0 + u * step < A.n) A.r[i0 + u * step] = q[u];
       leave(acc, A.out);
-      if (threadIdx.x == 0 && L.dead) atomicOr(err, static_cast<unsigned>(ERR_STALL));
+      if (threadIdx.x == 0 && L.dead) {
+        __hip_atomic_store(&A.lb->stalled, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(A.hstalled, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      }
     }
 
     __global__ __launch_bounds__(VT) void k_step(long n, double trust, double const* __restrict__ in, double* __restrict__ q,
-                                                 double* __restrict__ x, ListMove lm, double* __restrict__ hsum) {
+                                                 double* __restrict__ x, ListMove lm, unsigned const* __restrict__ stalled,
+                                                 double* __restrict__ hsum) {
       __shared__ double sh[VMAXB];
       double t[1];
+      unsigned const off = *stalled;   // its load is under way with the sums'
       collect(in, sh, t);
+      if (off) return;
       if (blockIdx.x == 0 && threadIdx.x == 0) *hsum = t[0];
       double const c = fmin(1.0, trust / sqrt(t[0]));
       vec_loop(
@@ -448,13 +473,15 @@ namespace flyg {
     }
 
     __global__ __launch_bounds__(VT) void k_rot_offset(long n, double dr, double const* __restrict__ ax,
-                                                       double* __restrict__ delta, ListMove lm) {
+                                                       double* __restrict__ delta, ListMove lm,
+                                                       unsigned const* __restrict__ stalled) {
+      bool const move = !stalled || !*stalled;
       vec_loop(
           n, [&](long i) { return M1{ax[i], to_move(lm, i)}; },
           [&](long i, M1 const& v) {
             double const o = -dr * v.a;
             delta[i] = o;
-            move_one(lm, v.m, o);
+            if (move) move_one(lm, v.m, o);
           });
     }
 
@@ -665,9 +692,12 @@ namespace flyg {
     return ListMove{reinterpret_cast<double*>(nl.pos.get()), reinterpret_cast<double*>(nl.gpos.get()), nl.rank.get()};
   }
 
-  void lb_first(flyg_ctx_s& ctx, long n, double const* x, double const* g, double* px, double* pg, double* r,
+  void lb_first(flyg_ctx_s& ctx, long n, LBScalars* lb, double const* x, double const* g, double* px, double* pg, double* r,
                 double const* w, double* out) {
-    FLYG_VEC_LAUNCH(k_lb_first, x, g, px, pg, r, w, out);
+    FLYG_VEC_LAUNCH(k_lb_first, lb, x, g, px, pg, r, w, out);
+  }
+  void lb_again(flyg_ctx_s& ctx, long n, LBScalars* lb, double const* s, double const* y, double const* pg, double* out) {
+    FLYG_VEC_LAUNCH(k_lb_again, lb, s, y, pg, out);
   }
   void lb_hist(flyg_ctx_s& ctx, long n, double const* x, double const* g, double* px, double* pg, double* s, double* y,
                double* out) {
@@ -694,15 +724,16 @@ namespace flyg {
     FLYG_VEC_LAUNCH(k_lb_loop2, j, lb, in, r, s, w, out);
   }
   void lb_newton(flyg_ctx_s& ctx, NewtonArgs const& a) {
-    k_lb_newton<<<vec_blocks(a.n), VT, 0, ctx.stream>>>(a, ctx.dflags.get());
+    k_lb_newton<<<vec_blocks(a.n), VT, 0, ctx.stream>>>(a);
     HIPCHK(hipGetLastError());
   }
   void lb_empty_slots(flyg_ctx_s& ctx, unsigned long long* slots, long count) {
     k_empty_slots<<<static_cast<unsigned>((count + VT - 1) / VT), VT, 0, ctx.stream>>>(slots, count);
     HIPCHK(hipGetLastError());
   }
-  void vec_step(flyg_ctx_s& ctx, long n, double trust, double const* in, double* q, double* x, ListMove lm, double* hsum) {
-    FLYG_VEC_LAUNCH(k_step, trust, in, q, x, lm, hsum);
+  void vec_step(flyg_ctx_s& ctx, long n, double trust, double const* in, double* q, double* x, ListMove lm,
+                unsigned const* stalled, double* hsum) {
+    FLYG_VEC_LAUNCH(k_step, trust, in, q, x, lm, stalled, hsum);
   }
   void vec_dots(flyg_ctx_s& ctx, long n, double const* a, double const* b, double const* c, double const* d, double* out,
                 unsigned* hflag) {
@@ -711,8 +742,8 @@ namespace flyg {
   void vec_diff(flyg_ctx_s& ctx, long n, double const* a, double const* b, double* o, double* out) {
     FLYG_VEC_LAUNCH(k_diff, a, b, o, out);
   }
-  void rot_offset(flyg_ctx_s& ctx, long n, double dr, double const* ax, double* delta, ListMove lm) {
-    FLYG_VEC_LAUNCH(k_rot_offset, dr, ax, delta, lm);
+  void rot_offset(flyg_ctx_s& ctx, long n, double dr, double const* ax, double* delta, ListMove lm, unsigned const* stalled) {
+    FLYG_VEC_LAUNCH(k_rot_offset, dr, ax, delta, lm, stalled);
   }
   void rot_diff(flyg_ctx_s& ctx, long n, double const* g1, double const* g0, double const* ax, double* dg, double* out) {
     FLYG_VEC_LAUNCH(k_rot_diff, g1, g0, ax, dg, out);

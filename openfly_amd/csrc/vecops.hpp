@@ -5,7 +5,7 @@
 // Reductions are deterministic: the grid depends on the vector length only (vec_blocks), each block
 // leaves its partial sums in part[k * VMAXB + block], and whoever needs the value adds the partials in
 // block order: the next kernel of the chain (every block for itself, from LDS), or the host, from a buffer
-// in pinned memory that the kernel writes directly.  No block waits for another one.
+// in pinned memory that the kernel writes directly.  No block waits for another one, but in lb_newton.
 //
 // What bounds them: at 16k atoms (48k elements) latency, not bytes.  A launch whose last block collected
 // the partials with device-scope loads in sequence took 14-16 us there, most of it that loop and its two
@@ -29,6 +29,7 @@ namespace flyg {
     double rho[32];
     double alpha[32];
     double h0;
+    unsigned stalled;   // set by a step of lb_newton that gave up, cleared by lb_first and lb_again
   };
 
   // The live positions of a neighbour list, moved by -u beside the kernel's own work (List::update).
@@ -42,11 +43,13 @@ namespace flyg {
   // L-BFGS two-loop stages (lbfgs_core.cpp:29-87).  `in`: the partial sums of the stage before; `out` must
   // be another buffer.
   // First call: px = x, pg = r = g; out: r.w (w = null: r.r).
-  void lb_first(flyg_ctx_s& ctx, long n, double const* x, double const* g, double* px, double* pg, double* r,
+  void lb_first(flyg_ctx_s& ctx, long n, LBScalars* lb, double const* x, double const* g, double* px, double* pg, double* r,
                 double const* w, double* out);
   // s = x - px, y = g - pg, px = x, pg = g; out: s.y, y.y, s.g.
   void lb_hist(flyg_ctx_s& ctx, long n, double const* x, double const* g, double* px, double* pg, double* s, double* y,
                double* out);
+  // The sums of lb_hist once more, for a pair that is stored already.
+  void lb_again(flyg_ctx_s& ctx, long n, LBScalars* lb, double const* s, double const* y, double const* pg, double* out);
   // alpha_j from `in` (newest: rho_j and h0 too), qout = q - alpha_j y; out: s_next.qout.
   void lb_loop1(flyg_ctx_s& ctx, long n, bool newest, int j, LBScalars* lb, double const* in, double const* q,
                 double const* y, double const* s_next, double* qout, double* out);
@@ -59,8 +62,9 @@ namespace flyg {
 
   // The whole two-loop in one launch, for vectors of at most NEWTON_BLOCKS blocks.  Pairs in order, oldest first (the
   // newest is written); j: their places in lb.  slots: two sets of NEWTON_SLOTS words in turn, those of `slots`
-  // empty, `spare` emptied for the next call.  out: r.w (w = null: r.r).  A workgroup that waits in vain (seconds)
-  // sets ERR_STALL and leaves.
+  // empty, `spare` emptied for the next call.  out: r.w (w = null: r.r).  A workgroup that polls `polls` times in vain
+  // gives up: the step sets lb->stalled and *hstalled (pinned) and leaves no r and no sums.  Pair, px and pg
+  // are in order all the same, so lb_again and the stage kernels can finish the step.
   constexpr int NEWTON_BLOCKS = 64;
   constexpr int NEWTON_SUMS = 2 * 32 + 3;
   constexpr int NEWTON_SLOTS = NEWTON_SUMS * NEWTON_BLOCKS;
@@ -76,6 +80,8 @@ namespace flyg {
     LBScalars* lb;
     unsigned long long* slots;
     unsigned long long* spare;
+    unsigned polls;
+    unsigned* hstalled;
     double* out;
     double* s[32];
     double* y[32];
@@ -84,8 +90,10 @@ namespace flyg {
   void lb_newton(flyg_ctx_s& ctx, NewtonArgs const& a);
   void lb_empty_slots(flyg_ctx_s& ctx, unsigned long long* slots, long count);
 
-  // Trust-region step: q *= min(1, trust / sqrt(in)), x -= q, the list follows; the sum itself goes to *hsum.
-  void vec_step(flyg_ctx_s& ctx, long n, double trust, double const* in, double* q, double* x, ListMove lm, double* hsum);
+  // Trust-region step: q *= min(1, trust / sqrt(in)), x -= q, the list follows; the sum itself goes to *hsum.  Nothing
+  // happens where *stalled is set.
+  void vec_step(flyg_ctx_s& ctx, long n, double trust, double const* in, double* q, double* x, ListMove lm,
+                unsigned const* stalled, double* hsum);
   // out: a.b and c.d (c null: one sum); the device error flags go to *hflag (null: not copied).
   void vec_dots(flyg_ctx_s& ctx, long n, double const* a, double const* b, double const* c, double const* d, double* out,
                 unsigned* hflag);
@@ -93,8 +101,8 @@ namespace flyg {
   void vec_diff(flyg_ctx_s& ctx, long n, double const* a, double const* b, double* o, double* out);
 
   // Rotor stages (rotor.cpp:49-164).
-  // delta = -dr ax, the list follows.
-  void rot_offset(flyg_ctx_s& ctx, long n, double dr, double const* ax, double* delta, ListMove lm);
+  // delta = -dr ax, the list follows, unless *stalled is set (stalled null: always).
+  void rot_offset(flyg_ctx_s& ctx, long n, double dr, double const* ax, double* delta, ListMove lm, unsigned const* stalled);
   // dg = g1 - g0; out: dg.ax.
   void rot_diff(flyg_ctx_s& ctx, long n, double const* g1, double const* g0, double const* ax, double* dg, double* out);
   // o = dg - in ax; out: the component sums of o when `sums`.

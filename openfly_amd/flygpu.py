@@ -132,6 +132,7 @@ _SIGS = {
     "flyg_ctx_destroy": [_vp],
     "flyg_ctx_last_error": [_vp],
     "flyg_ctx_synchronize": [_vp],
+    "flyg_ctx_set_step_polls": [_vp, C.c_uint],
     "flyg_ctx_stream": [_vp],
     "flyg_ctx_device_info": [_vp, C.c_char_p, C.c_size_t, C.POINTER(C.c_int)],
     "flyg_eam_load": [_vp, C.c_char_p, C.POINTER(_vp)],
@@ -338,6 +339,10 @@ class Context:
 
     def synchronize(self):
         self.check(lib().flyg_ctx_synchronize(self.h))
+
+    def set_step_polls(self, polls):
+        """Polls before a one-launch L-BFGS step gives up and is finished by stage launches (same bits)."""
+        self.check(lib().flyg_ctx_set_step_polls(self.h, polls))
 
     @property
     def stream(self):

@@ -5,9 +5,11 @@ same seeded start give barriers within 1e-4 eV of the oracle's.
 """
 import numpy as np
 import pytest
+import torch
 
 import openfly_amd as fa
 from openfly_amd import systems
+from openfly_amd.flygpu import DEVICE
 from oracle import pyoracle as po
 from tests import helpers as H
 
@@ -66,6 +68,62 @@ def test_steplbfgs_sizes(ctx, N):
         qg, qo = g_s.newton_step(x, g), o_s.newton_step(x, g)
         assert np.max(np.abs(qg - qo)) <= max(1e-12, N * 2.2e-16) * np.max(np.abs(qo)), it
         x = x - 0.5 * qo
+
+
+@pytest.fixture(params=[0, 1, 4])
+def impatient(request):
+    # Steps of the one-launch form give up before the first look, or after so many: some of them, any of them.
+    c = fa.Context(0)
+    c.set_step_polls(request.param)
+    return c
+
+
+@pytest.mark.parametrize("N,m", [(1, 3), (1025, 5), (9000, 32), (65536, 32)])
+def test_step_given_up_is_the_same_step(ctx, impatient, N, m):
+    # A step whose workgroups did not get the others' sums in time is finished by stage launches: the same bits,
+    # for histories of one pair up to m and beyond (m = 32: every place of the pair tables).  Device callers too.
+    rng = np.random.default_rng(N)
+    d = rng.uniform(1.0, 3.0, N)
+    a, b, c = fa.StepLBFGS(ctx, m), fa.StepLBFGS(impatient, m), fa.StepLBFGS(impatient, m)
+    x = rng.normal(size=N)
+    out = torch.zeros(N, dtype=torch.float64, device="cuda")
+    for it in range(m + 4):
+        g = d * x + 0.1 * np.sin(x)
+        q = a.newton_step(x, g)
+        assert np.all(np.isfinite(q)), it
+        assert np.array_equal(q, b.newton_step(x, g)), it
+        dx, dg = torch.from_numpy(x).cuda(), torch.from_numpy(g).cuda()
+        torch.cuda.synchronize()
+        impatient.check(fa.lib().flyg_steplbfgs_newton_step(c.h, dx.data_ptr(), dg.data_ptr(), N, out.data_ptr(), DEVICE))
+        impatient.synchronize()
+        assert np.array_equal(q, out.cpu().numpy()), it
+        x = x - 0.5 * q
+
+
+@pytest.mark.parametrize("frozen_frac", [0.0, 0.1])
+def test_relaxation_and_search_with_given_up_steps(ctx, impatient, frozen_frac):
+    # The minimiser, the dimer and the rotor undo nothing and lose nothing when a step gives up: every result has the
+    # bits, and every count the value, of a run whose steps all waited.
+    pos, basis = small_vacancy_system(cells=8, seed=4, a=2.855324, noise=0.05)
+    n = len(pos)
+    rng = np.random.default_rng(9)
+    t = np.zeros(n, np.uint32)
+    f = (rng.random(n) < frozen_frac).astype(np.uint8)
+    kick, axis = rng.normal(size=(2, n, 3)) * (f == 0)[:, None]
+    got = []
+    for c in (ctx, impatient):
+        pot, box = fa.EAM(c, H.WEN), fa.Box(basis)
+        mn = fa.LBFGS(c, box, f2norm=1e-5).minimise(pos, t, f, pot)
+        r = fa.Dimer(c, box, dimer=dict(max_steps=40, convex_max=100)).find_sp(mn[0] + 0.1 * kick, axis, t, f, mn[0], pot)
+        rot = fa.Rotor(c)
+        nl = fa.List(c, box, rot.r_cut(pot))
+        nl.rebuild(pos)
+        C, ax, eff = rot.eff_gradient(axis / np.linalg.norm(axis), t, f, pot, nl)
+        got.append((mn[0], mn[1], mn[2:], r["pos"], r["axis"], [r[k] for k in ("exit", "steps", "grads", "rebuilds", "curv")],
+                    C, ax, eff, nl.positions()))
+    for p, q in zip(*got):
+        assert np.array_equal(p, q)
+    assert got[0][5][1] > 5 and got[0][2][1] > 5
 
 
 def test_minimise_matches_oracle(ctx, wen):
