@@ -126,6 +126,9 @@ int flyg_list_update(flyg_list nl, const double* delta, int64_t n, int where);
 int flyg_list_size(flyg_list nl, int64_t* n);
 /* Number of ghost images made by the last rebuild (List::m_num_plus_ghosts - size(), list.hpp:178). */
 int flyg_list_num_ghosts(flyg_list nl, int64_t* n_ghosts);
+/* How the last rebuild laid the list out for the pair kernels (no reference counterpart): the cells of a tile along
+ * each axis and the entries of the fullest tile, or 0 0 0 and 0 for plain rows.  Results do not depend on it. */
+int flyg_list_form(flyg_list nl, int shape[3], int* fullest);
 /* Pairs with r < r_cut (List::for_neighbours, list.hpp:138-154): count, then export as CSR rows with
  * the real neighbour index, the image shift code (s0+1)+3(s1+1)+9(s2+1) and dr = r_n - r_i. */
 int flyg_list_count(flyg_list nl, double r_cut, int64_t* n_pairs);

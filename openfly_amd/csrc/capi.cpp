@@ -268,6 +268,14 @@ int flyg_list_size(flyg_list nl, int64_t* n) {
   return guard(nl->ctx, [&] { *n = nl->n; });
 }
 
+int flyg_list_form(flyg_list nl, int shape[3], int* fullest) {
+  return guard(nl->ctx, [&] {
+    require(nl->built, "List used before rebuild");
+    for (int k = 0; k < 3; ++k) shape[k] = nl->tiled ? nl->tile.d[k] : 0;
+    if (fullest) *fullest = nl->tile_most;
+  });
+}
+
 int flyg_list_num_ghosts(flyg_list nl, int64_t* g) {
   return guard(nl->ctx, [&] { *g = nl->nghost; });
 }

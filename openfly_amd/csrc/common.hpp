@@ -341,6 +341,7 @@ namespace flyg {
     }
   };
   constexpr int TILE_MOST = 1900;   // entries a tile may stage: with species and tables below 64 KB
+  constexpr int TILE_KINDS = 3;     // tile shapes to choose from
 
   // ----------------------------------------------------------------------------------------------
   // Wavefront helpers (64 lanes on CDNA).

@@ -126,15 +126,19 @@ struct flyg_list_s {
   // Lists that are not tiled keep packed (shift, slot) entries there instead, nbr's in the slot order.
   flyg::TileGrid tile{};
   bool tiled = false;            // rows and sslot belong to this build
-  int tile_level = 0;            // tile shapes found too full for LDS with this atom count are skipped
   int tile_most = 0;             // entries staged by the fullest tile
+  // Of the last build, for every tile shape: entries of the fullest tile, and tiles that hold atoms.  Valid for the
+  // next one while the atom count and the grid stay the same (tile_seen).
+  unsigned tile_full[flyg::TILE_KINDS] = {}, tile_used[flyg::TILE_KINDS] = {};
+  bool tile_seen = false;
+  int tile_shape[3] = {};        // the grid they belong to
   int rowK = 0;
   flyg::DBuf<unsigned> sslot;
   flyg::DBuf<unsigned> rows;
   flyg::DBuf<int> gcnt;          // entries per slot
   flyg::DBuf<int> scan_tmp;
   flyg::DBuf<double> stage;      // host staging of xyz vectors
-  flyg::DBuf<unsigned> lstate;   // device build counters: two sets, used in turn
+  flyg::DBuf<unsigned> lstate;   // device build counters: two sets of LIST_STATE words, used in turn
   int parity = 0;                // the set of the next build
   // ccount and that set are zero for a grid of so many cells + 1 (the search server gives one list object
   // system after system, each with its own box and grid).
@@ -161,7 +165,8 @@ namespace flyg {
   void list_rebuild(flyg_list_s& nl, double const* d_xyz, long n);
   void list_update(flyg_list_s& nl, double const* d_delta, long n);
   // Exclusive scan of src into dst (they may be the same; both hold scan_room(n) values, whatever lies past the
-  // n-th); clear_state: src and the four words there are zeroed.
+  // n-th); clear_state: src and the LIST_STATE words there are zeroed.
+  constexpr int LIST_STATE = 16;
   constexpr long scan_room(long n) { return (n + 3) & ~3l; }
   void exclusive_scan(flyg_ctx_s& ctx, int* src, int* dst, int n, flyg::DBuf<int>& tmp, unsigned* clear_state = nullptr);
 

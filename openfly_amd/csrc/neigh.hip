@@ -168,8 +168,16 @@ namespace flyg {
     }
 
     // ---- single-sync rebuild path ----------------------------------------------------------------
-    // lstate[0] ghosts generated, [1] longest row, [3] overflow bits.
+    // lstate[0] ghosts generated, [1] longest row, [3] overflow bits, [4 + l] entries of the fullest tile of shape l,
+    // [8 + l] tiles of shape l that hold atoms.
     enum : unsigned { OV_GHOST = 1u };
+
+    // The tile shapes a build could take; workgroups [first[l], first[l + 1]) of k_rank_place look at shape l, those
+    // after them place the entries.
+    struct TileKinds {
+      TileGrid g[TILE_KINDS];
+      unsigned first[TILE_KINDS + 1];
+    };
 
     // Slots for g images per thread, one atomic per workgroup of ETPB threads (prefix sums of the lanes' counts and
     // of the wavefronts' totals): the counter is one address, and an atomic per wavefront on it took 100 us
@@ -346,18 +354,46 @@ namespace flyg {
                                  int const* __restrict__ cstart, long nc1, unsigned const* __restrict__ usid,
                                  double4* __restrict__ spos, unsigned* __restrict__ sid, int* __restrict__ rslot,
                                  int* __restrict__ order, int* __restrict__ rank_of, double4* __restrict__ gpos,
-                                 TileGrid tg, unsigned* __restrict__ most) {
-      long e = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
-      if (e < tg.ntiles) {   // entries that tile e stages
-        int const t = static_cast<int>(e);
-        int sum = 0;
-        for (int q = 0; q < 16; ++q) {
-          int cb, ce;
-          tg.line(true, t % tg.nt[0], t / tg.nt[0] % tg.nt[1], t / (tg.nt[0] * tg.nt[1]), q, cb, ce);
-          sum += cstart[ce] - cstart[cb];
+                                 TileKinds tk, unsigned* __restrict__ seen) {
+      if (blockIdx.x < tk.first[TILE_KINDS]) {   // four lanes a tile: the entries it stages, and whether it holds atoms
+        int l = 0;
+        while (blockIdx.x >= tk.first[l + 1]) ++l;
+        TileGrid const& tg = tk.g[l];
+        int const w = static_cast<int>((blockIdx.x - tk.first[l]) * blockDim.x + threadIdx.x), t = w >> 2;
+        int sum = 0, own = 0;
+        if (t < tg.ntiles) {
+          int const tx = t % tg.nt[0], ty = t / tg.nt[0] % tg.nt[1], tz = t / (tg.nt[0] * tg.nt[1]);
+#pragma unroll
+          for (int y = 0; y < 4; ++y) {   // the lines of one z
+            int hb, he, ob, oe;
+            tg.line(true, tx, ty, tz, 4 * (w & 3) + y, hb, he);
+            tg.line(false, tx, ty, tz, 4 * (w & 3) + y, ob, oe);
+            sum += cstart[he] - cstart[hb];
+            own += cstart[nc1 + oe] - cstart[nc1 + ob];
+          }
         }
-        atomicMax(most, static_cast<unsigned>(sum));
+        for (int o = 1; o < 4; o <<= 1) {
+          sum += __shfl_xor(sum, o, 64);
+          own += __shfl_xor(own, o, 64);
+        }
+        // One pair of atomics a workgroup: they all go to one line, several nanoseconds each.
+        __shared__ int s_sum, s_used;
+        if (threadIdx.x == 0) s_sum = s_used = 0;
+        __syncthreads();
+        for (int o = 32; o > 2; o >>= 1) sum = max(sum, __shfl_xor(sum, o, 64));
+        int const used = __popcll(__ballot(own > 0)) / 4;
+        if ((threadIdx.x & 63) == 0) {
+          atomicMax(&s_sum, sum);
+          atomicAdd(&s_used, used);
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+          atomicMax(&seen[l], static_cast<unsigned>(s_sum));
+          atomicAdd(&seen[4 + l], static_cast<unsigned>(s_used));
+        }
+        return;
       }
+      long e = (blockIdx.x - tk.first[TILE_KINDS]) * static_cast<long>(blockDim.x) + threadIdx.x;
       if (e >= live_entries(st, n, gcap)) return;
       int c = ecell[e];
       unsigned id = eid[e];
@@ -395,8 +431,7 @@ namespace flyg {
     //
     // Each row is written twice: by atom with atom indices (nbr), and by slot, in a tiled list with indices into the
     // tile's stage (the candidate's place in the tile's halo: the lines' entries one after the other), otherwise with
-    // slots.  hst (pinned): [0] ghosts,
-    // [1] set when a row overflowed, [2] entries of the fullest tile, [3] overflow bits.
+    // slots.  hst (pinned): the build counters, but [1] set when a row overflowed.
     constexpr long BUILD_WIDE = 24000;
 
     template <int A, bool TILED>
@@ -408,11 +443,7 @@ namespace flyg {
                                                         TileGrid tg, unsigned* __restrict__ sslot, long live_cap,
                                                         unsigned* __restrict__ rows, int rowK, int* __restrict__ gcnt,
                                                         unsigned* __restrict__ hst) {
-      if (blockIdx.x == 0 && threadIdx.x == 0) {
-        hst[0] = st[0];
-        hst[2] = st[2];
-        hst[3] = st[3];
-      }
+      if (blockIdx.x == 0 && threadIdx.x < LIST_STATE && threadIdx.x != 1) hst[threadIdx.x] = st[threadIdx.x];
       if constexpr (TILED) {
         long const live = live_entries(st, n, live_cap);
         for (long s = blockIdx.x * static_cast<long>(TPB) + threadIdx.x; s < live; s += static_cast<long>(gridDim.x) * TPB) {
@@ -586,14 +617,14 @@ namespace flyg {
     constexpr int SCAN_B = 1024;
 
     // First level of an exclusive scan of src into dst (which may be src); clear: src is zeroed, and so are
-    // the four words at cst.
+    // the LIST_STATE words at cst.
     __global__ void k_scan_block(int* src, int* dst, int n, int* __restrict__ sums, bool clear, unsigned* cst) {
       __shared__ int wsum[SCAN_B / 64];
       int gi = blockIdx.x * SCAN_B + threadIdx.x;
       int v = gi < n ? src[gi] : 0;
       if (clear) {
         if (gi < n) src[gi] = 0;
-        if (gi < 4) cst[gi] = 0u;
+        if (gi < LIST_STATE) cst[gi] = 0u;
       }
       int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
       int inc = v;
@@ -644,7 +675,7 @@ namespace flyg {
 #pragma unroll
         for (int q = 0; q < SCAN_RUN; q += 4)
           if (q < per && b + q < n) *reinterpret_cast<int4*>(src + b + q) = make_int4(0, 0, 0, 0);
-        if (threadIdx.x < 4) cst[threadIdx.x] = 0u;
+        if (threadIdx.x < LIST_STATE) cst[threadIdx.x] = 0u;
       }
       int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
       int inc = v;
@@ -747,8 +778,7 @@ namespace flyg {
     // plain rows: 27.6k atoms (216 / 396 / 726 tiles) 86 / 67 / 53 / 53, 44k (343 / 637 / 1183) 96 / 75 / 78 / 81,
     // 93k (729 / 1377 / 2601) 122 / 134 / 134 / 153, 1.03M 500 / 550 / 640 / 750; below, the plain rows are faster
     // (16k: 40 us against 47).
-    constexpr int TILE_SHAPES[][3] = {{2, 2, 2}, {1, 2, 2}, {1, 1, 2}};
-    constexpr int TILE_KINDS = 3;
+    constexpr int TILE_SHAPES[TILE_KINDS][3] = {{2, 2, 2}, {1, 2, 2}, {1, 1, 2}};
     constexpr int TILE_LEAST = 600;
 
     TileGrid tile_grid(GridDesc const& g, int level) {
@@ -765,19 +795,22 @@ namespace flyg {
       return t;
     }
 
-    bool choose_tiles(flyg_list_s& nl, long n) {
+    // The tile shape for a build, or -1: plain rows.  seen: from what the build before counted, the tiles that hold atoms
+    // and the fullest one.  A first build takes the box to be filled evenly, and is done again if its own counts
+    // say otherwise (a particle in vacuum leaves most tiles empty and the chip idle: 16k atoms in eight times their volume took 74 us a
+    // gradient by tiles, 25 by rows).
+    int choose_tiles(flyg_list_s const& nl, long n, bool seen) {
       GridDesc const& g = nl.grid;
       double const inner = static_cast<double>(g.shape[0] - 2) * (g.shape[1] - 2) * (g.shape[2] - 2);
-      for (int level = nl.tile_level; level < TILE_KINDS; ++level) {
+      for (int level = 0; level < TILE_KINDS; ++level) {
         TileGrid const t = tile_grid(g, level);
-        double const staged = n / inner * (t.d[0] + 2) * (t.d[1] + 2) * (t.d[2] + 2);
-        if (staged > 0.9 * TILE_MOST || t.ntiles < TILE_LEAST) continue;
-        if (n < 16l * t.ntiles) return false;   // a gas: tiles of a few atoms
-        nl.tile = t;
-        nl.tile_level = level;
-        return true;
+        bool const full = seen ? nl.tile_full[level] > TILE_MOST
+                               : n / inner * (t.d[0] + 2) * (t.d[1] + 2) * (t.d[2] + 2) > 0.9 * TILE_MOST;
+        long const used = seen ? static_cast<long>(nl.tile_used[level]) : t.ntiles;
+        if (full || used < TILE_LEAST) continue;
+        return n < 16 * used ? -1 : level;   // a gas: tiles of a few atoms
       }
-      return false;
+      return -1;
     }
   }  // namespace
 
@@ -788,13 +821,14 @@ namespace flyg {
     require(n < MAX_ATOMS, "too many atoms for the packed neighbour format");
     flyg_ctx_s& ctx = *nl.ctx;
     hipStream_t st = ctx.stream;
-    if (!nl.hstate) HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&nl.hstate), 4 * sizeof(unsigned), hipHostMallocDefault));
+    if (!nl.hstate) HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&nl.hstate), LIST_STATE * sizeof(unsigned), hipHostMallocDefault));
     nl.built = false;
     if (n != nl.n) {
       nl.gcap = 0;
       nl.K = 0;
     }
-    if (n != nl.n || nl.clear_cells != nl.grid.ncells + 1) nl.tile_level = 0;
+    if (n != nl.n || !std::equal(nl.tile_shape, nl.tile_shape + 3, nl.grid.shape)) nl.tile_seen = false;
+    std::copy(nl.grid.shape, nl.grid.shape + 3, nl.tile_shape);
     nl.n = n;
     if (nl.gcap == 0) nl.gcap = std::max(4096l, n);
     if (nl.K == 0) {
@@ -807,7 +841,7 @@ namespace flyg {
     }
     int const nc = nl.grid.ncells;
     long const nc1 = nc + 1;
-    nl.lstate.reserve(8);
+    nl.lstate.reserve(2 * LIST_STATE);
     nl.ccount.reserve(scan_room(2 * nc1));
     nl.cstart.reserve(scan_room(2 * nc1));   // cell starts, then the first real slot of each cell (offset)
     nl.pos.reserve(n);
@@ -819,14 +853,16 @@ namespace flyg {
     nl.gcnt.reserve(n);
     if (nl.clear_cells != nc1) {   // a first build, another grid, or a build that ended in an error half way
       HIPCHK(hipMemsetAsync(nl.ccount.get(), 0, scan_room(2 * nc1) * sizeof(int), st));
-      HIPCHK(hipMemsetAsync(nl.lstate.get(), 0, 8 * sizeof(unsigned), st));
+      HIPCHK(hipMemsetAsync(nl.lstate.get(), 0, 2 * LIST_STATE * sizeof(unsigned), st));
     }
     nl.clear_cells = -1;
 
-    for (int attempt = 0; attempt < 3 + TILE_KINDS; ++attempt) {
+    TileKinds tk{};
+    for (int l = 0; l < TILE_KINDS; ++l) tk.g[l] = tile_grid(nl.grid, l);
+    for (int attempt = 0; attempt < 6; ++attempt) {
       // Two sets of state words in turn: the scan clears the other build's.
-      unsigned* dst = nl.lstate.get() + 4 * nl.parity;
-      unsigned* other = nl.lstate.get() + 4 * (1 - nl.parity);
+      unsigned* dst = nl.lstate.get() + LIST_STATE * nl.parity;
+      unsigned* other = nl.lstate.get() + LIST_STATE * (1 - nl.parity);
       nl.parity = 1 - nl.parity;
       long const cap = n + nl.gcap;
       nl.ent.reserve(cap);
@@ -837,8 +873,16 @@ namespace flyg {
       nl.sid.reserve(cap);
       nl.usid.reserve(cap);
       nl.nbr.reserve(static_cast<std::size_t>(n) * nl.K);
-      nl.tiled = choose_tiles(nl, n);
-      TileGrid const tg = nl.tiled ? nl.tile : TileGrid{};
+      int const level = choose_tiles(nl, n, nl.tile_seen);
+      nl.tiled = level >= 0;
+      // The shape in use is looked at in every build, the others (not those with more tiles than a quarter of the
+      // atoms) only while an even filling and what was seen disagree: three shapes take 5 us more at 54k atoms.
+      bool const all = n >= 16l * TILE_LEAST && (!nl.tile_seen || attempt > 0 || level != choose_tiles(nl, n, false));
+      for (int l = 0; l < TILE_KINDS; ++l) {
+        bool const look = l == level || (all && n >= 4l * tk.g[l].ntiles);
+        tk.first[l + 1] = tk.first[l] + (look ? nblk(4l * tk.g[l].ntiles, TPB) : 0);
+      }
+      TileGrid const tg = nl.tiled ? tk.g[level] : TileGrid{};
       nl.rowK = nl.tiled ? (nl.K + 31) / 32 * 32 : nl.K;
       if (nl.tiled) nl.sslot.reserve(cap);
       nl.rows.reserve(static_cast<std::size_t>(n) * nl.rowK / (nl.tiled ? 2 : 1));
@@ -855,9 +899,9 @@ namespace flyg {
       exclusive_scan(ctx, nl.ccount.get(), nl.cstart.get(), static_cast<int>(2 * nc1), nl.scan_tmp, other);
       k_scatter_ids<<<nblk(cap, TPB), TPB, 0, st>>>(nl.eid.get(), nl.ecell.get(), nl.earr.get(), n, nl.gcap, dst,
                                                     nl.cstart.get(), nl.usid.get());
-      k_rank_place<<<nblk(std::max<long>(cap, tg.ntiles), TPB), TPB, 0, st>>>(nl.ent.get(), nl.eid.get(), nl.ecell.get(), n, nl.gcap, dst,
-                                                   nl.cstart.get(), nc1, nl.usid.get(), nl.spos.get(), nl.sid.get(),
-                                                   nl.rslot.get(), nl.order.get(), nl.rank.get(), nl.gpos.get(), tg, dst + 2);
+      k_rank_place<<<tk.first[TILE_KINDS] + nblk(cap, TPB), TPB, 0, st>>>(
+          nl.ent.get(), nl.eid.get(), nl.ecell.get(), n, nl.gcap, dst, nl.cstart.get(), nc1, nl.usid.get(), nl.spos.get(),
+          nl.sid.get(), nl.rslot.get(), nl.order.get(), nl.rank.get(), nl.gpos.get(), tk, dst + 4);
       auto rows = [&](auto k, int A) {
         k<<<nblk(n, A * (TPB / 64)), TPB, 0, st>>>(nl.grid, nl.spos.get(), nl.sid.get(), nl.cstart.get(), nl.rslot.get(), n,
                                                    nl.nbr.get(), nl.ncnt.get(), nl.K, dst, nl.order.get(), nl.rank.get(),
@@ -878,16 +922,23 @@ namespace flyg {
       }
       nl.nghost = G;
       if (nl.hstate[1]) {   // a row overflowed: widen the rows and build again
-        HIPCHK(hipMemcpyAsync(nl.hstate, dst, 4 * sizeof(unsigned), hipMemcpyDeviceToHost, st));
+        HIPCHK(hipMemcpyAsync(nl.hstate, dst, LIST_STATE * sizeof(unsigned), hipMemcpyDeviceToHost, st));
         HIPCHK(hipStreamSynchronize(st));
         nl.K = (static_cast<int>(nl.hstate[1]) + 15) / 16 * 16 + 16;
         continue;
       }
-      nl.tile_most = static_cast<int>(nl.hstate[2]);
-      if (nl.tiled && nl.tile_most > TILE_MOST) {   // a tile too full for its stage: smaller tiles, or none
-        ++nl.tile_level;
-        continue;
-      }
+      bool const first = !nl.tile_seen;
+      for (int l = 0; l < TILE_KINDS; ++l)
+        if (all || l == level) {
+          nl.tile_full[l] = nl.hstate[4 + l];
+          nl.tile_used[l] = nl.hstate[8 + l];
+        }
+      nl.tile_seen = true;
+      // A tile too full for its stage, or a first build that took the wrong form: again, with what was seen.
+      if (nl.tiled && nl.tile_full[level] > TILE_MOST) continue;
+      if (first && choose_tiles(nl, n, true) != level) continue;
+      nl.tile = tg;
+      nl.tile_most = nl.tiled ? static_cast<int>(nl.tile_full[level]) : 0;
       static std::atomic<long> builds{0};
       nl.build_id = ++builds;
       nl.clear_cells = nc1;

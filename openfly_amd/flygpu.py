@@ -150,6 +150,7 @@ _SIGS = {
     "flyg_list_update": [_vp, _vp, C.c_int64, C.c_int],
     "flyg_list_size": [_vp, _i64],
     "flyg_list_num_ghosts": [_vp, _i64],
+    "flyg_list_form": [_vp, C.POINTER(C.c_int), C.POINTER(C.c_int)],
     "flyg_list_count": [_vp, C.c_double, _i64],
     "flyg_list_export": [_vp, C.c_double, _i64, _i32, _i32, _d],
     "flyg_list_positions": [_vp, _vp, C.c_int],
@@ -550,6 +551,12 @@ class List:
         g = C.c_int64()
         self.ctx.check(lib().flyg_list_num_ghosts(self.h, C.byref(g)))
         return g.value
+
+    def form(self):
+        """(cells of a tile along each axis, entries of the fullest tile), or None for plain rows."""
+        shape, most = (C.c_int * 3)(), C.c_int()
+        self.ctx.check(lib().flyg_list_form(self.h, shape, C.byref(most)))
+        return (tuple(shape), most.value) if shape[0] else None
 
     def pairs(self, r_cut=None):
         """(offsets, j, shift, dr) of every neighbour with r < r_cut (List::for_neighbours)."""

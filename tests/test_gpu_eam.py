@@ -438,7 +438,7 @@ def test_staged_atoms_follow_stage_calls_and_rebuilds(ctx, wen_orc):
 
 
 TILED = {   # cells: the tile shape a list with 0.6 A of skin takes
-    24: "1x1x2", 30: "1x2x2", 36: "2x2x2"}
+    24: (1, 1, 2), 30: (1, 2, 2), 36: (2, 2, 2)}
 
 
 @pytest.mark.parametrize("cells,tilt,slab,single", [(24, 0.0, False, False), (24, 0.1, True, True), (30, 0.07, False, False),
@@ -463,6 +463,7 @@ def test_tiled_passes_equal_plain_rows(ctx, cells, tilt, slab, single):
     nl = fa.List(ctx, fa.Box(basis, (1, 1, 0 if slab else 1)), 5.9)
     nl.rebuild(pos)
     nl.update(rng.uniform(-0.05, 0.05, pos.shape))
+    assert nl.form()[0] == TILED[cells]
     pot = fa.EAM(ctx, systems.potential_path(("Fe", "X")))
     for precision in (fa.FP64, fa.MIXED):
         pot.set_precision(precision)
@@ -481,19 +482,46 @@ def test_tiled_passes_equal_plain_rows(ctx, cells, tilt, slab, single):
     assert np.max(np.abs(hv[0] - hv[8])) <= 1e-13 * np.max(np.abs(hv[8]))
 
 
+def heap(count, spacing, at):
+    g = np.stack(np.meshgrid(*(np.arange(c) for c in count), indexing="ij"), axis=-1).reshape(-1, 3)
+    return at + spacing * g
+
+
 def test_crowded_cell_falls_back(ctx):
-    # 1300 more atoms around one cell of a 28k-atom system: no tile there fits the stage, the plain rows are used.
-    s = systems.fe_x_alloy(5, cells=24)
-    g = np.stack(np.meshgrid(np.arange(10), np.arange(10), np.arange(13), indexing="ij"), axis=-1).reshape(-1, 3)
-    pos = np.concatenate([s.pos, 10.0 + 1.85 * g])
-    types = np.concatenate([s.types, np.ones(len(g), np.uint32)])
-    frozen = np.zeros(len(pos), np.uint8)
+    # 2160 more atoms around one cell of a 54k-atom system: no tile there fits the stage, the plain rows are used; with
+    # 1300 of them the smallest tiles still fit.
+    s = systems.fe_x_alloy(5, cells=30)
     pot = fa.EAM(ctx, systems.potential_path(("Fe", "X")))
     nl = fa.List(ctx, fa.Box(s.basis), 5.9)
-    for p, t in ((s.pos, s.types), (pos, types), (s.pos, s.types)):   # tiles, too full for them, tiles again
+    none = np.zeros((0, 3))
+    for h, shape in ((none, (1, 2, 2)), (heap((12, 12, 15), 1.5, 12.6), None), (none, (1, 2, 2)),
+                     (heap((10, 10, 13), 1.85, 10.0), (1, 1, 2))):
+        p, t = np.concatenate([s.pos, h]), np.concatenate([s.types, np.ones(len(h), np.uint32)])
+        f = np.zeros(len(p), np.uint8)
         nl.rebuild(p)
-        f = frozen[:len(p)]
+        assert (nl.form() and nl.form()[0]) == shape
         pot.set_lanes(0)
         a = pot.gradient(t, f, nl).copy()
         pot.set_lanes(8)
         assert np.array_equal(a, pot.gradient(t, f, nl))
+
+
+def test_list_form_follows_the_atoms(ctx):
+    # The same atom count and box: atoms in a heap leave smaller tiles or none that fit their stage; when they are spread
+    # again, the rebuild after the next one goes back to the larger ones.  A particle in vacuum, most of whose tiles
+    # hold nothing, takes plain rows from its first build on.
+    s = systems.fe_x_alloy(5, cells=30)
+    rng = np.random.default_rng(0)
+    spread = rng.random((2160, 3)) @ s.basis
+    high, low = heap((12, 12, 15), 1.5, 12.6), np.concatenate([heap((10, 10, 13), 1.85, 10.0), spread[1300:]])
+    nl = fa.List(ctx, fa.Box(s.basis), 5.9)
+    for h, shape in ((spread, (1, 2, 2)), (low, (1, 1, 2)), (high, None), (high, None), (spread, None), (spread, (1, 2, 2)),
+                     (low, (1, 1, 2)), (low, (1, 1, 2))):
+        nl.rebuild(np.concatenate([s.pos, h]))
+        assert (nl.form() and nl.form()[0]) == shape
+    small = systems.fe_x_alloy(6, cells=20)
+    for periodic in ((1, 1, 1), (0, 0, 0)):
+        alone = fa.List(ctx, fa.Box(small.basis + np.diag([60.0] * 3), periodic), 5.9)
+        for _ in range(2):
+            alone.rebuild(small.pos + 30.0)
+            assert alone.form() is None
