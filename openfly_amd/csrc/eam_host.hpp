@@ -136,6 +136,9 @@ struct flyg_list_s {
   flyg::DBuf<unsigned> sslot;
   flyg::DBuf<unsigned> rows;
   flyg::DBuf<int> gcnt;          // entries per slot
+  // The plain rows in slot order of a tiled list, K entries of room each, made when a build's first call needs them.
+  flyg::DBuf<unsigned> srows;
+  long srows_build = -1;
   flyg::DBuf<int> scan_tmp;
   flyg::DBuf<double> stage;      // host staging of xyz vectors
   flyg::DBuf<unsigned> lstate;   // device build counters: two sets of LIST_STATE words, used in turn

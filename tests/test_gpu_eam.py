@@ -525,3 +525,28 @@ def test_list_form_follows_the_atoms(ctx):
         for _ in range(2):
             alone.rebuild(small.pos + 30.0)
             assert alone.form() is None
+
+
+def test_plain_rows_of_a_tiled_list(ctx):
+    # A fixed lane count on a tiled list walks plain rows in slot order, made for each build when first needed: the
+    # tiles' bits, for atoms in any order, after moves and rebuilds, with two handles on one list.
+    s = systems.fe_x_alloy(7, cells=30)
+    rng = np.random.default_rng(1)
+    mix = rng.permutation(s.n)
+    types, frozen = s.types[mix], (rng.random(s.n) < 0.2).astype(np.uint8)
+    path = systems.potential_path(("Fe", "X"))
+    tiles, rows, other = fa.EAM(ctx, path), fa.EAM(ctx, path), fa.EAM(ctx, path)
+    rows.set_lanes(8)
+    other.set_lanes(16)
+    nl = fa.List(ctx, fa.Box(s.basis), 5.9)
+    for build in range(3):
+        nl.rebuild(s.pos[mix] + rng.uniform(-0.05, 0.05, s.pos.shape))
+        assert nl.form() is not None
+        for step in range(2):
+            nl.update(rng.uniform(-0.03, 0.03, s.pos.shape))
+            for pot in (tiles, rows, other):
+                pot.set_precision(fa.MIXED if step else fa.FP64)
+            g, e = tiles.gradient(types, frozen, nl).copy(), tiles.energy(types, frozen, nl)
+            for pot in (rows, other):
+                assert np.array_equal(g, pot.gradient(types, frozen, nl))
+                assert e == pot.energy(types, frozen, nl)
