@@ -1104,9 +1104,13 @@ namespace flyg {
     // names a count: more lanes shorten each row's chain of dependent gathers, which is what bounds the sizes left to
     // these passes.  Density / force, us, FP64 at 16, 8 and 4 lanes: 8.2k atoms 6.6/8.1, 9.6/11.5, 13.4/17.8; 16k
     // 9.4/10.2, 8.5/13.4, 11.3/14.8.  Timing the three counts on a potential's first call cost 24 launches and
-    // could keep a slower one.
+    // could keep a slower one.  Eight lanes where 16 would take a second, nearly empty round of workgroups (2048 of
+    // 256 threads are resident, in the FP64 form with its registers fewer).  16 / 8 lanes, two species, list cut-offs
+    // 5.5 / 6.8 A: mixed 31k atoms 26.5/25.7 34.9/36.3, 35k 31.6/28.5 45.2/40.4, 44k 35.6/33.7 59.6/53.6, 54k equal;
+    // FP64 28k 33.0/33.2 40.9/44.6, 31k 37.9/33.1 50.8/45.6, 39k 44.2/40.1 65.8/58.8, 44k 47.9/48.7 74.9/69.9.
     void gradient_with(flyg_eam_s& E, Shifts const& S, PairArgs const& A, double* d_grad, int precision, double4* pf) {
-      int const L = E.lanes > 0 ? E.lanes : 16;
+      bool const eight = precision == FLYG_MIXED ? A.n > 32768 && A.n < 46000 : A.n >= 30000 && A.n < 41000;
+      int const L = E.lanes > 0 ? E.lanes : (eight ? 8 : 16);
       density_with(E, S, A, precision, L, pf);
       force_with(E, S, A, d_grad, precision, L, pf);
     }
@@ -1127,7 +1131,10 @@ namespace flyg {
       }
       HIPCHK(hipEventRecord(E.events[E.events_used].first, E.ctx->stream));
     }
-    if (nl.tiled && E.lanes <= 0) {
+    bool tiles = nl.tiled && E.lanes <= 0;
+    if (tiles && nl.grad_rows && nl.grad_build == nl.build_id) tiles = !slot_rows(E, nl);
+    nl.grad_build = nl.build_id;
+    if (tiles) {
       TileArgs A = tile_args(E, nl, types, frozen);
       tile_density(E, S, A, false, precision, E.posf.get());
       A.pos = E.posf.get();

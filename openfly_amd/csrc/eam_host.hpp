@@ -139,6 +139,8 @@ struct flyg_list_s {
   // The plain rows in slot order of a tiled list, K entries of room each, made when a build's first call needs them.
   flyg::DBuf<unsigned> srows;
   long srows_build = -1;
+  bool grad_rows = false;        // a tiled list whose gradients are faster by rows, from a build's second on
+  long grad_build = -1;          // the build of the last gradient
   flyg::DBuf<int> scan_tmp;
   flyg::DBuf<double> stage;      // host staging of xyz vectors
   flyg::DBuf<unsigned> lstate;   // device build counters: two sets of LIST_STATE words, used in turn

@@ -772,14 +772,20 @@ namespace flyg {
   }
 
   namespace {
-    // Tile shapes (cells), largest first.  A larger tile stages fewer entries per atom (8, 12, 18 of them) but
-    // there are fewer workgroups, each walking more rows: the largest shape that leaves TILE_LEAST tiles, a little
-    // over two for each of the 256 CUs, is taken.  Update + gradient, us, mixed form, one species, 2x2x2 / 1x2x2 / 1x1x2 /
-    // plain rows: 27.6k atoms (216 / 396 / 726 tiles) 86 / 67 / 53 / 53, 44k (343 / 637 / 1183) 96 / 75 / 78 / 81,
-    // 93k (729 / 1377 / 2601) 122 / 134 / 134 / 153, 1.03M 500 / 550 / 640 / 750; below, the plain rows are faster
-    // (16k: 40 us against 47).
+    // Tile shapes (cells), largest first.  A larger tile stages fewer entries per atom (8, 12, 18 of them) but there are
+    // fewer workgroups, each walking more rows.  Which is best depends on how the tiles fill the chip: three
+    // workgroups of 512 threads run on each of 256 CUs, so 1000 tiles take little less than 1500 would.  Gradient,
+    // us, one species, list cut-off 5.9 A, mixed / FP64, by 2x2x2 (tiles) / 1x2x2 / 1x1x2 / plain rows in slot order:
+    //   27.6k atoms  42.5/51.6 (216)   31.3/39.8 (396)   24.4/33.4 (726)   21.8/30.0
+    //   43.9k        48.7/64.2 (343)   36.2/49.6 (637)   39.2/53.0 (1183)  33.0/43.4
+    //   54.0k        47.6/63.1 (343)   36.9/50.4 (686)   40.5/54.5 (1372)  38.2/50.5
+    //   110k         64.0/93.4 (729)   69.9/97.6 (1458)  73.7/101 (2916)   81.7/111
+    //   128k         102/151 (1000)    81.8/119 (1900)   92.0/124 (3610)   92.8/128
+    //   686k         348/505 (4913)    346/501 (9537)    415/560 (18513)   581/815
     constexpr int TILE_SHAPES[TILE_KINDS][3] = {{2, 2, 2}, {1, 2, 2}, {1, 1, 2}};
-    constexpr int TILE_LEAST = 600;
+    constexpr long TILE_ATOMS = 27000;      // fewer: plain rows are faster or equal in the passes together
+    constexpr long TILE_LEAST = 600;        // a little over two for each CU
+    constexpr double TILE_SLOTS = 768.0;    // workgroups resident at once
 
     TileGrid tile_grid(GridDesc const& g, int level) {
       TileGrid t{};
@@ -795,22 +801,57 @@ namespace flyg {
       return t;
     }
 
-    // The tile shape for a build, or -1: plain rows.  seen: from what the build before counted, the tiles that hold atoms
-    // and the fullest one.  A first build takes the box to be filled evenly, and is done again if its own counts
-    // say otherwise (a particle in vacuum leaves most tiles empty and the chip idle: 16k atoms in eight times their volume took 74 us a
+    // What an atom costs in tiles of a shape, in the cost of full tiles of 2x2x2 that fill every round of workgroups:
+    // the shape's own factor, a stage so large that a CU holds fewer workgroups (40 KB for four of a gradient's
+    // and two of an HVP's), the last round's idle slots at half their time (its workgroups have more of a CU to
+    // themselves), and cells that the last tile of an axis lacks.
+    double tile_cost(TileGrid const& t, int level, double used, double staged) {
+      constexpr double factor[TILE_KINDS] = {1.0, 1.12, 1.3};
+      double const rounds = used / TILE_SLOTS;
+      double inner = 1, most = t.ntiles;
+      for (int k = 0; k < 3; ++k) {
+        inner *= t.shape[k] - 2;
+        most *= t.d[k];
+      }
+      return factor[level] * (staged > 1100 ? 1.1 : 1.0) * (0.5 + 0.5 * std::ceil(rounds) / rounds) * (most / inner);
+    }
+
+    // The tile shape for a build, or -1: plain rows.  The largest shape that leaves TILE_LEAST tiles, if no other is
+    // clearly cheaper.  seen: from what the build before counted, the tiles that hold atoms and the fullest one.
+    // A first build takes the box to be filled evenly, and is done again if its own counts say otherwise (a particle
+    // in vacuum leaves most tiles empty and the chip idle: 16k atoms in eight times their volume took 74 us a
     // gradient by tiles, 25 by rows).
-    int choose_tiles(flyg_list_s const& nl, long n, bool seen) {
+    int choose_tiles(flyg_list_s const& nl, long n, bool seen, double* cost = nullptr) {
+      if (n < TILE_ATOMS) return -1;
       GridDesc const& g = nl.grid;
       double const inner = static_cast<double>(g.shape[0] - 2) * (g.shape[1] - 2) * (g.shape[2] - 2);
+      int best = -1;
+      bool first = true;
+      double least = 2.0;   // dearer than plain rows
       for (int level = 0; level < TILE_KINDS; ++level) {
         TileGrid const t = tile_grid(g, level);
-        bool const full = seen ? nl.tile_full[level] > TILE_MOST
-                               : n / inner * (t.d[0] + 2) * (t.d[1] + 2) * (t.d[2] + 2) > 0.9 * TILE_MOST;
+        double const staged = n / inner * (t.d[0] + 2) * (t.d[1] + 2) * (t.d[2] + 2);
+        bool const full = staged > 0.9 * TILE_MOST || (seen && nl.tile_full[level] > TILE_MOST);
         long const used = seen ? static_cast<long>(nl.tile_used[level]) : t.ntiles;
-        if (full || used < TILE_LEAST) continue;
-        return n < 16 * used ? -1 : level;   // a gas: tiles of a few atoms
+        if (full || used == 0 || n < 16 * used) continue;   // (the last: a gas, tiles of a few atoms)
+        double const c = tile_cost(t, level, static_cast<double>(used), staged);
+        double const compared = first && used >= TILE_LEAST ? 0.93 * c : c;
+        if (used >= TILE_LEAST) first = false;
+        if (compared < least) {
+          least = compared;
+          best = level;
+          if (cost) *cost = c;
+        }
       }
-      return -1;
+      return best;
+    }
+
+    // Neighbours within the list's cut-off in a box filled evenly.
+    double mean_row(flyg_list_s const& nl, long n) {
+      double const vol = std::fabs(nl.box.B[0][0] * (nl.box.B[1][1] * nl.box.B[2][2] - nl.box.B[1][2] * nl.box.B[2][1]) -
+                                   nl.box.B[0][1] * (nl.box.B[1][0] * nl.box.B[2][2] - nl.box.B[1][2] * nl.box.B[2][0]) +
+                                   nl.box.B[0][2] * (nl.box.B[1][0] * nl.box.B[2][1] - nl.box.B[1][1] * nl.box.B[2][0]));
+      return static_cast<double>(n) / vol * 4.18879 * nl.rc * nl.rc * nl.rc;
     }
   }  // namespace
 
@@ -833,11 +874,7 @@ namespace flyg {
     if (nl.gcap == 0) nl.gcap = std::max(4096l, n);
     if (nl.K == 0) {
       // Room for the rows of a uniform system and a fifth more: a first guess of 64 built most lists twice.
-      double const vol = std::fabs(nl.box.B[0][0] * (nl.box.B[1][1] * nl.box.B[2][2] - nl.box.B[1][2] * nl.box.B[2][1]) -
-                                   nl.box.B[0][1] * (nl.box.B[1][0] * nl.box.B[2][2] - nl.box.B[1][2] * nl.box.B[2][0]) +
-                                   nl.box.B[0][2] * (nl.box.B[1][0] * nl.box.B[2][1] - nl.box.B[1][1] * nl.box.B[2][0]));
-      double const mean = static_cast<double>(n) / vol * 4.18879 * nl.rc * nl.rc * nl.rc;
-      nl.K = std::max(64, (static_cast<int>(std::min(1.2 * mean, 512.0)) + 15) / 16 * 16);
+      nl.K = std::max(64, (static_cast<int>(std::min(1.2 * mean_row(nl, n), 512.0)) + 15) / 16 * 16);
     }
     int const nc = nl.grid.ncells;
     long const nc1 = nc + 1;
@@ -873,11 +910,16 @@ namespace flyg {
       nl.sid.reserve(cap);
       nl.usid.reserve(cap);
       nl.nbr.reserve(static_cast<std::size_t>(n) * nl.K);
-      int const level = choose_tiles(nl, n, nl.tile_seen);
+      double cost = 0;
+      int const level = choose_tiles(nl, n, nl.tile_seen, &cost);
       nl.tiled = level >= 0;
+      // Where tiles fill the chip badly a gradient is up to 15 % faster by rows in slot order (which take a pass of
+      // their own); the other passes are not (HVP at 35k to 44k atoms by tiles: 0.63 to 0.9 of the time by rows).
+      // Longer rows favour the tiles (44k atoms, cut-off 6.8 A, mixed: 38.6 us by tiles at a cost of 1.6, 47 by rows).
+      nl.grad_rows = nl.tiled && n < 46000 && cost > (mean_row(nl, n) < 90.0 ? 1.3 : 1.62);
       // The shape in use is looked at in every build, the others (not those with more tiles than a quarter of the
       // atoms) only while an even filling and what was seen disagree: three shapes take 5 us more at 54k atoms.
-      bool const all = n >= 16l * TILE_LEAST && (!nl.tile_seen || attempt > 0 || level != choose_tiles(nl, n, false));
+      bool const all = n >= TILE_ATOMS && (!nl.tile_seen || attempt > 0 || level != choose_tiles(nl, n, false));
       for (int l = 0; l < TILE_KINDS; ++l) {
         bool const look = l == level || (all && n >= 4l * tk.g[l].ntiles);
         tk.first[l + 1] = tk.first[l] + (look ? nblk(4l * tk.g[l].ntiles, TPB) : 0);
@@ -908,10 +950,11 @@ namespace flyg {
                                                    tg, nl.sslot.get(), nl.gcap, nl.rows.get(), nl.rowK, nl.gcnt.get(),
                                                    nl.hstate);
       };
-      if (n < BUILD_WIDE) {
-        nl.tiled ? rows(k_build_rows<1, true>, 1) : rows(k_build_rows<1, false>, 1);
+      static_assert(TILE_ATOMS >= BUILD_WIDE, "a tiled list has enough atoms for four a wavefront");
+      if (nl.tiled) {
+        rows(k_build_rows<4, true>, 4);
       } else {
-        nl.tiled ? rows(k_build_rows<4, true>, 4) : rows(k_build_rows<4, false>, 4);
+        n < BUILD_WIDE ? rows(k_build_rows<1, false>, 1) : rows(k_build_rows<4, false>, 4);
       }
       HIPCHK(hipGetLastError());
       HIPCHK(hipStreamSynchronize(st));

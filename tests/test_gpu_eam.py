@@ -5,6 +5,7 @@ component); mixed precision (FP32 pair arithmetic, FP64 accumulation) within 2e-
 """
 import numpy as np
 import pytest
+import torch
 
 import openfly_amd as fa
 from openfly_amd import systems
@@ -437,17 +438,15 @@ def test_staged_atoms_follow_stage_calls_and_rebuilds(ctx, wen_orc):
         pot.gradient(None, None, nl)
 
 
-TILED = {   # cells: the tile shape a list with 0.6 A of skin takes
-    24: (1, 1, 2), 30: (1, 2, 2), 36: (2, 2, 2)}
-
-
-@pytest.mark.parametrize("cells,tilt,slab,single", [(24, 0.0, False, False), (24, 0.1, True, True), (30, 0.07, False, False),
-                                                    (30, 0.0, True, True), (36, 0.0, False, False)])
-def test_tiled_passes_equal_plain_rows(ctx, cells, tilt, slab, single):
+@pytest.mark.parametrize("cells,rc,tilt,slab,single,shape", [
+    (26, 6.8, 0.0, False, False, (1, 1, 2)), (26, 6.8, 0.1, True, True, None), (30, 5.9, 0.0, False, True, (1, 2, 2)),
+    (30, 5.9, 0.07, False, False, None), (30, 5.9, 0.0, True, True, (1, 2, 2)), (30, 5.47, 0.0, False, False, (2, 2, 2)),
+    (36, 5.9, 0.0, False, False, (2, 2, 2))])
+def test_tiled_passes_equal_plain_rows(ctx, cells, rc, tilt, slab, single, shape):
     # Lists of these sizes evaluate tile by tile; a handle with a fixed lane count walks the plain rows.  The
     # same entries in the same order: gradients and energies are equal bit for bit, in periodic, sheared and slab boxes
     # (edge tiles, image shifts), with frozen atoms, after moves, and with atoms on the box faces.
-    print(f"case tiles {TILED[cells]} tilt={tilt} slab={slab} single={single}", flush=True)
+    print(f"case {cells}^3 cells, cut-off {rc}, tiles {shape} tilt={tilt} slab={slab} single={single}", flush=True)
     s = systems.fe_x_alloy(cells, cells=cells)
     basis = s.basis.copy()
     pos = s.pos.copy()
@@ -460,10 +459,11 @@ def test_tiled_passes_equal_plain_rows(ctx, cells, tilt, slab, single):
     types = np.zeros_like(s.types) if single else s.types
     rng = np.random.default_rng(cells)
     frozen = (rng.random(s.n) < 0.2).astype(np.uint8)
-    nl = fa.List(ctx, fa.Box(basis, (1, 1, 0 if slab else 1)), 5.9)
+    nl = fa.List(ctx, fa.Box(basis, (1, 1, 0 if slab else 1)), rc)
     nl.rebuild(pos)
     nl.update(rng.uniform(-0.05, 0.05, pos.shape))
-    assert nl.form()[0] == TILED[cells]
+    form = nl.form()[0]
+    assert shape is None or form == shape
     pot = fa.EAM(ctx, systems.potential_path(("Fe", "X")))
     for precision in (fa.FP64, fa.MIXED):
         pot.set_precision(precision)
@@ -550,3 +550,28 @@ def test_plain_rows_of_a_tiled_list(ctx):
             for pot in (rows, other):
                 assert np.array_equal(g, pot.gradient(types, frozen, nl))
                 assert e == pot.energy(types, frozen, nl)
+
+
+@pytest.mark.parametrize("precision", [fa.FP64, fa.MIXED])
+@pytest.mark.parametrize("cells,rc,tiled", [(23, 5.9, False), (24, 5.9, True), (25, 5.47, True), (28, 5.9, True), (28, 5.47, True)])
+def test_gradients_where_forms_meet(ctx, cells, rc, tiled, precision):
+    # Sizes around the least that are tiled, where a build's first gradient goes by tiles and the later ones may go by
+    # rows in slot order, with 8 or 16 lanes: the bits of the call that needs no scratch and walks rows by atom.
+    s = systems.fe_x_alloy(cells, cells=cells)
+    rng = np.random.default_rng(3)
+    frozen = (rng.random(s.n) < 0.2).astype(np.uint8)
+    pot = fa.EAM(ctx, systems.potential_path(("Fe", "X")))
+    pot.set_precision(precision)
+    nl = fa.List(ctx, fa.Box(s.basis), rc)
+    t, f = (torch.from_numpy(a).cuda() for a in (s.types, frozen))
+    out = torch.zeros((s.n, 3), dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    for build in range(2):
+        nl.rebuild(s.pos + rng.uniform(-0.05, 0.05, s.pos.shape))
+        assert (nl.form() is not None) == tiled
+        for step in range(3):
+            g = pot.gradient(s.types, frozen, nl)
+            ctx.check(fa.lib().flyg_eam_gradient_noalloc(pot.h, nl.h, t.data_ptr(), f.data_ptr(), s.n, out.data_ptr()))
+            ctx.synchronize()
+            assert np.array_equal(g, out.cpu().numpy())
+            nl.update(rng.uniform(-0.03, 0.03, s.pos.shape))
