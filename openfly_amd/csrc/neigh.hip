@@ -433,6 +433,9 @@ namespace flyg {
     // tile's stage (the candidate's place in the tile's halo: the lines' entries one after the other), otherwise with
     // slots.  hst (pinned): the build counters, but [1] set when a row overflowed.
     constexpr long BUILD_WIDE = 24000;
+    // Atoms a cell below which eight lanes an atom are faster than four atoms a wavefront.  Rebuild, us, by the two:
+    // 26k atoms at 1, 4, 6, 8 atoms a cell 63.6/80.1, 59.1/68.5, 61.4/66.8, 66.0/65.1; 1M at 0.3 and 2 533/1095, 579/985.
+    constexpr double SPARSE = 6.0;
 
     template <int A, bool TILED>
     __global__ __launch_bounds__(TPB) void k_build_rows(GridDesc g, double4 const* __restrict__ spos,
@@ -609,6 +612,78 @@ namespace flyg {
         // atomic per atom on the one counter serialised the kernel (half of its time).
         if (c > K) {
           atomicMax(&st[1], static_cast<unsigned>(c));
+          hst[1] = 1u;
+        }
+      }
+    }
+
+    // The same for a dilute system, whose ranges hold a few candidates each: eight lanes an atom, so a wavefront walks the
+    // blocks of eight atoms at once instead of a mostly empty chunk of 64 after the other.  Lists of plain rows only.
+    constexpr int SPARSE_LANES = 8;
+    constexpr int SPARSE_UNROLL = 4;   // chunks of candidates loaded before the first is tested
+
+    __global__ __launch_bounds__(TPB) void k_build_rows_sparse(GridDesc g, double4 const* __restrict__ spos,
+                                                               unsigned const* __restrict__ sid,
+                                                               int const* __restrict__ cstart, int const* __restrict__ rslot,
+                                                               long n, unsigned* __restrict__ nbr, int* __restrict__ ncnt,
+                                                               int K, unsigned* __restrict__ st,
+                                                               int const* __restrict__ order, int const* __restrict__ rank_of,
+                                                               unsigned* __restrict__ rows, int* __restrict__ gcnt,
+                                                               unsigned* __restrict__ hst) {
+      if (blockIdx.x == 0 && threadIdx.x < LIST_STATE && threadIdx.x != 1) hst[threadIdx.x] = st[threadIdx.x];
+      constexpr int L = SPARSE_LANES, U = SPARSE_UNROLL;
+      long const gid = xcd_block(blockIdx.x, gridDim.x) * static_cast<long>(TPB) + threadIdx.x, slot = gid / L;
+      int const lane = static_cast<int>(gid % L), gbase = static_cast<int>(threadIdx.x & 63) - lane;
+      if (slot >= n) return;   // whole groups leave together
+      int const atom = order[slot], self = rslot[atom];
+      double4 const p = spos[self];
+      double const xi[3] = {p.x, p.y, p.z}, rc2 = g.rc * g.rc;
+      int c3[3];
+      cell_idx(g, xi, c3);
+      int cnt = 0;
+      unsigned* row = nbr + atom * static_cast<long>(K);
+      unsigned* srow = rows + slot * K;
+      int const x0 = max(c3[0] - 1, 0), x1 = min(c3[0] + 2, g.shape[0]);
+      for (int z = max(c3[2] - 1, 0); z < min(c3[2] + 2, g.shape[2]); ++z)
+        for (int y = max(c3[1] - 1, 0); y < min(c3[1] + 2, g.shape[1]); ++y) {
+          int const line = y * g.prod[1] + z * g.prod[2];
+          int const b = cstart[x0 * g.prod[0] + line], end = cstart[(x1 - 1) * g.prod[0] + line + 1];
+          for (int s0 = b; s0 < end; s0 += U * L) {
+            bool hit[U];
+            unsigned en[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+              int const s = s0 + u * L + lane;
+              hit[u] = false;
+              en[u] = 0;
+              if (s < end && s != self) {
+                double4 const q = spos[s];
+                en[u] = sid[s];
+                double const xn[3] = {q.x, q.y, q.z};
+                hit[u] = dist2(xi, xn) < rc2;
+              }
+            }
+            int rk[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) rk[u] = hit[u] ? rank_of[en[u] & NB_IDX_MASK] : 0;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+              unsigned long long const m = __ballot(hit[u]);
+              unsigned const gm = static_cast<unsigned>((m >> gbase) & ((1ull << L) - 1ull));
+              int const k = cnt + __popc(gm & ((1u << lane) - 1u));
+              if (hit[u] && k < K) {
+                row[k] = en[u];
+                srow[k] = (en[u] & ~NB_IDX_MASK) | static_cast<unsigned>(rk[u]);
+              }
+              cnt += __popc(gm);
+            }
+          }
+        }
+      if (lane == 0) {
+        ncnt[atom] = cnt;
+        gcnt[slot] = cnt;
+        if (cnt > K) {
+          atomicMax(&st[1], static_cast<unsigned>(cnt));
           hst[1] = 1u;
         }
       }
@@ -953,6 +1028,11 @@ namespace flyg {
       static_assert(TILE_ATOMS >= BUILD_WIDE, "a tiled list has enough atoms for four a wavefront");
       if (nl.tiled) {
         rows(k_build_rows<4, true>, 4);
+      } else if (n >= BUILD_WIDE &&
+                 n < SPARSE * (nl.grid.shape[0] - 2) * (nl.grid.shape[1] - 2) * (nl.grid.shape[2] - 2)) {
+        k_build_rows_sparse<<<nblk(n, TPB / SPARSE_LANES), TPB, 0, st>>>(
+            nl.grid, nl.spos.get(), nl.sid.get(), nl.cstart.get(), nl.rslot.get(), n, nl.nbr.get(), nl.ncnt.get(), nl.K, dst,
+            nl.order.get(), nl.rank.get(), nl.rows.get(), nl.gcnt.get(), nl.hstate);
       } else {
         n < BUILD_WIDE ? rows(k_build_rows<1, false>, 1) : rows(k_build_rows<4, false>, 4);
       }

@@ -85,6 +85,34 @@ def test_large_lists_equal_pair_sets(ctx, n, rc, tilt):
     assert np.array_equal(H.pair_set(go, gj, gs), H.pair_set(oo, oj, os_))
 
 
+@pytest.mark.parametrize("n,rc,tilt,clump", [(24001, 2.0, 0.0, 0), (26007, 2.3, 4.0, 0), (30001, 1.7, 0.0, 300), (24000, 8.0, 0.0, 2)])
+def test_dilute_lists_equal_pair_sets(ctx, n, rc, tilt, clump):
+    # Few atoms a cell (eight lanes walk an atom's cells): less than one, one to two, a clump whose rows overflow the first
+    # row table in a box otherwise empty, and pairs of atoms far from all others.  In order, too: rows are sequences.
+    rng = np.random.default_rng(n)
+    L = np.array([61.0, 55.0, 64.0]) if clump != 2 else np.array([410.0, 380.0, 400.0])
+    basis = np.diag(L)
+    basis[0, 1] = tilt
+    periodic = np.array([1, 1, 0], np.int32)
+    pos = rng.random((n, 3)) @ basis.T
+    if clump == 300:
+        pos[:clump] = 20.0 + rng.random((clump, 3)) * rc
+    elif clump == 2:
+        pos[1::2] = np.clip(pos[::2] + rng.normal(0.0, 1.0, (n // 2, 3)), 0.0, L - 1e-6)
+    nl = fa.List(ctx, fa.Box(basis, periodic), rc)
+    nl.rebuild(pos[::-1].copy())
+    nl.rebuild(pos)
+    assert nl.form() is None
+    _, (oo, oj, os_, _) = oracle_pairs(basis, periodic, pos, rc)
+    go, gj, gs, _ = nl.pairs()
+    assert np.array_equal(go, oo)
+    assert np.array_equal(H.pair_set(go, gj, gs), H.pair_set(oo, oj, os_))
+    first = (gj.copy(), gs.copy())
+    nl.rebuild(pos)
+    go, gj, gs, _ = nl.pairs()
+    assert np.array_equal(gj, first[0]) and np.array_equal(gs, first[1])
+
+
 def test_update_matches_brute_force(ctx):
     rng = np.random.default_rng(77)
     for _ in range(4):
