@@ -1108,9 +1108,14 @@ namespace flyg {
     // 256 threads are resident, in the FP64 form with its registers fewer).  16 / 8 lanes, two species, list cut-offs
     // 5.5 / 6.8 A: mixed 31k atoms 26.5/25.7 34.9/36.3, 35k 31.6/28.5 45.2/40.4, 44k 35.6/33.7 59.6/53.6, 54k equal;
     // FP64 28k 33.0/33.2 40.9/44.6, 31k 37.9/33.1 50.8/45.6, 39k 44.2/40.1 65.8/58.8, 44k 47.9/48.7 74.9/69.9.
-    void gradient_with(flyg_eam_s& E, Shifts const& S, PairArgs const& A, double* d_grad, int precision, double4* pf) {
-      bool const eight = precision == FLYG_MIXED ? A.n > 32768 && A.n < 46000 : A.n >= 30000 && A.n < 41000;
-      int const L = E.lanes > 0 ? E.lanes : (eight ? 8 : 16);
+    // Fewer also where a dilute system's rows would leave most of 16 idle, 16 / 8 / 4 lanes, mixed, 216k atoms with rows
+    // of 4, 8, 17, 34, 46: 43/28/25, 51/32/31, 79/50/49, 84/72/81, 91/95/99; 33k: 11/10/10, 12/11/10, 16/13/14,
+    // 17/16/22, 18/19/26; below 20k they are equal.
+    void gradient_with(flyg_eam_s& E, Shifts const& S, PairArgs const& A, double row, double* d_grad, int precision,
+                       double4* pf) {
+      bool const eight = (precision == FLYG_MIXED ? A.n > 32768 && A.n < 46000 : A.n >= 30000 && A.n < 41000) ||
+                         (A.n >= 20000 && row < 40.0);
+      int const L = E.lanes > 0 ? E.lanes : (A.n >= 20000 && row < 7.0 ? 4 : (eight ? 8 : 16));
       density_with(E, S, A, precision, L, pf);
       force_with(E, S, A, d_grad, precision, L, pf);
     }
@@ -1140,7 +1145,7 @@ namespace flyg {
       A.pos = E.posf.get();
       tile_force(E, S, A, d_grad, precision);
     } else {
-      gradient_with(E, S, slot_args(E, nl, types, frozen), d_grad, precision, E.posf.get());
+      gradient_with(E, S, slot_args(E, nl, types, frozen), nl.mean_row, d_grad, precision, E.posf.get());
     }
     if (E.timing) HIPCHK(hipEventRecord(E.events[E.events_used++].second, E.ctx->stream));
     HIPCHK(hipGetLastError());
@@ -1186,7 +1191,7 @@ namespace flyg {
     require(pf != nullptr, "no scratch address for this device (its context was not created)");
     Shifts S = shifts_of(nl.box);
     PairArgs A = pair_args(E, nl, d_types, d_frozen);
-    gradient_with(E, S, A, d_grad, precision, pf);
+    gradient_with(E, S, A, nl.mean_row, d_grad, precision, pf);
     HIPCHK(hipGetLastError());
   }
 
@@ -1214,14 +1219,23 @@ namespace flyg {
       return;
     }
     PairArgs A = pair_args(E, nl, types, frozen);
-    constexpr int L = 16;
-    unsigned g = grid_for(nl.n, L);
-    if (A.t0 < 0) {
-      k_hvp_density<L, true><<<g, NT, 0, st>>>(E.dtab.get(), S, A, d_v, E.dfp.get(), err);
-      k_hvp_force<L, true><<<g, NT, 0, st>>>(E.dtab.get(), S, A, d_v, E.dfp.get(), d_hv, err);
+    auto rows = [&](auto lanes) {
+      constexpr int L = decltype(lanes)::value;
+      unsigned const g = grid_for(nl.n, L);
+      if (A.t0 < 0) {
+        k_hvp_density<L, true><<<g, NT, 0, st>>>(E.dtab.get(), S, A, d_v, E.dfp.get(), err);
+        k_hvp_force<L, true><<<g, NT, 0, st>>>(E.dtab.get(), S, A, d_v, E.dfp.get(), d_hv, err);
+      } else {
+        k_hvp_density<L, false><<<g, NT, 0, st>>>(E.dtab.get(), S, A, d_v, E.dfp.get(), err);
+        k_hvp_force<L, false><<<g, NT, 0, st>>>(E.dtab.get(), S, A, d_v, E.dfp.get(), d_hv, err);
+      }
+    };
+    // Rows of a dilute system would leave most of 16 lanes idle: 216k atoms with rows of 8, 17, 25, us, 16 / 8 lanes:
+    // 73/53, 122/110, 132/136.
+    if (nl.mean_row < 22.0) {
+      rows(std::integral_constant<int, 8>{});
     } else {
-      k_hvp_density<L, false><<<g, NT, 0, st>>>(E.dtab.get(), S, A, d_v, E.dfp.get(), err);
-      k_hvp_force<L, false><<<g, NT, 0, st>>>(E.dtab.get(), S, A, d_v, E.dfp.get(), d_hv, err);
+      rows(std::integral_constant<int, 16>{});
     }
     HIPCHK(hipGetLastError());
   }

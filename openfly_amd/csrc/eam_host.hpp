@@ -133,6 +133,7 @@ struct flyg_list_s {
   bool tile_seen = false;
   int tile_shape[3] = {};        // the grid they belong to
   int rowK = 0;
+  double mean_row = 0;           // entries of a row, roughly
   flyg::DBuf<unsigned> sslot;
   flyg::DBuf<unsigned> rows;
   flyg::DBuf<int> gcnt;          // entries per slot

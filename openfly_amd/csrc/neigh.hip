@@ -169,7 +169,7 @@ namespace flyg {
 
     // ---- single-sync rebuild path ----------------------------------------------------------------
     // lstate[0] ghosts generated, [1] longest row, [3] overflow bits, [4 + l] entries of the fullest tile of shape l,
-    // [8 + l] tiles of shape l that hold atoms.
+    // [8 + l] tiles of shape l that hold atoms, [12] atoms sampled, [13] others that share their cells.
     enum : unsigned { OV_GHOST = 1u };
 
     // The tile shapes a build could take; workgroups [first[l], first[l + 1]) of k_rank_place look at shape l, those
@@ -354,7 +354,7 @@ namespace flyg {
                                  int const* __restrict__ cstart, long nc1, unsigned const* __restrict__ usid,
                                  double4* __restrict__ spos, unsigned* __restrict__ sid, int* __restrict__ rslot,
                                  int* __restrict__ order, int* __restrict__ rank_of, double4* __restrict__ gpos,
-                                 TileKinds tk, unsigned* __restrict__ seen) {
+                                 TileKinds tk, unsigned* __restrict__ seen, unsigned* __restrict__ sample) {
       if (blockIdx.x < tk.first[TILE_KINDS]) {   // four lanes a tile: the entries it stages, and whether it holds atoms
         int l = 0;
         while (blockIdx.x >= tk.first[l + 1]) ++l;
@@ -398,6 +398,15 @@ namespace flyg {
       int c = ecell[e];
       unsigned id = eid[e];
       int b = cstart[c], end = cstart[c + 1];
+      unsigned const block = blockIdx.x - tk.first[TILE_KINDS];
+      if (block % 64 == 0 && (block + 1) * static_cast<long>(blockDim.x) <= n) {   // a sample of the atoms' surroundings
+        int others = end - b - 1;
+        for (int o = 32; o > 0; o >>= 1) others += __shfl_xor(others, o, 64);
+        if ((threadIdx.x & 63) == 0) {
+          atomicAdd(&sample[0], 64u);
+          atomicAdd(&sample[1], static_cast<unsigned>(others));
+        }
+      }
       int rank = 0, reals_before = 0;
       for (int q = b; q < end; ++q) {
         unsigned const u = usid[q];
@@ -860,6 +869,9 @@ namespace flyg {
     constexpr int TILE_SHAPES[TILE_KINDS][3] = {{2, 2, 2}, {1, 2, 2}, {1, 1, 2}};
     constexpr long TILE_ATOMS = 27000;      // fewer: plain rows are faster or equal in the passes together
     constexpr long TILE_LEAST = 600;        // a little over two for each CU
+    // Atoms a cell below which a tile's rows are too few and too short.  512k atoms at 4, 6, 8, 11 a cell (metals have 13
+    // and more), mixed gradient, us, by tiles / by rows: 217/103, 180/133, 172/181, 188/216.
+    constexpr long TILE_CELL = 8;
     constexpr double TILE_SLOTS = 768.0;    // workgroups resident at once
 
     TileGrid tile_grid(GridDesc const& g, int level) {
@@ -908,7 +920,7 @@ namespace flyg {
         double const staged = n / inner * (t.d[0] + 2) * (t.d[1] + 2) * (t.d[2] + 2);
         bool const full = staged > 0.9 * TILE_MOST || (seen && nl.tile_full[level] > TILE_MOST);
         long const used = seen ? static_cast<long>(nl.tile_used[level]) : t.ntiles;
-        if (full || used == 0 || n < 16 * used) continue;   // (the last: a gas, tiles of a few atoms)
+        if (full || used == 0 || n < TILE_CELL * t.d[0] * t.d[1] * t.d[2] * used) continue;
         double const c = tile_cost(t, level, static_cast<double>(used), staged);
         double const compared = first && used >= TILE_LEAST ? 0.93 * c : c;
         if (used >= TILE_LEAST) first = false;
@@ -988,10 +1000,6 @@ namespace flyg {
       double cost = 0;
       int const level = choose_tiles(nl, n, nl.tile_seen, &cost);
       nl.tiled = level >= 0;
-      // Where tiles fill the chip badly a gradient is up to 15 % faster by rows in slot order (which take a pass of
-      // their own); the other passes are not (HVP at 35k to 44k atoms by tiles: 0.63 to 0.9 of the time by rows).
-      // Longer rows favour the tiles (44k atoms, cut-off 6.8 A, mixed: 38.6 us by tiles at a cost of 1.6, 47 by rows).
-      nl.grad_rows = nl.tiled && n < 46000 && cost > (mean_row(nl, n) < 90.0 ? 1.3 : 1.62);
       // The shape in use is looked at in every build, the others (not those with more tiles than a quarter of the
       // atoms) only while an even filling and what was seen disagree: three shapes take 5 us more at 54k atoms.
       bool const all = n >= TILE_ATOMS && (!nl.tile_seen || attempt > 0 || level != choose_tiles(nl, n, false));
@@ -1018,7 +1026,8 @@ namespace flyg {
                                                     nl.cstart.get(), nl.usid.get());
       k_rank_place<<<tk.first[TILE_KINDS] + nblk(cap, TPB), TPB, 0, st>>>(
           nl.ent.get(), nl.eid.get(), nl.ecell.get(), n, nl.gcap, dst, nl.cstart.get(), nc1, nl.usid.get(), nl.spos.get(),
-          nl.sid.get(), nl.rslot.get(), nl.order.get(), nl.rank.get(), nl.gpos.get(), tk, dst + 4);
+          nl.sid.get(), nl.rslot.get(), nl.order.get(), nl.rank.get(), nl.gpos.get(), tk, dst + 4,
+          dst + 12);
       auto rows = [&](auto k, int A) {
         k<<<nblk(n, A * (TPB / 64)), TPB, 0, st>>>(nl.grid, nl.spos.get(), nl.sid.get(), nl.cstart.get(), nl.rslot.get(), n,
                                                    nl.nbr.get(), nl.ncnt.get(), nl.K, dst, nl.order.get(), nl.rank.get(),
@@ -1060,6 +1069,13 @@ namespace flyg {
       // A tile too full for its stage, or a first build that took the wrong form: again, with what was seen.
       if (nl.tiled && nl.tile_full[level] > TILE_MOST) continue;
       if (first && choose_tiles(nl, n, true) != level) continue;
+      // The mean row, from the sample: a box is not always filled evenly.
+      double const cell = nl.grid.cell[0] * nl.grid.cell[1] * nl.grid.cell[2];
+      nl.mean_row = nl.hstate[12] > 0 ? 4.18879 * nl.rc * nl.rc * nl.rc / cell * nl.hstate[13] / nl.hstate[12] : mean_row(nl, n);
+      // Where tiles fill the chip badly a gradient is up to 15 % faster by rows in slot order (which take a pass of
+      // their own); the other passes are not (HVP at 35k to 44k atoms by tiles: 0.63 to 0.9 of the time by rows).
+      // Longer rows favour the tiles (44k atoms, cut-off 6.8 A, mixed: 38.6 us by tiles at a cost of 1.6, 47 by rows).
+      nl.grad_rows = nl.tiled && n < 46000 && cost > (nl.mean_row < 90.0 ? 1.3 : 1.62);
       nl.tile = tg;
       nl.tile_most = nl.tiled ? static_cast<int>(nl.tile_full[level]) : 0;
       static std::atomic<long> builds{0};
