@@ -8,7 +8,9 @@
 //       K = k'' u u^T + (m / r) (I - u u^T),  m = V' + F'_g phi'_{a->g} + F'_a phi'_{g->a}, k'' the same of second derivatives,
 //     + sum over atoms b, frozen ones included, of F''_b (grad rho_b)(grad rho_b)^T.
 // D holds dF'_b by moved coordinate for every atom b next to a mobile one; a row of H is then the pair
-// blocks plus a short sum of rows of D (one per neighbour), so both kernels stream whole rows.  Assembly from
+// blocks plus a short sum of rows of D (one per neighbour), so both kernels stream whole rows.  Mobile atoms scattered
+// through a large system have up to 66 times as many neighbours: D is made for a panel of columns at a time, of at
+// most HESS_PANEL, instead of 20 times H.  Assembly from
 // the columns' Hessian-vector products took five launches and two passes over the whole system for
 // each of the 3M coordinates: 11 ms at 120 mobile atoms in a 2000-atom cell, now 60 us.
 //
@@ -16,8 +18,9 @@
 // one launch a column that applies the previous reflection and multiplies by the next one in the same
 // pass over the block; then each eigenvalue by multisection on Sturm counts (Givens' bisection), a
 // wavefront per eigenvalue testing 64 points of its interval at once.  Both are
-// backward stable: errors of a few units of 1e-16 of the largest eigenvalue.  Bound by one launch per column
-// up to some 1000 coordinates, then by the memory traffic of the shrinking block.  Cyclic Jacobi rotations
+// backward stable: errors of a few units of 1e-16 of the largest eigenvalue.  Bound by one launch per column, 5 us, up
+// to some 550 coordinates; above, a column also waits for the shrinking block and its vectors from the caches (8 us
+// at 780 coordinates, 11 at 1200).  Cyclic Jacobi rotations
 // needed ten sweeps of 3M rounds of two launches: 36 ms at 360 coordinates.
 #include <algorithm>
 #include <cmath>
@@ -31,6 +34,7 @@ namespace flyg {
 
     constexpr int NTB = 256;
     constexpr std::size_t HESS_KEEP = 64u << 20;   // largest workspace kept in the potential handle between calls
+    constexpr std::size_t HESS_PANEL = 256u << 20;   // largest panel of D
 
     constexpr int EC = 256;   // neighbour entries staged at a time
 
@@ -109,11 +113,11 @@ namespace flyg {
       return p;
     }
 
-    // Row b of D: F''_b d rho_b / d (coordinate) for the 3 nm mobile coordinates.  One workgroup per region atom:
+    // Row b of D: F''_b d rho_b / d (coordinate) for mobile coordinates c0 .. c0 + w - 1.  One workgroup per region atom:
     // its entries are staged in LDS, then every thread sums those that touch its columns, in row order.
     __global__ __launch_bounds__(NTB) void k_drow(EAMTables T, Shifts S, PairArgs A, double2 const* __restrict__ ff,
-                                                  int const* __restrict__ region, int const* __restrict__ mob, long n3m,
-                                                  double* __restrict__ D, unsigned* __restrict__ err) {
+                                                  int const* __restrict__ region, int const* __restrict__ mob, long c0,
+                                                  long w, double* __restrict__ D, unsigned* __restrict__ err) {
       __shared__ double s_g[3][EC];
       __shared__ int s_m[EC];
       long const b = region[blockIdx.x];
@@ -123,7 +127,7 @@ namespace flyg {
       int const mb = mob[b];
       double const fpp = ff[b].y;
       int const c = min(A.cnt[b], A.K);
-      double* row = D + blockIdx.x * n3m;
+      double* row = D + blockIdx.x * w;
       for (int k0 = 0; k0 == 0 || k0 < c; k0 += EC) {
         int const nk = min(EC, c - k0);
         __syncthreads();
@@ -136,26 +140,26 @@ namespace flyg {
           s_m[k] = p.in ? mob[p.j] : -2;
         }
         __syncthreads();
-        for (long col = threadIdx.x; col < n3m; col += NTB) {
-          int const m = static_cast<int>(col / 3), d = static_cast<int>(col % 3);
-          double v = k0 ? row[col] : 0.0;
+        for (long q = threadIdx.x; q < w; q += NTB) {
+          int const m = static_cast<int>((c0 + q) / 3), d = static_cast<int>((c0 + q) % 3);
+          double v = k0 ? row[q] : 0.0;
           if (m == mb) {
             for (int k = 0; k < nk; ++k) v += (s_m[k] == m ? s_g[d][k] : 0.0) - s_g[d][k];
           } else {
             for (int k = 0; k < nk; ++k)
               if (s_m[k] == m) v += s_g[d][k];
           }
-          row[col] = v;
+          row[q] = v;
         }
       }
       if (e) atomicOr(err, e);
     }
 
-    // Rows 3g .. 3g + 2 of the mass-weighted block.  One workgroup per mobile atom g.
+    // Columns c0 .. c0 + w - 1 of rows 3g .. 3g + 2 of the mass-weighted block.  One workgroup per mobile atom g.
     __global__ __launch_bounds__(NTB) void k_hrow(EAMTables T, Shifts S, PairArgs A, double2 const* __restrict__ ff,
                                                   int const* __restrict__ atoms, int const* __restrict__ mob,
                                                   int const* __restrict__ loc, double const* __restrict__ rmass, long n3m,
-                                                  double const* __restrict__ D, double* __restrict__ H,
+                                                  long c0, long w, double const* __restrict__ D, double* __restrict__ H,
                                                   unsigned* __restrict__ err) {
       __shared__ double s_u[3][EC], s_g[EC], s_a[EC], s_k[EC], s_t[EC];   // u, phi'_{a->g}, phi'_{g->a}, k'' - m / r, m / r
       __shared__ int s_m[EC], s_l[EC];
@@ -166,7 +170,7 @@ namespace flyg {
       int const tg = A.t0 < 0 ? checked_type(A.types[g], T.ntypes, e) : A.t0;
       double const fg = ff[g].x;
       int const c = min(A.cnt[g], A.K);
-      double const* Dg = D + static_cast<long>(loc[g]) * n3m;
+      double const* Dg = D + static_cast<long>(loc[g]) * w;
       double* h0 = H + 3l * mg * n3m;
       for (int k0 = 0; k0 == 0 || k0 < c; k0 += EC) {
         int const nk = min(EC, c - k0);
@@ -196,20 +200,21 @@ namespace flyg {
           s_l[k] = p.in ? loc[p.j] : loc[g];
         }
         __syncthreads();
-        for (long col = threadIdx.x; col < n3m; col += NTB) {
+        for (long at = threadIdx.x; at < w; at += NTB) {
+          long const col = c0 + at;
           int const m = static_cast<int>(col / 3), d = static_cast<int>(col % 3);
-          double const dg = Dg[col], rc = rmass[col];
+          double const dg = Dg[at], rc = rmass[col];
           double h[3] = {0, 0, 0};
 #pragma unroll 4
           for (int k = 0; k < nk; ++k) {
-            double const q = s_g[k] * dg + s_a[k] * D[s_l[k] * n3m + col];
+            double const q = s_g[k] * dg + s_a[k] * D[s_l[k] * w + at];
 #pragma unroll
             for (int r = 0; r < 3; ++r) h[r] -= s_u[r][k] * q;
-            double const w = (m == mg ? 1.0 : 0.0) - (m == s_m[k] ? 1.0 : 0.0);
-            if (w != 0.0) {
+            double const on = (m == mg ? 1.0 : 0.0) - (m == s_m[k] ? 1.0 : 0.0);
+            if (on != 0.0) {
               double const ud = s_u[d][k] * s_k[k];
 #pragma unroll
-              for (int r = 0; r < 3; ++r) h[r] += w * (s_u[r][k] * ud + (r == d ? s_t[k] : 0.0));
+              for (int r = 0; r < 3; ++r) h[r] += on * (s_u[r][k] * ud + (r == d ? s_t[k] : 0.0));
             }
           }
 #pragma unroll
@@ -590,8 +595,9 @@ namespace flyg {
     HIPCHK(hipStreamSynchronize(st));
     long const nreg = static_cast<long>(ctx.hflags[2]);
 
-    // One workspace: H, D, (F', F'') by atom, 1 / sqrt(m), and eight vectors of the reduction.
-    std::size_t const need = static_cast<std::size_t>(n3m) * (n3m + nreg + 9) + 2 * n + 16;
+    // One workspace: H, a panel of D, (F', F'') by atom, 1 / sqrt(m), and eight vectors of the reduction.
+    long const panel = std::min(n3m, std::max<long>(1, HESS_PANEL / sizeof(double) / nreg));
+    std::size_t const need = static_cast<std::size_t>(n3m) * (n3m + 9) + static_cast<std::size_t>(panel) * nreg + 2 * n + 16;
     DBuf<double> own;
     bool const keep = need * sizeof(double) <= HESS_KEEP;
     DBuf<double>& work = keep ? E.hess : own;
@@ -599,7 +605,7 @@ namespace flyg {
     double2* ff = reinterpret_cast<double2*>(work.get());
     double* H = work.get() + 2 * n;
     double* D = H + n3m * n3m;
-    double* rm = D + nreg * n3m;
+    double* rm = D + nreg * panel;
     double* v[2] = {rm + n3m, rm + 2 * n3m};
     double* p[2] = {rm + 3 * n3m, rm + 4 * n3m};
     double* diag = rm + 5 * n3m;
@@ -610,8 +616,11 @@ namespace flyg {
     double* lim = rm + 9 * n3m + 2;
     HIPCHK(hipMemcpyAsync(rm, rmass.data(), n3m * sizeof(double), hipMemcpyHostToDevice, st));
     k_embed<8><<<blocks(n * 8, NTB), NTB, 0, st>>>(E.tab, S, A, ff, err);
-    k_drow<<<static_cast<unsigned>(nreg), NTB, 0, st>>>(E.tab, S, A, ff, region, mob, n3m, D, err);
-    k_hrow<<<static_cast<unsigned>(nm), NTB, 0, st>>>(E.tab, S, A, ff, atoms, mob, loc, rm, n3m, D, H, err);
+    for (long c0 = 0; c0 < n3m; c0 += panel) {
+      long const w = std::min(panel, n3m - c0);
+      k_drow<<<static_cast<unsigned>(nreg), NTB, 0, st>>>(E.tab, S, A, ff, region, mob, c0, w, D, err);
+      k_hrow<<<static_cast<unsigned>(nm), NTB, 0, st>>>(E.tab, S, A, ff, atoms, mob, loc, rm, n3m, c0, w, D, H, err);
+    }
     k_mirror_lower<<<blocks(n3m * n3m, NTB), NTB, 0, st>>>(H, n3m);
     for (long k = 0; k + 2 < n3m; ++k) {
       long const rows = n3m - k - 1;

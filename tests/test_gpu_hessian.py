@@ -5,6 +5,7 @@ and weighted by the oracle's masses: eigenvalues within 1e-9 of the largest in m
 saddle the spectrum has exactly one negative mode and the three translation zero modes (find.cpp:849-866)."""
 import numpy as np
 import pytest
+import torch
 
 import openfly_amd as fa
 from openfly_amd import systems
@@ -89,6 +90,71 @@ def test_spectrum_of_few_atoms(ctx, wen, species, mobile):
     wo = oracle_block(data, basis, pos, t, f)
     assert len(w) == 3 * mobile and np.all(np.diff(w) >= 0)
     assert np.max(np.abs(w - wo)) <= 1e-12 * np.abs(wo).max()
+
+
+def block_of_products(pot, data, t, f, nl):
+    # eigvalsh of the block whose columns are Hessian-vector products (FP64, another route through the tables).
+    n, dof = len(t), np.nonzero(np.repeat(f == 0, 3))[0]
+    td, fd = torch.from_numpy(t).cuda(), torch.from_numpy(f).cuda()
+    v = torch.zeros(3 * n, dtype=torch.float64, device="cuda")
+    hv = torch.zeros((n, 3), dtype=torch.float64, device="cuda")
+    rows = torch.from_numpy(dof).cuda()
+    cols = []
+    for c in dof:
+        v[c] = 1.0
+        torch.cuda.synchronize()
+        pot.hvp(td, fd, nl, v.view(n, 3), out=hv)
+        pot.ctx.synchronize()
+        cols.append(hv.view(-1)[rows].clone())
+        v[c] = 0.0
+    m = np.repeat(data.masses[t], 3)[dof]
+    B = torch.stack(cols, 1).cpu().numpy() / np.sqrt(np.outer(m, m))
+    return np.linalg.eigvalsh(0.5 * (B + B.T))
+
+
+@pytest.mark.parametrize("scattered", [True, False])
+def test_spectrum_of_large_blocks(ctx, wen, scattered):
+    # 500 mobile atoms scattered through 54k (the derivatives of F' are made in several panels), and 1030 together (3090
+    # coordinates: more than the Sturm counts keep in LDS, and a workspace too large to be kept).
+    # Bound: 60 terms an element, and the reduction is backward stable: n x 1e-16 of the largest eigenvalue.
+    rng = np.random.default_rng(8)
+    if scattered:
+        path = systems.potential_path(("Fe", "X"))
+        pot, data = fa.EAM(ctx, path), po.DataEAM(path)
+        s = systems.fe_x_alloy(3, cells=30)
+        pos, basis, t, mobile = s.pos, s.basis, s.types, rng.choice(s.n, 500, replace=False)
+    else:
+        pot, data = wen
+        pos, basis = vacancy_cell(9)
+        t, mobile = np.zeros(len(pos), np.uint32), np.arange(1030)
+    pos = pos + rng.normal(0, 0.03, pos.shape)
+    f = np.ones(len(pos), np.uint8)
+    f[mobile] = 0
+    nl = fa.List(ctx, fa.Box(basis), pot.r_cut() + 0.1)
+    nl.rebuild(pos)
+    w = pot.hessian_eigenvalues(t, f, nl)
+    wo = block_of_products(pot, data, t, f, nl)
+    assert len(w) == 3 * len(mobile) and np.all(np.diff(w) >= 0)
+    assert np.max(np.abs(w - wo)) <= 1e-12 * np.abs(wo).max()
+    assert np.array_equal(w, pot.hessian_eigenvalues(t, f, nl))
+
+
+def test_spectrum_on_long_rows(ctx, wen):
+    # Rows of 305 entries are staged in two pieces, the second added to rows already written; most entries lie beyond the
+    # potential's cut-off, so the spectrum is that on the short list.  Bound as above.
+    pot, data = wen
+    pos, basis = vacancy_cell(10)
+    rng = np.random.default_rng(2)
+    pos = pos + rng.normal(0, 0.04, pos.shape)
+    t, f = np.zeros(len(pos), np.uint32), np.ones(len(pos), np.uint8)
+    f[rng.choice(len(pos), 41, replace=False)] = 0
+    w = []
+    for rc in (pot.r_cut(), 9.5):
+        nl = fa.List(ctx, fa.Box(basis), rc)
+        nl.rebuild(pos)
+        w.append(pot.hessian_eigenvalues(t, f, nl))
+    assert np.diff(nl.pairs()[0]).max() > 256
+    assert np.max(np.abs(w[0] - w[1])) <= 1e-12 * np.abs(w[0]).max()
 
 
 def test_saddle_spectrum_and_prefactor(ctx, wen):
