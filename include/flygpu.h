@@ -99,8 +99,9 @@ int flyg_eam_info(flyg_eam eam, int* ntypes, double* r_cut, double* masses, char
 /* FLYG_FP64 (default) or FLYG_MIXED for gradient / HVP pair arithmetic.  Energies are always FP64. */
 int flyg_eam_set_precision(flyg_eam eam, int precision);
 /* Lanes of a wavefront that share one atom's neighbour row: 4, 8 or 16, which also selects the row-by-row
- * gradient and energy kernels, or 0 (default) for the library's choice of kernel by size.  Results are bitwise
- * identical for every choice. */
+ * kernels (gradients, energies and Hessian-vector products; the latter two keep their own lane counts), or 0
+ * (default) for the library's choice of kernel and lanes by size.  Gradients and energies are bitwise identical for
+ * every choice. */
 int flyg_eam_set_lanes(flyg_eam eam, int lanes);
 /* Kernel timing of gradient calls (no reference counterpart; for benchmarks): while on, each gradient
  * call records a HIP event pair on the context's stream around its density + force kernels.
@@ -158,8 +159,10 @@ int flyg_eam_energy(flyg_eam eam, flyg_list nl, const uint32_t* types, const uin
 int flyg_eam_gradient(flyg_eam eam, flyg_list nl, const uint32_t* types, const uint8_t* frozen, int64_t n, int where,
                       double* grad);
 /* No counterpart in the reference: EAM::gradient for callers that cannot allocate device memory (code under
- * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).  Same kernels and results as
- * flyg_eam_gradient with FLYG_DEVICE pointers (types, frozen, grad on the context's device), but the
+ * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).  The results of
+ * flyg_eam_gradient with FLYG_DEVICE pointers (types, frozen, grad on the context's device), bit for bit, by
+ * the row kernels on the rows by atom: from about 50,000 atoms, and wherever the atoms are in no spatial order, that is
+ * slower than flyg_eam_gradient, whose layout in cell order needs a species gather.  The
  * density pass's output goes to a library-held device array of at most 131072 atoms (32 B per atom, one
  * copy per GPU, held until the process ends) instead of a per-handle buffer.  Larger systems are refused
  * (FLYG_INVALID_ARG).  Calls that overlap on one GPU share that array and race.  Asynchronous on the

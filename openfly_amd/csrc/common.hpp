@@ -340,7 +340,9 @@ namespace flyg {
       e = (halo ? halo_hi(0, tx) : hi(0, tx)) * prod[0] + l;
     }
   };
-  constexpr int TILE_MOST = 1900;   // entries a tile may stage: with species and tables below 64 KB
+  // Entries a tile may stage: 33 bytes each in a gradient, 64 KB with the tables (two workgroups a CU), 65 in an HVP's
+  // force pass, 125 KB (one; above 1200 entries already).
+  constexpr int TILE_MOST = 1900;
   constexpr int TILE_KINDS = 3;     // tile shapes to choose from
 
   // ----------------------------------------------------------------------------------------------

@@ -1195,6 +1195,10 @@ namespace flyg {
     HIPCHK(hipGetLastError());
   }
 
+  // The largest stage of any pass fits the 160 KB of LDS a workgroup of gfx950 can have.
+  static_assert((TILE_MOST + 15) / 16 * 16 * 65 + sizeof(TileLds) + 2 * MAX_TYPES * MAX_TYPES * sizeof(SplineDesc) <= 160 * 1024,
+                "an HVP's stage does not fit in LDS");
+
   void eam_hvp(flyg_eam_s& E, flyg_list_s& nl, uint32_t const* types, uint8_t const* frozen, double const* d_v,
                double* d_hv) {
     require(nl.built, "List used before rebuild");
