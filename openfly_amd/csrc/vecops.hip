@@ -236,8 +236,9 @@ namespace flyg {
     }
 
     // ---- The two-loop in one launch ------------------------------------------------------------------
-    // Its 2 m sums are a chain, each needed by every element before the next.  As launches a link costs 4 us at
-    // 48k elements (an empty launch 2.35); here it is a store and a poll through the device's memory, under 2.  A
+    // Its 2 m sums are a chain, each needed by every element before the next.  As launches a link costs 3.6 us at
+    // 65k elements (an empty launch 2.35); here it is a store and a poll through the device's memory, 1.1 us at 3k
+    // elements, 2.8 at 30k and 3.5 at 65k, where the two meet (NEWTON_BLOCKS).  A
     // thread keeps its (at most four) elements of q and r in registers from the first stage to the last, so no
     // vector data crosses workgroups, only partial sums do: a workgroup writes its sum to a slot of its own, and one
     // wavefront of every workgroup reads all of them until none is empty.  An empty slot holds a
