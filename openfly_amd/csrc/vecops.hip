@@ -292,6 +292,7 @@ namespace flyg {
               L.dead = 1;
               break;
             }
+            __builtin_amdgcn_s_sleep(1);   // 64 clocks, as the clock that was read here before took
           }
           L.sh[k][lane] = __longlong_as_double(static_cast<long long>(v));
         }
