@@ -70,6 +70,21 @@ def test_steplbfgs_sizes(ctx, N):
         x = x - 0.5 * qo
 
 
+def test_steplbfgs_longest_history(ctx):
+    # The longest history (32 pairs), filled and wrapped round, in the one-launch form.
+    # Bound: a step is a chain of 64 sums of N terms, each rounded up to N times in another order.
+    N, m = 9000, 32
+    rng = np.random.default_rng(32)
+    d = rng.uniform(1.0, 3.0, N)
+    g_s, o_s = fa.StepLBFGS(ctx, m), po.StepLBFGS(m)
+    x = rng.normal(size=N)
+    for it in range(m + 6):
+        g = d * x + 0.1 * np.sin(x)
+        qg, qo = g_s.newton_step(x, g), o_s.newton_step(x, g)
+        assert np.max(np.abs(qg - qo)) <= 2 * m * N * 2.2e-16 * np.max(np.abs(qo)), it
+        x = x - 0.1 * qo
+
+
 @pytest.fixture(params=[0, 1, 4])
 def impatient(request):
     # Steps of the one-launch form give up before the first look, or after so many: some of them, any of them.
