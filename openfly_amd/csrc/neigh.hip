@@ -890,7 +890,7 @@ namespace flyg {
 
     // What an atom costs in tiles of a shape, in the cost of full tiles of 2x2x2 that fill every round of workgroups:
     // the shape's own factor, a stage so large that a CU holds fewer workgroups (40 KB for four of a gradient's
-    // and two of an HVP's), the last round's idle slots at half their time (its workgroups have more of a CU to
+    // and two of an HVP's, 54 KB for three), the last round's idle slots at half their time (its workgroups have more of a CU to
     // themselves), and cells that the last tile of an axis lacks.
     double tile_cost(TileGrid const& t, int level, double used, double staged) {
       constexpr double factor[TILE_KINDS] = {1.0, 1.12, 1.3};
@@ -900,7 +900,8 @@ namespace flyg {
         inner *= t.shape[k] - 2;
         most *= t.d[k];
       }
-      return factor[level] * (staged > 1100 ? 1.1 : 1.0) * (0.5 + 0.5 * std::ceil(rounds) / rounds) * (most / inner);
+      double const large = staged > 1530 ? 1.5 : (staged > 1100 ? 1.1 : 1.0);
+      return factor[level] * large * (0.5 + 0.5 * std::ceil(rounds) / rounds) * (most / inner);
     }
 
     // The tile shape for a build, or -1: plain rows.  The largest shape that leaves TILE_LEAST tiles, if no other is
